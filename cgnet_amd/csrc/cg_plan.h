@@ -4,6 +4,7 @@
 #pragma once
 #include <vector>
 
+#include "cg_pair.h"
 #include "common.h"
 
 namespace cgnet {
@@ -90,6 +91,7 @@ struct cgnet_cg_plan {
     size_t fwd_lds = 0, bwd_lds = 0;
     bool fwd_mm = false;                         // the forward runs cg_forward_mm_kernel (product on the matrix cores)
     bool bwd_general_ok = true;                  // cg_backward_kernel's LDS need fits (else only the unit kernels serve)
+    cgnet::FwdPairSet pairs;                     // the forward's other form: units of cg_forward_pair_kernel (empty: never used)
     std::vector<int> fwd_class_begin;            // forward tasks by LDS class: class k = tasks [begin[k], begin[k+1])
     std::vector<size_t> fwd_class_lds;           // LDS bytes of a work-group of class k
     int bwd_threads = 256;                       // work-group size of the backward kernel

@@ -10,6 +10,8 @@
 // terms), the tile is written to LDS in output order and streamed out with contiguous stores.
 // Optionally the per-channel sums of |z| and |z|^2 are taken from the staged tile.
 //
+// The forward of many shapes with few channels runs in another form, organised by pairs (l1, l2): cg_pair.hip.
+//
 // Backward: one work-group per (sample, group of tasks).  The gradient of the whole sample's
 // fragments is accumulated in LDS while the group's gFF tiles stream through LDS once; each
 // output element is owned by one 2^k-lane row of threads that splits the channel reduction
@@ -1977,7 +1979,17 @@ int bwd_groups_for(const cgnet_cg_plan* p, int B) {
 
 }  // namespace
 
-int samples_per_group_for(int B, int ntasks) {
+// The pair kernel (built only for at most 16 channels per degree, fewer than all in 8..16) against the task kernel,
+// forward with statistics, measured over lmax 2..20, 1..36 channels, 1..64 samples: with 16 samples or more 1.0 .. 3.5 times
+// faster up to lmax 15 and, above, up to 4 channels (lmax 11, 5 channels, B = 32: 70 -> 40 us; lmax 20, 1 channel, B = 64:
+// 485 -> 168 us); equal at 4 samples; slower at 1 from lmax 15 on (15 -> 18 us), where a wave has few lanes to fill.  More
+// channels at high degrees leave room for one output degree per unit (lmax 20, 7 channels: 0.82 times the speed), more than 16
+// channels fill the task kernel's register tiles (lmax 8, 20 channels: 0.86 times).
+static bool cg_forward_uses_pairs(const cgnet_cg_plan* p, int B) { return !p->pairs.units.empty() && B >= 4; }
+
+int cg_forward_spg(const cgnet_cg_plan* p, int B) {
+    if (cg_forward_uses_pairs(p, B)) return fwd_pairs_spg(p->pairs, B);
+    const int ntasks = (int)p->fwd_tasks.size();
     // enough work-groups to fill 256 CUs a few times over, while each group amortises the
     // staging of its CG table over several samples
     int groups = std::max(1, std::min(B, (6144 + ntasks - 1) / std::max(1, ntasks)));
@@ -1989,6 +2001,7 @@ using namespace cgnet;
 
 static void free_plan(cgnet_cg_plan* plan) {
     if (!plan) return;
+    free_fwd_pairs(&plan->pairs);
     if (plan->d_fwd_tasks) (void)hipFree(plan->d_fwd_tasks);
     if (plan->d_bwd_tasks) (void)hipFree(plan->d_bwd_tasks);
     if (plan->d_bwd_group_table) (void)hipFree(plan->d_bwd_group_table);
@@ -2504,6 +2517,20 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
     // set-up time: the statistics area of cgnet_sparse_forward_stats_static gets its address on this device
     // (a plan is usable without it: a failure here is reported by that entry point, which resolves the address again)
     if (!resolve_static_scratch()) clear_error();
+    // Few channels: the units of cg_forward_pair_kernel beside the tasks (cg_forward_uses_pairs decides per call).
+    // CGNET_FWD_PAIRS=0 keeps the tasks alone.
+    {
+        int max_tau = 0, sum_tau = 0;
+        for (int l = 0; l < n1; ++l) { max_tau = std::max(max_tau, h_t_F[l]); sum_tau += h_t_F[l]; }
+        const char* e = getenv("CGNET_FWD_PAIRS");
+        if (!p->fwd_mm && max_tau <= 16 && (L <= 15 || sum_tau <= 4 * n1) && !(e && e[0] == '0')) {
+            std::vector<PairTriple> triples(nllls);
+            for (int i = 0; i < nllls; ++i)
+                triples[i] = {tl[i], tl1[i], tl2[i], cgo[i], p->cumFF[tl[i]] + p->t_off[i] * (2 * tl[i] + 1),
+                              p->cumT[tl[i]] + p->t_off[i]};
+            if (int rc = build_fwd_pairs(triples, p->t_F, p->cumF, p->nFF, p->sumT, &p->pairs)) return rc;
+        }
+    }
     if (!p->fwd_tasks.empty()) {
         CGNET_HIP(hipMalloc((void**)&p->d_fwd_tasks, sizeof(CgTask) * p->fwd_tasks.size()));
         CGNET_HIP(hipMemcpy(p->d_fwd_tasks, p->fwd_tasks.data(), sizeof(CgTask) * p->fwd_tasks.size(), hipMemcpyHostToDevice));
@@ -2551,7 +2578,9 @@ extern "C" int cgnet_cg_plan_sizes(const cgnet_cg_plan* plan, int sizes[5]) {
     return CGNET_OK;
 }
 
-extern "C" size_t cgnet_cg_plan_forward_lds(const cgnet_cg_plan* plan) { return plan ? plan->fwd_lds : 0; }
+extern "C" size_t cgnet_cg_plan_forward_lds(const cgnet_cg_plan* plan) {
+    return plan ? std::max(plan->fwd_lds, plan->pairs.lds) : 0;
+}
 
 extern "C" int cgnet_cg_plan_backward_groups(const cgnet_cg_plan* plan) {
     if (!plan) return 0;
@@ -2577,6 +2606,7 @@ extern "C" int cgnet_cg_plan_channels(const cgnet_cg_plan* plan, int* h_t_FF, in
 
 int cgnet::cg_launch_forward(const cgnet_cg_plan* p, const float* d_F, float* d_FF, const float* d_CG, int B,
                           double* d_part, int spg, hipStream_t s, const CgTask* d_tasks, int nFF, int sumT) {
+    if (cg_forward_uses_pairs(p, B)) return launch_fwd_pairs(p->pairs, d_F, d_FF, d_CG, p->nF, B, d_part, spg, s);
     if (!d_tasks) {
         d_tasks = p->d_fwd_tasks;
         nFF = p->nFF;
@@ -2609,13 +2639,13 @@ extern "C" int cgnet_sparse_forward(const cgnet_cg_plan* plan, const float* d_F,
     CGNET_REQUIRE(B >= 0, CGNET_ERR_ARG, "B=%d is negative", B);
     if (B == 0 || plan->nFF == 0) return CGNET_OK;
     CGNET_REQUIRE(d_F && d_FF && d_CG, CGNET_ERR_ARG, "null device pointer");
-    const int spg = samples_per_group_for(B, (int)plan->fwd_tasks.size());
+    const int spg = cg_forward_spg(plan, B);
     return cg_launch_forward(plan, d_F, d_FF, d_CG, B, nullptr, spg, (hipStream_t)stream);
 }
 
 extern "C" size_t cgnet_sparse_forward_stats_workspace(const cgnet_cg_plan* plan, int B) {
     if (!plan || B <= 0) return 0;
-    const int spg = samples_per_group_for(B, (int)plan->fwd_tasks.size());
+    const int spg = cg_forward_spg(plan, B);
     const int ngroups = (B + spg - 1) / spg;
     return align_up(sizeof(double) * 2 * (size_t)plan->sumT * ngroups, 256);
 }
@@ -2640,7 +2670,7 @@ extern "C" int cgnet_sparse_forward_stats(const cgnet_cg_plan* plan, const float
     const size_t need = cgnet_sparse_forward_stats_workspace(plan, B);
     CGNET_REQUIRE(d_workspace && workspace_bytes >= need, CGNET_ERR_WORKSPACE,
                   "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
-    const int spg = samples_per_group_for(B, (int)plan->fwd_tasks.size());
+    const int spg = cg_forward_spg(plan, B);
     const int ngroups = (B + spg - 1) / spg;
     int rc = cg_launch_forward(plan, d_F, d_FF, d_CG, B, (double*)d_workspace, spg, s);
     if (rc != CGNET_OK) return rc;
@@ -2675,7 +2705,7 @@ extern "C" int cgnet_sparse_forward_stats_static(const cgnet_cg_plan* plan, cons
                   "(use cgnet_sparse_forward_stats with a caller workspace)", need, kStaticScratchBytes);
     void* area = resolve_static_scratch();   // resolved when the plan was created on this device; a lookup here
     if (!area) return CGNET_ERR_HIP;         // resolve_static_scratch has recorded the message
-    const int spg = samples_per_group_for(B, (int)plan->fwd_tasks.size());
+    const int spg = cg_forward_spg(plan, B);
     const int ngroups = (B + spg - 1) / spg;
     // every partial sum [group][channel][2] of this call is written by the product kernel before the
     // reduction reads it, so what an earlier call left in the area needs no clearing
@@ -3090,7 +3120,7 @@ int launch_forward_fused(const cgnet_cg_plan* p, const FwdLink& link, const floa
                          float* d_Opart, float* d_O, int B, hipStream_t s) {
     CGNET_REQUIRE(link.ok, CGNET_ERR_UNSUPPORTED, "the fused inference forward does not take this pair of plans");
     const int ntasks = (int)p->fwd_tasks.size();
-    const int spg = samples_per_group_for(B, ntasks);
+    const int spg = cg_forward_spg(p, B);
     const int ngroups = (B + spg - 1) / spg;
     CGNET_REQUIRE((long long)ntasks * ngroups < (1LL << 31), CGNET_ERR_UNSUPPORTED,
                   "%d tasks x %d sample groups exceed the grid limit", ntasks, ngroups);

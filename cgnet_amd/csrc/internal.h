@@ -20,7 +20,7 @@ int wmm_gradw_raw(const cgnet_wmm_plan* plan, const float* d_gO, const float* d_
                   hipStream_t s);
 
 // ---- cg_product.hip
-int samples_per_group_for(int B, int ntasks);
+int cg_forward_spg(const cgnet_cg_plan* p, int B);       // samples per work-group of the product forward
 // the product kernels of one call; d_part != nullptr: also the per-group partial statistics [group][sumT][2]
 // d_tasks: another table of the plan's forward tasks, in the same order, whose tiles lie elsewhere in the product
 // tensor (nFF complex entries and sumT channels per sample); nullptr = the plan's own

@@ -190,7 +190,7 @@ SavedAreas saved_areas(const cgnet_layer_plan* lp, int B) {
 struct FwdAreas { size_t part, wp, opart, total; int spg, ngroups; };
 FwdAreas forward_areas(const cgnet_layer_plan* lp, int B) {
     FwdAreas a{};
-    a.spg = samples_per_group_for(B, (int)lp->cg->fwd_tasks.size());
+    a.spg = cg_forward_spg(lp->cg, B);
     a.ngroups = (B + a.spg - 1) / a.spg;
     // sized for either layout of the product tensor
     size_t wp = wmm_forward_wp_bytes(lp->wmm), opart = wmm_forward_opart_bytes(lp->wmm, B);
