@@ -24,68 +24,98 @@ namespace cgnet {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kStatTileBytes = 32 * 1024;
+constexpr int kStatStageBytes = 12 * 1024;   // statistics: LDS bytes of a wave's stage (six waves with two stages share a compute unit)
 constexpr int kStatGroups = 8;
 constexpr int kGradWChunk = 32;     // samples whose weight-gradient sums one work-group forms, at most (the chunks of a
                                     // batch are made equal: 100 samples are four chunks of 25, not 32 + 32 + 32 + 4)
 constexpr int kGradWFold = 1;       // samples per matrix-core chain inside a chunk
 
 // --------------------------------------------------------------------------- statistics
-// sums of |z| and |z|^2 over (b, m) per mid channel, from FF
-__global__ void __launch_bounds__(kThreads)
+// sqrt(n) from the hardware's reciprocal square root and one correction step: half an ulp but for rare ties, at a third of
+// the instructions of sqrtf (which also scales arguments below 2^-96; their roots count for nothing in the sums).
+__device__ __forceinline__ float modulus(float n) {
+    const float y = __builtin_amdgcn_rsqf(fmaxf(n, 1e-37f));
+    const float r = n * y;
+    return fmaf(fmaf(-r, r, n), 0.5f * y, r);
+}
+
+// Sums of |z| and |z|^2 over (b, m) per mid channel, from FF.  Bound by reading FF once.  A wave works alone: a lane is a
+// channel, the run of its up to 64 channels (contiguous in a sample) is copied into LDS by LDS-direct loads one stage
+// ahead, as many samples a stage as fit kStatStageBytes, and no barrier holds the stream up.  (A work-group that loaded
+// one sample's tile through registers between two barriers ran at 2.7 TB/s: lmax 11, 12 channels, B = 50, 383 MB of FF:
+// 141 us, now 81 us.)
+__global__ void __launch_bounds__(64)
 fn_stats_kernel(const float2* __restrict__ FF, const WmmDeg* __restrict__ degs,
                 const WmmChanUnit* __restrict__ units, int nFF, int B, int samples_per_group,
-                double* __restrict__ part, int sumT) {
+                double* __restrict__ part, int sumT, int stage_bytes) {
     extern __shared__ __align__(16) unsigned char smem[];
-    float2* tile = reinterpret_cast<float2*>(smem);
     const UnitPart up = part_major((B + samples_per_group - 1) / samples_per_group);
     const WmmChanUnit u = units[up.unit];
     const WmmDeg d = degs[u.deg];
-    const int n = u.nc * d.M;
-    const int tid = threadIdx.x;
-    double s1 = 0., s2 = 0.;
+    const int lane = threadIdx.x, M = d.M;
+    const int n = u.nc * M, pitch = (8 * n + 15) & ~15;          // entries / LDS bytes of one sample
+    const int G = max(1, stage_bytes / pitch);                   // samples of a stage
     const int b0 = up.part * samples_per_group, b1 = min(B, b0 + samples_per_group);
-    for (int b = b0; b < b1; ++b) {
-        const float2* src = FF + (size_t)b * nFF + d.cumFF + (size_t)u.c0 * d.M;
-        for (int e = tid; e < n; e += kThreads) tile[e] = src[e];
-        __syncthreads();
-        if (tid < u.nc) {
-            // both sums run over the same rounded |z| in double (no cancellation between
-            // inconsistently rounded terms when the variance is formed)
-            for (int mm = 0; mm < d.M; ++mm) {
-                const float2 z = tile[tid * d.M + mm];
-                const double r = (double)sqrtf(fmaf(z.x, z.x, z.y * z.y));
-                s1 += r;
-                s2 = fma(r, r, s2);
+    const int ni = (((n >> 1) + 63) >> 6) + (n & 1);             // copy instructions of a sample
+    const float2* src = FF + d.cumFF + (size_t)u.c0 * M;
+    auto issue = [&](int b, int par) {
+        for (int g = 0; g < G && b + g < b1; ++g) {
+            const float2* from = src + (size_t)(b + g) * nFF;
+            unsigned char* to = smem + par * stage_bytes + g * pitch;
+            dma16<64>(from, to, n >> 1, lane);
+            if (n & 1) dma8(from + (n - 1), to + 8 * (size_t)(n - 1), lane);
+        }
+    };
+    double s1 = 0., s2 = 0.;
+    if (b0 < b1) issue(b0, 0);
+    int par = 0;
+    for (int b = b0; b < b1; b += G, par ^= 1) {
+        const int next = min(G, b1 - b - G);                     // samples of the following stage
+        if (next > 0) {
+            issue(b + G, par ^ 1);
+            wait_vmcnt(next * ni);
+        } else {
+            dma_wait();
+        }
+        if (lane < u.nc) {
+            for (int g = 0; g < G && b + g < b1; ++g) {
+                const float2* row = reinterpret_cast<const float2*>(smem + par * stage_bytes + g * pitch) + lane * M;
+                // both sums run over the same rounded |z| in double (no cancellation between inconsistently rounded terms
+                // when the variance is formed)
+#pragma unroll 4
+                for (int mm = 0; mm < M; ++mm) {
+                    const float2 z = row[mm];
+                    const double r = (double)modulus(fmaf(z.x, z.x, z.y * z.y));
+                    s1 += r;
+                    s2 = fma(r, r, s2);
+                }
             }
         }
-        __syncthreads();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the buffer has been read before the next copy into it
     }
-    if (tid < u.nc) {
-        double* p = part + ((size_t)up.part * sumT + d.cumT + u.c0 + tid) * 2;
+    if (lane < u.nc) {
+        double* p = part + ((size_t)up.part * sumT + d.cumT + u.c0 + lane) * 2;
         p[0] = s1;
         p[1] = s2;
     }
 }
 
+// stds[c] <- stds[c] * cnt/(cnt+1) + std_batch[c] / (cnt+1), from the sums of `ngroups` groups of samples (added in order)
 __global__ void __launch_bounds__(256)
-fn_sum_groups_kernel(const double* __restrict__ part, double* __restrict__ sums, int n2, int ngroups) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n2) return;
-    double s = 0.;
-    for (int g = 0; g < ngroups; ++g) s += part[(size_t)g * n2 + i];
-    sums[i] = s;
-}
-
-// stds[c] <- stds[c] * cnt/(cnt+1) + std_batch[c] / (cnt+1)
-__global__ void __launch_bounds__(256)
-fn_update_std_kernel(const double* __restrict__ sums, float* __restrict__ stds,
+fn_update_std_kernel(const double* __restrict__ part, int ngroups, float* __restrict__ stds,
                      const WmmDeg* __restrict__ degs, int ndeg, int sumT, int B, float cnt) {
     __shared__ int s_tab[kMaxLookup];
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     const int di = lookup_in_group(ndeg, c, [&](int k) { return degs[k].cumT; }, s_tab);
     if (c >= sumT) return;
-    stds[c] = updated_std(stds[c], sums[2 * c], sums[2 * c + 1], (double)B * (double)degs[di].M, cnt);
+    double s1 = 0., s2 = 0.;
+#pragma unroll 4
+    for (int g = 0; g < ngroups; ++g) {
+        const double2 v = reinterpret_cast<const double2*>(part)[(size_t)g * sumT + c];
+        s1 += v.x;
+        s2 += v.y;
+    }
+    stds[c] = updated_std(stds[c], s1, s2, (double)B * (double)degs[di].M, cnt);
 }
 
 // --------------------------------------------------------------------------- weight packing
@@ -677,14 +707,12 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(float* p, size_t n) {
 int stat_groups_for(int B) { return std::max(1, std::min(B, kStatGroups)); }
 
 struct FwdWorkspace {
-    size_t sums, part, wp, opart, total;
+    size_t part, wp, opart, total;
 };
 
 FwdWorkspace fwd_workspace(const cgnet_wmm_plan* p, int B) {
     FwdWorkspace w;
     size_t o = 0;
-    w.sums = o;
-    o += align_up(sizeof(double) * 2 * (size_t)p->sumT, 256);
     w.part = o;
     o += align_up(sizeof(double) * 2 * (size_t)p->sumT * stat_groups_for(B), 256);
     w.wp = o;
@@ -793,10 +821,9 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
     for (int di = 0; di < ndeg; ++di) {
         const WmmDeg& d = p->degs[di];
         if (d.K == 0) continue;
-        const int per_stat = std::max(1, std::min(kThreads, kStatTileBytes / (8 * d.M)));
+        const int per_stat = d.M <= 24 ? 64 : d.M <= 48 ? 32 : 16;
         for (int c0 = 0; c0 < d.K; c0 += per_stat)
             p->stat_units.push_back(WmmChanUnit{di, 0, c0, std::min(per_stat, d.K - c0)});
-        p->stat_lds = std::max(p->stat_lds, (size_t)8 * per_stat * d.M);
         const int per_gff = std::max(1, 4096 / d.M);
         for (int c0 = 0; c0 < d.K; c0 += per_gff) {
             p->gff_units.push_back(WmmChanUnit{di, 0, c0, std::min(per_gff, d.K - c0)});
@@ -900,21 +927,19 @@ extern "C" int cgnet_FN_WMM_forward(const cgnet_wmm_plan* plan, const float* d_F
 
     if (upd && plan->sumT > 0) {
         const double* sums = d_sums;
+        int nsums = 1;
         if (!sums) {
             const int ng = stat_groups_for(B);
             const int spg = (B + ng - 1) / ng;
             const int ngroups = (B + spg - 1) / spg;
-            CGNET_LAUNCH(fn_stats_kernel, dim3(grid_1d(plan->stat_units.size(), ngroups)), dim3(kThreads),
-                               plan->stat_lds, s, (const float2*)d_FF, plan->d_degs, plan->d_stat_units, plan->nFF,
-                               B, spg, (double*)(base + ws.part), plan->sumT);
+            CGNET_LAUNCH(fn_stats_kernel, dim3(grid_1d(plan->stat_units.size(), ngroups)), dim3(64), 2 * kStatStageBytes, s,
+                         (const float2*)d_FF, plan->d_degs, plan->d_stat_units, plan->nFF, B, spg, (double*)(base + ws.part),
+                         plan->sumT, kStatStageBytes);
             CGNET_HIP(hipGetLastError());
-            const int n2 = 2 * plan->sumT;
-            CGNET_LAUNCH(fn_sum_groups_kernel, dim3((n2 + 255) / 256), dim3(256), 0, s,
-                               (const double*)(base + ws.part), (double*)(base + ws.sums), n2, ngroups);
-            CGNET_HIP(hipGetLastError());
-            sums = (const double*)(base + ws.sums);
+            sums = (const double*)(base + ws.part);
+            nsums = ngroups;
         }
-        CGNET_LAUNCH(fn_update_std_kernel, dim3((plan->sumT + 255) / 256), dim3(256), 0, s, sums, d_stds,
+        CGNET_LAUNCH(fn_update_std_kernel, dim3((plan->sumT + 255) / 256), dim3(256), 0, s, sums, nsums, d_stds,
                            plan->d_degs, ndeg, plan->sumT, B, cnt);
         CGNET_HIP(hipGetLastError());
     }

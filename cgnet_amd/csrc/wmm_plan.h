@@ -49,7 +49,7 @@ struct cgnet_wmm_plan {
     cgnet::WmmChanUnit* d_gff_zero_units = nullptr;   // channels of degrees without outputs: their gradient is zero
     cgnet::WmmChanUnit* d_stat_units = nullptr;
     int* d_cumO = nullptr;      // per deg index: cumO, and S, interleaved: [ndeg+1] cumO then [ndeg] S
-    size_t stat_lds = 0, gff_lds = 0;
+    size_t gff_lds = 0;
 };
 
 
