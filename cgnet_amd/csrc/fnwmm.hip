@@ -153,8 +153,19 @@ pack_w_backward_kernel(const float2* __restrict__ W, const float* __restrict__ s
 // is a vmcnt wait that leaves the younger stages in flight.
 constexpr int kFwdKC = 8;        // channels per stage (two k-steps of 4)
 constexpr int kFwdMaxT = 6;      // column tiles per wave (96 complex columns)
-constexpr int kFwdDepth = 3;
-constexpr int kFwdSlice = 256;   // channels per k-slice: short enough that the groups pack the CUs evenly
+constexpr int kFwdDepth = 3;       // longer rings cost more (fewer waves a compute unit, more to clear) than they hide,
+                                   // also where few waves run: 120 -> 145 us with four stages (net of kFwdSlices)
+// Channels per k-slice: the longest that gives kFwdFill waves.  A wave walks its slice as one serial chain of stages, so few
+// waves leave the chip waiting on latency; shorter slices than needed cost partial outputs.  Mixing + slice sum of all
+// layers, us, for slices of 256 | 128 | 64 | 32 (waves of the widest layer):
+//   lmax 10, five layers of 12..3 channels, B=100   179 | 142 | 159 | 165   (1465 | 2789 | 5408 | 10443)
+//   the same, B=1                                   130 |  91 |  68 |  60   (31 | 58 | 112 | 215)
+//   lmax 11, 5 channels, B=32                        41 |  27 |  27 |  29   (881 | 1676 | 3233 | 6368)
+//   lmax 13, MST triples, 16..4 channels, B=27      109 |  85 |  76 |  80   (643 | 1184 | 2273 | 4444)
+//   lmax 11, 12 channels, B=100                     195 | 206 | 239 | 320   (14427 | 28513 | ...)
+constexpr int kFwdSlices[] = {256, 128, 64, 32};
+constexpr int kFwdFill = 1600;
+constexpr int kFwdWhole = 128;     // degrees up to this many channels stay whole: 16 stages cost less than a launch that adds slices
 
 template <int T>
 __device__ __forceinline__ void wmm_forward_wave(const float2* __restrict__ FF, const float* __restrict__ Wp,
@@ -706,6 +717,18 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(float* p, size_t n) {
 
 int stat_groups_for(int B) { return std::max(1, std::min(B, kStatGroups)); }
 
+// The split a batch of this size runs with (kFwdSlices).
+const WmmFwdSplit& fwd_split(const cgnet_wmm_plan* p, int B) {
+    if (p->maxK <= kFwdWhole) return p->fwd_splits.front();
+    for (const WmmFwdSplit& sp : p->fwd_splits) {
+        size_t waves = 0;
+        for (size_t di = 0; di < p->degs.size(); ++di)
+            waves += (size_t)sp.deg_units[di] * ((B + p->degs[di].G - 1) / p->degs[di].G);
+        if (waves >= kFwdFill) return sp;
+    }
+    return p->fwd_splits.back();
+}
+
 struct FwdWorkspace {
     size_t part, wp, opart, total;
 };
@@ -718,7 +741,7 @@ FwdWorkspace fwd_workspace(const cgnet_wmm_plan* p, int B) {
     w.wp = o;
     o += align_up(sizeof(float) * 64 * (size_t)p->wp_blocks, 256);
     w.opart = o;
-    if (p->maxS > 1) o += align_up(sizeof(float) * 2 * (size_t)p->nO * B * p->maxS, 256);
+    o += align_up(wmm_forward_opart_bytes(p, B), 256);
     w.total = o;
     return w;
 }
@@ -730,10 +753,14 @@ using namespace cgnet;
 
 static void free_plan(cgnet_wmm_plan* plan) {
     if (!plan) return;
-    void* ptrs[] = {plan->d_degs, plan->d_fwd_units, plan->d_gw_units, plan->d_gw_units_rc0, plan->d_gff_units, plan->d_gff_zero_units,
-                    plan->d_stat_units, plan->d_cumO};
+    void* ptrs[] = {plan->d_degs, plan->d_gw_units, plan->d_gw_units_rc0, plan->d_gff_units, plan->d_gff_zero_units,
+                    plan->d_stat_units};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
+    for (const WmmFwdSplit& sp : plan->fwd_splits) {
+        if (sp.d_units) (void)hipFree(sp.d_units);
+        if (sp.d_cumO_S) (void)hipFree(sp.d_cumO_S);
+    }
     delete plan;
 }
 
@@ -776,8 +803,6 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
         }
         d.G = bestG;
         d.NC = bestNC;
-        // k-slices of about kFwdSlice channels (multiples of 8)
-        d.S = std::max(1, (K + kFwdSlice - 1) / kFwdSlice);
         d.nks_b = std::max(1, (2 * tO + 3) / 4);
         d.ap_base = p->ap_blocks;
         p->ap_blocks += ((K + 15) / 16) * d.nks_b;
@@ -797,16 +822,8 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
         const WmmDeg& d = p->degs[di];
         if (d.K == 0 || d.tO == 0) continue;
         CGNET_REQUIRE(d.NC <= kFwdMaxT, CGNET_ERR_UNSUPPORTED, "degree %d has more than 96 columns per sample", d.l);
-        p->maxS = std::max(p->maxS, d.S);
-        p->maxG = std::max(p->maxG, d.G);
+        p->maxK = std::max(p->maxK, d.K);
         p->fwd_stage_cap = std::max(p->fwd_stage_cap, 1024 + d.G * kFwdKC * d.M * 8);   // bytes: weights + runs
-        const int steps = (d.K + 7) / 8;
-        const int per = ((steps + d.S - 1) / d.S) * 8;
-        for (int rc = 0; rc < d.nrc; ++rc)
-            for (int s = 0; s < d.S; ++s) {
-                WmmFwdUnit u{di, rc, s, std::min(d.K, s * per), std::min(d.K, (s + 1) * per)};
-                p->fwd_units.push_back(u);
-            }
         int gw_nc = 64;
         // both stages of the unit's FF rows and of the 16 gO rows fit 64 KB of LDS
         while (gw_nc > 16 && 16 * ((size_t)gw_nc * d.M + 2 + 16 * (size_t)d.M + 2) > 64 * 1024) gw_nc /= 2;
@@ -834,18 +851,9 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
     // the matrix-core gradient kernel keeps a tile and two operand buffers per wave inside 64 KB of LDS
     if ((size_t)p->gff_out_cap + 2 * (size_t)p->gff_go_cap > 64 * 1024) p->gff_mfma = false;
     CGNET_REQUIRE(p->gff_lds <= 64 * 1024, CGNET_ERR_UNSUPPORTED, "t_O*(2l+1) too large for the gradient kernel");
-    // heavier forward units first
-    std::stable_sort(p->fwd_units.begin(), p->fwd_units.end(), [&](const WmmFwdUnit& a, const WmmFwdUnit& b) {
-        return (long long)(a.k_end - a.k_begin) * p->degs[a.deg].M > (long long)(b.k_end - b.k_begin) * p->degs[b.deg].M;
-    });
     std::stable_sort(p->gw_units.begin(), p->gw_units.end(), [&](const WmmChanUnit& a, const WmmChanUnit& b) {
         return p->degs[a.deg].M > p->degs[b.deg].M;
     });
-
-    std::vector<int> cumO_S(2 * ndeg + 1);
-    for (int di = 0; di < ndeg; ++di) cumO_S[di] = p->degs[di].cumO;
-    cumO_S[ndeg] = p->nO;
-    for (int di = 0; di < ndeg; ++di) cumO_S[ndeg + 1 + di] = (p->degs[di].K == 0 || p->degs[di].tO == 0) ? 0 : p->degs[di].S;
 
     auto upload = [&](const void* src, size_t bytes, void** dst) -> int {
         if (bytes == 0) return CGNET_OK;
@@ -855,19 +863,37 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
     };
     int rc;
     if ((rc = upload(p->degs.data(), sizeof(WmmDeg) * ndeg, (void**)&p->d_degs))) return rc;
-    {
+    for (const int slice : kFwdSlices) {
+        WmmFwdSplit& sp = p->fwd_splits.emplace_back();
+        std::vector<int> cumO_S(2 * ndeg + 1);
+        sp.deg_units.assign(ndeg, 0);
+        for (int di = 0; di < ndeg; ++di) {
+            const WmmDeg& d = p->degs[di];
+            cumO_S[di] = d.cumO;
+            if (d.K == 0 || d.tO == 0) continue;
+            // k-slices of about `slice` channels (multiples of 8)
+            const int S = (d.K + slice - 1) / slice, steps = (d.K + 7) / 8, per = ((steps + S - 1) / S) * 8;
+            cumO_S[ndeg + 1 + di] = S;
+            sp.maxS = std::max(sp.maxS, S);
+            sp.deg_units[di] = S * d.nrc;
+            for (int rc2 = 0; rc2 < d.nrc; ++rc2)
+                for (int s = 0; s < S; ++s)
+                    sp.units.push_back(WmmFwdUnit{di, rc2, s, std::min(d.K, s * per), std::min(d.K, (s + 1) * per)});
+        }
+        cumO_S[ndeg] = p->nO;
         // longest units first, so that the last groups to start are short ones
         auto work = [&](const WmmFwdUnit& u) {
             const WmmDeg& d = p->degs[u.deg];
             return (long long)(u.k_end - u.k_begin) * d.M * d.G;
         };
-        std::stable_sort(p->fwd_units.begin(), p->fwd_units.end(),
+        std::stable_sort(sp.units.begin(), sp.units.end(),
                          [&](const WmmFwdUnit& a, const WmmFwdUnit& b) { return work(a) > work(b); });
-        auto mid = std::stable_partition(p->fwd_units.begin(), p->fwd_units.end(),
+        auto mid = std::stable_partition(sp.units.begin(), sp.units.end(),
                                          [&](const WmmFwdUnit& u) { return p->degs[u.deg].NC <= 3; });
-        p->fwd_units_small = (int)(mid - p->fwd_units.begin());
+        sp.units_small = (int)(mid - sp.units.begin());
+        if ((rc = upload(sp.units.data(), sizeof(WmmFwdUnit) * sp.units.size(), (void**)&sp.d_units))) return rc;
+        if ((rc = upload(cumO_S.data(), sizeof(int) * cumO_S.size(), (void**)&sp.d_cumO_S))) return rc;
     }
-    if ((rc = upload(p->fwd_units.data(), sizeof(WmmFwdUnit) * p->fwd_units.size(), (void**)&p->d_fwd_units))) return rc;
     if ((rc = upload(p->gw_units.data(), sizeof(WmmChanUnit) * p->gw_units.size(), (void**)&p->d_gw_units))) return rc;
     for (const WmmChanUnit& u : p->gw_units)
         if (u.rc == 0) p->gw_units_rc0.push_back(u);
@@ -875,7 +901,6 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
     if ((rc = upload(p->gff_units.data(), sizeof(WmmChanUnit) * p->gff_units.size(), (void**)&p->d_gff_units))) return rc;
     if ((rc = upload(p->gff_zero_units.data(), sizeof(WmmChanUnit) * p->gff_zero_units.size(), (void**)&p->d_gff_zero_units))) return rc;
     if ((rc = upload(p->stat_units.data(), sizeof(WmmChanUnit) * p->stat_units.size(), (void**)&p->d_stat_units))) return rc;
-    if ((rc = upload(cumO_S.data(), sizeof(int) * cumO_S.size(), (void**)&p->d_cumO))) return rc;
     *plan = guard.release();
     return CGNET_OK;
 }
@@ -945,7 +970,7 @@ extern "C" int cgnet_FN_WMM_forward(const cgnet_wmm_plan* plan, const float* d_F
     }
     if (plan->nO == 0) return CGNET_OK;
     float* Wp = (float*)(base + ws.wp);
-    if (!plan->fwd_units.empty()) {
+    if (!plan->fwd_splits[0].units.empty()) {
         const int total = plan->wp_blocks * 16;   // one thread per four packed floats
         CGNET_LAUNCH(pack_w_forward_kernel, dim3((total + 255) / 256), dim3(256), 0, s, (const float2*)d_W,
                            bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Wp, plan->wp_blocks);
@@ -957,7 +982,8 @@ extern "C" int cgnet_FN_WMM_forward(const cgnet_wmm_plan* plan, const float* d_F
 namespace cgnet {
 size_t wmm_forward_wp_bytes(const cgnet_wmm_plan* plan) { return sizeof(float) * 64 * (size_t)plan->wp_blocks; }
 size_t wmm_forward_opart_bytes(const cgnet_wmm_plan* plan, int B) {
-    return plan->maxS > 1 ? sizeof(float) * 2 * (size_t)plan->nO * B * plan->maxS : 0;
+    const WmmFwdSplit& sp = fwd_split(plan, B);
+    return sp.maxS > 1 ? sizeof(float) * 2 * (size_t)plan->nO * B * sp.maxS : 0;
 }
 
 // The mixing itself, with the weights already packed (pack_w_forward_thread): O = sum over channel slices.
@@ -965,7 +991,8 @@ int wmm_forward_packed(const cgnet_wmm_plan* plan, const float* d_FF, float* d_O
                        void* d_opart, hipStream_t s) {
     const int ndeg = (int)plan->degs.size();
     if (plan->nO == 0 || B == 0) return CGNET_OK;
-    if (plan->fwd_units.empty()) {   // degrees with outputs but no mid channels produce zeros
+    const WmmFwdSplit& sp = fwd_split(plan, B);
+    if (sp.units.empty()) {   // degrees with outputs but no mid channels produce zeros
         const size_t n = (size_t)2 * plan->nO * B;
         CGNET_LAUNCH(fill_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_O, n);
         CGNET_HIP(hipGetLastError());
@@ -974,9 +1001,9 @@ int wmm_forward_packed(const cgnet_wmm_plan* plan, const float* d_FF, float* d_O
     // degrees with t_O > 0 but no mid channels are never written by the product kernel
     bool holes = false;
     for (const WmmDeg& d : plan->degs) holes |= (d.tO > 0 && d.K == 0);
-    float2* out = plan->maxS > 1 ? (float2*)d_opart : (float2*)d_O;
+    float2* out = sp.maxS > 1 ? (float2*)d_opart : (float2*)d_O;
     if (holes) {
-        const size_t n = (size_t)2 * plan->nO * B * (plan->maxS > 1 ? plan->maxS : 1);
+        const size_t n = (size_t)2 * plan->nO * B * sp.maxS;
         CGNET_LAUNCH(fill_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (float*)out, n);
         CGNET_HIP(hipGetLastError());
     }
@@ -992,23 +1019,23 @@ int wmm_forward_packed(const cgnet_wmm_plan* plan, const float* d_FF, float* d_O
     const int depth = (int)std::min<size_t>(want_depth, (64 * 1024) / (wpg * (size_t)plan->fwd_stage_cap));
     CGNET_REQUIRE(depth >= 2, CGNET_ERR_UNSUPPORTED, "forward stage of %d bytes does not fit the LDS ring", plan->fwd_stage_cap);
     const size_t lds = wpg * (size_t)depth * plan->fwd_stage_cap;
-    if (plan->fwd_units_small > 0) {
-        CGNET_LAUNCH(wmm_forward_kernel<3>, dim3(grid_1d(plan->fwd_units_small, ygroups)), dim3(64 * wpg), lds, s,
-                     (const float2*)d_FF, Wp, out, plan->d_degs, plan->d_fwd_units, B, plan->nFF, plan->nO,
+    if (sp.units_small > 0) {
+        CGNET_LAUNCH(wmm_forward_kernel<3>, dim3(grid_1d(sp.units_small, ygroups)), dim3(64 * wpg), lds, s,
+                     (const float2*)d_FF, Wp, out, plan->d_degs, sp.d_units, B, plan->nFF, plan->nO,
                      plan->fwd_stage_cap, depth, ygroups);
         CGNET_HIP(hipGetLastError());
     }
-    if ((int)plan->fwd_units.size() > plan->fwd_units_small) {
-        CGNET_LAUNCH(wmm_forward_kernel<6>, dim3(grid_1d(plan->fwd_units.size() - plan->fwd_units_small, ygroups)),
+    if ((int)sp.units.size() > sp.units_small) {
+        CGNET_LAUNCH(wmm_forward_kernel<6>, dim3(grid_1d(sp.units.size() - sp.units_small, ygroups)),
                      dim3(64 * wpg), lds, s, (const float2*)d_FF, Wp, out, plan->d_degs,
-                     plan->d_fwd_units + plan->fwd_units_small, B, plan->nFF, plan->nO, plan->fwd_stage_cap, depth,
+                     sp.d_units + sp.units_small, B, plan->nFF, plan->nO, plan->fwd_stage_cap, depth,
                      ygroups);
         CGNET_HIP(hipGetLastError());
     }
-    if (plan->maxS > 1) {
+    if (sp.maxS > 1) {
         const size_t n = (size_t)plan->nO * B;
         CGNET_LAUNCH(wmm_sum_slices_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           (const float2*)out, (float2*)d_O, plan->d_cumO, ndeg, B, plan->nO);
+                           (const float2*)out, (float2*)d_O, sp.d_cumO_S, ndeg, B, plan->nO);
         CGNET_HIP(hipGetLastError());
     }
     return CGNET_OK;

@@ -430,7 +430,7 @@ extern "C" int cgnet_CGBN_forward(const cgnet_layer_plan* plan, const float* d_F
     }
     // the operands of the mixing forward and (when asked for) of the backward
     float* Wp = (float*)(ws + fa.wp);
-    const bool pack_fwd = wmm->nO > 0 && !wmm->fwd_units.empty();
+    const bool pack_fwd = wmm->nO > 0 && !wmm->fwd_splits[0].units.empty();
     const int nb_fwd = pack_fwd ? (wmm->wp_blocks * 16 + 255) / 256 : 0;
     const int nb_gen = save ? (plan->link.npack + 3) / 4 : 0;
     const int nbF = save ? (int)(((size_t)cg->bwd_nFp * B + 255) / 256) : 0;

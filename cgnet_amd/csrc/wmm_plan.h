@@ -16,12 +16,20 @@ struct WmmDeg {
     int nrc;           // row chunks of 16 output channels
     int wp_base;       // first 64-float block of the degree in the packed weights
     int G, NC;         // forward: samples per work-group, 32-column chunks per wave
-    int S;             // forward: number of k-slices
     int nks_b;         // gradient wrt FF: k-steps of 4 over the 2*tO real rows (re, im interleaved)
     int ap_base;       // first 64-float block of the degree in the packed conj(W)/div operand
 };
 
 struct WmmFwdUnit { int deg, rc, slice, k_begin, k_end; };
+// The forward's units for one length of the k-slices (units of degrees with NC <= 3 first, longest first).
+struct WmmFwdSplit {
+    int maxS = 1;               // slices of the degree that has most of them
+    int units_small = 0;        // units of degrees with NC <= 3
+    std::vector<WmmFwdUnit> units;
+    std::vector<int> deg_units; // units of each degree
+    WmmFwdUnit* d_units = nullptr;
+    int* d_cumO_S = nullptr;    // [ndeg + 1] cumO, then [ndeg] slices of the degree
+};
 struct WmmChanUnit { int deg, rc, c0, nc; };   // a chunk of mid channels of one degree
 
 }  // namespace cgnet
@@ -33,22 +41,19 @@ struct cgnet_wmm_plan {
     int ap_blocks = 0;     // 64-float blocks of the packed operand of the FF-gradient kernel
     bool gff_mfma = true;  // every degree has t_O <= 16 (the operand then fits eight registers)
     int gw_ff_cap = 2, gw_go_cap = 2;   // LDS capacities (complex entries) of one stage of the weight-gradient kernel
+    int maxK = 0;          // channels of the largest degree with outputs
     int fwd_stage_cap = 16;             // LDS bytes of one stage of one wave of the forward kernel
     int gff_out_cap = 16, gff_go_cap = 16; // LDS bytes per wave of the FF-gradient kernel: result tile / one gO buffer
-    int maxS = 1, maxG = 1;
     std::vector<cgnet::WmmDeg> degs;
-    std::vector<cgnet::WmmFwdUnit> fwd_units;   // units of degrees with NC <= 3 first
-    int fwd_units_small = 0;
+    std::vector<cgnet::WmmFwdSplit> fwd_splits;   // longest slices first
     std::vector<cgnet::WmmChanUnit> gw_units, gw_units_rc0, gff_units, gff_zero_units, stat_units;
     std::vector<int> cumO_all, cumFF_all;   // L+2 entries, for element -> degree lookups
     cgnet::WmmDeg* d_degs = nullptr;
-    cgnet::WmmFwdUnit* d_fwd_units = nullptr;
     cgnet::WmmChanUnit* d_gw_units = nullptr;
     cgnet::WmmChanUnit* d_gw_units_rc0 = nullptr;   // one entry per 64-channel chunk (row chunk 0 only)
     cgnet::WmmChanUnit* d_gff_units = nullptr;
     cgnet::WmmChanUnit* d_gff_zero_units = nullptr;   // channels of degrees without outputs: their gradient is zero
     cgnet::WmmChanUnit* d_stat_units = nullptr;
-    int* d_cumO = nullptr;      // per deg index: cumO, and S, interleaved: [ndeg+1] cumO then [ndeg] S
     size_t gff_lds = 0;
 };
 
