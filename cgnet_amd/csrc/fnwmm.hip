@@ -28,6 +28,10 @@ constexpr int kStatStageBytes = 12 * 1024;   // statistics: LDS bytes of a wave'
 constexpr int kStatGroups = 8;
 constexpr int kGradWChunk = 32;     // samples whose weight-gradient sums one work-group forms, at most (the chunks of a
                                     // batch are made equal: 100 samples are four chunks of 25, not 32 + 32 + 32 + 4)
+// A batch is cut into more chunks where that fills the chip: kGradWFill work-groups wanted, kGradWMin samples a chunk at least
+// (a chunk's sums are written once and added by the finishing kernel).  lmax 10, five layers of 12..3 channels, B=100 (112
+// units): chunks of 32 145 us, 1280 groups 99 us, 2560 groups 106 us; lmax 13, MST, 16..4 channels, B=27: 101 -> 45 us.
+constexpr int kGradWFill = 1280, kGradWMin = 4;
 constexpr int kGradWFold = 1;       // samples per matrix-core chain inside a chunk
 
 // --------------------------------------------------------------------------- statistics
@@ -471,6 +475,7 @@ wmm_gradw_finish_kernel(const float2* __restrict__ part, const float* __restrict
     const int di = lookup_in_group(ndeg, idx, [&](int k) { return degs[k].cumW; }, s_tab);
     if (idx >= nW) return;
     float2 s = part[idx];
+#pragma unroll 8
     for (int k = 1; k < nchunks; ++k) {
         const float2 v = part[(size_t)k * nW + idx];
         s.x += v.x;
@@ -565,6 +570,9 @@ pack_w_gradff_kernel(const float2* __restrict__ W, const float* __restrict__ std
 // NT = column tiles worked on together; ONE: these are all column tiles of the degree, so the B
 // operands are built once per sample and shared by the channel tiles.
 constexpr int kGffSub = 4;     // channel tiles per wave
+// Waves wanted (at least eight groups of samples are made in any case), samples a wave keeps at least: it loads its operand
+// once.  lmax 10, layers of 12..3 channels, B=100 (112 units), us: 8 groups 151, 2048 waves 95, 4096 waves 84, 8192 waves 87.
+constexpr int kGffFill = 4096, kGffMin = 2;
 template <int NKS, int NT, bool ONE>
 __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, const float* __restrict__ Ap,
                                                 float2* __restrict__ gFF, const WmmDeg& d, const WmmChanUnit& u, int B,
@@ -1053,17 +1061,22 @@ int wmm_plan_degree(const cgnet_wmm_plan* plan, int l, WmmDegInfo* info) {
 }
 }  // namespace cgnet
 
-static int gradw_chunks(int B) { return (B + kGradWChunk - 1) / kGradWChunk; }
+static int gradw_chunks(const cgnet_wmm_plan* plan, int B) {
+    const int least = (B + kGradWChunk - 1) / kGradWChunk;
+    if (plan->gw_units.empty()) return least;
+    const int units = (int)plan->gw_units.size();
+    return std::max(least, std::min((kGradWFill + units - 1) / units, (B + kGradWMin - 1) / kGradWMin));
+}
 
 namespace cgnet {
 size_t wmm_gradw_part_bytes(const cgnet_wmm_plan* plan, int B) {
-    return sizeof(float) * 2 * (size_t)plan->nW * gradw_chunks(B);
+    return sizeof(float) * 2 * (size_t)plan->nW * gradw_chunks(plan, B);
 }
 int wmm_gradw_raw(const cgnet_wmm_plan* plan, const float* d_gO, const float* d_FF, float* d_part, int B, int* nchunks_out,
                   hipStream_t s) {
     // equal chunks of at most kGradWChunk samples; the kernel derives the number of chunks from their size
-    const int spc = (B + gradw_chunks(B) - 1) / gradw_chunks(B);
-    const int nchunks = (B + spc - 1) / spc;             // <= gradw_chunks(B), what the partial area holds
+    const int spc = (B + gradw_chunks(plan, B) - 1) / gradw_chunks(plan, B);
+    const int nchunks = (B + spc - 1) / spc;             // <= gradw_chunks(plan, B), what the partial area holds
     const size_t lds = sizeof(float2) * 2 * ((size_t)plan->gw_ff_cap + plan->gw_go_cap);
     CGNET_LAUNCH(wmm_gradw_kernel, dim3(grid_1d(plan->gw_units.size(), nchunks)), dim3(kThreads), lds, s,
                  (const float2*)d_gO, (const float2*)d_FF, (float2*)d_part, plan->d_degs, plan->d_gw_units, B, spc,
@@ -1081,7 +1094,7 @@ extern "C" size_t cgnet_FN_WMM_backward_workspace(const cgnet_wmm_plan* plan, in
     if (!plan || B <= 0) return 0;
     // [operand of the FF-gradient kernel] [raw weight-gradient sums per chunk of samples]
     return align_up(gff_operand_bytes(plan), 256) +
-           align_up(sizeof(float) * 2 * (size_t)plan->nW * gradw_chunks(B), 256);
+           align_up(sizeof(float) * 2 * (size_t)plan->nW * gradw_chunks(plan, B), 256);
 }
 
 extern "C" int cgnet_FN_WMM_backward(const cgnet_wmm_plan* plan, const float* d_gO, float* d_gFF, float* d_gW,
@@ -1126,7 +1139,8 @@ extern "C" int cgnet_FN_WMM_backward(const cgnet_wmm_plan* plan, const float* d_
             CGNET_LAUNCH(pack_w_gradff_kernel, dim3((total + 255) / 256), dim3(256), 0, s, (const float2*)d_W,
                          bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap, plan->ap_blocks);
             CGNET_HIP(hipGetLastError());
-            const int groups = std::max(1, std::min(B, 8));
+            const int units = (int)plan->gw_units_rc0.size();
+            const int groups = std::max(std::min(B, 8), std::min((kGffFill + units - 1) / units, (B + kGffMin - 1) / kGffMin));
             const int spg = (B + groups - 1) / groups;
             const int out_bytes = plan->gff_out_cap, go_bytes = plan->gff_go_cap;   // per wave
             const size_t lds = (size_t)out_bytes + 2 * (size_t)go_bytes;

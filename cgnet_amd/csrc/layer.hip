@@ -113,6 +113,7 @@ gradw_unfold_kernel(const float2* __restrict__ part, int nchunks, int nWc, const
     const int cc = (e & 0x7fffffff) - d.cumT;                     // compact channel inside the degree
     const size_t src = (size_t)d.cumW + (size_t)to * d.K + cc;
     float2 s = part[src];
+#pragma unroll 8
     for (int k = 1; k < nchunks; ++k) {
         const float2 v = part[(size_t)k * nWc + src];
         s.x += v.x;
