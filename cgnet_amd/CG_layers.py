@@ -209,8 +209,12 @@ def _straight(fragments):
         row = base.shape[1] * 2
         for v in fragments:
             n = v.numel() // B if B else 0
-            if (v._base is not base or v.dim() != 4 or v.shape[0] != B or v.shape[3] != 2
-                    or v.storage_offset() != off or v.stride() != (row, v.shape[2] * 2, 2, 1)):
+            if v._base is not base or v.dim() != 4 or v.shape[0] != B or v.shape[3] != 2 or v.storage_offset() != off:
+                ok = False
+                break
+            t, m, s = v.shape[1], v.shape[2], v.stride()
+            # the stride of a dimension of size one means nothing (one sample, one channel, degree 0)
+            if n and (s[3] != 1 or (m > 1 and s[2] != 2) or (t > 1 and s[1] != 2 * m) or (B > 1 and s[0] != row)):
                 ok = False
                 break
             off += n
@@ -374,14 +378,15 @@ class _CGBN_fused(torch.autograd.Function):
     visible outside the node, so the backward may skip grad_FF altogether (``fused_backward``)."""
 
     @staticmethod
-    def forward(ctx, Fs, W, layer_plan, CG, bn_stds, bn_cnt, bn_eps, training, fused_backward=True):
+    def forward(ctx, Fs, W, layer_plan, CG, bn_stds, bn_cnt, bn_eps, training, fused_backward=True, wants_grad=True):
         cg_plan, wmm_plan = layer_plan.cg_plan, layer_plan.wmm_plan
         Fs = Fs.contiguous()
         W = W.contiguous()
         B = Fs.shape[0]
         dev = Fs.device
         flags = (BN_FLAG if bn_stds is not None else 0) | (UPDATESTD_FLAG if training else 0)
-        need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
+        # needs_input_grad does not know of torch.no_grad; the caller does
+        need_grad = wants_grad and (ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
         ctx.fused_backward = bool(fused_backward) and layer_plan.fused_backward_supported
         # With the one-kernel backward nothing reads FF but the mixing and the weight gradient, and the layer keeps
         # it in its compact layout (one channel per pair of a diagonal triple) where it has one.
@@ -391,7 +396,7 @@ class _CGBN_fused(torch.autograd.Function):
         out = torch.empty(B, wmm_plan.nO, 2, device=dev, dtype=torch.float)
         # the operands of the one-kernel backward are prepared beside those of the mixing forward, in the same launch
         saved_ops = layer_plan.forward(Fs, FF, out, W, CG, B, bn_stds, float(bn_cnt), float(bn_eps), flags,
-                                       save=ctx.fused_backward and ctx.needs_input_grad[0])
+                                       save=ctx.fused_backward and need_grad and ctx.needs_input_grad[0])
         # bn_stds was updated in place; backward must see the value used for this batch: the copy the forward left
         # among the saved operands, else a clone
         saved_stds = None
@@ -419,13 +424,13 @@ class _CGBN_fused(torch.autograd.Function):
             if need_F:
                 ctx.layer_plan.backward_fused(Fs, grad_F, grad_output, W, CG, ctx.B, stds, ctx.eps,
                                               ctx.flags & (BN_FLAG | UPDATESTD_FLAG), saved_ops)
-            return grad_F, grad_W, None, None, None, None, None, None, None
+            return grad_F, grad_W, None, None, None, None, None, None, None, None
         grad_FF = torch.empty_like(FF) if need_F else None
         if need_F or need_W:
             wmm_plan.backward(grad_output, grad_FF, grad_W, FF, W, ctx.B, stds, ctx.eps, ctx.flags)
         if need_F:
             cg_plan.backward(Fs, grad_F, grad_FF, CG, ctx.B)
-        return grad_F, grad_W, None, None, None, None, None, None, None
+        return grad_F, grad_W, None, None, None, None, None, None, None, None
 
 
 class CGBN_cuda(nn.Module):
@@ -478,7 +483,7 @@ class CGBN_cuda(nn.Module):
                                      bn.bn_stds, bn._eps_host, BN_FLAG if bn.bn_stds is not None else 0)
             else:
                 new_fs = _CGBN_fused.apply(fs, bn.W, lp, self.cg.CGspace, bn.bn_stds, bn.bn_cnt, bn._eps_host, bn.training,
-                                           self.fused_backward)
+                                           self.fused_backward, wants_grad)
             if updates:
                 bn.bn_cnt += 1
         else:
