@@ -1988,12 +1988,18 @@ int bwd_groups_for(const cgnet_cg_plan* p, int B) {
 static bool cg_forward_uses_pairs(const cgnet_cg_plan* p, int B) { return !p->pairs.units.empty() && B >= 4; }
 
 int cg_forward_spg(const cgnet_cg_plan* p, int B) {
-    if (cg_forward_uses_pairs(p, B)) return fwd_pairs_spg(p->pairs, B);
     const int ntasks = (int)p->fwd_tasks.size();
     // enough work-groups to fill 256 CUs a few times over, while each group amortises the
     // staging of its CG table over several samples
-    int groups = std::max(1, std::min(B, (6144 + ntasks - 1) / std::max(1, ntasks)));
-    return (B + groups - 1) / groups;
+    const int groups = std::max(1, std::min(B, (6144 + ntasks - 1) / std::max(1, ntasks)));
+    const int spg = (B + groups - 1) / groups;
+    if (!cg_forward_uses_pairs(p, B)) return spg;
+    // The pair kernel's groups grow with the batch and the task kernel's do not: longer groups where the partial statistics
+    // would outgrow the fixed area of cgnet_sparse_forward_stats_static and those of the task kernel fit in it.
+    const size_t most = p->sumT ? kStaticScratchBytes / (sizeof(double) * 2 * (size_t)p->sumT) : (size_t)B;
+    const int pair_spg = fwd_pairs_spg(p->pairs, B);
+    if ((size_t)((B + spg - 1) / spg) > most || most >= (size_t)B) return pair_spg;
+    return std::max(pair_spg, (int)((B + most - 1) / most));
 }
 }  // namespace cgnet
 

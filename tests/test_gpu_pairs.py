@@ -55,3 +55,33 @@ def test_pair_forward_and_statistics(dev, lmax, taus, bsz, mode):  # noqa: F811
         o += n
     s1, s2 = (torch.cat([(c ** k).sum((0, 2)) for c in parts]) for k in (1, 2))
     assert torch.allclose(sums[:, 0], s1, rtol=4e-7, atol=1e-12) and torch.allclose(sums[:, 1], s2, rtol=8e-7, atol=1e-12)
+
+
+def test_large_batches_fit_the_static_statistics_area(dev):  # noqa: F811
+    """The groups of the pair kernel grow with the batch; their partial statistics stay inside the fixed area wherever
+    there is room for the task kernel's groups (29 of them here), at any batch."""
+    from cgnet_amd import CG_layers, _lib
+    lib = _lib.load()
+    limit = int(lib.cgnet_sparse_forward_stats_static_limit())
+    mod = CG_layers.CG_woFilter_cuda(8, [8, 7, 6, 8, 6, 8, 7, 5, 8], device=dev)
+    plan = mod.native_plan()
+    for bsz in (4, 31, 128, 1000, 4097, 1000003):
+        assert 0 < lib.cgnet_sparse_forward_stats_workspace(plan._h, bsz) <= limit, bsz
+    bsz = 8 * (limit // (16 * plan.sum_tFF)) + 13                      # eight samples a group would be too many groups
+    g = torch.Generator(device=dev).manual_seed(8)
+    x = torch.randn(bsz, plan.nF, 2, generator=g, device=dev)
+    ff, ff_s = (torch.full((bsz, plan.nFF, 2), float("nan"), device=dev) for _ in range(2))
+    sums, sums_s = (torch.full((plan.sum_tFF, 2), float("nan"), device=dev, dtype=torch.float64) for _ in range(2))
+    plan.forward_stats(x, ff, mod.CGspace, bsz, sums)
+    plan.forward_stats_static(x, ff_s, mod.CGspace, bsz, sums_s)
+    assert torch.equal(ff, ff_s) and torch.equal(sums, sums_s)
+    o = 0
+    for l, t in enumerate(int(v) for v in mod.t_FF):                   # the last sample's and the sums of one degree's channels
+        n = t * (2 * l + 1)
+        if l == 5:
+            z = ff[:, o:o + n].double().pow(2).sum(-1).sqrt().reshape(bsz, t, 2 * l + 1)
+            c = int(sum(int(v) for v in mod.t_FF[:l]))
+            assert torch.allclose(sums[c:c + t, 0], z.sum((0, 2)), rtol=4e-7, atol=1e-12)
+        o += n
+    alone = mod(x[-4:], straight_output=True)
+    assert torch.equal(alone, ff[-4:])
