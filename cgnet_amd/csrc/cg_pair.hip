@@ -12,6 +12,7 @@
 // coefficients through scalar registers or row broadcasts therefore cost twice as much.)
 #include <algorithm>
 #include <array>
+#include <cstring>
 #include <map>
 
 #include "cg_pair.h"
@@ -540,11 +541,14 @@ int build_fwd_pairs(const std::vector<PairTriple>& triples, const std::vector<in
     out->nFF = nFF;
     out->sumT = sumT;
     if (!out->units.empty()) {
-        const size_t bytes = sizeof(FwdPair) * out->units.size();
-        CGNET_HIP(hipMalloc((void**)&out->d_units, bytes));
-        CGNET_HIP(hipMemcpy(out->d_units, out->units.data(), bytes, hipMemcpyHostToDevice));
-        CGNET_HIP(hipMalloc((void**)&out->d_items, sizeof(FwdItem) * its.size()));
-        CGNET_HIP(hipMemcpy(out->d_items, its.data(), sizeof(FwdItem) * its.size(), hipMemcpyHostToDevice));
+        // units and items in one allocation, filled by one copy
+        const size_t bytes = sizeof(FwdPair) * out->units.size(), at = align_up(bytes, 256), more = sizeof(FwdItem) * its.size();
+        std::vector<unsigned char> tables(at + more);
+        memcpy(tables.data(), out->units.data(), bytes);
+        memcpy(tables.data() + at, its.data(), more);
+        CGNET_HIP(hipMalloc((void**)&out->d_units, tables.size()));
+        out->d_items = reinterpret_cast<FwdItem*>(reinterpret_cast<unsigned char*>(out->d_units) + at);
+        CGNET_HIP(hipMemcpy(out->d_units, tables.data(), tables.size(), hipMemcpyHostToDevice));
         const void* kernels[] = {(const void*)cg_forward_pair_kernel<true, false>, (const void*)cg_forward_pair_kernel<false, false>,
                                  (const void*)cg_forward_pair_kernel<true, true>, (const void*)cg_forward_pair_kernel<false, true>};
         for (const void* k : kernels)
@@ -555,7 +559,6 @@ int build_fwd_pairs(const std::vector<PairTriple>& triples, const std::vector<in
 
 void free_fwd_pairs(FwdPairSet* set) {
     if (set->d_units) (void)hipFree(set->d_units);
-    if (set->d_items) (void)hipFree(set->d_items);
     *set = FwdPairSet();
 }
 

@@ -48,6 +48,7 @@ struct cgnet_wmm_plan {
     std::vector<cgnet::WmmFwdSplit> fwd_splits;   // longest slices first
     std::vector<cgnet::WmmChanUnit> gw_units, gw_units_rc0, gff_units, gff_zero_units, stat_units;
     std::vector<int> cumO_all, cumFF_all;   // L+2 entries, for element -> degree lookups
+    unsigned char* d_tables = nullptr;          // owns the tables that the pointers below and those of fwd_splits point to
     cgnet::WmmDeg* d_degs = nullptr;
     cgnet::WmmChanUnit* d_gw_units = nullptr;
     cgnet::WmmChanUnit* d_gw_units_rc0 = nullptr;   // one entry per 64-channel chunk (row chunk 0 only)
