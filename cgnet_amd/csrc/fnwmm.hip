@@ -730,13 +730,8 @@ int stat_groups_for(int B) { return std::max(1, std::min(B, kStatGroups)); }
 
 // The split a batch of this size runs with (kFwdSlices).
 const WmmFwdSplit& fwd_split(const cgnet_wmm_plan* p, int B) {
-    if (p->maxK <= kFwdWhole) return p->fwd_splits.front();
-    for (const WmmFwdSplit& sp : p->fwd_splits) {
-        size_t waves = 0;
-        for (size_t di = 0; di < p->degs.size(); ++di)
-            waves += (size_t)sp.deg_units[di] * ((B + p->degs[di].G - 1) / p->degs[di].G);
-        if (waves >= kFwdFill) return sp;
-    }
+    for (const WmmFwdSplit& sp : p->fwd_splits)
+        if (B >= sp.min_batch) return sp;
     return p->fwd_splits.back();
 }
 
@@ -874,7 +869,7 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
     for (const int slice : kFwdSlices) {
         WmmFwdSplit& sp = p->fwd_splits.emplace_back();
         std::vector<int> cumO_S(2 * ndeg + 1);
-        sp.deg_units.assign(ndeg, 0);
+        std::vector<int> deg_units(ndeg, 0);
         for (int di = 0; di < ndeg; ++di) {
             const WmmDeg& d = p->degs[di];
             cumO_S[di] = d.cumO;
@@ -883,12 +878,27 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
             const int S = (d.K + slice - 1) / slice, steps = (d.K + 7) / 8, per = ((steps + S - 1) / S) * 8;
             cumO_S[ndeg + 1 + di] = S;
             sp.maxS = std::max(sp.maxS, S);
-            sp.deg_units[di] = S * d.nrc;
+            deg_units[di] = S * d.nrc;
             for (int rc2 = 0; rc2 < d.nrc; ++rc2)
                 for (int s = 0; s < S; ++s)
                     sp.units.push_back(WmmFwdUnit{di, rc2, s, std::min(d.K, s * per), std::min(d.K, (s + 1) * per)});
         }
         cumO_S[ndeg] = p->nO;
+        // the smallest batch that gives kFwdFill waves (a larger one never gives fewer; kFwdFill samples are enough for any unit
+        // of a group of at most 48)
+        auto fills = [&](int batch) {
+            size_t waves = 0;
+            for (int di = 0; di < ndeg; ++di) waves += (size_t)deg_units[di] * ((batch + p->degs[di].G - 1) / p->degs[di].G);
+            return waves >= kFwdFill;
+        };
+        if (p->maxK > kFwdWhole && slice != std::end(kFwdSlices)[-1]) {
+            int low = 0, high = 48 * kFwdFill;
+            while (high - low > 1) {
+                const int batch = (low + high) / 2;
+                (fills(batch) ? high : low) = batch;
+            }
+            sp.min_batch = high;
+        }
         // longest units first, so that the last groups to start are short ones
         auto work = [&](const WmmFwdUnit& u) {
             const WmmDeg& d = p->degs[u.deg];
@@ -993,8 +1003,17 @@ extern "C" int cgnet_FN_WMM_forward(const cgnet_wmm_plan* plan, const float* d_F
 namespace cgnet {
 size_t wmm_forward_wp_bytes(const cgnet_wmm_plan* plan) { return sizeof(float) * 64 * (size_t)plan->wp_blocks; }
 size_t wmm_forward_opart_bytes(const cgnet_wmm_plan* plan, int B) {
-    const WmmFwdSplit& sp = fwd_split(plan, B);
-    return sp.maxS > 1 ? sizeof(float) * 2 * (size_t)plan->nO * B * sp.maxS : 0;
+    // a smaller batch may run with shorter slices: the largest of what this batch and every smaller one need, so that a
+    // workspace made for a batch serves the smaller ones too
+    size_t most = 0;
+    int batch = B;
+    for (const WmmFwdSplit& sp : plan->fwd_splits) {
+        if (batch >= std::max(1, sp.min_batch)) {
+            if (sp.maxS > 1) most = std::max(most, sizeof(float) * 2 * (size_t)plan->nO * batch * sp.maxS);
+            batch = sp.min_batch - 1;
+        }
+    }
+    return most;
 }
 
 // The mixing itself, with the weights already packed (pack_w_forward_thread): O = sum over channel slices.

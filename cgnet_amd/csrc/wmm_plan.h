@@ -23,10 +23,10 @@ struct WmmDeg {
 struct WmmFwdUnit { int deg, rc, slice, k_begin, k_end; };
 // The forward's units for one length of the k-slices (units of degrees with NC <= 3 first, longest first).
 struct WmmFwdSplit {
+    int min_batch = 0;          // batches from here on run with this split, smaller ones with a later one
     int maxS = 1;               // slices of the degree that has most of them
     int units_small = 0;        // units of degrees with NC <= 3
     std::vector<WmmFwdUnit> units;
-    std::vector<int> deg_units; // units of each degree
     WmmFwdUnit* d_units = nullptr;
     int* d_cumO_S = nullptr;    // [ndeg + 1] cumO, then [ndeg] slices of the degree
 };

@@ -55,3 +55,14 @@ def test_mixing_splits(dev, lmax, t_ff, t_o, bsz):  # noqa: F811
             else:
                 assert a.abs().sum() == 0
         offs = [offs[0] + k * m, offs[1] + n * m, offs[2] + k * n, offs[3] + k]
+
+
+@pytest.mark.parametrize("lmax,tau", [(3, 16), (8, 9), (11, 5)])
+def test_workspace_of_a_batch_serves_smaller_ones(dev, lmax, tau):  # noqa: F811
+    """Smaller batches take shorter slices, which leave more partial outputs a sample."""
+    from cgnet_amd import CG_layers, CGutils, _lib
+    pairs = CGutils.SparseLtuples.compute_default_ltuples(lmax)
+    mod = CG_layers.MyBatchNormWeightMM_cuda(lmax, [len(p) * tau * tau for p in pairs], [tau] * (lmax + 1))
+    plan = mod.native_plan()
+    sizes = [_lib.load().cgnet_FN_WMM_forward_workspace(plan._h, b) for b in range(1, 400)]
+    assert sizes == sorted(sizes) and sizes[0] > 0
