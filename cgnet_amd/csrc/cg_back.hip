@@ -1,0 +1,420 @@
+// Backward of the Clebsch-Gordan product organised by pairs of input degrees: plans, packing kernels and launches.  The kernel
+// and what it does: cg_back_kernel.h.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <map>
+#include <memory>
+#include <numeric>
+
+#include "cg_back_args.h"
+#include "internal.h"
+
+namespace cgnet {
+namespace {
+
+// The coefficients of all pairs, one work-group per (pair, M).
+__global__ void __launch_bounds__(256)
+pack_coef_back_kernel(const float* __restrict__ CG, const BackPair* __restrict__ pairs, const int2* __restrict__ map, int grid0,
+                      float* __restrict__ coef) {
+    pack_coef_back_block(CG, pairs, map[blockIdx.x], grid0, coef);
+}
+
+// Packed gO of the layer source: [chunk of eight M][degree][step][lane (k, (M, re / im))], k = (channel, re / im); zero past the
+// degree's channels and values.  A work-group takes a (chunk, degree) of a sample.  degs: per degree cumO, t_O.
+__global__ void __launch_bounds__(64)
+pack_go_back_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs, float* __restrict__ Go, int ndeg, int pairs,
+                    int grid0, int nO, int nGo) {
+    const int l = (int)blockIdx.x % ndeg, c = (int)blockIdx.x / ndeg;
+    const int2 d = degs[l];
+    const int lane = threadIdx.x, i = lane & 15, kk = lane >> 4;
+    const int x = grid0 + 8 * c + (i >> 1) + l, r = i & 1;
+    const float2* src = gO + (size_t)blockIdx.y * nO + d.x;
+    float* dst = Go + (size_t)blockIdx.y * nGo + (size_t)blockIdx.x * 128 * pairs + lane;
+    for (int s = 0; s < 2 * pairs; ++s) {
+        const int k = 4 * s + kk, to = k >> 1, sel = k & 1;
+        float v = 0.f;
+        if (to < d.y && x >= 0 && x <= 2 * l) {
+            const float2 z = src[to * (2 * l + 1) + x];
+            v = (r == sel) ? (r ? -z.x : z.x) : z.y;
+        }
+        dst[64 * s] = v;
+    }
+}
+
+// Input gradient from the units' partial ones: a row's shares added in the order of its list.
+// meta: [L+2] cumF | [L+2] first row of a degree | [rows + 1] list begin | offsets of the shares
+__global__ void __launch_bounds__(256)
+cg_backward_rows_kernel(const float2* __restrict__ part, float2* __restrict__ gF, const int* __restrict__ meta, int L, int nF, int P,
+                        int B) {
+    __shared__ int s_tab[kMaxLookup];
+    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int b = (int)(idx / nF), e = (int)(idx % nF);
+    const int* cum_rows = meta + (L + 2);
+    const int* begin = cum_rows + (L + 2);
+    const int* at = begin + cum_rows[L + 1] + 1;
+    const int l = lookup_in_group(L + 1, e, [&](int k) { return meta[k]; }, s_tab);
+    if (idx >= (size_t)B * nF) return;
+    const int M = 2 * l + 1, rel = e - s_tab[l], t = rel / M, x = rel - t * M;
+    const int row = cum_rows[l] + t;
+    const float2* from = part + (size_t)b * P + x;
+    float2 s = make_float2(0.f, 0.f);
+#pragma unroll 8
+    for (int k = begin[row]; k < begin[row + 1]; ++k) {
+        const float2 v = from[at[k]];
+        s.x += v.x;
+        s.y += v.y;
+    }
+    gF[idx] = s;
+}
+
+// Packed weights of the layer source, one work-group of four waves per (pair, degree).
+__global__ void __launch_bounds__(256)
+pack_w_back_kernel(const float2* __restrict__ W, const float* __restrict__ stds, float eps, const BackGenW* __restrict__ gens,
+                   float* __restrict__ Wp) {
+    pack_w_back_wave(W, stds, eps, gens[blockIdx.x], (int)(threadIdx.x >> 6), threadIdx.x & 63, Wp);
+}
+
+constexpr int kVariants = 4;                       // kernel variants, by the largest degree
+constexpr int kVariantL[kVariants] = {7, 11, 15, kBackMaxL};
+
+const void* variant_kernel(int v, int pairs) {
+    return v == 0 ? back_kernel_0(pairs) : v == 1 ? back_kernel_1(pairs) : v == 2 ? back_kernel_2(pairs) : back_kernel_3(pairs);
+}
+
+int launch_back(const BackSet& set, const BackLevel& lv, int pairs, BackArgs a, hipStream_t s) {
+    a.pairs = set.d_pairs; a.units = lv.d_units; a.P = lv.P; a.grid0 = set.grid0;
+    a.lds_wave = (int)(set.lds / (4 * kBackWaves));
+    a.nunits = (int)lv.units.size();
+    const int quads = (a.B + kBackWaves - 1) / kBackWaves;
+    CGNET_REQUIRE((long long)a.nunits * quads < (1LL << 31), CGNET_ERR_UNSUPPORTED, "%d units x %d sample groups exceed the grid limit",
+                  a.nunits, quads);
+    const dim3 grid((unsigned)(a.nunits * quads));
+    auto* launch = set.variant == 0 ? back_launch_0 : set.variant == 1 ? back_launch_1 : set.variant == 2 ? back_launch_2 : back_launch_3;
+    launch(pairs, grid, set.lds, s, a);
+    CGNET_HIP(hipGetLastError());
+    return CGNET_OK;
+}
+
+}  // namespace
+
+const BackLevel& back_level(const BackSet& set, int B) {
+    // units wanted of a sample: enough waves that the longest of them is a small part of the call
+    const int want = (5120 + B - 1) / std::max(1, B);
+    for (const BackLevel& lv : set.levels)
+        if (want <= lv.most_units) return lv;
+    return set.levels.back();
+}
+
+int launch_back_combine(const BackLevel& lv, const float* d_part, float* d_gF, int L, int nF, int B, hipStream_t s) {
+    const size_t n = (size_t)nF * B;
+    CGNET_LAUNCH(cg_backward_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const float2*)d_part, (float2*)d_gF,
+                 lv.d_combine, L, nF, lv.P, B);
+    CGNET_HIP(hipGetLastError());
+    return CGNET_OK;
+}
+
+int back_most_batch(const BackSet& set, int L, double per_mac, double slack) {
+    const double more = (set.blocks + 0.6 * set.steps - per_mac * set.macs) * 1e-4;
+    const double most = slack * (20. + 0.25 * L * L);
+    return more <= 0. || most / more >= 1e6 ? INT32_MAX : (int)(most / more);
+}
+
+void free_back_set(BackSet* set) {
+    if (set->d_tables) (void)hipFree(set->d_tables);
+    *set = BackSet();
+}
+
+int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int>& t_F, const std::vector<int>& cumF, int L, int nFF,
+                   BackSet* out) {
+    free_back_set(out);
+    if (L > kBackMaxL || nFF < 2 || nFF >= 1 << 28) return CGNET_OK;       // (32-bit byte offsets in a sample, sixteen bytes a load)
+    for (int t : t_F)
+        if (t > kBackMaxTau) return CGNET_OK;
+    // triples by pair, largest output degree first; the n-th repetition of a triple goes into a list of its own
+    std::map<std::vector<int>, std::vector<const PairTriple*>> lists;          // (l1, l2, repetition)
+    std::map<std::vector<int>, int> seen;
+    for (const PairTriple& t : triples)
+        if (t_F[t.l1] > 0 && t_F[t.l2] > 0) lists[{t.l1, t.l2, seen[{t.l1, t.l2, t.l}]++}].push_back(&t);
+    if (lists.empty()) return CGNET_OK;
+    // The grid of chunks: of the eight places of its origin the one with the fewest chunks in all.
+    int best = -1;
+    for (int shift = 0; shift < 8; ++shift) {
+        const int g0 = -L - shift;
+        int n = 0;
+        for (const PairTriple& t : triples) n += (t.l - g0) / 8 - (-t.l - g0) / 8 + 1;
+        if ((L - g0) / 8 + 1 > (2 * L + 1 + 7) / 8) continue;                  // no more chunks than needed
+        if (best < 0 || n < best) { best = n; out->grid0 = g0; }
+    }
+    out->nchunks = (L - out->grid0) / 8 + 1;
+    for (int v = kVariants - 1; v >= 0; --v)
+        if (L <= kVariantL[v]) out->variant = v;
+    std::vector<double> tile_cost;
+    std::vector<int2> coefmap;
+    size_t coef = 0, lds = 0;
+    for (auto& entry : lists) {
+        std::vector<const PairTriple*>& ts = entry.second;
+        std::stable_sort(ts.begin(), ts.end(), [](const PairTriple* x, const PairTriple* y) { return x->l > y->l; });
+        BackPair p{};
+        p.l1 = entry.first[0]; p.l2 = entry.first[1];
+        p.tau1 = t_F[p.l1]; p.tau2 = t_F[p.l2];
+        p.nl = (int)ts.size();
+        p.nks = (p.nl + 3) / 4;
+        p.nt = (2 * p.l2 + 1 + 15) / 16;
+        // Whole rows t1 in a tile, or sixteen columns wherever they begin, where that makes fewer tiles (tau2 = 12: nine for 144
+        // channels, not twelve); the latter repeat their t2 after tau2 / gcd(16, tau2) tiles.
+        const int C = p.tau1 * p.tau2, whole = std::min(std::min(kBackMaxTau / p.tau2, p.tau1), kBackMaxRows);
+        p.ncol = whole * p.tau2;
+        p.tstep = 1;
+        if ((C + 15) / 16 < (p.tau1 + whole - 1) / whole && (14 + p.tau2) / p.tau2 + 1 <= kBackMaxRows) {
+            p.ncol = kBackMaxTau;
+            p.tstep = p.tau2 / std::gcd(16, p.tau2);
+        }
+        p.ntiles = (C + p.ncol - 1) / p.ncol;
+        for (int t = 0; t < p.ntiles; ++t)
+            p.nrows = std::max(p.nrows, (std::min(C, (t + 1) * p.ncol) - 1) / p.tau2 - t * p.ncol / p.tau2 + 1);
+        p.inv_tau2 = (65536 + p.tau2 - 1) / p.tau2;
+        p.inv_M1 = ((1 << 20) + 2 * p.l1) / (2 * p.l1 + 1);
+        p.inv_M2 = ((1 << 20) + 2 * p.l2) / (2 * p.l2 + 1);
+        const int lm = ts[0]->l;
+        p.c0 = (-lm - out->grid0) / 8;
+        p.nch = (lm - out->grid0) / 8 - p.c0 + 1;
+        p.offF1 = cumF[p.l1]; p.offF2 = cumF[p.l2];
+        p.coef = (int)coef;
+        for (int q = 0; q < p.nl; ++q) {
+            p.l[q] = ts[q]->l;
+            p.cg[q] = ts[q]->cg;
+            p.offFF[q] = ts[q]->offFF;
+            if (p.offFF[q] == 0) p.ends |= 1;
+            if (p.offFF[q] + p.tau1 * p.tau2 * (2 * p.l[q] + 1) == nFF) p.ends |= 2;
+        }
+        // cycles of a tile: matrix instructions of H, the vector half, making (or fetching and turning) G
+        double cost = 3000;
+        for (int x = 0; x < 8 * p.nch; ++x) {
+            const int M = out->grid0 + 8 * p.c0 + x;
+            int n = 0, tiles = 0;
+            for (int q = 0; q < p.nl; ++q) n += std::abs(M) <= p.l[q];
+            for (int rt = 0; rt < p.nt && n > 0; ++rt) {
+                const int lo = std::max(-p.l2, M - p.l1), hi = std::min(p.l2, M + p.l1);
+                if (lo <= -p.l2 + 16 * rt + 15 && hi >= -p.l2 + 16 * rt) tiles |= 1 << rt;
+            }
+            const int nk = tiles ? (n + 3) / 4 : 0;
+            p.steps[x >> 3] |= nk << (4 * (x & 7));
+            p.tiles[x >> 3] |= tiles << (4 * (x & 7));
+            p.degs[x >> 3] = std::max(p.degs[x >> 3], n);
+            const int entries = std::min(p.l2, M + p.l1) - std::max(-p.l2, M - p.l1) + 1;
+            if (n > 0) out->macs += (double)C * n * entries;
+            out->blocks += (double)p.ntiles * __builtin_popcount(tiles);
+            out->steps += 2. * p.ntiles * nk * __builtin_popcount(tiles);
+            if (nk > 0) coefmap.push_back(make_int2((int)out->pairs.size(), x));
+            cost += 60 + __builtin_popcount(tiles) * (64. * nk + 110.);
+        }
+        for (int c = 0; c < p.nch; ++c) cost += ((p.degs[c] + 3) / 4) * 4 * 220.;
+        tile_cost.push_back(cost);
+        coef += (size_t)8 * p.nch * p.nks * p.nt * 64;
+        lds = std::max(lds, (size_t)back_lds_floats(p.nch, p.nt, p.nrows));
+        out->pairs.push_back(p);
+    }
+    CGNET_REQUIRE(coef < (1u << 30), CGNET_ERR_UNSUPPORTED, "packed coefficients of the backward exceed 2^30 floats");
+    out->coef_floats = coef + 64 * 6 * 3;          // a chunk's last reads may run past its own groups
+    out->ncoefmap = (int)coefmap.size();
+    out->lds = 4 * lds * kBackWaves;
+    // levels: pieces of at most 1 / n of a sample's work
+    double all = 0;
+    for (size_t k = 0; k < tile_cost.size(); ++k) all += tile_cost[k] * out->pairs[k].ntiles;
+    std::vector<int> cum_rows(L + 2, 0);
+    for (int l = 0; l <= L; ++l) cum_rows[l + 1] = cum_rows[l] + t_F[l];
+    std::vector<std::vector<int>> combine;
+    for (const int n : {64, 256, 1 << 30}) {
+        BackLevel lv;
+        lv.most_units = n;
+        const double target = n == 1 << 30 ? 0. : all / n;
+        std::vector<std::pair<double, BackUnit>> units;
+        std::vector<std::vector<int>> rows(cum_rows[L + 1]);        // per row (degree, channel): where its shares lie
+        int at = 0;
+        for (size_t k = 0; k < out->pairs.size(); ++k) {
+            const BackPair& p = out->pairs[k];
+            const int M1 = 2 * p.l1 + 1, M2 = 2 * p.l2 + 1;
+            for (int phase = 0; phase < std::min(p.tstep, p.ntiles); ++phase) {
+                const int nt = (p.ntiles - phase + p.tstep - 1) / p.tstep;
+                const int pieces = target > 0. ? std::max(1, (int)std::min((double)nt, std::ceil(nt * tile_cost[k] / target))) : nt;
+                for (int i = 0; i < pieces; ++i) {
+                    const int t0 = nt * i / pieces, n = nt * (i + 1) / pieces - t0;
+                    BackUnit u{(int)k, phase + t0 * p.tstep, n, at, 0};
+                    for (int t = 0; t < n; ++t) {
+                        const int c0 = (u.tile0 + t * p.tstep) * p.ncol, c1 = std::min(p.tau1 * p.tau2, c0 + p.ncol);
+                        for (int r = c0 / p.tau2; r <= (c1 - 1) / p.tau2; ++r)
+                            rows[cum_rows[p.l1] + r].push_back(at + (t * p.nrows + r - c0 / p.tau2) * M1);
+                    }
+                    at += n * p.nrows * M1;
+                    u.p2off = at;
+                    for (int r = 0; r < p.tau2; ++r) rows[cum_rows[p.l2] + r].push_back(at + r * M2);
+                    at += p.tau2 * M2;
+                    units.push_back({tile_cost[k] * n, u});
+                }
+            }
+        }
+        std::stable_sort(units.begin(), units.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+        for (const auto& x : units) lv.units.push_back(x.second);
+        lv.P = at;
+        // meta of cg_backward_rows_kernel: [L+2] cumF | [L+2] first row of a degree | [rows + 1] list begin | offsets
+        std::vector<int> meta(cumF.begin(), cumF.end());
+        meta.insert(meta.end(), cum_rows.begin(), cum_rows.end());
+        int run = 0;
+        for (const auto& r : rows) { meta.push_back(run); run += (int)r.size(); }
+        meta.push_back(run);
+        for (const auto& r : rows) meta.insert(meta.end(), r.begin(), r.end());
+        bool finest = true;
+        for (const BackUnit& u : lv.units) finest &= u.ntiles == 1;
+        out->levels.push_back(lv);
+        combine.push_back(meta);
+        if (finest) break;
+    }
+    // everything in one allocation, filled by one copy
+    size_t bytes = 0;
+    auto place = [&](size_t n) { const size_t at = bytes; bytes += align_up(n, 256); return at; };
+    const size_t at_pairs = place(sizeof(BackPair) * out->pairs.size()), at_map = place(sizeof(int2) * coefmap.size());
+    std::vector<size_t> at_units, at_meta;
+    for (size_t k = 0; k < out->levels.size(); ++k) {
+        at_units.push_back(place(sizeof(BackUnit) * out->levels[k].units.size()));
+        at_meta.push_back(place(sizeof(int) * combine[k].size()));
+    }
+    const std::unique_ptr<unsigned char[]> host(new unsigned char[bytes]());
+    memcpy(host.get() + at_pairs, out->pairs.data(), sizeof(BackPair) * out->pairs.size());
+    memcpy(host.get() + at_map, coefmap.data(), sizeof(int2) * coefmap.size());
+    for (size_t k = 0; k < out->levels.size(); ++k) {
+        memcpy(host.get() + at_units[k], out->levels[k].units.data(), sizeof(BackUnit) * out->levels[k].units.size());
+        memcpy(host.get() + at_meta[k], combine[k].data(), sizeof(int) * combine[k].size());
+    }
+    CGNET_HIP(hipMalloc((void**)&out->d_tables, bytes));
+    CGNET_HIP(hipMemcpy(out->d_tables, host.get(), bytes, hipMemcpyHostToDevice));
+    out->d_pairs = reinterpret_cast<BackPair*>(out->d_tables + at_pairs);
+    out->d_coefmap = reinterpret_cast<int2*>(out->d_tables + at_map);
+    for (size_t k = 0; k < out->levels.size(); ++k) {
+        out->levels[k].d_units = reinterpret_cast<BackUnit*>(out->d_tables + at_units[k]);
+        out->levels[k].d_combine = reinterpret_cast<int*>(out->d_tables + at_meta[k]);
+    }
+    return raise_dynamic_lds(variant_kernel(out->variant, 0), out->lds);
+}
+
+int launch_pack_coef_back(const BackSet& set, const float* d_CG, float* d_coef, hipStream_t s) {
+    CGNET_LAUNCH(pack_coef_back_kernel, dim3((unsigned)set.ncoefmap), dim3(256), 0, s, d_CG, set.d_pairs, set.d_coefmap, set.grid0,
+                 d_coef);
+    CGNET_HIP(hipGetLastError());
+    return CGNET_OK;
+}
+
+int launch_back_memory(const BackSet& set, const BackLevel& lv, const float* d_F, const float* d_gFF, const float* d_coef,
+                       float* d_part, int nF, int nFF, int B, hipStream_t s) {
+    BackArgs a{};
+    a.F = (const float2*)d_F; a.gFF = (const float2*)d_gFF;
+    a.coef = d_coef; a.part = (float2*)d_part;
+    a.nF = nF; a.nFF = nFF; a.B = B;
+    return launch_back(set, lv, 0, a, s);
+}
+
+// ---- layer source --------------------------------------------------------------------------------
+void free_back_link(BackLink* link) {
+    if (link->d_tables) (void)hipFree(link->d_tables);
+    *link = BackLink();
+}
+
+int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* link) {
+    free_back_link(link);
+    CGNET_REQUIRE(wmm_plan_degrees(w) == p->L + 1, CGNET_ERR_ARG, "the two plans have different lmax");
+    std::vector<WmmDegInfo> info(p->L + 1);
+    for (int l = 0; l <= p->L; ++l) {
+        if (int rc = wmm_plan_degree(w, l, &info[l])) return rc;
+        CGNET_REQUIRE(info[l].K == p->t_FF[l], CGNET_ERR_ARG,
+                      "degree %d: the mixing plan has %d mid channels, the product %d", l, info[l].K, p->t_FF[l]);
+    }
+    const BackSet& set = p->back;
+    CGNET_REQUIRE(set.ok(), CGNET_ERR_UNSUPPORTED,
+                  "the fused backward needs lmax <= %d and at most %d channels in every input degree", kBackMaxL, kBackMaxTau);
+    CGNET_REQUIRE(wmm_gradff_operand_ok(w), CGNET_ERR_UNSUPPORTED, "the fused backward needs t_O <= 16 in every degree");
+    link->nO = info[p->L].cumO + info[p->L].tO * (2 * p->L + 1);
+    // every degree takes the pairs of steps (four output channels each) of the one with most outputs
+    std::vector<int2> degs(p->L + 1);
+    for (int l = 0; l <= p->L; ++l) {
+        degs[l] = make_int2(info[l].cumO, info[l].tO);
+        link->pairs = std::max(link->pairs, std::max(1, (info[l].tO + 3) / 4));
+    }
+    link->go_floats = set.nchunks * (p->L + 1) * 128 * link->pairs;
+    std::vector<BackGenPair> gps(set.pairs.size());
+    std::vector<BackGenW> gens;
+    size_t at = 0;
+    for (size_t k = 0; k < set.pairs.size(); ++k) {
+        const BackPair& b = set.pairs[k];
+        BackGenPair& g = gps[k];
+        g = BackGenPair{};
+        g.w = (int)at;
+        for (int grp = 0; grp < b.nks; ++grp) {
+            const int n = std::min(4, b.nl - 4 * grp);
+            for (int q = 0; q < n; ++q) {
+                const int l = b.l[4 * grp + q];
+                BackGenW e{};
+                e.chan0 = (b.offFF[4 * grp + q] - p->cumFF[l]) / (2 * l + 1);
+                e.nch = b.tau1 * b.tau2;
+                e.tO = info[l].tO; e.cumW = info[l].cumW; e.K = info[l].K; e.cumT = info[l].cumT;
+                e.pairs = link->pairs;
+                e.at = (int)at + g.wtile + 256 * (q / 2) + 2 * (q & 1);
+                e.ncol = b.ncol;
+                e.ntiles = b.ntiles;
+                gens.push_back(e);
+            }
+            g.wtile += 512 * link->pairs;
+        }
+        for (size_t i = gens.size() - b.nl; i < gens.size(); ++i) gens[i].wtile = g.wtile;
+        at += (size_t)g.wtile * b.ntiles;
+        CGNET_REQUIRE(at < (1u << 30), CGNET_ERR_UNSUPPORTED, "packed weights of the fused backward exceed 2^30 floats");
+    }
+    link->w_floats = at;
+    link->ngens = (int)gens.size();
+    size_t bytes = 0;
+    auto place = [&](size_t n) { const size_t o = bytes; bytes += align_up(n, 256); return o; };
+    const size_t at_gp = place(sizeof(BackGenPair) * gps.size()), at_gd = place(sizeof(int2) * degs.size());
+    const size_t at_gw = place(sizeof(BackGenW) * gens.size());
+    const std::unique_ptr<unsigned char[]> host(new unsigned char[bytes]());
+    memcpy(host.get() + at_gp, gps.data(), sizeof(BackGenPair) * gps.size());
+    memcpy(host.get() + at_gd, degs.data(), sizeof(int2) * degs.size());
+    memcpy(host.get() + at_gw, gens.data(), sizeof(BackGenW) * gens.size());
+    CGNET_HIP(hipMalloc((void**)&link->d_tables, bytes));
+    if (hipMemcpy(link->d_tables, host.get(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
+        free_back_link(link);
+        set_error("copying the tables of the fused backward failed");
+        return CGNET_ERR_HIP;
+    }
+    link->d_gp = reinterpret_cast<BackGenPair*>(link->d_tables + at_gp);
+    link->d_degs = reinterpret_cast<int2*>(link->d_tables + at_gd);
+    link->d_gens = reinterpret_cast<BackGenW*>(link->d_tables + at_gw);
+    link->ndeg = p->L + 1;
+    link->most_B = back_most_batch(set, p->L, 0.0075, 0.2);
+    if (int rc = raise_dynamic_lds(variant_kernel(set.variant, link->pairs), set.lds)) {
+        free_back_link(link);
+        return rc;
+    }
+    link->ok = true;
+    return CGNET_OK;
+}
+
+int launch_pack_w_back(const BackLink& link, const float* d_W, const float* d_stds, float eps, float* d_Wp, hipStream_t s) {
+    CGNET_LAUNCH(pack_w_back_kernel, dim3((unsigned)link.ngens), dim3(256), 0, s, (const float2*)d_W, d_stds, eps, link.d_gens, d_Wp);
+    CGNET_HIP(hipGetLastError());
+    return CGNET_OK;
+}
+
+int launch_back_layer(const BackSet& set, const BackLink& link, const BackLevel& lv, const float* d_F, const float* d_gO,
+                      const float* d_Wp, const float* d_coef, float* d_Go, float* d_part, int nF, int B, hipStream_t s) {
+    CGNET_REQUIRE(B <= 65535, CGNET_ERR_UNSUPPORTED, "B=%d above 65535", B);
+    const int per_chunk = link.ndeg * 128 * link.pairs;
+    CGNET_LAUNCH(pack_go_back_kernel, dim3((unsigned)(set.nchunks * link.ndeg), (unsigned)B), dim3(64), 0, s, (const float2*)d_gO,
+                 link.d_degs, d_Go, link.ndeg, link.pairs, set.grid0, link.nO, link.go_floats);
+    CGNET_HIP(hipGetLastError());
+    BackArgs a{};
+    a.F = (const float2*)d_F; a.Go = d_Go; a.W = d_Wp; a.gp = link.d_gp;
+    a.coef = d_coef; a.part = (float2*)d_part;
+    a.nF = nF; a.nGo = link.go_floats; a.go_chunk = per_chunk; a.go_degree = 128 * link.pairs; a.B = B;
+    return launch_back(set, lv, link.pairs, a, s);
+}
+
+}  // namespace cgnet

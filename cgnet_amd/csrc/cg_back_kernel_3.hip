@@ -1,0 +1,5 @@
+#include "cg_back_kernel.h"
+
+namespace cgnet {
+CGNET_BACK_VARIANT(3, 6, 3)
+}  // namespace cgnet

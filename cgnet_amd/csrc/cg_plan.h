@@ -4,6 +4,7 @@
 #pragma once
 #include <vector>
 
+#include "cg_back.h"
 #include "cg_pair.h"
 #include "common.h"
 
@@ -91,6 +92,8 @@ struct cgnet_cg_plan {
     size_t fwd_lds = 0, bwd_lds = 0;
     bool fwd_mm = false;                         // the forward runs cg_forward_mm_kernel (product on the matrix cores)
     bool bwd_general_ok = true;                  // cg_backward_kernel's LDS need fits (else only the unit kernels serve)
+    cgnet::BackSet back;                         // the backward by pairs (empty: the unit or the general kernel serves)
+    int back_most_B = 0;                         // ... and the largest batch it is taken for
     cgnet::PairSet pairs;                     // the forward's other form: units of cg_forward_pair_kernel (empty: never used)
     std::vector<int> fwd_class_begin;            // forward tasks by LDS class: class k = tasks [begin[k], begin[k+1])
     std::vector<size_t> fwd_class_lds;           // LDS bytes of a work-group of class k

@@ -1989,6 +1989,8 @@ static bool cg_forward_uses_pairs(const cgnet_cg_plan* p, int B) {
     return !set.units.empty() && B >= 4 && (B >= 8 || set.lanes >= 40 || (long long)B * set.ntriples >= 145LL * (p->L + 1));
 }
 
+static bool cg_backward_uses_pairs(const cgnet_cg_plan* p, int B) { return p->back.ok() && B <= p->back_most_B; }
+
 int cg_forward_spg(const cgnet_cg_plan* p, int B) {
     const int ntasks = (int)p->fwd_tasks.size();
     // enough work-groups to fill 256 CUs a few times over, while each group amortises the
@@ -2012,6 +2014,7 @@ using namespace cgnet;
 static void free_plan(cgnet_cg_plan* plan) {
     if (!plan) return;
     free_fwd_pairs(&plan->pairs);
+    free_back_set(&plan->back);
     if (plan->d_fwd_tasks) (void)hipFree(plan->d_fwd_tasks);
     if (plan->d_bwd_tasks) (void)hipFree(plan->d_bwd_tasks);
     if (plan->d_bwd_group_table) (void)hipFree(plan->d_bwd_group_table);
@@ -2255,6 +2258,21 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
         }
     }
 
+    // ---- backward by pairs of input degrees; the units below are made where it leaves larger batches to them
+    // CGNET_BWD_GENERAL=1 forces the LDS-accumulator kernel (kept for shapes the unit scheme cannot hold)
+    const char* force_general = getenv("CGNET_BWD_GENERAL");
+    const bool general = force_general && force_general[0] == '1';
+    std::vector<PairTriple> triples(nllls);
+    for (int i = 0; i < nllls; ++i)
+        triples[i] = {tl[i], tl1[i], tl2[i], cgo[i], p->cumFF[tl[i]] + p->t_off[i] * (2 * tl[i] + 1), p->cumT[tl[i]] + p->t_off[i]};
+    if (!general) {
+        if (int rc = build_back_set(triples, p->t_F, p->cumF, L, p->nFF, &p->back)) return rc;
+        bool matrix = true;                          // the units would take slot 2 on the matrix cores
+        for (int l = 0; l < n1; ++l) matrix &= h_t_F[l] == 0 || (h_t_F[l] >= 8 && h_t_F[l] <= 16);
+        p->back_most_B = back_most_batch(p->back, L, 0.005, matrix ? 0.2 : 0.4);
+    }
+    const bool want_units = !general && (!p->back.ok() || p->back_most_B < INT32_MAX);
+
     // ---- register-resident backward: units = (l1, range of t1 rows), tasks ordered by (l2, l)
     std::vector<int> combine_meta, pad_meta;
     // First with slot 2 on the matrix cores where the shapes allow it: with the largest tiles that let four work-groups
@@ -2265,7 +2283,7 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
     const int hyb_tiles_kb[] = {30, 28, 24, 20, 16, 12, 40, 36, 32, 28, 24, 20, 16, 12, 8, 4};
     const int n_hyb4 = 6;
     const int n_hyb = (int)(sizeof(hyb_tiles_kb) / sizeof(hyb_tiles_kb[0]));
-    for (int attempt = 0; attempt < n_hyb + 2 && !p->bwd_fast; ++attempt) {
+    for (int attempt = 0; attempt < n_hyb + 2 && want_units && !p->bwd_fast; ++attempt) {
         bool ok = true;
         int P2 = 0;
         size_t lds_max = 0;
@@ -2476,9 +2494,6 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
             }
             p->bwd_units.swap(cut);
         }
-        // CGNET_BWD_GENERAL=1 forces the LDS-accumulator kernel (kept for shapes the unit scheme cannot hold)
-        const char* force_general = getenv("CGNET_BWD_GENERAL");
-        if (force_general && force_general[0] == '1') ok = false;
         if (ok && !p->bwd_units.empty() && lds_max <= (hybrid ? hyb_lds_limit : kMaxUnitLds)) {
             p->bwd_hybrid = hybrid;
             p->bwd_hyb_groups = hybrid ? hyb_groups : 0;
@@ -2523,6 +2538,8 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
         }
     }
 
+    if (!p->bwd_fast) p->back_most_B = INT32_MAX;
+
     CGNET_HIP(hipGetDevice(&p->device));
     // set-up time: the statistics area of cgnet_sparse_forward_stats_static gets its address on this device
     // (a plan is usable without it: a failure here is reported by that entry point, which resolves the address again)
@@ -2534,10 +2551,6 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
         for (int l = 0; l < n1; ++l) { max_tau = std::max(max_tau, h_t_F[l]); sum_tau += h_t_F[l]; }
         const char* e = getenv("CGNET_FWD_PAIRS");
         if (!p->fwd_mm && max_tau <= 16 && (L <= 15 || sum_tau <= 4 * n1) && !(e && e[0] == '0')) {
-            std::vector<PairTriple> triples(nllls);
-            for (int i = 0; i < nllls; ++i)
-                triples[i] = {tl[i], tl1[i], tl2[i], cgo[i], p->cumFF[tl[i]] + p->t_off[i] * (2 * tl[i] + 1),
-                              p->cumT[tl[i]] + p->t_off[i]};
             if (int rc = build_fwd_pairs(triples, p->t_F, p->cumF, p->nFF, p->sumT, &p->pairs)) return rc;
         }
     }
@@ -2596,14 +2609,14 @@ extern "C" int cgnet_cg_plan_backward_groups(const cgnet_cg_plan* plan) {
     if (!plan) return 0;
     const size_t lds = cgnet_cg_plan_backward_lds(plan);
     const int by_lds = lds ? (int)std::min<size_t>(16, cgnet::kMaxLds / lds) : 16;
-    // register budgets: the hybrid kernel 64 or 80 registers with eight waves per group, the unit kernel 128 with four
-    const int by_regs = !plan->bwd_fast ? 8 : plan->bwd_hybrid ? std::max(2, std::min(4, plan->bwd_hyb_groups)) : 4;
+    // register budgets: the kernel by pairs 168 or 256 registers with four waves per group, the hybrid kernel 64 or 80 registers with eight waves per group, the unit kernel 128 with four
+    const int by_regs = plan->back.ok() ? (plan->L <= 7 ? 3 : 2) : !plan->bwd_fast ? 8 : plan->bwd_hybrid ? std::max(2, std::min(4, plan->bwd_hyb_groups)) : 4;
     return std::max(1, std::min(by_lds, by_regs));
 }
 
 extern "C" size_t cgnet_cg_plan_backward_lds(const cgnet_cg_plan* plan) {
     if (!plan) return 0;
-    return plan->bwd_fast ? plan->bwd_fast_lds : plan->bwd_lds;
+    return plan->back.ok() ? plan->back.lds : plan->bwd_fast ? plan->bwd_fast_lds : plan->bwd_lds;
 }
 
 extern "C" int cgnet_cg_plan_channels(const cgnet_cg_plan* plan, int* h_t_FF, int* h_t_offsets) {
@@ -2728,6 +2741,9 @@ extern "C" int cgnet_sparse_forward_stats_static(const cgnet_cg_plan* plan, cons
 
 extern "C" size_t cgnet_sparse_backward_workspace(const cgnet_cg_plan* plan, int B) {
     if (!plan || B <= 0) return 0;
+    if (cg_backward_uses_pairs(plan, B))
+        return align_up(sizeof(float) * 2 * (size_t)back_level(plan->back, B).P * B, 256) +
+               align_up(sizeof(float) * plan->back.coef_floats, 256);
     if (plan->bwd_fast)
         return align_up(sizeof(float) * 2 * (size_t)plan->nF * B, 256) +
                align_up(sizeof(float) * 2 * (size_t)plan->bwd_P2 * B, 256) +
@@ -2762,6 +2778,15 @@ extern "C" int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F
     const size_t need = cgnet_sparse_backward_workspace(plan, B);
     CGNET_REQUIRE(need == 0 || (d_workspace && workspace_bytes >= need), CGNET_ERR_WORKSPACE,
                   "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
+    if (cg_backward_uses_pairs(plan, B)) {
+        CGNET_REQUIRE(((uintptr_t)d_workspace & 15) == 0, CGNET_ERR_ARG, "workspace must be 16-byte aligned");
+        const BackLevel& lv = back_level(plan->back, B);
+        float* part = (float*)d_workspace;
+        float* coef = (float*)((char*)d_workspace + align_up(sizeof(float) * 2 * (size_t)lv.P * B, 256));
+        if (int rc = launch_pack_coef_back(plan->back, d_CG, coef, s)) return rc;
+        if (int rc = launch_back_memory(plan->back, lv, d_F, d_gFF, coef, part, plan->nF, plan->nFF, B, s)) return rc;
+        return launch_back_combine(lv, part, d_gF, plan->L, plan->nF, B, s);
+    }
     if (plan->bwd_fast) {
         float2* part1 = (float2*)d_workspace;
         float2* part2 = (float2*)((char*)part1 + align_up(sizeof(float) * 2 * (size_t)plan->nF * B, 256));

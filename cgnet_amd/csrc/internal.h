@@ -44,6 +44,35 @@ int launch_fused_backward(const cgnet_cg_plan* p, const FusedLink& link, const f
                           const float* d_Fp, const float* d_CGP, float* d_Bg, float* d_part1, float* d_part2,
                           float* d_gF, int B, hipStream_t s);
 
+// ---- cg_back.hip: backward by pairs of input degrees
+// `triples`: every kept triple with its place in the product tensor.  Leaves the set empty where the shape is not taken.
+int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int>& t_F, const std::vector<int>& cumF, int L, int nFF,
+                   BackSet* out);
+void free_back_set(BackSet* set);
+const BackLevel& back_level(const BackSet& set, int B);              // the cut for a batch of B samples
+// Largest batch the backward by pairs is taken for, against a kernel that works triple by triple: where a pair has few output
+// degrees, or rows and columns of its tiles are empty, the other spends fewer instructions, and large batches show it.
+// Measured over lmax 2..23, 1..16 channels (constant and falling with the degree), default and minimum-spanning-tree (MST)
+// triples, 1..64 samples (1365 shapes; geometric means against the other kernels):
+//   stand-alone   always 0.72 of their time, 15 % of the shapes more than 5 % slower, at worst 2.25 times (lmax 8, MST, 14 channels,
+//                 B = 64: 81 -> 181 us); by the rule 0.70, 5 %, 1.54 times
+//   layer, 8..16 channels   always 0.63, 10 %, 1.59 times; by the rule 0.63, 3 %, 1.59 times (lmax 20, MST, 9 channels, B = 16)
+//   layer, other shapes     always 0.49 of the two kernels' time, 1 % slower
+// per_mac: blocks of 256 products that the other kernel makes up for by a multiply-add; slack: of the time a small batch saves.
+int back_most_batch(const BackSet& set, int L, double per_mac, double slack);
+int launch_pack_coef_back(const BackSet& set, const float* d_CG, float* d_coef, hipStream_t s);
+// d_part: lv.P * B complex entries, added up by launch_back_combine
+int launch_back_memory(const BackSet& set, const BackLevel& lv, const float* d_F, const float* d_gFF, const float* d_coef,
+                       float* d_part, int nF, int nFF, int B, hipStream_t s);
+// The same with the gradient of the product made in registers from packed weights and gO.  link->ok says whether the pair of
+// plans is taken; when it is not, the return code is CGNET_ERR_UNSUPPORTED and cgnet_last_error() names the reason.
+int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* link);
+void free_back_link(BackLink* link);
+int launch_pack_w_back(const BackLink& link, const float* d_W, const float* d_stds, float eps, float* d_Wp, hipStream_t s);
+int launch_back_layer(const BackSet& set, const BackLink& link, const BackLevel& lv, const float* d_F, const float* d_gO,
+                      const float* d_Wp, const float* d_coef, float* d_Go, float* d_part, int nF, int B, hipStream_t s);
+int launch_back_combine(const BackLevel& lv, const float* d_part, float* d_gF, int L, int nF, int B, hipStream_t s);
+
 // ---- fused inference forward (cg_product.hip)
 int build_fwd_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, FwdLink* link);
 void free_fwd_link(FwdLink* link);

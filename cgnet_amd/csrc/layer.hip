@@ -27,7 +27,8 @@ struct CompactLink {
 struct cgnet_layer_plan {
     const cgnet_cg_plan* cg = nullptr;
     const cgnet_wmm_plan* wmm = nullptr;
-    cgnet::FusedLink link;
+    cgnet::BackLink link;        // one-kernel backward by pairs of input degrees
+    cgnet::FusedLink fused;      // ... by triples, for the batches the other leaves to it
     char reason[512] = "";       // why the fused backward does not take this layer ("" if it does)
     cgnet::FwdLink fwd;
     char fwd_reason[512] = "";   // why the fused inference forward does not take it
@@ -135,19 +136,19 @@ gradw_unfold_kernel(const float2* __restrict__ part, int nchunks, int nWc, const
 // one launch; the work-groups are dealt out by role:
 //   [0, nb_fwd)      packed weights of the mixing forward               (pack_w_forward_thread; `degs` is the plan the
 //                    mixing runs with: the layer's, or the compact one together with degs_full and cmap)
-//   [.., + nb_gen)   packed weights of the fused backward, four (task, row tile) pairs each   (pack_w_gen_lane)
-//   [.., + nbF)      fragments with a zero behind every row             (pad_fragments_block)
-//   [.., + ntab)     every triple's table between zero rows             (pad_table_block)
+//   [.., + nb_gen)   packed weights of the one-kernel backward, a (pair, degree) each   (pack_w_back_wave)
+//   [.., + nbF)      a copy of the fragments
+//   [.., + ncoef)    packed coefficients of the one-kernel backward, a (pair, M) each   (pack_coef_back_block)
 //   [.., + nb_std)   a copy of the stds (the running values move on with the next batch; the backward of this one
 //                    needs those it was normalised with)
 __global__ void __launch_bounds__(256)
 layer_prepare_kernel(const float2* __restrict__ W, const float* __restrict__ stds, float eps,
                      const WmmDeg* __restrict__ degs, int ndeg, float* __restrict__ Wp, int wp_blocks, int nb_fwd,
                      const WmmDeg* __restrict__ degs_full, const int2* __restrict__ cmap,
-                     const GenTask* __restrict__ gens, const int* __restrict__ packmap, int npack, float* __restrict__ Ag,
-                     int nb_gen, const float2* __restrict__ F, const float* __restrict__ CG, float2* __restrict__ Fp,
-                     float* __restrict__ CGP, const int* __restrict__ padmeta, int L, int nF, int nFp, int B, int nbF,
-                     int ntab, float* __restrict__ stds_copy, int sumT) {
+                     const BackGenW* __restrict__ gens, float* __restrict__ Wb, int nb_gen, const float2* __restrict__ F,
+                     float2* __restrict__ F_copy, size_t n_copy, int nbF, const float* __restrict__ CG,
+                     const BackPair* __restrict__ pairs, const int2* __restrict__ coefmap, int ncoef, int grid0,
+                     float* __restrict__ coef, float* __restrict__ stds_copy, int sumT) {
     __shared__ int s_tab[kMaxLookup];
     int blk = (int)blockIdx.x;
     if (blk < nb_fwd) {
@@ -156,34 +157,39 @@ layer_prepare_kernel(const float2* __restrict__ W, const float* __restrict__ std
     }
     blk -= nb_fwd;
     if (blk < nb_gen) {
-        const int pair = blk * 4 + (int)(threadIdx.x >> 6);
-        if (pair < npack) pack_w_gen_lane(W, stds, eps, gens[packmap[2 * pair]], packmap[2 * pair + 1], threadIdx.x & 63, Ag);
+        pack_w_back_wave(W, stds, eps, gens[blk], (int)(threadIdx.x >> 6), threadIdx.x & 63, Wb);
         return;
     }
     blk -= nb_gen;
     if (blk < nbF) {
-        pad_fragments_block(F, Fp, padmeta, L, nF, nFp, B, blk, s_tab);
+        const size_t e = (size_t)blk * 256 + threadIdx.x;
+        if (e < n_copy) F_copy[e] = F[e];
         return;
     }
     blk -= nbF;
-    if (blk < ntab) {
-        pad_table_block(CG, CGP, padmeta + 2 * (L + 2) + kPadMetaInts * blk);
+    if (blk < ncoef) {
+        pack_coef_back_block(CG, pairs, coefmap[blk], grid0, coef);
         return;
     }
-    blk -= ntab;
+    blk -= ncoef;
     const int c = blk * 256 + (int)threadIdx.x;
     if (c < sumT) stds_copy[c] = stds[c];
 }
 
-struct SavedAreas { size_t stds, Ag, Fp, CGP, total; };
+bool backward_ok(const cgnet_layer_plan* lp) { return lp->link.ok || lp->fused.ok; }
+bool backward_uses_pairs(const cgnet_layer_plan* lp, int B) { return lp->link.ok && (!lp->fused.ok || B <= lp->link.most_B); }
+
+// By pairs: packed weights, fragments, packed coefficients; by triples: packed weights, padded fragments, padded tables.
+struct SavedAreas { size_t stds, Wb, F, coef, total; };
 SavedAreas saved_areas(const cgnet_layer_plan* lp, int B) {
     SavedAreas a{};
-    if (!lp->link.ok || B <= 0) return a;
+    if (!backward_ok(lp) || B <= 0) return a;
+    const bool pairs = backward_uses_pairs(lp, B);
     size_t o = 0;
     a.stds = o; o += align_up(sizeof(float) * (size_t)lp->cg->sumT, 256);   // the stds this batch was normalised with
-    a.Ag = o;   o += align_up(sizeof(float) * lp->link.operand_floats, 256);
-    a.Fp = o;   o += align_up(sizeof(float) * 2 * (size_t)lp->cg->bwd_nFp * B, 256);
-    a.CGP = o;  o += align_up(sizeof(float) * (size_t)lp->cg->bwd_cgp_len, 256);
+    a.Wb = o;   o += align_up(sizeof(float) * (pairs ? lp->link.w_floats : lp->fused.operand_floats), 256);
+    a.F = o;    o += align_up(sizeof(float) * 2 * (size_t)(pairs ? lp->cg->nF : lp->cg->bwd_nFp) * B, 256);
+    a.coef = o; o += align_up(sizeof(float) * (pairs ? lp->cg->back.coef_floats : (size_t)lp->cg->bwd_cgp_len), 256);
     a.total = o;
     return a;
 }
@@ -287,13 +293,21 @@ int build_compact_link(const cgnet_cg_plan* cg, const cgnet_wmm_plan* wmm, Compa
     return CGNET_OK;
 }
 
-struct BwdFusedAreas { BwdAreas own; size_t Ag, Bg, total; };
+struct BwdFusedAreas { BwdAreas own; size_t part, Wb, coef, Go, total; };
 BwdFusedAreas backward_areas(const cgnet_layer_plan* lp, int B) {
     BwdFusedAreas a{};
-    a.own = bwd_areas(lp->cg, B);
-    size_t o = a.own.total;
-    a.Ag = o; o += align_up(sizeof(float) * lp->link.operand_floats, 256);
-    a.Bg = o; o += align_up(sizeof(float) * (size_t)lp->link.bop_floats * B, 256);
+    size_t o = 0;
+    if (backward_uses_pairs(lp, B)) {
+        a.part = o; o += align_up(sizeof(float) * 2 * (size_t)back_level(lp->cg->back, B).P * B, 256);
+        a.Wb = o;   o += align_up(sizeof(float) * lp->link.w_floats, 256);
+        a.coef = o; o += align_up(sizeof(float) * lp->cg->back.coef_floats, 256);
+        a.Go = o;   o += align_up(sizeof(float) * (size_t)lp->link.go_floats * B, 256);
+    } else {
+        a.own = bwd_areas(lp->cg, B);
+        o = a.own.total;
+        a.Wb = o;   o += align_up(sizeof(float) * lp->fused.operand_floats, 256);
+        a.Go = o;   o += align_up(sizeof(float) * (size_t)lp->fused.bop_floats * B, 256);
+    }
     a.total = o;
     return a;
 }
@@ -318,7 +332,7 @@ extern "C" int cgnet_layer_plan_create(cgnet_layer_plan** plan, const cgnet_cg_p
     std::unique_ptr<cgnet_layer_plan> p(new cgnet_layer_plan());
     p->cg = cg_plan;
     p->wmm = wmm_plan;
-    const int rc = build_fused_link(cg_plan, wmm_plan, &p->link);
+    const int rc = build_back_link(cg_plan, wmm_plan, &p->link);
     if (rc == CGNET_ERR_UNSUPPORTED) {
         // the layer still runs, with the two-kernel backward
         std::strncpy(p->reason, cgnet_last_error(), sizeof(p->reason) - 1);
@@ -326,20 +340,31 @@ extern "C" int cgnet_layer_plan_create(cgnet_layer_plan** plan, const cgnet_cg_p
     } else if (rc != CGNET_OK) {
         return rc;
     }
+    if (!p->link.ok || p->link.most_B < INT32_MAX) {
+        const int rc1 = build_fused_link(cg_plan, wmm_plan, &p->fused);
+        if (rc1 == CGNET_ERR_UNSUPPORTED) {
+            clear_error();
+        } else if (rc1 != CGNET_OK) {
+            free_back_link(&p->link);
+            return rc1;
+        }
+    }
     const int rc2 = build_fwd_link(cg_plan, wmm_plan, &p->fwd);
     if (rc2 == CGNET_ERR_UNSUPPORTED) {
         std::strncpy(p->fwd_reason, cgnet_last_error(), sizeof(p->fwd_reason) - 1);
         clear_error();
     } else if (rc2 != CGNET_OK) {
-        free_fused_link(&p->link);
+        free_back_link(&p->link);
+        free_fused_link(&p->fused);
         return rc2;
     }
     // the compact product tensor serves the route whose backward never reads FF as a whole: the one-kernel backward
-    if (p->link.ok) {
+    if (backward_ok(p.get())) {
         const int rc3 = build_compact_link(cg_plan, wmm_plan, &p->compact);
         if (rc3 != CGNET_OK) {
             free_fwd_link(&p->fwd);
-            free_fused_link(&p->link);
+            free_back_link(&p->link);
+            free_fused_link(&p->fused);
             return rc3;
         }
     }
@@ -352,13 +377,14 @@ extern "C" int cgnet_layer_plan_destroy(cgnet_layer_plan* plan) {
     if (!plan) return CGNET_OK;
     free_compact_link(&plan->compact);
     free_fwd_link(&plan->fwd);
-    free_fused_link(&plan->link);
+    free_back_link(&plan->link);
+    free_fused_link(&plan->fused);
     delete plan;
     return CGNET_OK;
 }
 
 extern "C" int cgnet_CGBN_backward_fused_supported(const cgnet_layer_plan* plan) {
-    return plan && plan->link.ok ? 1 : 0;
+    return plan && backward_ok(plan) ? 1 : 0;
 }
 
 extern "C" const char* cgnet_CGBN_backward_fused_reason(const cgnet_layer_plan* plan) {
@@ -370,7 +396,7 @@ extern "C" size_t cgnet_CGBN_saved_bytes(const cgnet_layer_plan* plan, int B) {
 }
 
 extern "C" size_t cgnet_CGBN_saved_stds_bytes(const cgnet_layer_plan* plan, int B) {
-    if (!plan || !plan->link.ok || B <= 0) return 0;
+    if (!plan || !backward_ok(plan) || B <= 0) return 0;
     return sizeof(float) * (size_t)plan->cg->sumT;          // the copy sits at the start of the area
 }
 
@@ -433,25 +459,31 @@ extern "C" int cgnet_CGBN_forward(const cgnet_layer_plan* plan, const float* d_F
     float* Wp = (float*)(ws + fa.wp);
     const bool pack_fwd = wmm->nO > 0 && !wmm->fwd_splits[0].units.empty();
     const int nb_fwd = pack_fwd ? (wmm->wp_blocks * 16 + 255) / 256 : 0;
-    const int nb_gen = save ? (plan->link.npack + 3) / 4 : 0;
-    const int nbF = save ? (int)(((size_t)cg->bwd_nFp * B + 255) / 256) : 0;
-    const int ntab = save ? cg->nllls : 0;
+    const bool save_pairs = save && backward_uses_pairs(plan, B);
+    const int nb_gen = save_pairs ? plan->link.ngens : 0;
+    const int nbF = save_pairs ? (int)(((size_t)cg->nF * B + 255) / 256) : 0;
+    const int ncoef = save_pairs ? cg->back.ncoefmap : 0;
     const int nb_std = save && bn ? (cg->sumT + 255) / 256 : 0;
-    if (nb_fwd + nb_gen + nbF + ntab + nb_std > 0) {
+    if (nb_fwd + nb_gen + nbF + ncoef + nb_std > 0) {
         char* sv = (char*)d_saved;
-        CGNET_LAUNCH(layer_prepare_kernel, dim3((unsigned)(nb_fwd + nb_gen + nbF + ntab + nb_std)), dim3(256), 0, s,
+        CGNET_LAUNCH(layer_prepare_kernel, dim3((unsigned)(nb_fwd + nb_gen + nbF + ncoef + nb_std)), dim3(256), 0, s,
                      (const float2*)d_W, bn ? d_stds : nullptr, eps, wmm->d_degs, ndeg, Wp, wmm->wp_blocks, nb_fwd,
-                     compact ? plan->wmm->d_degs : nullptr, compact ? plan->compact.d_cmap : nullptr, plan->link.d_gens, plan->link.d_packmap, plan->link.npack, save ? (float*)(sv + sa.Ag) : nullptr,
-                     nb_gen, (const float2*)d_F, d_CG, save ? (float2*)(sv + sa.Fp) : nullptr,
-                     save ? (float*)(sv + sa.CGP) : nullptr, cg->d_bwd_padmeta, cg->L, cg->nF, cg->bwd_nFp, B, nbF, ntab,
-                     save ? (float*)(sv + sa.stds) : nullptr, cg->sumT);
+                     compact ? plan->wmm->d_degs : nullptr, compact ? plan->compact.d_cmap : nullptr, plan->link.d_gens,
+                     save ? (float*)(sv + sa.Wb) : nullptr, nb_gen, (const float2*)d_F, save ? (float2*)(sv + sa.F) : nullptr,
+                     (size_t)cg->nF * B, nbF, d_CG, cg->back.d_pairs, cg->back.d_coefmap, ncoef, cg->back.grid0,
+                     save ? (float*)(sv + sa.coef) : nullptr, save ? (float*)(sv + sa.stds) : nullptr, cg->sumT);
         CGNET_HIP(hipGetLastError());
+    }
+    if (save && !save_pairs) {
+        char* sv = (char*)d_saved;
+        if (int rc = launch_pack_w_gen(plan->fused, d_W, bn ? d_stds : nullptr, eps, (float*)(sv + sa.Wb), s)) return rc;
+        if (int rc = launch_backward_pad(cg, d_F, d_CG, (float*)(sv + sa.F), (float*)(sv + sa.coef), B, s)) return rc;
     }
     return wmm_forward_packed(wmm, d_FF, d_O, Wp, B, ws + fa.opart, s);
 }
 
 extern "C" size_t cgnet_CGBN_backward_fused_workspace(const cgnet_layer_plan* plan, int B) {
-    if (!plan || B <= 0 || !plan->link.ok) return 0;
+    if (!plan || B <= 0 || !backward_ok(plan)) return 0;
     return backward_areas(plan, B).total;
 }
 
@@ -464,7 +496,7 @@ extern "C" int cgnet_CGBN_backward_fused(const cgnet_layer_plan* plan, const flo
     CGNET_REQUIRE(B >= 0, CGNET_ERR_ARG, "B=%d is negative", B);
     const cgnet_cg_plan* cg = plan->cg;
     if (B == 0 || cg->nF == 0) return CGNET_OK;
-    CGNET_REQUIRE(plan->link.ok, CGNET_ERR_UNSUPPORTED, "%s", plan->reason);
+    CGNET_REQUIRE(backward_ok(plan), CGNET_ERR_UNSUPPORTED, "%s", plan->reason);
     const bool bn = flags & CGNET_FN_BATCHNORM;
     CGNET_REQUIRE(d_gF && d_gO, CGNET_ERR_ARG, "null device pointer");
     const BwdFusedAreas ba = backward_areas(plan, B);
@@ -473,27 +505,43 @@ extern "C" int cgnet_CGBN_backward_fused(const cgnet_layer_plan* plan, const flo
     CGNET_REQUIRE(((uintptr_t)d_workspace & 15) == 0, CGNET_ERR_ARG, "workspace must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)d_workspace;
-    const float *Ag, *Fp, *CGP;
+    const bool pairs = backward_uses_pairs(plan, B);
+    const float *Wb, *F, *coef;
     if (d_saved) {
         const SavedAreas sa = saved_areas(plan, B);
         CGNET_REQUIRE(saved_bytes >= sa.total, CGNET_ERR_WORKSPACE, "saved-operand area of %zu bytes given, %zu needed",
                       saved_bytes, sa.total);
         CGNET_REQUIRE(((uintptr_t)d_saved & 15) == 0, CGNET_ERR_ARG, "the saved-operand area must be 16-byte aligned");
         const char* sv = (const char*)d_saved;
-        Ag = (const float*)(sv + sa.Ag);
-        Fp = (const float*)(sv + sa.Fp);
-        CGP = (const float*)(sv + sa.CGP);
+        Wb = (const float*)(sv + sa.Wb);
+        F = (const float*)(sv + sa.F);
+        coef = (const float*)(sv + sa.coef);
     } else {
         CGNET_REQUIRE(!bn || d_stds, CGNET_ERR_ARG, "batch-norm flag set but d_stds is NULL");
         CGNET_REQUIRE(d_F && d_W && d_CG, CGNET_ERR_ARG, "null device pointer");
-        if (int rc = launch_pack_w_gen(plan->link, d_W, bn ? d_stds : nullptr, eps, (float*)(ws + ba.Ag), s)) return rc;
-        if (int rc = launch_backward_pad(cg, d_F, d_CG, (float*)(ws + ba.own.Fp), (float*)(ws + ba.own.CGP), B, s)) return rc;
-        Ag = (const float*)(ws + ba.Ag);
-        Fp = (const float*)(ws + ba.own.Fp);
-        CGP = (const float*)(ws + ba.own.CGP);
+        float* own_Wb = (float*)(ws + ba.Wb);
+        Wb = own_Wb;
+        if (pairs) {
+            if (int rc = launch_pack_w_back(plan->link, d_W, bn ? d_stds : nullptr, eps, own_Wb, s)) return rc;
+            if (int rc = launch_pack_coef_back(cg->back, d_CG, (float*)(ws + ba.coef), s)) return rc;
+            F = d_F;
+            coef = (const float*)(ws + ba.coef);
+        } else {
+            float *Fp = (float*)(ws + ba.own.Fp), *CGP = (float*)(ws + ba.own.CGP);
+            if (int rc = launch_pack_w_gen(plan->fused, d_W, bn ? d_stds : nullptr, eps, own_Wb, s)) return rc;
+            if (int rc = launch_backward_pad(cg, d_F, d_CG, Fp, CGP, B, s)) return rc;
+            F = Fp;
+            coef = CGP;
+        }
     }
-    return launch_fused_backward(cg, plan->link, d_gO, Ag, Fp, CGP, (float*)(ws + ba.Bg), (float*)(ws + ba.own.part1),
-                                 (float*)(ws + ba.own.part2), d_gF, B, s);
+    if (!pairs)
+        return launch_fused_backward(cg, plan->fused, d_gO, Wb, F, coef, (float*)(ws + ba.Go), (float*)(ws + ba.own.part1),
+                                     (float*)(ws + ba.own.part2), d_gF, B, s);
+    const BackLevel& lv = back_level(cg->back, B);
+    if (int rc = launch_back_layer(cg->back, plan->link, lv, F, d_gO, Wb, coef, (float*)(ws + ba.Go), (float*)(ws + ba.part),
+                                   cg->nF, B, s))
+        return rc;
+    return launch_back_combine(lv, (const float*)(ws + ba.part), d_gF, cg->L, cg->nF, B, s);
 }
 
 // ---- compact product tensor: sizes, weight gradient --------------------------------------------------

@@ -178,8 +178,8 @@ typedef struct cgnet_layer_plan cgnet_layer_plan;
 int cgnet_layer_plan_create(cgnet_layer_plan** plan, const cgnet_cg_plan* cg_plan, const cgnet_wmm_plan* wmm_plan);
 int cgnet_layer_plan_destroy(cgnet_layer_plan* plan);
 
-/* 1 if cgnet_CGBN_backward_fused takes this layer (every input channel count in 8..16, lmax <= 23, t_O <= 16,
- * LDS within limits), else 0; cgnet_CGBN_backward_fused_reason then names what is missing. */
+/* 1 if cgnet_CGBN_backward_fused takes this layer (at most 16 channels in every input degree, lmax <= 23,
+ * t_O <= 16), else 0; cgnet_CGBN_backward_fused_reason then names what is missing. */
 int cgnet_CGBN_backward_fused_supported(const cgnet_layer_plan* plan);
 const char* cgnet_CGBN_backward_fused_reason(const cgnet_layer_plan* plan);
 
@@ -187,8 +187,8 @@ const char* cgnet_CGBN_backward_fused_reason(const cgnet_layer_plan* plan);
  * cgnet_FN_WMM_forward(d_sums = ...), same arithmetic and same results bit for bit, in fewer launches: the
  * statistics are reduced and the running stds updated in one kernel, and one further kernel packs the weights of
  * the mixing and -- when d_saved is given -- the three operands cgnet_CGBN_backward_fused would otherwise build
- * itself (packed W / max(eps, stds) per task, F with a zero behind every row, the tables between zero rows), all of
- * which depend only on what the forward already holds.  d_FF (B x nFF complex) is written as by
+ * itself (packed W / max(eps, stds), the fragments, the packed coefficients), all of which depend only on what the
+ * forward already holds.  d_FF (B x nFF complex) is written as by
  * cgnet_sparse_forward: the weight gradient needs it.  d_saved: cgnet_CGBN_saved_bytes(plan, B) bytes, 16-byte
  * aligned, or NULL (inference; also when the fused backward is not supported, where the size is 0).
  * d_stds / cnt / eps / flags as in cgnet_FN_WMM_forward. */
