@@ -439,6 +439,18 @@ class _CGBN_fused(torch.autograd.Function):
         return grad_F, grad_W, None, None, None, None, None, None, None, None
 
 
+_GLOBAL_HOOKS = [getattr(nn.modules.module, name) for name in
+                 ("_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks", "_global_backward_pre_hooks")]
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+
+
+def plain_call(layer):
+    """Whether calling ``layer`` runs ``CGBN_cuda.forward`` and nothing that sees its arguments or its result."""
+    d = layer.__dict__
+    return (type(layer) is CGBN_cuda and CGBN_cuda.forward is _CGBN_FORWARD and "forward" not in d
+            and not any(d.get(name) for name in _HOOKS) and not any(_GLOBAL_HOOKS))
+
+
 class CGBN_cuda(nn.Module):
     def __init__(self, lmax, taus_fs, tau_out, batchnorm=True, sparse_flag=False, device='cuda',
                  weight_scale=0.05, init='random', eps=1e-5):
@@ -498,3 +510,6 @@ class CGBN_cuda(nn.Module):
         if not straight_output:
             new_fs = CGutils.reshape_out(new_fs, self.tau_out)
         return new_fs
+
+
+_CGBN_FORWARD = CGBN_cuda.forward
