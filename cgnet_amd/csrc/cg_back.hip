@@ -1,9 +1,9 @@
 // Backward of the Clebsch-Gordan product organised by pairs of input degrees: plans, packing kernels and launches.  The kernel
 // and what it does: cg_back_kernel.h.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
-#include <map>
 #include <memory>
 #include <numeric>
 
@@ -132,11 +132,15 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
     for (int t : t_F)
         if (t > kBackMaxTau) return CGNET_OK;
     // triples by pair, largest output degree first; the n-th repetition of a triple goes into a list of its own
-    std::map<std::vector<int>, std::vector<const PairTriple*>> lists;          // (l1, l2, repetition)
-    std::map<std::vector<int>, int> seen;
-    for (const PairTriple& t : triples)
-        if (t_F[t.l1] > 0 && t_F[t.l2] > 0) lists[{t.l1, t.l2, seen[{t.l1, t.l2, t.l}]++}].push_back(&t);
-    if (lists.empty()) return CGNET_OK;
+    std::vector<std::array<int, 5>> order;                                     // l1, l2, repetition, -l, triple
+    for (size_t k = 0; k < triples.size(); ++k)
+        if (t_F[triples[k].l1] > 0 && t_F[triples[k].l2] > 0) order.push_back({triples[k].l1, triples[k].l2, 0, -triples[k].l, (int)k});
+    if (order.empty()) return CGNET_OK;
+    std::sort(order.begin(), order.end());
+    for (size_t k = 1; k < order.size(); ++k)
+        if (order[k][0] == order[k - 1][0] && order[k][1] == order[k - 1][1] && order[k][3] == order[k - 1][3])
+            order[k][2] = order[k - 1][2] + 1;
+    std::sort(order.begin(), order.end());
     // The grid of chunks: of the eight places of its origin the one with the fewest chunks in all.
     int best = -1;
     for (int shift = 0; shift < 8; ++shift) {
@@ -152,13 +156,13 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
     std::vector<double> tile_cost;
     std::vector<int2> coefmap;
     size_t coef = 0, lds = 0;
-    for (auto& entry : lists) {
-        std::vector<const PairTriple*>& ts = entry.second;
-        std::stable_sort(ts.begin(), ts.end(), [](const PairTriple* x, const PairTriple* y) { return x->l > y->l; });
+    for (size_t from = 0, to; from < order.size(); from = to) {
+        to = from + 1;
+        while (to < order.size() && std::equal(order[to].begin(), order[to].begin() + 3, order[from].begin())) ++to;
         BackPair p{};
-        p.l1 = entry.first[0]; p.l2 = entry.first[1];
+        p.l1 = order[from][0]; p.l2 = order[from][1];
         p.tau1 = t_F[p.l1]; p.tau2 = t_F[p.l2];
-        p.nl = (int)ts.size();
+        p.nl = (int)(to - from);
         p.nks = (p.nl + 3) / 4;
         p.nt = (2 * p.l2 + 1 + 15) / 16;
         // Whole rows t1 in a tile, or sixteen columns wherever they begin, where that makes fewer tiles (tau2 = 12: nine for 144
@@ -176,15 +180,16 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         p.inv_tau2 = (65536 + p.tau2 - 1) / p.tau2;
         p.inv_M1 = ((1 << 20) + 2 * p.l1) / (2 * p.l1 + 1);
         p.inv_M2 = ((1 << 20) + 2 * p.l2) / (2 * p.l2 + 1);
-        const int lm = ts[0]->l;
+        const int lm = -order[from][3];
         p.c0 = (-lm - out->grid0) / 8;
         p.nch = (lm - out->grid0) / 8 - p.c0 + 1;
         p.offF1 = cumF[p.l1]; p.offF2 = cumF[p.l2];
         p.coef = (int)coef;
         for (int q = 0; q < p.nl; ++q) {
-            p.l[q] = ts[q]->l;
-            p.cg[q] = ts[q]->cg;
-            p.offFF[q] = ts[q]->offFF;
+            const PairTriple& t = triples[order[from + q][4]];
+            p.l[q] = t.l;
+            p.cg[q] = t.cg;
+            p.offFF[q] = t.offFF;
             if (p.offFF[q] == 0) p.ends |= 1;
             if (p.offFF[q] + p.tau1 * p.tau2 * (2 * p.l[q] + 1) == nFF) p.ends |= 2;
         }
@@ -230,7 +235,7 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         lv.most_units = n;
         const double target = n == 1 << 30 ? 0. : all / n;
         std::vector<std::pair<double, BackUnit>> units;
-        std::vector<std::vector<int>> rows(cum_rows[L + 1]);        // per row (degree, channel): where its shares lie
+        std::vector<int2> shares;                                   // (row of a degree, where a share of it lies)
         int at = 0;
         for (size_t k = 0; k < out->pairs.size(); ++k) {
             const BackPair& p = out->pairs[k];
@@ -244,11 +249,11 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
                     for (int t = 0; t < n; ++t) {
                         const int c0 = (u.tile0 + t * p.tstep) * p.ncol, c1 = std::min(p.tau1 * p.tau2, c0 + p.ncol);
                         for (int r = c0 / p.tau2; r <= (c1 - 1) / p.tau2; ++r)
-                            rows[cum_rows[p.l1] + r].push_back(at + (t * p.nrows + r - c0 / p.tau2) * M1);
+                            shares.push_back(make_int2(cum_rows[p.l1] + r, at + (t * p.nrows + r - c0 / p.tau2) * M1));
                     }
                     at += n * p.nrows * M1;
                     u.p2off = at;
-                    for (int r = 0; r < p.tau2; ++r) rows[cum_rows[p.l2] + r].push_back(at + r * M2);
+                    for (int r = 0; r < p.tau2; ++r) shares.push_back(make_int2(cum_rows[p.l2] + r, at + r * M2));
                     at += p.tau2 * M2;
                     units.push_back({tile_cost[k] * n, u});
                 }
@@ -260,10 +265,13 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         // meta of cg_backward_rows_kernel: [L+2] cumF | [L+2] first row of a degree | [rows + 1] list begin | offsets
         std::vector<int> meta(cumF.begin(), cumF.end());
         meta.insert(meta.end(), cum_rows.begin(), cum_rows.end());
-        int run = 0;
-        for (const auto& r : rows) { meta.push_back(run); run += (int)r.size(); }
-        meta.push_back(run);
-        for (const auto& r : rows) meta.insert(meta.end(), r.begin(), r.end());
+        const size_t head = meta.size(), nrows = cum_rows[L + 1];
+        meta.resize(head + nrows + 1 + shares.size());
+        int* begin = meta.data() + head;                            // (counted one place on, then summed)
+        for (const int2& x : shares) ++begin[x.x + 1];
+        for (size_t r = 0; r < nrows; ++r) begin[r + 1] += begin[r];
+        std::vector<int> next(begin, begin + nrows);
+        for (const int2& x : shares) begin[nrows + 1 + next[x.x]++] = x.y;
         bool finest = true;
         for (const BackUnit& u : lv.units) finest &= u.ntiles == 1;
         out->levels.push_back(lv);
