@@ -10,13 +10,13 @@ struct PairTriple;
 
 constexpr int kBackMaxL = 23;      // 2L+1 <= 48 rows: three row tiles of sixteen values of m2
 constexpr int kBackMaxTau = 16;    // channels of degree l2: the columns of a tile
-constexpr int kBackNL = 24;        // output degrees of a pair, in groups of four
+constexpr int kBackNL = 16;        // output degrees of a pair, in groups of four
 constexpr int kBackChunks = 6;     // chunks of eight values of M = m1 + m2
 constexpr int kBackWaves = 4;      // waves of a work-group: samples of the same unit
 constexpr int kBackMaxRows = 8;    // rows t1 of a tile at most (their fragments are staged twice)
 
-// A pair (l1, l2) with its output degrees, largest first.  Its tau1 x tau2 channels (t1, t2) are cut into tiles of ncol columns; the
-// tiles of a unit lie tstep apart, so that a column has the same t2 in all of them.
+// A pair (l1, l2) with its output degrees, largest first (at most kBackNL: more make a pair of their own).  Its tau1 x tau2 channels
+// (t1, t2) are cut into tiles of ncol columns; the tiles of a unit lie tstep apart, so that a column has the same t2 in all of them.
 struct BackPair {
     int l1, l2, tau1, tau2;
     int nl, nks;                   // output degrees, groups of four

@@ -77,6 +77,12 @@ pack_w_back_kernel(const float2* __restrict__ W, const float* __restrict__ stds,
 
 constexpr int kVariants = 4;                       // kernel variants, by the largest degree
 constexpr int kVariantL[kVariants] = {7, 11, 15, kBackMaxL};
+// Groups of four output degrees: the smallest number that holds all of a pair, up to lmax 15.  Above it that took 256 registers, 177
+// of them spilled, at six groups; a pair of more than sixteen degrees is cut, its smaller ones make a pair of their own that spans few M
+// (layer, lmax 20, 16 channels, B = 32: 2.39 -> 2.18 ms, five groups 2.28, three 2.27; from memory at B = 16: 1.54 -> 1.14 ms).  Where
+// all fit, cutting only repeats the vector half (lmax 11, 12 channels, B = 100: 424 us, cut at two groups 452; lmax 15, 16 channels,
+// B = 64: 1.52 ms, cut at three groups 1.64).
+constexpr int kVariantKS[kVariants] = {2, 3, 4, 4};
 
 const void* variant_kernel(int v, int pairs) {
     return v == 0 ? back_kernel_0(pairs) : v == 1 ? back_kernel_1(pairs) : v == 2 ? back_kernel_2(pairs) : back_kernel_3(pairs);
@@ -153,12 +159,13 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
     out->nchunks = (L - out->grid0) / 8 + 1;
     for (int v = kVariants - 1; v >= 0; --v)
         if (L <= kVariantL[v]) out->variant = v;
+    const size_t most = 4 * kVariantKS[out->variant];                          // output degrees of a pair
     std::vector<double> tile_cost;
     std::vector<int2> coefmap;
     size_t coef = 0, lds = 0;
     for (size_t from = 0, to; from < order.size(); from = to) {
         to = from + 1;
-        while (to < order.size() && std::equal(order[to].begin(), order[to].begin() + 3, order[from].begin())) ++to;
+        while (to < order.size() && to - from < most && std::equal(order[to].begin(), order[to].begin() + 3, order[from].begin())) ++to;
         BackPair p{};
         p.l1 = order[from][0]; p.l2 = order[from][1];
         p.tau1 = t_F[p.l1]; p.tau2 = t_F[p.l2];
@@ -221,7 +228,7 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         out->pairs.push_back(p);
     }
     CGNET_REQUIRE(coef < (1u << 30), CGNET_ERR_UNSUPPORTED, "packed coefficients of the backward exceed 2^30 floats");
-    out->coef_floats = coef + 64 * 6 * 3;          // a chunk's last reads may run past its own groups
+    out->coef_floats = coef + 64 * 4 * 3;          // a chunk's last reads may run past its own groups
     out->ncoefmap = (int)coefmap.size();
     out->lds = 4 * lds * kBackWaves;
     // levels: pieces of at most 1 / n of a sample's work

@@ -29,7 +29,7 @@
 // lane and half of that to 8 bytes, and out of L2, for which the work-groups of a sample stay on one XCD.  Adding the sums in LDS with
 // ds_add_f32 is no alternative to read and write: 18 times slower (measured alone).
 // Against the kernels that work triple by triple (whole input gradient, us): lmax 11, 12 channels, B = 100, layer 561 -> 450; lmax 20,
-// 16 channels, B = 32, layer 3960 -> 2440; lmax 15, 16 channels, B = 64, stand-alone 1760 -> 1420; lmax 10, 4 channels, B = 100,
+// 16 channels, B = 32, layer 3960 -> 2290; lmax 15, 16 channels, B = 64, stand-alone 1760 -> 1420; lmax 10, 4 channels, B = 100,
 // stand-alone 116 -> 66, layer (two kernels before) 155 -> 66.
 #pragma once
 #include <utility>
@@ -352,7 +352,7 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
         // memory source: a lane past the last channel repeats the last row's of its t2
         if constexpr (PAIRS == 0) w.chan = min(t1, p->tau1 - 1) * tau2 + (t1 < p->tau1 ? c0 + jj - t1 * tau2 : t2);
         // all loads of a chunk go out during the one before it where there are registers for them
-        constexpr bool AHEAD = PAIRS == 0 && KS <= 4;
+        constexpr bool AHEAD = PAIRS == 0 && KS + NT <= 6;
         const bool ends = (p->ends & 1 && c0 == 0) || (p->ends & 2 && c0 + ncol == C);
         f32x4 next[KS][4];
         if constexpr (AHEAD) {
@@ -361,7 +361,6 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
         w.cp = a.coef + p->coef;
         for (int c = 0; c < p->nch; ++c) {
             const int steps8 = p->steps[c], tiles8 = p->tiles[c], nd = p->degs[c];
-            constexpr int K1 = KS <= 4 ? 1 : 2, K2 = KS <= 4 ? 2 : 4;
             const int Mc = M0 + 8 * c, c1 = min(c + 1, p->nch - 1), next_M0 = M0 + 8 * c1, next_nd = p->degs[c1];
             if constexpr (PAIRS > 0) {
                 back_make<PAIRS, KS>(w, p->c0 + c, nd, G);
@@ -373,8 +372,8 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
                 if (ends) mem_ends<KS>(w, Mc, nd, G);
             }
             turn_all<KS>(nd, G);
-            if (nd <= 4 * K1) back_chunk<KS, NT, K1, AHEAD>(w, A, G, steps8, tiles8, next, next_M0, next_nd);
-            else if (KS == K2 || nd <= 4 * K2) back_chunk<KS, NT, K2, AHEAD>(w, A, G, steps8, tiles8, next, next_M0, next_nd);
+            if (nd <= 4) back_chunk<KS, NT, 1, AHEAD>(w, A, G, steps8, tiles8, next, next_M0, next_nd);
+            else if (KS == 2 || nd <= 8) back_chunk<KS, NT, 2, AHEAD>(w, A, G, steps8, tiles8, next, next_M0, next_nd);
             else back_chunk<KS, NT, KS, AHEAD>(w, A, G, steps8, tiles8, next, next_M0, next_nd);
         }
         // the three sums that have not seen their last row
@@ -430,7 +429,7 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
 }
 
 template <int KS, int NTMAX, int PAIRS>
-__global__ void __launch_bounds__(kBackThreads, PAIRS == 0 ? (NTMAX == 1 ? 3 : 2) : NTMAX == 1 ? 4 : KS <= 3 ? 3 : 2)
+__global__ void __launch_bounds__(kBackThreads, PAIRS == 0 ? (NTMAX == 1 ? 3 : 2) : NTMAX == 1 ? 4 : KS + NTMAX <= 5 ? 3 : 2)
 cg_backward_pair_kernel(BackArgs a) {
     extern __shared__ __align__(16) float back_lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;

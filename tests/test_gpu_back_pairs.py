@@ -23,8 +23,8 @@ CASES = [
     (11, [12] * 12, 2, "default"),
     (13, [1] * 13 + [15], 7, "mst"),
     (15, [4, 16] * 8, 2, "default"),                                  # 31 values of m2, sixteen output degrees
-    (16, [1, 2] * 8 + [3], 2, "default"),                             # 33: three row tiles, one row in the third
-    (20, [2] * 21, 1, "default"),                                     # 21 output degrees: six groups
+    (16, [1, 2] * 8 + [3], 2, "default"),                             # 33: three row tiles, one row in the third; 17 degrees: cut, 16 and 1
+    (20, [2] * 21, 1, "default"),                                     # 21 output degrees: cut, 16 and 5
     (23, [1, 2, 1] * 8, 3, "edge"),
     (3, [2, 3, 1, 2], 13, [[(1, 1)], [(1, 1), (2, 1), (2, 1)], [(2, 2), (2, 2), (3, 1)], [(3, 0)]]),   # kept twice
 ]
@@ -87,6 +87,7 @@ def test_non_finite_gradients_stay_in_their_sample(dev, lmax, taus, bsz, mode): 
     (6, [3, 0, 16, 1, 9, 2, 4], [1, 5, 0, 16, 2, 3, 8], 6, True),     # no inputs, no outputs
     (9, [1] * 10, [4] * 10, 1, False),
     (16, [1] * 17, [2] * 17, 2, True),
+    (20, [1] * 21, [1] * 21, 2, False),                               # pairs of up to 21 output degrees, cut after sixteen
 ])
 def test_layer_backward_of_few_channels(dev, monkeypatch, lmax, tin, tout, bsz, sparse):  # noqa: F811
     """The one-kernel backward makes the product's gradient in the order of the gFF kernel and goes on as the stand-alone
