@@ -52,7 +52,7 @@ def profiled_traffic():
     table, rev = {}, "unknown revision"
     try:
         for line in open(path):
-            m = re.match(r"^(\w+)(?:<\d+>)?\s+([\d.]+) MB\s+([\d.]+) MB\s+([\d.]+) MB\s+([\d.]+) MB\s+[\d.]+\s*$", line)
+            m = re.match(r"^(\w+)(?:<[\d,]+>)?\s+([\d.]+) MB\s+([\d.]+) MB\s+([\d.]+) MB\s+([\d.]+) MB\s+[\d.]+\s*$", line)
             if m:
                 table[m.group(1)] = float(m.group(4)) * 1e6
             m = re.match(r"^source revision:\s*(\S+)", line)
@@ -216,7 +216,7 @@ def main():
     lib.cgnet_profile_reset()
     candidates = ("cg_forward_kernel", "cg_forward_mm_kernel", "wmm_forward_kernel", "wmm_gradw_kernel",
                   "wmm_gradff_mfma_kernel", "wmm_gradff_kernel", "cg_backward_unit_kernel", "cg_backward_hybrid_kernel",
-                  "cg_backward_kernel", "cgbn_backward_fused_kernel")
+                  "cg_backward_kernel", "cg_backward_pair_kernel", "cgbn_backward_fused_kernel")
     dominant = max((n for n in survey if n in candidates), key=lambda n: survey[n][0])
     lib.cgnet_profile_select(dominant.encode())
     lib.cgnet_profile_enable(1)
@@ -249,9 +249,10 @@ def main():
         "cg_backward_hybrid_kernel": 8 * (bsz * n_ff + 2 * bsz * n_f),
         "cg_backward_kernel": 8 * (bsz * n_ff + 2 * bsz * n_f),
     }
-    # the one-kernel layer backward stands for two of the five passes (grad FF written, grad FF read); it is priced
+    # the one-kernel layer backward (by pairs of input degrees, or triple by triple) stands for two of the five passes (grad FF written, grad FF read); it is priced
     # against the bytes those passes would move although it moves neither (what it really moves: `traffic`)
     algo["cgbn_backward_fused_kernel"] = algo["wmm_gradff_mfma_kernel"] + algo["cg_backward_hybrid_kernel"]
+    algo["cg_backward_pair_kernel"] = algo["cgbn_backward_fused_kernel"] if layer.fused_backward else algo["cg_backward_hybrid_kernel"]
     measured_traffic, traffic_source = profiled_traffic()
     step_bytes = 8 * (5 * bsz * n_ff + bsz * (3 * n_f + 3 * n_o) + 3 * n_w) + 4 * (2 * sum_t + cg_len)
     kernels = {}

@@ -23,7 +23,7 @@
 // same values to the bit.
 //
 // Bounded by issue where enough waves run: a vector multiply-add holds a SIMD for four cycles, a matrix instruction for 32, and the two
-// take turns.  lmax 11, 12 channels, B = 100, inside the layer: 9.7e7 vector and 1.1e7 matrix instructions, 84 % of the cycles of
+// take turns.  lmax 11, 12 channels, B = 100, inside the layer: 8.6e7 vector and 1.1e7 matrix instructions, 75 % of the cycles of
 // 1024 SIMDs; three waves a SIMD (168 registers; from lmax 12 on two, 256).  Without the loads of packed gO and weights it takes
 // 345 us, without the vector half 414 of then 494: the loads come out of L1, which gives 64 bytes a cycle to loads of 4 or 16 bytes a
 // lane and half of that to 8 bytes, and out of L2, for which the work-groups of a sample stay on one XCD.  Adding the sums in LDS with
