@@ -42,7 +42,7 @@ struct BackUnit { int pair, tile0, ntiles, p1off, p2off; };
 
 // A cut of all pairs into units for a range of batch sizes.
 struct BackLevel {
-    int most_units = 0;            // taken while this many units (or fewer) are wanted for one sample
+    int least_B = 1;               // taken from this batch on (levels from coarse to fine, the last from one sample on)
     std::vector<BackUnit> units;   // longest first
     BackUnit* d_units = nullptr;
     int* d_combine = nullptr;      // meta of cg_backward_rows_kernel

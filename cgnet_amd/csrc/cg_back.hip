@@ -105,10 +105,8 @@ int launch_back(const BackSet& set, const BackLevel& lv, int pairs, BackArgs a, 
 }  // namespace
 
 const BackLevel& back_level(const BackSet& set, int B) {
-    // units wanted of a sample: enough waves that the longest of them is a small part of the call
-    const int want = (5120 + B - 1) / std::max(1, B);
     for (const BackLevel& lv : set.levels)
-        if (want <= lv.most_units) return lv;
+        if (B >= lv.least_B) return lv;
     return set.levels.back();
 }
 
@@ -231,7 +229,8 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
     out->coef_floats = coef + 64 * 4 * 3;          // a chunk's last reads may run past its own groups
     out->ncoefmap = (int)coefmap.size();
     out->lds = 4 * lds * kBackWaves;
-    // levels: pieces of at most 1 / n of a sample's work
+    // levels: pieces of at most 1 / n of a sample's work, for batches that make about 5120 units of them: enough waves that the longest
+    // is a small part of the call
     double all = 0;
     for (size_t k = 0; k < tile_cost.size(); ++k) all += tile_cost[k] * out->pairs[k].ntiles;
     std::vector<int> cum_rows(L + 2, 0);
@@ -239,7 +238,7 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
     std::vector<std::vector<int>> combine;
     for (const int n : {64, 256, 1 << 30}) {
         BackLevel lv;
-        lv.most_units = n;
+        lv.least_B = n == 1 << 30 ? 1 : (5120 + n - 1) / n;
         const double target = n == 1 << 30 ? 0. : all / n;
         std::vector<std::pair<double, BackUnit>> units;
         std::vector<int2> shares;                                   // (row of a degree, where a share of it lies)
@@ -283,7 +282,10 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         for (const BackUnit& u : lv.units) finest &= u.ntiles == 1;
         out->levels.push_back(lv);
         combine.push_back(meta);
-        if (finest) break;
+        if (finest) {
+            out->levels.back().least_B = 1;
+            break;
+        }
     }
     // everything in one allocation, filled by one copy
     size_t bytes = 0;

@@ -2739,8 +2739,7 @@ extern "C" int cgnet_sparse_forward_stats_static(const cgnet_cg_plan* plan, cons
     return CGNET_OK;
 }
 
-extern "C" size_t cgnet_sparse_backward_workspace(const cgnet_cg_plan* plan, int B) {
-    if (!plan || B <= 0) return 0;
+static size_t backward_bytes(const cgnet_cg_plan* plan, int B) {
     if (cg_backward_uses_pairs(plan, B))
         return align_up(sizeof(float) * 2 * (size_t)back_level(plan->back, B).P * B, 256) +
                align_up(sizeof(float) * plan->back.coef_floats, 256);
@@ -2752,6 +2751,11 @@ extern "C" size_t cgnet_sparse_backward_workspace(const cgnet_cg_plan* plan, int
     const int ng = bwd_groups_for(plan, B);
     if (ng <= 1) return 0;
     return align_up(sizeof(float) * 2 * (size_t)plan->nF * B * ng, 256);
+}
+
+extern "C" size_t cgnet_sparse_backward_workspace(const cgnet_cg_plan* plan, int B) {
+    if (!plan || B <= 0) return 0;
+    return back_bytes_up_to(plan->back, plan->back_most_B, B, [&](int b) { return backward_bytes(plan, b); });
 }
 
 extern "C" int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F, float* d_gF,
@@ -2775,7 +2779,7 @@ extern "C" int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F
     }
     CGNET_REQUIRE(d_F && d_gFF && d_CG, CGNET_ERR_ARG, "null device pointer");
     const int ng = bwd_groups_for(plan, B);
-    const size_t need = cgnet_sparse_backward_workspace(plan, B);
+    const size_t need = backward_bytes(plan, B);
     CGNET_REQUIRE(need == 0 || (d_workspace && workspace_bytes >= need), CGNET_ERR_WORKSPACE,
                   "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
     if (cg_backward_uses_pairs(plan, B)) {

@@ -1,5 +1,7 @@
 // Host-side functions the translation units of libcgnet_hip call in each other (not part of the C ABI).
 #pragma once
+#include <algorithm>
+
 #include "common.h"
 #include "cg_plan.h"
 #include "wmm_plan.h"
@@ -50,6 +52,19 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
                    BackSet* out);
 void free_back_set(BackSet* set);
 const BackLevel& back_level(const BackSet& set, int B);              // the cut for a batch of B samples
+// Bytes that serve a batch of B samples and every smaller one, from bytes(b), those of b samples alone.  A smaller batch may take a
+// finer cut (more partial gradients a sample) or, up to most_B samples, go by pairs where this one does not: in between bytes(b)
+// grows with b.
+template <typename Bytes>
+size_t back_bytes_up_to(const BackSet& set, int most_B, int B, Bytes&& bytes) {
+    size_t most = bytes(B);
+    auto look = [&](int b) { if (b >= 1 && b < B) most = std::max(most, (size_t)bytes(b)); };
+    if (!set.ok()) return most;
+    look(most_B);
+    for (const BackLevel& lv : set.levels)
+        if (lv.least_B - 1 <= most_B) look(lv.least_B - 1);
+    return most;
+}
 // Largest batch the backward by pairs is taken for, against a kernel that works triple by triple: where a pair has few output
 // degrees, or rows and columns of its tiles are empty, the other spends fewer instructions, and large batches show it.
 // Measured over lmax 2..23, 1..16 channels (constant and falling with the degree), default and minimum-spanning-tree (MST)

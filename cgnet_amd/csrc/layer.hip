@@ -177,7 +177,9 @@ layer_prepare_kernel(const float2* __restrict__ W, const float* __restrict__ std
 }
 
 bool backward_ok(const cgnet_layer_plan* lp) { return lp->link.ok || lp->fused.ok; }
-bool backward_uses_pairs(const cgnet_layer_plan* lp, int B) { return lp->link.ok && (!lp->fused.ok || B <= lp->link.most_B); }
+// the largest batch that goes by pairs
+int most_by_pairs(const cgnet_layer_plan* lp) { return !lp->link.ok ? 0 : lp->fused.ok ? lp->link.most_B : INT32_MAX; }
+bool backward_uses_pairs(const cgnet_layer_plan* lp, int B) { return B <= most_by_pairs(lp); }
 
 // By pairs: packed weights, fragments, packed coefficients; by triples: packed weights, padded fragments, padded tables.
 struct SavedAreas { size_t stds, Wb, F, coef, total; };
@@ -392,7 +394,8 @@ extern "C" const char* cgnet_CGBN_backward_fused_reason(const cgnet_layer_plan* 
 }
 
 extern "C" size_t cgnet_CGBN_saved_bytes(const cgnet_layer_plan* plan, int B) {
-    return plan ? saved_areas(plan, B).total : 0;
+    if (!plan || B <= 0) return 0;
+    return back_bytes_up_to(plan->cg->back, most_by_pairs(plan), B, [&](int b) { return saved_areas(plan, b).total; });
 }
 
 extern "C" size_t cgnet_CGBN_saved_stds_bytes(const cgnet_layer_plan* plan, int B) {
@@ -484,7 +487,7 @@ extern "C" int cgnet_CGBN_forward(const cgnet_layer_plan* plan, const float* d_F
 
 extern "C" size_t cgnet_CGBN_backward_fused_workspace(const cgnet_layer_plan* plan, int B) {
     if (!plan || B <= 0 || !backward_ok(plan)) return 0;
-    return backward_areas(plan, B).total;
+    return back_bytes_up_to(plan->cg->back, most_by_pairs(plan), B, [&](int b) { return backward_areas(plan, b).total; });
 }
 
 extern "C" int cgnet_CGBN_backward_fused(const cgnet_layer_plan* plan, const float* d_F, float* d_gF, const float* d_gO,

@@ -1,0 +1,57 @@
+"""The backward goes by pairs of input degrees up to a batch, triple by triple above it, and cuts its work finer for small batches:
+what a caller sees of that besides the results."""
+import ctypes
+
+import pytest
+import torch
+
+from tests.test_gpu_parity import dev  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lmax,tau,sparse", [
+    (11, 12, False),                                       # by pairs throughout, three cuts
+    (20, 3, False),
+    (8, 12, True),                                         # pairs, then triples
+    (11, 5, True),
+    (15, 16, True),
+])
+def test_buffers_of_a_batch_serve_smaller_ones(dev, lmax, tau, sparse):  # noqa: F811
+    """A caller allocates for its full batch and passes a shorter last one: sizes never fall with the batch, and a call on a small
+    batch takes the buffers of a large one."""
+    from cgnet_amd import CG_layers, _lib
+    taus = [tau] * (lmax + 1)
+    mod = CG_layers.CGBN_cuda(lmax, taus, [2] * (lmax + 1), sparse_flag=sparse, device=dev)
+    lib, lp = _lib.load(), mod.native_layer_plan()
+    cg = lp.cg_plan
+    queries = {"backward": (lib.cgnet_sparse_backward_workspace, cg._h), "saved": (lib.cgnet_CGBN_saved_bytes, lp._h),
+               "layer backward": (lib.cgnet_CGBN_backward_fused_workspace, lp._h)}
+    batches = range(1, 260)
+    sizes = {name: [query(plan, b) for b in batches] for name, (query, plan) in queries.items()}
+    for name, got in sizes.items():
+        assert got[0] > 0 and got == sorted(got), name
+    big = {name: torch.empty(got[-1], dtype=torch.uint8, device=dev) for name, got in sizes.items()}
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    s = torch.cuda.current_stream(dev).cuda_stream
+    ffs = torch.empty(30, cg.nFF, 2, device=dev)
+    g = torch.Generator(device=dev).manual_seed(lmax)
+    for b in (1, 19, 30):
+        x, out = torch.randn(b, cg.nF, 2, generator=g, device=dev), torch.empty(b, lp.wmm_plan.nO, 2, device=dev)
+        go, gff = torch.randn(out.shape, generator=g, device=dev), torch.randn(b, cg.nFF, 2, generator=g, device=dev)
+        want, got = torch.empty_like(x), torch.empty_like(x)
+        cg.backward(x, want, gff, mod.cg.CGspace, b)
+        _lib.check(lib.cgnet_sparse_backward(cg._h, ptr(x), ptr(got), ptr(gff), ptr(mod.cg.CGspace), b, ptr(big["backward"]),
+                                             big["backward"].numel(), s))
+        assert torch.equal(got, want)
+        args = mod.bnWMM.W.detach(), mod.cg.CGspace, b, mod.bnWMM.bn_stds, 1., 1e-5, _lib.FN_BATCHNORM
+        own = lp.forward(x, ffs[:b], out, *args)
+        lp.backward_fused(x, want, go, mod.bnWMM.W.detach(), mod.cg.CGspace, b, mod.bnWMM.bn_stds, 1e-5, _lib.FN_BATCHNORM, own)
+        ws = torch.empty(lib.cgnet_CGBN_forward_workspace(lp._h, b), dtype=torch.uint8, device=dev)
+        _lib.check(lib.cgnet_CGBN_forward(lp._h, ptr(x), ptr(ffs), ptr(out), ptr(mod.bnWMM.W), ptr(mod.cg.CGspace), b,
+                                          ptr(mod.bnWMM.bn_stds), 1., 1e-5, _lib.FN_BATCHNORM, ptr(big["saved"]),
+                                          big["saved"].numel(), ptr(ws), ws.numel(), s))
+        _lib.check(lib.cgnet_CGBN_backward_fused(lp._h, None, ptr(got), ptr(go), None, None, b, None, 1e-5, _lib.FN_BATCHNORM,
+                                                 ptr(big["saved"]), big["saved"].numel(), ptr(big["layer backward"]),
+                                                 big["layer backward"].numel(), s))
+        assert torch.equal(got, want)
