@@ -120,7 +120,10 @@ int cgnet_sparse_forward_stats_static(const cgnet_cg_plan* plan, const float* d_
  *   gF[b,l1,t1,m1] = sum CG * gFF[b,l,t,m1+m2] * conj(F[b,l2,t2,m2])  + the same with the
  *   roles of the two slots exchanged (a diagonal triple l1 == l2 contributes through both).
  * Replaces CG_cuda_ops.sparse_backward (cudaCG_all.cpp:73-108; kernel cudaCG_sparse.cu:186-298).
- * Deterministic.  Every element of d_gF is written. */
+ * Deterministic.  Every element of d_gF is written.
+ * A workspace of cgnet_sparse_backward_workspace(plan, B) bytes serves every batch of up to B samples (a smaller one may
+ * need more than B samples alone do); the same holds for cgnet_CGBN_backward_fused_workspace and
+ * cgnet_CGBN_saved_bytes below. */
 size_t cgnet_sparse_backward_workspace(const cgnet_cg_plan* plan, int B);
 int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F, float* d_gF,
                           const float* d_gFF, const float* d_CG, int B,
