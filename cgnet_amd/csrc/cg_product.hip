@@ -2758,6 +2758,13 @@ extern "C" size_t cgnet_sparse_backward_workspace(const cgnet_cg_plan* plan, int
     return back_bytes_up_to(plan->back, plan->back_most_B, B, [&](int b) { return backward_bytes(plan, b); });
 }
 
+int cgnet::launch_zero_gradient(const cgnet_cg_plan* plan, float* d_gF, int B, hipStream_t s) {
+    const size_t nf = 2 * (size_t)plan->nF * B;
+    CGNET_LAUNCH(fill_zero_f32_kernel, dim3((unsigned)std::min<size_t>((nf + 255) / 256, 4096)), dim3(256), 0, s, d_gF, nf);
+    CGNET_HIP(hipGetLastError());
+    return CGNET_OK;
+}
+
 extern "C" int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F, float* d_gF,
                                      const float* d_gFF, const float* d_CG, int B, void* d_workspace,
                                      size_t workspace_bytes, void* stream) {
@@ -2772,10 +2779,7 @@ extern "C" int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F
     if (ng_max <= 0 || plan->bwd_tasks.empty()) {
         // no triple contributes: the gradient is zero (a fill kernel, not hipMemsetAsync: the call may be recorded
         // into a graph)
-        const size_t nf = 2 * (size_t)plan->nF * B;
-        CGNET_LAUNCH(fill_zero_f32_kernel, dim3((unsigned)std::min<size_t>((nf + 255) / 256, 4096)), dim3(256), 0, s, d_gF, nf);
-        CGNET_HIP(hipGetLastError());
-        return CGNET_OK;
+        return launch_zero_gradient(plan, d_gF, B, s);
     }
     CGNET_REQUIRE(d_F && d_gFF && d_CG, CGNET_ERR_ARG, "null device pointer");
     const int ng = bwd_groups_for(plan, B);

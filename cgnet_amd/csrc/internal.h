@@ -46,6 +46,8 @@ int launch_fused_backward(const cgnet_cg_plan* p, const FusedLink& link, const f
                           const float* d_Fp, const float* d_CGP, float* d_Bg, float* d_part1, float* d_part2,
                           float* d_gF, int B, hipStream_t s);
 
+int launch_zero_gradient(const cgnet_cg_plan* p, float* d_gF, int B, hipStream_t s);      // a fill kernel: may be recorded
+
 // ---- cg_back.hip: backward by pairs of input degrees
 // `triples`: every kept triple with its place in the product tensor.  Leaves the set empty where the shape is not taken.
 int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int>& t_F, const std::vector<int>& cumF, int L, int nFF,

@@ -501,7 +501,8 @@ extern "C" int cgnet_CGBN_backward_fused(const cgnet_layer_plan* plan, const flo
     if (B == 0 || cg->nF == 0) return CGNET_OK;
     CGNET_REQUIRE(backward_ok(plan), CGNET_ERR_UNSUPPORTED, "%s", plan->reason);
     const bool bn = flags & CGNET_FN_BATCHNORM;
-    CGNET_REQUIRE(d_gF && d_gO, CGNET_ERR_ARG, "null device pointer");
+    CGNET_REQUIRE(d_gF && (d_gO || plan->wmm->nO == 0), CGNET_ERR_ARG, "null device pointer");
+    if (plan->wmm->nO == 0) return launch_zero_gradient(cg, d_gF, B, (hipStream_t)stream);     // nothing comes out of the layer
     const BwdFusedAreas ba = backward_areas(plan, B);
     CGNET_REQUIRE(d_workspace && workspace_bytes >= ba.total, CGNET_ERR_WORKSPACE,
                   "workspace of %zu bytes given, %zu needed", workspace_bytes, ba.total);

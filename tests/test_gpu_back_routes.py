@@ -55,3 +55,15 @@ def test_buffers_of_a_batch_serve_smaller_ones(dev, lmax, tau, sparse):  # noqa:
                                                  ptr(big["saved"]), big["saved"].numel(), ptr(big["layer backward"]),
                                                  big["layer backward"].numel(), s))
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tau", [3, 9])
+def test_layer_without_outputs(dev, tau):  # noqa: F811
+    """No output channel in any degree: the output is empty (and lies nowhere), the gradients are zeros."""
+    from cgnet_amd import CG_layers
+    mod = CG_layers.CGBN_cuda(2, [tau] * 3, [0] * 3, device=dev)
+    x = torch.randn(4, tau * 9, 2, device=dev, requires_grad=True)
+    out = mod(x, straight_output=True)
+    assert out.shape == (4, 0, 2)
+    out.backward(torch.empty_like(out))
+    assert x.grad.shape == x.shape and not x.grad.any()
