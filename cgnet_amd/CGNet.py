@@ -44,13 +44,14 @@ class SphericalCNN(nn.Module):
             first = f_input[:, 0:int(self.taus[0][0]), :].reshape(B, -1)
         embedding = [first] if self.skipconn else []
         fs = f_input
-        for i, layer in enumerate(self.cgs):
-            # The fragments of a layer's output are views that only a hook or another class in its place can see; the next
-            # layer takes the straight tensor they are views of.  (Making and looking over 11 views a layer took 160 of 450 us
-            # of a five-layer classifier on one sample.)
-            if cglayers.plain_call(layer):
+        plain = [cglayers.plain_call(layer) for layer in self.cgs]
+        for layer, alone in zip(self.cgs, (a and b for a, b in zip(plain, plain[1:] + [True]))):
+            # The fragments of a layer's output are views that only a hook, or another class in the layer's or in the next one's
+            # place, can see; the next layer takes the straight tensor they are views of.  (Making and looking over 11 views a
+            # layer took 160 of 450 us of a five-layer classifier on one sample.)
+            if alone:
                 fs = layer(fs, straight_output=True)
-                first = fs[:, :int(self.taus[i + 1][0])]
+                first = fs[:, :int(layer.tau_out[0])]
             else:
                 fs = layer(fs, straight_output=False)
                 first = fs[0]

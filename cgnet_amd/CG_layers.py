@@ -445,9 +445,10 @@ _HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_
 
 
 def plain_call(layer):
-    """Whether calling ``layer`` runs ``CGBN_cuda.forward`` and nothing that sees its arguments or its result."""
+    """Whether calling ``layer`` runs ``CGBN_cuda.forward`` and nothing that sees its arguments or its result.  (Without ``fused``
+    the layer hands its arguments on to its product module.)"""
     d = layer.__dict__
-    return (type(layer) is CGBN_cuda and CGBN_cuda.forward is _CGBN_FORWARD and "forward" not in d
+    return (type(layer) is CGBN_cuda and layer.fused and CGBN_cuda.forward is _CGBN_FORWARD and "forward" not in d
             and not any(d.get(name) for name in _HOOKS) and not any(_GLOBAL_HOOKS))
 
 
