@@ -2262,10 +2262,12 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
     // CGNET_BWD_GENERAL=1 forces the LDS-accumulator kernel (kept for shapes the unit scheme cannot hold)
     const char* force_general = getenv("CGNET_BWD_GENERAL");
     const bool general = force_general && force_general[0] == '1';
+    // CGNET_BWD_PAIRS=0 leaves every batch to the kernels that work triple by triple
+    const char* by_pairs = getenv("CGNET_BWD_PAIRS");
     std::vector<PairTriple> triples(nllls);
     for (int i = 0; i < nllls; ++i)
         triples[i] = {tl[i], tl1[i], tl2[i], cgo[i], p->cumFF[tl[i]] + p->t_off[i] * (2 * tl[i] + 1), p->cumT[tl[i]] + p->t_off[i]};
-    if (!general) {
+    if (!general && !(by_pairs && by_pairs[0] == '0')) {
         if (int rc = build_back_set(triples, p->t_F, p->cumF, L, p->nFF, &p->back)) return rc;
         bool matrix = true;                          // the units would take slot 2 on the matrix cores
         for (int l = 0; l < n1; ++l) matrix &= h_t_F[l] == 0 || (h_t_F[l] >= 8 && h_t_F[l] <= 16);

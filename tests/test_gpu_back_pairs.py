@@ -1,6 +1,6 @@
 """The backward organised by pairs of input degrees (cg_backward_pair_kernel) where its pieces have edges: tiles of whole rows and
 of sixteen columns wherever they begin, a last tile that is short, one to three row tiles (and one row in the last), one to six
-chunks of values of m, one to six groups of output degrees, a triple kept twice, empty degrees, units cut for small batches, work-groups
+chunks of values of m, one to four groups of output degrees, a triple kept twice, empty degrees, units cut for small batches, work-groups
 with samples left over; both sources of the product's gradient; and the rule that chooses the kernel.  Against the oracle the
 tolerance of tests/test_gpu_parity.py: the strict bar, or three times what float32 arithmetic on the CPU is off by."""
 import pytest

@@ -5,6 +5,8 @@ import ctypes
 import pytest
 import torch
 
+from tests import test_gpu_parity as parity
+from tests.test_gpu_back_pairs import _kernels
 from tests.test_gpu_parity import dev  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +69,37 @@ def test_layer_without_outputs(dev, tau):  # noqa: F811
     assert out.shape == (4, 0, 2)
     out.backward(torch.empty_like(out))
     assert x.grad.shape == x.shape and not x.grad.any()
+
+
+# The kernels that work triple by triple serve the large batches of reduced triples; with CGNET_BWD_PAIRS=0 at plan creation they take
+# the small batches that the oracle can follow too.
+PRODUCTS = ([c for c in parity.CG_CASES if max(c[1]) <= 16] + parity._random_matrix_core_cases(12, 5) +
+            parity._random_matrix_core_cases_high(6, 9) + [c for c in parity._random_cg_cases(24, 11) if max(c[1]) <= 16] +
+            [(13, [16] * 14, 2, "mst"), (20, [9] * 21, 1, "mst"), (18, [8, 13, 16] * 6 + [10], 1, "mst"), (20, [3] * 21, 2, "mst")])
+
+
+@pytest.mark.parametrize("lmax,taus,bsz,mode", PRODUCTS)
+def test_product_triple_by_triple(dev, monkeypatch, lmax, taus, bsz, mode):  # noqa: F811
+    """Ragged channels, row blocks cut by the LDS, partial last steps, one to three column tiles, empty degrees, against the oracle."""
+    monkeypatch.setenv("CGNET_BWD_PAIRS", "0")
+    names = _kernels(lambda: parity.test_cg_forward_backward(dev, lmax, taus, bsz, mode))
+    matrix = all(t == 0 or 8 <= t <= 16 for t in taus)
+    backward = {n for n in names if n in ("cg_backward_hybrid_kernel", "cg_backward_unit_kernel", "cg_backward_pair_kernel")}
+    assert backward == {"cg_backward_hybrid_kernel" if matrix else "cg_backward_unit_kernel"}, names
+
+
+@pytest.mark.parametrize("lmax,tin,tout,bsz,sparse,bn", parity.LAYER_CASES)
+def test_layer_triple_by_triple(dev, monkeypatch, lmax, tin, tout, bsz, sparse, bn):  # noqa: F811
+    monkeypatch.setenv("CGNET_BWD_PAIRS", "0")
+    names = _kernels(lambda: parity.test_layer_forward_backward(dev, lmax, tin, tout, bsz, sparse, bn, "fused_backward"))
+    one = all(t == 0 or 8 <= t <= 16 for t in tin) and max(tout) <= 16
+    assert "cg_backward_pair_kernel" not in names and ("cgbn_backward_fused_kernel" in names) == one, names
+
+
+@pytest.mark.parametrize("test", [parity.test_invalid_table_slots_are_never_used, parity.test_fused_backward_builds_its_own_operands,
+                                  parity.test_layer_steps_back_to_back])
+def test_layer_properties_triple_by_triple(dev, monkeypatch, test):  # noqa: F811
+    """The masked tables, the operands a backward makes itself, steps without a wait between them: as for the pairs."""
+    monkeypatch.setenv("CGNET_BWD_PAIRS", "0")
+    names = _kernels(lambda: test(dev))
+    assert "cgbn_backward_fused_kernel" in names and "cg_backward_pair_kernel" not in names, names

@@ -254,7 +254,8 @@ def test_cg_random_shapes(dev, lmax, taus, bsz, mode):
 
 
 def _random_matrix_core_cases(n, seed):
-    """Shapes whose backward takes the kernel with one gradient on the matrix cores: every channel count in 8..16."""
+    """Shapes that the kernel with one gradient on the matrix cores takes: every channel count in 8..16.  (The plan goes by pairs of
+    input degrees here; tests/test_gpu_back_routes.py runs the same shapes triple by triple.)"""
     rng = np.random.default_rng(seed)
     cases = []
     for _ in range(n):
@@ -525,8 +526,8 @@ def check_layer_step(dev, mod, ora, twin, w64, x64, go64):
 @pytest.mark.parametrize("lmax,tin,tout,bsz,sparse,bn", LAYER_CASES)
 def test_layer_forward_backward(dev, lmax, tin, tout, bsz, sparse, bn, fused):
     """fused: one autograd node for the layer (statistics inside the product kernel); "fused_backward": in addition the
-    backward runs from grad_output to the input gradient in one kernel where the shapes allow it (the two 11-degree
-    cases here), without grad_FF in memory; False: the reference's two Functions chained."""
+    backward runs from grad_output to the input gradient in one kernel where the shapes allow it (at most 16 channels),
+    without grad_FF in memory; False: the reference's two Functions chained."""
     mod, ora, twin, w64 = build_layer_pair(dev, lmax, tin, tout, sparse, bn, seed=lmax + bsz)
     mod.fused = bool(fused)
     mod.fused_backward = fused == "fused_backward"
@@ -595,17 +596,24 @@ def _fused_backward_cases(n, seed):
                     (20, [16] * 21, [16] * 21, 1, False, True, n + 2)]
 
 
-@pytest.mark.parametrize("fold", [False, True])
+@pytest.mark.parametrize("fold", [False, True, "pairs"])
 @pytest.mark.parametrize("lmax,tin,tout,bsz,sparse,bn,k", _fused_backward_cases(12, 31))
 def test_fused_backward_equals_two_kernel_backward(dev, monkeypatch, lmax, tin, tout, bsz, sparse, bn, k, fold):
-    """The one-kernel backward (gFF tiles formed in LDS) against the gFF kernel followed by the product's backward, for the
-    input gradient and the weight gradient, in training mode.  Without the fold of the diagonal triples
-    (CGNET_DIAG_FOLD=0 when the layer plan is made) the two routes agree bit for bit; with it (the default) the triples
-    with l1 = l2 are summed in another order (symmetrised tile, one slot's arithmetic), so the input gradients agree to
-    rounding.  The product tensor keeps the reference's layout on both routes here (the compact layout, which only the
-    one-kernel route can use, has a test of its own below).  The small cases are also held against the oracle."""
-    monkeypatch.setenv("CGNET_DIAG_FOLD", "1" if fold else "0")
-    from cgnet_amd import CG_layers
+    """The one-kernel backward against the gFF kernel followed by the product's backward, for the input gradient and the
+    weight gradient, in training mode: by pairs of input degrees ("pairs", gFF made in registers), and triple by triple (gFF
+    tiles formed in LDS; the kernels that large batches of reduced triples run).  By pairs the two routes agree bit for bit; so
+    they do triple by triple without the fold of the diagonal triples (CGNET_DIAG_FOLD=0 when the layer plan is made).  With
+    it (the default) the triples with l1 = l2 are summed in another order (symmetrised tile, one slot's arithmetic), so the
+    input gradients agree to rounding.  The product tensor keeps the reference's layout on both routes here (the compact
+    layout, which only the one-kernel route can use, has a test of its own below).  The small cases are also held against the
+    oracle."""
+    by_pairs = fold == "pairs"
+    fold = fold is True
+    if not by_pairs:
+        monkeypatch.setenv("CGNET_BWD_PAIRS", "0")
+        monkeypatch.setenv("CGNET_DIAG_FOLD", "1" if fold else "0")
+    from cgnet_amd import CG_layers, _lib
+    lib = _lib.load()
     monkeypatch.setattr(CG_layers, "_COMPACT_FF", False)
     mod, ora, twin, w64 = build_layer_pair(dev, lmax, tin, tout, sparse, bn, seed=400 + k)
     lp = mod.native_layer_plan()
@@ -624,7 +632,16 @@ def test_fused_backward_equals_two_kernel_backward(dev, monkeypatch, lmax, tin, 
                 mod.bnWMM.bn_stds.copy_(stds0)
         mod.bnWMM.W.grad = None
         x = x64.float().to(dev).requires_grad_(True)
+        lib.cgnet_profile_reset()
+        lib.cgnet_profile_enable(1)
         mod(x, straight_output=True).backward(go)
+        torch.cuda.synchronize()
+        lib.cgnet_profile_enable(0)
+        names = set(_lib.kernel_times())
+        if n_o:
+            assert ("cg_backward_pair_kernel" in names) == by_pairs, names
+            assert ("cgbn_backward_fused_kernel" in names) == (fb and not by_pairs), names
+            assert ("cg_backward_hybrid_kernel" in names) == (not fb and not by_pairs), names
         grads.append((x.grad.clone(), mod.bnWMM.W.grad.clone() if mod.bnWMM.W.numel() else None))
     if fold:
         # per degree: the difference is rounding of sums of that degree's magnitude
