@@ -2607,19 +2607,24 @@ extern "C" size_t cgnet_cg_plan_forward_lds(const cgnet_cg_plan* plan) {
     return plan ? std::max(plan->fwd_lds, plan->pairs.lds) : 0;
 }
 
-extern "C" int cgnet_cg_plan_backward_groups(const cgnet_cg_plan* plan) {
-    if (!plan) return 0;
-    const size_t lds = cgnet_cg_plan_backward_lds(plan);
-    const int by_lds = lds ? (int)std::min<size_t>(16, cgnet::kMaxLds / lds) : 16;
-    // register budgets: the kernel by pairs 168 or 256 registers with four waves per group, the hybrid kernel 64 or 80 registers with eight waves per group, the unit kernel 128 with four
-    const int by_regs = plan->back.ok() ? (plan->L <= 7 ? 3 : 2) : !plan->bwd_fast ? 8 : plan->bwd_hybrid ? std::max(2, std::min(4, plan->bwd_hyb_groups)) : 4;
-    return std::max(1, std::min(by_lds, by_regs));
+// LDS of a work-group of the backward and how many of them share a compute unit (LDS and registers decide).  A plan that goes by
+// pairs up to a batch and triple by triple above it reports the kernel that occupies more.
+static std::pair<size_t, int> backward_use(const cgnet_cg_plan* plan) {
+    std::pair<size_t, int> most = {0, 0};
+    auto kernel = [&](size_t lds, int by_regs) {
+        const int groups = std::max(1, std::min(lds ? (int)std::min<size_t>(16, kMaxLds / lds) : 16, by_regs));
+        if (most.second == 0 || lds * groups > most.first * most.second) most = {lds, groups};
+    };
+    // by pairs, gFF from memory: 168 or 256 registers, four waves a group; hybrid: 64 or 80, eight waves; unit: 128, four waves
+    if (plan->back.ok()) kernel(plan->back.lds, plan->L <= 7 ? 3 : 2);
+    if (plan->bwd_fast) kernel(plan->bwd_fast_lds, plan->bwd_hybrid ? std::max(2, std::min(4, plan->bwd_hyb_groups)) : 4);
+    else if (!plan->back.ok()) kernel(plan->bwd_lds, 8);
+    return most;
 }
 
-extern "C" size_t cgnet_cg_plan_backward_lds(const cgnet_cg_plan* plan) {
-    if (!plan) return 0;
-    return plan->back.ok() ? plan->back.lds : plan->bwd_fast ? plan->bwd_fast_lds : plan->bwd_lds;
-}
+extern "C" int cgnet_cg_plan_backward_groups(const cgnet_cg_plan* plan) { return plan ? backward_use(plan).second : 0; }
+
+extern "C" size_t cgnet_cg_plan_backward_lds(const cgnet_cg_plan* plan) { return plan ? backward_use(plan).first : 0; }
 
 extern "C" int cgnet_cg_plan_channels(const cgnet_cg_plan* plan, int* h_t_FF, int* h_t_offsets) {
     clear_error();

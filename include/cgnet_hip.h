@@ -78,13 +78,13 @@ int cgnet_cg_plan_destroy(cgnet_cg_plan* plan);
 int cgnet_cg_plan_sizes(const cgnet_cg_plan* plan, int sizes[5]);
 /* h_t_FF[L+1], h_t_offsets[nllls]; either may be NULL */
 int cgnet_cg_plan_channels(const cgnet_cg_plan* plan, int* h_t_FF, int* h_t_offsets);
-/* LDS bytes one work-group of the product's backward kernel holds (0 without a plan).  No counterpart in the
- * reference: a scheduling hint for callers that run another kernel on a second stream beside the backward
+/* LDS bytes one work-group of the product's backward kernel holds (0 without a plan); of a plan whose kernel depends on the
+ * batch, those of the kernel that occupies more of a compute unit.  No counterpart in the reference: a scheduling hint for callers that run another kernel on a second stream beside the backward
  * (a compute unit has 160 KB; what two such groups leave decides whether the other kernel fits beside them). */
 size_t cgnet_cg_plan_backward_lds(const cgnet_cg_plan* plan);
 /* The same for the forward kernel (its largest launch class).  No counterpart in the reference. */
 size_t cgnet_cg_plan_forward_lds(const cgnet_cg_plan* plan);
-/* Work-groups of the backward kernel that share a compute unit (its LDS need and register budget decide); with
+/* Work-groups of that backward kernel that share a compute unit (its LDS need and register budget decide); with
  * cgnet_cg_plan_backward_lds the LDS the backward occupies.  No counterpart in the reference. */
 int cgnet_cg_plan_backward_groups(const cgnet_cg_plan* plan);
 

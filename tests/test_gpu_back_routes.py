@@ -103,3 +103,16 @@ def test_layer_properties_triple_by_triple(dev, monkeypatch, test):  # noqa: F81
     monkeypatch.setenv("CGNET_BWD_PAIRS", "0")
     names = _kernels(lambda: test(dev))
     assert "cgbn_backward_fused_kernel" in names and "cg_backward_pair_kernel" not in names, names
+
+
+@pytest.mark.parametrize("lmax,tau,sparse", [(15, 16, True), (8, 12, True), (11, 5, True), (11, 12, False)])
+def test_occupancy_covers_every_kernel_of_a_plan(dev, monkeypatch, lmax, tau, sparse):  # noqa: F811
+    """What a caller schedules by holds for each kernel the plan may launch."""
+    from cgnet_amd import CG_layers
+    make = lambda: CG_layers.CG_woFilter_cuda(lmax, [tau] * (lmax + 1), lll_mode="mst" if sparse else None, device=dev).native_plan()  # noqa: E731
+    plan = make()
+    monkeypatch.setenv("CGNET_BWD_PAIRS", "0")
+    triples = make()
+    assert triples.backward_groups >= 1 and plan.backward_groups * plan.backward_lds <= 160 * 1024
+    if sparse:                                             # small batches by pairs, large ones triple by triple
+        assert plan.backward_groups * plan.backward_lds >= triples.backward_groups * triples.backward_lds
