@@ -33,7 +33,7 @@ struct BackPair {
     int offFF[kBackNL];            // complex offset inside a sample's gFF of channel (0, 0)
     int inv_tau2, inv_M1, inv_M2;  // ceil(2^16 / tau2), ceil(2^20 / (2 l1 + 1)), ceil(2^20 / (2 l2 + 1))
     int ends;                      // bit 0 / 1: the first / last channel of a degree is the first / last of a sample's product
-    int pad;
+    int nbuf;                      // buffers of F1 rows
 };
 
 // One wave's share of a pair: tiles tile0, tile0 + tstep, ...  Its partial gradients inside a sample's: nrows rows of degree l1 per

@@ -222,7 +222,8 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         for (int c = 0; c < p.nch; ++c) cost += ((p.degs[c] + 3) / 4) * 4 * 220.;
         tile_cost.push_back(cost);
         coef += (size_t)8 * p.nch * p.nks * p.nt * 64;
-        lds = std::max(lds, (size_t)back_lds_floats(p.nch, p.nt, p.nrows));
+        p.nbuf = p.ntiles > p.tstep ? 2 : 1;
+        lds = std::max(lds, (size_t)back_lds_floats(p.nch, p.nt, p.nrows, p.nbuf));
         out->pairs.push_back(p);
     }
     CGNET_REQUIRE(coef < (1u << 30), CGNET_ERR_UNSUPPORTED, "packed coefficients of the backward exceed 2^30 floats");

@@ -17,14 +17,18 @@ struct BackArgs {
     int nF, nFF, go_chunk, go_degree, nGo, P, grid0, B, nunits, lds_wave;
 };
 
-// LDS of a wave (floats): sums [rows][kBackPitch] complex | a row of zeros | two buffers of nrows rows of degree l1 between zeros.
-// Row r stands for m1 = first M + l2 - 16 nt + 1 + r.
+// LDS of a wave (floats): sums [rows][kBackPitch] complex | a row of zeros | nbuf buffers of nrows rows of degree l1 between zeros (two
+// where a unit has several tiles: the next one's rows are fetched ahead).  Row r stands for m1 = first M + l2 - 16 nt + 1 + r.  The row
+// of zeros begins in the unused columns of the last sum and ends in the first entry of a fragment row, which stands for no m1
+// (16 nt - 1 - l2 - l1 + lm >= 16 nt - 1 - 2 l2 > 0 entries lie before m1 = -l1): with three rows t1 at lmax 20..23 this is what lets two
+// work-groups share a compute unit (81 920 bytes each).
 constexpr int kBackPitch = 20;                 // complex entries per m1 of the LDS sums: sixteen columns, rows four apart fall on other banks
+constexpr int kBackSpare = kBackPitch - 16;    // columns of a sum that nothing is added to
 __host__ __device__ inline int back_rows(int nch, int nt) { return 8 * nch + 16 * nt - 1; }
-__host__ __device__ inline int back_row_pitch(int rows) { return rows | 1; }
-__host__ __device__ inline int back_lds_floats(int nch, int nt, int nrows) {
+__host__ __device__ inline int back_row_pitch(int rows) { return rows; }     // (odd)
+__host__ __device__ inline int back_lds_floats(int nch, int nt, int nrows, int nbuf) {
     const int rows = back_rows(nch, nt);
-    return (2 * (rows * kBackPitch + (2 * nrows + 1) * back_row_pitch(rows)) + 3) & ~3;
+    return (2 * (rows * kBackPitch - kBackSpare + (nbuf * nrows + 1) * back_row_pitch(rows) - 1) + 3) & ~3;
 }
 
 // a variant's kernel for the layer source with so many pairs of steps (0: memory source), and its launch

@@ -284,15 +284,15 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
     const int M0 = a.grid0 + 8 * p->c0;
     const int row0 = -l1 - (M0 + l2 - 16 * NT + 1);                // row of m1 = -l1
     v2f* const sums = reinterpret_cast<v2f*>(lds);
-    v2f* const zeros = sums + rows * kBackPitch;
-    v2f* const f1buf = zeros + pitch;                              // [2][nrows][pitch]
+    v2f* const zeros = sums + rows * kBackPitch - kBackSpare;
+    v2f* const f1buf = zeros + pitch - 1;                          // [nbuf][nrows][pitch]
     const int C = p->tau1 * tau2;
     const int inv2 = p->inv_tau2;
     const int first2 = u.tile0 * p->ncol - div16(u.tile0 * p->ncol, inv2) * tau2;     // t2 of the first column
     const int t2 = first2 + j - div16(first2 + j, inv2) * tau2;
     {
         f32x4* z = reinterpret_cast<f32x4*>(lds);
-        const int n = back_lds_floats(p->nch, NT, nrows) >> 2;
+        const int n = back_lds_floats(p->nch, NT, nrows, p->nbuf) >> 2;
         for (int e = lane; e < n; e += 64) z[e] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // the zeros precede the copies

@@ -116,3 +116,15 @@ def test_occupancy_covers_every_kernel_of_a_plan(dev, monkeypatch, lmax, tau, sp
     assert triples.backward_groups >= 1 and plan.backward_groups * plan.backward_lds <= 160 * 1024
     if sparse:                                             # small batches by pairs, large ones triple by triple
         assert plan.backward_groups * plan.backward_lds >= triples.backward_groups * triples.backward_lds
+
+
+@pytest.mark.parametrize("lmax,tau", [(20, 3), (20, 9), (20, 13), (21, 5), (23, 4), (23, 10), (23, 11), (23, 16)])
+def test_two_groups_share_a_compute_unit(dev, lmax, tau):  # noqa: F811
+    """The LDS of the pair kernel, whatever number of rows t1 its tiles touch; and the layout that this takes, against the oracle:
+    a row of zeros between the sums and the fragments, one buffer of fragments where no unit has a second tile."""
+    from cgnet_amd import CG_layers
+    taus = [tau] * (lmax + 1)
+    plan = CG_layers.CG_woFilter_cuda(lmax, taus, device=dev).native_plan()
+    assert plan.backward_groups == 2 and 2 * plan.backward_lds <= 160 * 1024
+    names = _kernels(lambda: parity.test_cg_forward_backward(dev, lmax, taus, 2 if tau < 10 else 1, "debug"))
+    assert "cg_backward_pair_kernel" in names
