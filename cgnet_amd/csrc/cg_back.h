@@ -61,9 +61,9 @@ struct BackSet {
     int nchunks = 0;                       // chunks of the grid
     int variant = 0;                       // kernel variant (groups x row tiles)
     size_t lds = 0;                        // LDS bytes of a work-group
-    // of one sample: 16 x 16 blocks of H that the vector ALUs multiply, matrix instructions that make them, multiply-adds of one
-    // gradient triple by triple
-    double blocks = 0., steps = 0., macs = 0.;
+    // of one sample: 16 x 16 blocks of H that the vector ALUs multiply, tiles of channels, multiply-adds of one gradient triple by
+    // triple
+    double blocks = 0., tiles = 0., macs = 0.;
     bool ok() const { return !pairs.empty(); }
 };
 

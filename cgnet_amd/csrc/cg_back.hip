@@ -118,9 +118,9 @@ int launch_back_combine(const BackLevel& lv, const float* d_part, float* d_gF, i
     return CGNET_OK;
 }
 
-int back_most_batch(const BackSet& set, int L, double per_mac, double slack) {
-    const double more = (set.blocks + 0.6 * set.steps - per_mac * set.macs) * 1e-4;
-    const double most = slack * (20. + 0.25 * L * L);
+int back_most_batch(const BackSet& set, int L, int nFF, int ntasks, const BackRule& rule) {
+    const double more = 1e-4 * (rule.block * set.blocks + rule.tile * set.tiles - rule.mac * set.macs - rule.entry * nFF - rule.task * ntasks);
+    const double most = rule.start + rule.start_L2 * L * L;
     return more <= 0. || most / more >= 1e6 ? INT32_MAX : (int)(most / more);
 }
 
@@ -215,10 +215,10 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
             const int entries = std::min(p.l2, M + p.l1) - std::max(-p.l2, M - p.l1) + 1;
             if (n > 0) out->macs += (double)C * n * entries;
             out->blocks += (double)p.ntiles * __builtin_popcount(tiles);
-            out->steps += 2. * p.ntiles * nk * __builtin_popcount(tiles);
             if (nk > 0) coefmap.push_back(make_int2((int)out->pairs.size(), x));
             cost += 60 + __builtin_popcount(tiles) * (64. * nk + 110.);
         }
+        out->tiles += p.ntiles;
         for (int c = 0; c < p.nch; ++c) cost += ((p.degs[c] + 3) / 4) * 4 * 220.;
         tile_cost.push_back(cost);
         coef += (size_t)8 * p.nch * p.nks * p.nt * 64;
@@ -406,7 +406,7 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
     link->d_degs = reinterpret_cast<int2*>(link->d_tables + at_gd);
     link->d_gens = reinterpret_cast<BackGenW*>(link->d_tables + at_gw);
     link->ndeg = p->L + 1;
-    link->most_B = back_most_batch(set, p->L, 0.0075, 0.2);
+    link->most_B = p->bwd_hybrid ? back_most_batch(set, p->L, p->nFF, (int)p->bwd_utasks.size(), kBackRuleLayer) : INT32_MAX;
     if (int rc = raise_dynamic_lds(variant_kernel(set.variant, link->pairs), set.lds)) {
         free_back_link(link);
         return rc;

@@ -2271,7 +2271,9 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
         if (int rc = build_back_set(triples, p->t_F, p->cumF, L, p->nFF, &p->back)) return rc;
         bool matrix = true;                          // the units would take slot 2 on the matrix cores
         for (int l = 0; l < n1; ++l) matrix &= h_t_F[l] == 0 || (h_t_F[l] >= 8 && h_t_F[l] <= 16);
-        p->back_most_B = back_most_batch(p->back, L, 0.005, matrix ? 0.2 : 0.4);
+        // a task per triple is the least the units need (a triple whose tile is cut has more): no batch for them, no units
+        const int ntasks = (int)std::count_if(triples.begin(), triples.end(), [&](const PairTriple& t) { return h_t_F[t.l1] > 0 && h_t_F[t.l2] > 0; });
+        p->back_most_B = back_most_batch(p->back, L, p->nFF, ntasks, matrix ? kBackRuleHybrid : kBackRuleUnit);
     }
     const bool want_units = !general && (!p->back.ok() || p->back_most_B < INT32_MAX);
 
@@ -2540,7 +2542,10 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
         }
     }
 
-    if (!p->bwd_fast) p->back_most_B = INT32_MAX;
+    if (!p->bwd_fast)
+        p->back_most_B = INT32_MAX;
+    else if (p->back.ok())
+        p->back_most_B = back_most_batch(p->back, L, p->nFF, (int)p->bwd_utasks.size(), p->bwd_hybrid ? kBackRuleHybrid : kBackRuleUnit);
 
     CGNET_HIP(hipGetDevice(&p->device));
     // set-up time: the statistics area of cgnet_sparse_forward_stats_static gets its address on this device

@@ -67,16 +67,27 @@ size_t back_bytes_up_to(const BackSet& set, int most_B, int B, Bytes&& bytes) {
         if (lv.least_B - 1 <= most_B) look(lv.least_B - 1);
     return most;
 }
-// Largest batch the backward by pairs is taken for, against a kernel that works triple by triple: where a pair has few output
-// degrees, or rows and columns of its tiles are empty, the other spends fewer instructions, and large batches show it.
-// Measured over lmax 2..23, 1..16 channels (constant and falling with the degree), default and minimum-spanning-tree (MST)
-// triples, 1..64 samples (1365 shapes; geometric means against the other kernels):
-//   stand-alone   always 0.72 of their time, 15 % of the shapes more than 5 % slower, at worst 2.25 times (lmax 8, MST, 14 channels,
-//                 B = 64: 81 -> 181 us); by the rule 0.70, 5 %, 1.54 times
-//   layer, 8..16 channels   always 0.63, 10 %, 1.59 times; by the rule 0.63, 3 %, 1.59 times (lmax 20, MST, 9 channels, B = 16)
-//   layer, other shapes     always 0.49 of the two kernels' time, 1 % slower
-// per_mac: blocks of 256 products that the other kernel makes up for by a multiply-add; slack: of the time a small batch saves.
-int back_most_batch(const BackSet& set, int L, double per_mac, double slack);
+// Largest batch the backward by pairs is taken for, against a kernel that works triple by triple.  By pairs a call ends earlier
+// however few samples it has; where a pair has few output degrees, or rows and columns of its tiles are empty, the other spends
+// less on a sample, and large batches show it.  Both sides are sums over a sample's work, the constants fitted to the choice
+// (not to the times: a rule's terms are right up to a common factor) over lmax 3..23, 1..16 channels (constant and falling with
+// the degree), default and minimum-spanning-tree (MST) triples, 1..128 samples, 5447 calls of 25 us and more:
+//   stand-alone, hybrid kernel   by the rule 0.67 of the time triple by triple, 0.3 % of the calls more than 5 % slower, at worst
+//                                1.12 times; always by pairs 0.75, 33 %, 2.55 times
+//   stand-alone, unit kernel     by the rule 0.59, 0.6 %, 1.16 times; always 0.60, 8 %, 1.66 times
+//   layer, 8..16 channels        by the rule 0.62, 1.4 %, 1.26 times (lmax 16, MST, 11 channels, B = 128: 1090 -> 1376 us); always
+//                                0.63, 14 %, 1.64 times
+// A layer with other channels has no other kernel but the two of the chain: always by pairs, 0.48 of their time, 0.3 % of 2325 calls
+// slower, at worst 1.14 times.
+struct BackRule {
+    double block, tile;            // 1e-4 us of a sample by pairs: per block of 16 x 16 entries of H, per tile of channels
+    double mac, entry, task;       // ... triple by triple: per multiply-add, per entry of the product, per task of a unit
+    double start, start_L2;        // us that a small batch saves: at lmax 0, times lmax squared
+};
+constexpr BackRule kBackRuleUnit = {3.0, 49., 0.0095, 0., 15.7, 16., 0.186};
+constexpr BackRule kBackRuleHybrid = {1.8, 37., 0., 0.041, 13., 8., 0.21};
+constexpr BackRule kBackRuleLayer = {1.2, 46., 0., 0.059, 51., 13., 0.04};
+int back_most_batch(const BackSet& set, int L, int nFF, int ntasks, const BackRule& rule);
 int launch_pack_coef_back(const BackSet& set, const float* d_CG, float* d_coef, hipStream_t s);
 // d_part: lv.P * B complex entries, added up by launch_back_combine
 int launch_back_memory(const BackSet& set, const BackLevel& lv, const float* d_F, const float* d_gFF, const float* d_coef,

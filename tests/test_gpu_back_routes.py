@@ -128,3 +128,32 @@ def test_two_groups_share_a_compute_unit(dev, lmax, tau):  # noqa: F811
     assert plan.backward_groups == 2 and 2 * plan.backward_lds <= 160 * 1024
     names = _kernels(lambda: parity.test_cg_forward_backward(dev, lmax, taus, 2 if tau < 10 else 1, "debug"))
     assert "cg_backward_pair_kernel" in names
+
+
+@pytest.mark.parametrize("lmax,tau,sparse,layer,most", [
+    (10, 12, False, False, 33),                            # by pairs 1.25 times as long at 64 samples
+    (5, 7, False, False, 48),                              # 1.17 at 64
+    (8, 14, True, False, 9),                               # 2.5 at 128
+    (14, 10, True, True, 25),                              # 1.34 at 40
+    (12, 15, True, True, 11),                              # 1.12 at 16
+    (11, 12, False, True, None),                           # 0.76 at 128: every batch
+    (11, 5, False, False, None),                           # 0.75 at 128
+    (15, 16, False, False, None),
+    (13, 16, True, True, None),
+])
+def test_largest_batch_by_pairs(dev, lmax, tau, sparse, layer, most):  # noqa: F811
+    """The rule that leaves large batches to the kernels that work triple by triple, where those are the faster ones."""
+    from cgnet_amd import CG_layers
+    taus = [tau] * (lmax + 1)
+    mod = CG_layers.CGBN_cuda(lmax, taus, [1] * (lmax + 1), sparse_flag=sparse, device=dev)
+    plan, lp = mod.cg.native_plan(), mod.native_layer_plan()
+    for bsz in (1, most, most + 1) if most else (1, 70):
+        x = torch.randn(bsz, plan.nF, 2, device=dev)
+        gx = torch.empty_like(x)
+        if layer:
+            go = torch.randn(bsz, lp.wmm_plan.nO, 2, device=dev)
+            names = _kernels(lambda: lp.backward_fused(x, gx, go, mod.bnWMM.W.detach(), mod.cg.CGspace, bsz, None, 1e-5, 0))
+        else:
+            gff = torch.zeros(bsz, plan.nFF, 2, device=dev)
+            names = _kernels(lambda: plan.backward(x, gx, gff, mod.cg.CGspace, bsz))
+        assert ("cg_backward_pair_kernel" in names) == (not most or bsz <= most), (bsz, names)
