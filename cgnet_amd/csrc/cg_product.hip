@@ -2146,44 +2146,6 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
         if (h_t_F[l] != 0 && (h_t_F[l] < 8 || h_t_F[l] > 16)) p->fwd_mm = false;
     if (const char* e = getenv("CGNET_FWD_MM"); e && e[0] == '0') p->fwd_mm = false;
     build(p->fwd_mm ? kFwdMmTileBytes : kFwdTileBytes, &p->fwd_tasks, 0, p->fwd_mm);
-    p->bwd_tasks.clear();
-    build(kBwdTileBytes, &p->bwd_tasks, kPadLo + kPadHi);
-    // Backward tiling.  Per slot a thread owns TI output channels x 2 m and RW lanes split the
-    // reduced channels.  cost = passes over the work-group * sequential steps of a lane * TI;
-    // the work-group size that wastes the fewest lane-steps over all tasks is kept.
-    {
-        const int cand[3] = {128, 192, 256};
-        double best_total = -1;
-        for (int ci = 0; ci < 3; ++ci) {
-            const int wg = cand[ci];
-            double total = 0;
-            std::vector<CgTask> tmp = p->bwd_tasks;
-            for (CgTask& t : tmp) {
-                for (int slot = 0; slot < 2; ++slot) {
-                    const int n_o = slot == 0 ? t.rows : t.tau2, n_r = slot == 0 ? t.tau2 : t.rows;
-                    const int M_o = slot == 0 ? 2 * t.l1 + 1 : 2 * t.l2 + 1;
-                    const int M_r = slot == 0 ? 2 * t.l2 + 1 : 2 * t.l1 + 1;
-                    double best = -1;
-                    for (int ti = 1; ti <= 4; ++ti)
-                        for (int rw = 1; rw <= 16; rw *= 2) {
-                            if (rw > 1 && rw / 2 >= n_r) continue;
-                            const int items = ((n_o + ti - 1) / ti) * ((M_o + 1) / 2);
-                            const int rows_blk = wg / rw;
-                            const double passes = (items + rows_blk - 1) / rows_blk;
-                            // steps of one lane; the row reduction costs about 2*ti*log2(rw) more
-                            double c = passes * (((n_r + rw - 1) / rw) * (double)M_r * (ti + 0.75) + 1.5 * ti * rw);
-                            if (best < 0 || c < best) { best = c; t.bTI[slot] = ti; t.bRW[slot] = rw; }
-                        }
-                    total += best * wg;
-                }
-            }
-            if (best_total < 0 || total < best_total) {
-                best_total = total;
-                p->bwd_threads = wg;
-                p->bwd_tasks = tmp;
-            }
-        }
-    }
     // heaviest forward tasks first: a short tail when the grid drains
     std::stable_sort(p->fwd_tasks.begin(), p->fwd_tasks.end(), [](const CgTask& a, const CgTask& b) {
         return (long long)a.rows * a.tau2 * (2 * a.l + 1) * (2 * a.l2 + 1) >
@@ -2207,57 +2169,15 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
         p->fwd_class_lds.back() = std::max(p->fwd_class_lds.back(), fwd_need(p->fwd_tasks[k]));
     }
     p->fwd_class_begin.push_back((int)p->fwd_tasks.size());
-    size_t fl = 0, bl = 0;
+    size_t fl = 0;
     for (const CgTask& t : p->fwd_tasks) {
         fl = std::max(fl, fwd_need(t));
         CGNET_REQUIRE(2 * fwd_frag_lds(t) <= kMaxUnitLds, CGNET_ERR_UNSUPPORTED,
                       "fragment slabs of %zu bytes exceed the LDS staging window", 2 * fwd_frag_lds(t));
     }
-    for (const CgTask& t : p->bwd_tasks) bl = std::max(bl, bwd_task_lds(t));
     p->fwd_lds = align_up(fl, 16);
-    p->bwd_lds = align_up(bl, 16) + 8 * (size_t)p->nF;
     CGNET_REQUIRE(p->fwd_lds <= kMaxLds, CGNET_ERR_UNSUPPORTED,
                   "a single output row needs %zu bytes of LDS (limit %zu)", p->fwd_lds, kMaxLds);
-    // The LDS-accumulator backward keeps a sample's whole input gradient in LDS.  Where that does not fit, the
-    // backward depends on the unit kernels below; where they do not fit either, the plan serves the forward only and
-    // cgnet_sparse_backward reports the shape as unsupported.
-    p->bwd_general_ok = p->bwd_lds <= kMaxLds;
-
-    // backward groups: contiguous task ranges of roughly equal cost, at most kMaxBwdGroups
-    {
-        const int nt = (int)p->bwd_tasks.size();
-        const int ng = std::min(kMaxBwdGroups, nt);
-        std::vector<double> cost(nt);
-        double total = 0;
-        for (int i = 0; i < nt; ++i) {
-            const CgTask& t = p->bwd_tasks[i];
-            cost[i] = (double)t.rows * t.tau2 * (2 * t.l + 1) * (2.0 * t.l1 + 2.0 * t.l2 + 2.0) + 2000.0;
-            total += cost[i];
-        }
-        p->bwd_group_begin.clear();
-        p->bwd_group_begin.push_back(0);
-        double run = 0;
-        for (int i = 0, gcount = 1; i < nt; ++i) {
-            run += cost[i];
-            if (gcount < ng && run >= total * gcount / ng && i + 1 < nt) {
-                p->bwd_group_begin.push_back(i + 1);
-                ++gcount;
-            }
-        }
-        p->bwd_group_begin.push_back(nt);
-        if (nt == 0) p->bwd_group_begin.assign(1, 0);
-    }
-    // boundaries of every coarser grouping (ng = 1 .. finest), concatenated
-    std::vector<int> gtab;
-    {
-        const int ng_max = (int)p->bwd_group_begin.size() - 1;
-        p->bwd_group_table_off.assign(ng_max + 1, 0);
-        for (int ng = 1; ng <= ng_max; ++ng) {
-            p->bwd_group_table_off[ng] = (int)gtab.size();
-            for (int g = 0; g <= ng; ++g) gtab.push_back(p->bwd_group_begin[(size_t)g * ng_max / ng]);
-        }
-    }
-
     // ---- backward by pairs of input degrees; the units below are made where it leaves larger batches to them
     // CGNET_BWD_GENERAL=1 forces the LDS-accumulator kernel (kept for shapes the unit scheme cannot hold)
     const char* force_general = getenv("CGNET_BWD_GENERAL");
@@ -2547,6 +2467,90 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
     else if (p->back.ok())
         p->back_most_B = back_most_batch(p->back, L, p->nFF, (int)p->bwd_utasks.size(), p->bwd_hybrid ? kBackRuleHybrid : kBackRuleUnit);
 
+    // ---- the LDS-accumulator backward, where nothing else takes the shape (its tiles and groups are half of the time of a large plan)
+    std::vector<int> gtab;
+    const bool want_general = !p->bwd_fast && !p->back.ok();
+    if (want_general) {
+        p->bwd_tasks.clear();
+        build(kBwdTileBytes, &p->bwd_tasks, kPadLo + kPadHi);
+        // Backward tiling.  Per slot a thread owns TI output channels x 2 m and RW lanes split the
+        // reduced channels.  cost = passes over the work-group * sequential steps of a lane * TI;
+        // the work-group size that wastes the fewest lane-steps over all tasks is kept.
+        {
+            const int cand[3] = {128, 192, 256};
+            double best_total = -1;
+            for (int ci = 0; ci < 3; ++ci) {
+                const int wg = cand[ci];
+                double total = 0;
+                std::vector<CgTask> tmp = p->bwd_tasks;
+                for (CgTask& t : tmp) {
+                    for (int slot = 0; slot < 2; ++slot) {
+                        const int n_o = slot == 0 ? t.rows : t.tau2, n_r = slot == 0 ? t.tau2 : t.rows;
+                        const int M_o = slot == 0 ? 2 * t.l1 + 1 : 2 * t.l2 + 1;
+                        const int M_r = slot == 0 ? 2 * t.l2 + 1 : 2 * t.l1 + 1;
+                        double best = -1;
+                        for (int ti = 1; ti <= 4; ++ti)
+                            for (int rw = 1; rw <= 16; rw *= 2) {
+                                if (rw > 1 && rw / 2 >= n_r) continue;
+                                const int items = ((n_o + ti - 1) / ti) * ((M_o + 1) / 2);
+                                const int rows_blk = wg / rw;
+                                const double passes = (items + rows_blk - 1) / rows_blk;
+                                // steps of one lane; the row reduction costs about 2*ti*log2(rw) more
+                                double c = passes * (((n_r + rw - 1) / rw) * (double)M_r * (ti + 0.75) + 1.5 * ti * rw);
+                                if (best < 0 || c < best) { best = c; t.bTI[slot] = ti; t.bRW[slot] = rw; }
+                            }
+                        total += best * wg;
+                    }
+                }
+                if (best_total < 0 || total < best_total) {
+                    best_total = total;
+                    p->bwd_threads = wg;
+                    p->bwd_tasks = tmp;
+                }
+            }
+        }
+        size_t bl = 0;
+        for (const CgTask& t : p->bwd_tasks) bl = std::max(bl, bwd_task_lds(t));
+        p->bwd_lds = align_up(bl, 16) + 8 * (size_t)p->nF;
+        // It keeps a sample's whole input gradient in LDS.  Where that does not fit, the plan serves the forward only and
+        // cgnet_sparse_backward reports the shape as unsupported.
+        p->bwd_general_ok = p->bwd_lds <= kMaxLds;
+
+        // backward groups: contiguous task ranges of roughly equal cost, at most kMaxBwdGroups
+        {
+            const int nt = (int)p->bwd_tasks.size();
+            const int ng = std::min(kMaxBwdGroups, nt);
+            std::vector<double> cost(nt);
+            double total = 0;
+            for (int i = 0; i < nt; ++i) {
+                const CgTask& t = p->bwd_tasks[i];
+                cost[i] = (double)t.rows * t.tau2 * (2 * t.l + 1) * (2.0 * t.l1 + 2.0 * t.l2 + 2.0) + 2000.0;
+                total += cost[i];
+            }
+            p->bwd_group_begin.clear();
+            p->bwd_group_begin.push_back(0);
+            double run = 0;
+            for (int i = 0, gcount = 1; i < nt; ++i) {
+                run += cost[i];
+                if (gcount < ng && run >= total * gcount / ng && i + 1 < nt) {
+                    p->bwd_group_begin.push_back(i + 1);
+                    ++gcount;
+                }
+            }
+            p->bwd_group_begin.push_back(nt);
+            if (nt == 0) p->bwd_group_begin.assign(1, 0);
+        }
+        // boundaries of every coarser grouping (ng = 1 .. finest), concatenated
+        {
+            const int ng_max = (int)p->bwd_group_begin.size() - 1;
+            p->bwd_group_table_off.assign(ng_max + 1, 0);
+            for (int ng = 1; ng <= ng_max; ++ng) {
+                p->bwd_group_table_off[ng] = (int)gtab.size();
+                for (int g = 0; g <= ng; ++g) gtab.push_back(p->bwd_group_begin[(size_t)g * ng_max / ng]);
+            }
+        }
+    }
+
     CGNET_HIP(hipGetDevice(&p->device));
     // set-up time: the statistics area of cgnet_sparse_forward_stats_static gets its address on this device
     // (a plan is usable without it: a failure here is reported by that entry point, which resolves the address again)
@@ -2564,6 +2568,8 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
     if (!p->fwd_tasks.empty()) {
         CGNET_HIP(hipMalloc((void**)&p->d_fwd_tasks, sizeof(CgTask) * p->fwd_tasks.size()));
         CGNET_HIP(hipMemcpy(p->d_fwd_tasks, p->fwd_tasks.data(), sizeof(CgTask) * p->fwd_tasks.size(), hipMemcpyHostToDevice));
+    }
+    if (!p->bwd_tasks.empty()) {
         CGNET_HIP(hipMalloc((void**)&p->d_bwd_tasks, sizeof(CgTask) * p->bwd_tasks.size()));
         CGNET_HIP(hipMemcpy(p->d_bwd_tasks, p->bwd_tasks.data(), sizeof(CgTask) * p->bwd_tasks.size(), hipMemcpyHostToDevice));
         CGNET_HIP(hipMalloc((void**)&p->d_bwd_group_table, sizeof(int) * gtab.size()));
@@ -2585,7 +2591,7 @@ extern "C" int cgnet_cg_plan_create(cgnet_cg_plan** plan, int L, const int* h_t_
             return rc;
     }
     if (int rc = raise_dynamic_lds(p->fwd_mm ? (const void*)cg_forward_mm_kernel : (const void*)cg_forward_kernel, p->fwd_lds)) return rc;
-    if (p->bwd_general_ok)
+    if (want_general && p->bwd_general_ok)
         if (int rc = raise_dynamic_lds((const void*)cg_backward_kernel, p->bwd_lds)) return rc;
     *plan = guard.release();
     return CGNET_OK;
@@ -2787,14 +2793,12 @@ extern "C" int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F
     CGNET_REQUIRE(d_gF, CGNET_ERR_ARG, "d_gF is NULL");
     CGNET_REQUIRE(B <= 65535, CGNET_ERR_UNSUPPORTED, "B=%d above 65535", B);
     hipStream_t s = (hipStream_t)stream;
-    const int ng_max = (int)plan->bwd_group_begin.size() - 1;
-    if (ng_max <= 0 || plan->bwd_tasks.empty()) {
+    if (plan->fwd_tasks.empty()) {
         // no triple contributes: the gradient is zero (a fill kernel, not hipMemsetAsync: the call may be recorded
         // into a graph)
         return launch_zero_gradient(plan, d_gF, B, s);
     }
     CGNET_REQUIRE(d_F && d_gFF && d_CG, CGNET_ERR_ARG, "null device pointer");
-    const int ng = bwd_groups_for(plan, B);
     const size_t need = backward_bytes(plan, B);
     CGNET_REQUIRE(need == 0 || (d_workspace && workspace_bytes >= need), CGNET_ERR_WORKSPACE,
                   "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
@@ -2847,6 +2851,7 @@ extern "C" int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F
     CGNET_REQUIRE(plan->bwd_general_ok, CGNET_ERR_UNSUPPORTED,
                   "backward needs %zu bytes of LDS (limit %zu): too many input channels for this lmax; the plan serves "
                   "the forward only", plan->bwd_lds, kMaxLds);
+    const int ng = bwd_groups_for(plan, B);
     const int* d_gb = plan->d_bwd_group_table + plan->bwd_group_table_off[ng];
     float2* dst = ng > 1 ? (float2*)d_workspace : (float2*)d_gF;
     CGNET_LAUNCH(cg_backward_kernel, dim3(ng, B), dim3(plan->bwd_threads), plan->bwd_lds, s,
