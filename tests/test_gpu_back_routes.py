@@ -157,3 +157,73 @@ def test_largest_batch_by_pairs(dev, lmax, tau, sparse, layer, most):  # noqa: F
             gff = torch.zeros(bsz, plan.nFF, 2, device=dev)
             names = _kernels(lambda: plan.backward(x, gx, gff, mod.cg.CGspace, bsz))
         assert ("cg_backward_pair_kernel" in names) == (not most or bsz <= most), (bsz, names)
+
+
+def _reached(plan, l, m, channel=None):
+    """Entries of F whose gradient holds entry m of degree l of the product's gradient: of one of its channels, or of all."""
+    from cgnet_amd import CGutils
+    n1 = plan.lmax + 1
+    at = [0]
+    for d in range(n1):
+        at.append(at[-1] + plan.t_F[d] * (2 * d + 1))
+    hit = torch.zeros(plan.nF, dtype=torch.bool)
+    for (out, l1, l2), first in zip(CGutils.SparseLtuples.get_iter(plan.lmax, plan.llls), plan.t_offsets):
+        t1, t2 = plan.t_F[l1], plan.t_F[l2]
+        if out != l or not t1 * t2 or (channel is not None and not first <= channel < first + t1 * t2):
+            continue
+        a, b = (slice(None),) * 2 if channel is None else divmod(channel - first, t2)
+        lo, hi = max(-l1, m - l2), min(l1, m + l2)
+        hit[at[l1]:at[l1 + 1]].view(t1, -1)[a, l1 + lo:l1 + hi + 1] = True
+        hit[at[l2]:at[l2 + 1]].view(t2, -1)[b, l2 + m - hi:l2 + m - lo + 1] = True
+    return hit
+
+
+@pytest.mark.parametrize("lmax,taus,sparse", [
+    (0, [3], False),
+    (1, [1, 2], False),
+    (3, [2] * 4, False),
+    (5, [12, 0, 7, 12, 1, 10], False),
+    (9, [3] * 10, True),
+    (11, [12] * 12, False),                                # tiles that begin inside a row
+    (15, [4, 16] * 8, False),
+    (20, [2] * 21, True),
+])
+def test_entries_that_are_not_finite_reach_what_depends_on_them(dev, lmax, taus, sparse):  # noqa: F811
+    """Zero coefficients stand for no value of m, no degree and no channel, and zero times infinity is no zero: an infinity or NaN in
+    the gradient that comes in changes the gradients it is a term of, and no other entry of its sample or of the batch."""
+    from cgnet_amd import CG_layers
+    mod = CG_layers.CGBN_cuda(lmax, taus, [2] * (lmax + 1), sparse_flag=sparse, device=dev).eval()
+    plan, lp = mod.cg.native_plan(), mod.native_layer_plan()
+    g = torch.Generator().manual_seed(lmax)
+    with torch.no_grad():
+        mod.bnWMM.W.copy_(torch.randn(mod.bnWMM.W.shape, generator=g))
+        mod.bnWMM.bn_stds.fill_(1.)
+    x = torch.randn(3, plan.nF, 2, generator=g).to(dev)
+
+    def places(width):                                     # (degree, m, channel, entry): the ends of every degree, and some between
+        begin = 0
+        for l, t in enumerate(width):
+            n = t * (2 * l + 1)
+            for e in sorted({0, 2 * l, n // 3, n - 1}) if n else ():
+                yield l, e % (2 * l + 1) - l, e // (2 * l + 1), begin + e
+            begin += n
+    for width, n, of_channel in ((plan.t_FF, plan.nFF, True), ([2] * (lmax + 1), lp.wmm_plan.nO, False)):
+        gy = torch.randn(3, n, 2, generator=g).to(dev)
+        want, got = torch.empty_like(x), torch.empty_like(x)
+
+        def backward(grad):
+            if of_channel:
+                plan.backward(x, grad, gy, mod.cg.CGspace, 3)
+            else:
+                lp.backward_fused(x, grad, gy, mod.bnWMM.W.detach(), mod.cg.CGspace, 3, mod.bnWMM.bn_stds.data, 1e-5, 1)
+        names = _kernels(lambda: backward(want))
+        assert "cg_backward_pair_kernel" in names
+        for k, (l, m, channel, entry) in enumerate(places(width)):
+            keep = gy[1, entry].clone()
+            gy[1, entry, k % 2] = (float("inf"), float("nan"), -float("inf"))[k % 3]
+            backward(got)
+            gy[1, entry] = keep
+            hit = torch.zeros(3, plan.nF, dtype=torch.bool)
+            hit[1] = _reached(plan, l, m, channel if of_channel else None)
+            assert torch.equal((~torch.isfinite(got)).any(-1).cpu(), hit), (of_channel, l, m, channel)
+            assert torch.equal(got[~hit.to(dev)], want[~hit.to(dev)])
