@@ -349,6 +349,8 @@ extern "C" int cgnet_layer_plan_create(cgnet_layer_plan** plan, const cgnet_cg_p
         } else if (rc1 != CGNET_OK) {
             free_back_link(&p->link);
             return rc1;
+        } else {
+            p->reason[0] = 0;
         }
     }
     const int rc2 = build_fwd_link(cg_plan, wmm_plan, &p->fwd);

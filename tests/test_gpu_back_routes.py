@@ -96,6 +96,15 @@ def test_layer_triple_by_triple(dev, monkeypatch, lmax, tin, tout, bsz, sparse, 
     assert "cg_backward_pair_kernel" not in names and ("cgbn_backward_fused_kernel" in names) == one, names
 
 
+def test_reason_of_a_layer_that_is_taken(dev, monkeypatch):  # noqa: F811
+    """A layer that only the kernel by triples takes has no reason why it is not taken; one that neither takes has."""
+    from cgnet_amd import CG_layers
+    monkeypatch.setenv("CGNET_BWD_PAIRS", "0")
+    for tau, taken in ((9, True), (3, False)):
+        lp = CG_layers.CGBN_cuda(2, [tau] * 3, [2] * 3, device=dev).native_layer_plan()
+        assert lp.fused_backward_supported == taken and bool(lp.fused_backward_reason) != taken
+
+
 @pytest.mark.parametrize("test", [parity.test_invalid_table_slots_are_never_used, parity.test_fused_backward_builds_its_own_operands,
                                   parity.test_layer_steps_back_to_back])
 def test_layer_properties_triple_by_triple(dev, monkeypatch, test):  # noqa: F811
