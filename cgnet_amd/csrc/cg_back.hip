@@ -42,11 +42,111 @@ pack_go_back_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs
     }
 }
 
+// What an entry of the input gradient is a sum of, straight from the operands of the pair kernel.
+struct BackTerms {
+    const float2 *F, *gFF, *gO;    // gFF: memory source, else gO
+    const float* W;                // layer source: packed weights
+    const BackGenPair* gp;
+    const int2* degs;
+    const float* coef;
+    const BackPair* pairs;
+    int npairs, nFF, nO, ndeg, steps, grid0;   // steps: pairs of steps over the output channels
+};
+
+__device__ __forceinline__ bool finite(float2 z) {
+    return (__float_as_uint(z.x) & 0x7f800000u) != 0x7f800000u && (__float_as_uint(z.y) & 0x7f800000u) != 0x7f800000u;
+}
+
+// G of (pair k, channel c), its degree q, value M.
+__device__ float2 back_gradient(const BackTerms& a, const BackPair& p, int k, int c, int q, int M, int b) {
+    const int l = p.l[q];
+    if (a.gFF) return a.gFF[(size_t)b * a.nFF + p.offFF[q] + c * (2 * l + 1) + M + l];
+    const int tile = c / p.ncol, j = c - tile * p.ncol;
+    const float* w = a.W + a.gp[k].w + (size_t)tile * a.gp[k].wtile + 512 * a.steps * (q >> 2) + 256 * ((q >> 1) & 1) + 2 * (q & 1) + 4 * j;
+    const float2* g = a.gO + (size_t)b * a.nO + a.degs[l].x + M + l;
+    float2 s = make_float2(0.f, 0.f);
+    for (int to = 0; to < a.degs[l].y; ++to) {
+        // places of the real and the imaginary part: operand rows 2 to, 2 to + 1 of steps of four
+        const float* at = w + 512 * (to >> 2) + ((to >> 1) & 1) + 128 * (to & 1);
+        const float x = at[0], y = at[64];
+        const float2 z = g[to * (2 * l + 1)];
+        s.x += z.x * x + z.y * y;
+        s.y += z.y * x - z.x * y;
+    }
+    return s;
+}
+
+// f(pair, its number, the other degree's channels, degree and offset in F, whether degree l is the pair's l2) for all pairs that hold
+// degree l, until it returns true.
+template <typename F>
+__device__ __forceinline__ bool any_pair(const BackTerms& a, int l, F&& f) {
+    for (int k = 0; k < a.npairs; ++k) {
+        const BackPair& p = a.pairs[k];
+        if (p.l1 == l && f(p, k, p.tau2, p.l2, p.offF2, false)) return true;
+        if (p.l2 == l && f(p, k, p.tau1, p.l1, p.offF1, true)) return true;
+    }
+    return false;
+}
+
+// Entry m of row t of degree l, term by term; `sum` if a term is not finite.
+__device__ float2 back_entry(const BackTerms& a, int b, int nF, int l, int t, int m, float2 sum) {
+    const float2* const Fb = a.F + (size_t)b * nF;
+    // what makes most entries of a sample not finite is looked at first: (the layer) an entry of gO, which is in every channel's G, or a
+    // fragment
+    for (int d = 0; d < a.ndeg && !a.gFF; ++d) {
+        const float2* g = a.gO + (size_t)b * a.nO + a.degs[d].x;
+        for (int e = 0; e < a.degs[d].y * (2 * d + 1); ++e) {
+            if (finite(g[e])) continue;
+            const int M = e % (2 * d + 1) - d;
+            if (any_pair(a, l, [&](const BackPair& p, int, int, int lo, int, bool) {
+                    for (int q = 0; q < p.nl; ++q)
+                        if (p.l[q] == d) return abs(M - m) <= lo;
+                    return false;
+                }))
+                return sum;
+        }
+    }
+    if (any_pair(a, l, [&](const BackPair& p, int, int n, int lo, int off, bool) {
+            for (int o = 0; o < n; ++o)
+                for (int mo = max(-lo, -p.l[0] - m); mo <= min(lo, p.l[0] - m); ++mo)
+                    if (!finite(Fb[off + o * (2 * lo + 1) + lo + mo])) return true;
+            return false;
+        }))
+        return sum;
+    float2 s = make_float2(0.f, 0.f);
+    if (any_pair(a, l, [&](const BackPair& p, int k, int n, int lo, int off, bool second) {
+            for (int o = 0; o < n; ++o)
+                for (int mo = max(-lo, -p.l[0] - m); mo <= min(lo, p.l[0] - m); ++mo) {
+                    const int M = m + mo, m2 = p.l2 + (second ? m : mo), c = second ? o * p.tau2 + t : t * p.tau2 + o;
+                    const float* coef = a.coef + p.coef + ((M - a.grid0 - 8 * p.c0) * p.nks * p.nt + (m2 >> 4)) * 64 + (m2 & 15);
+                    float2 h = make_float2(0.f, 0.f);
+                    for (int q = 0; q < p.nl && abs(M) <= p.l[q]; ++q) {
+                        const float2 g = back_gradient(a, p, k, c, q, M, b);
+                        if (!finite(g)) return true;
+                        const float v = coef[(q >> 2) * p.nt * 64 + 16 * (q & 3)];
+                        h.x += v * g.x;
+                        h.y += v * g.y;
+                    }
+                    const float2 z = Fb[off + o * (2 * lo + 1) + lo + mo];
+                    s.x += h.x * z.x + h.y * z.y;
+                    s.y += h.y * z.x - h.x * z.y;
+                }
+            return false;
+        }))
+        return sum;
+    return s;
+}
+
 // Input gradient from the units' partial ones: a row's shares added in the order of its list.
+// The pair kernel multiplies places that stand for no value of m, no degree or no channel by zero coefficients, and zero times
+// infinity is no zero: a sum that is not finite is looked at term by term, so that an entry of G that is not finite reaches what
+// depends on it and nothing else.  (Masks in the pair kernel itself, even as a second pass off its hot path, cost it 1 .. 6 %: more
+// registers to spill, and a check per unit.  Here finite gradients cost nothing: lmax 11, 12 channels, B = 100 14 us, as without; 43 us where
+// all of gO is NaN, 46 with one infinity in each sample; lmax 10, 4 channels, with entries to add up again in every sample, 8 -> 1370.)
 // meta: [L+2] cumF | [L+2] first row of a degree | [rows + 1] list begin | offsets of the shares
 __global__ void __launch_bounds__(256)
 cg_backward_rows_kernel(const float2* __restrict__ part, float2* __restrict__ gF, const int* __restrict__ meta, int L, int nF, int P,
-                        int B) {
+                        int B, BackTerms terms) {
     __shared__ int s_tab[kMaxLookup];
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int b = (int)(idx / nF), e = (int)(idx % nF);
@@ -65,6 +165,7 @@ cg_backward_rows_kernel(const float2* __restrict__ part, float2* __restrict__ gF
         s.x += v.x;
         s.y += v.y;
     }
+    if (__builtin_expect(!finite(s), 0)) s = back_entry(terms, b, nF, l, t, x - l, s);
     gF[idx] = s;
 }
 
@@ -88,7 +189,7 @@ const void* variant_kernel(int v, int pairs) {
     return v == 0 ? back_kernel_0(pairs) : v == 1 ? back_kernel_1(pairs) : v == 2 ? back_kernel_2(pairs) : back_kernel_3(pairs);
 }
 
-int launch_back(const BackSet& set, const BackLevel& lv, int pairs, BackArgs a, hipStream_t s) {
+int launch_back(const BackSet& set, const BackLevel& lv, int pairs, BackArgs a, BackTerms t, float* d_gF, int L, hipStream_t s) {
     a.pairs = set.d_pairs; a.units = lv.d_units; a.P = lv.P; a.grid0 = set.grid0;
     a.lds_wave = (int)(set.lds / (4 * kBackWaves));
     a.nunits = (int)lv.units.size();
@@ -99,6 +200,11 @@ int launch_back(const BackSet& set, const BackLevel& lv, int pairs, BackArgs a, 
     auto* launch = set.variant == 0 ? back_launch_0 : set.variant == 1 ? back_launch_1 : set.variant == 2 ? back_launch_2 : back_launch_3;
     launch(pairs, grid, set.lds, s, a);
     CGNET_HIP(hipGetLastError());
+    t.F = a.F; t.coef = a.coef; t.pairs = set.d_pairs; t.npairs = (int)set.pairs.size(); t.grid0 = set.grid0;
+    const size_t n = (size_t)a.nF * a.B;
+    CGNET_LAUNCH(cg_backward_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.part, (float2*)d_gF, lv.d_combine, L,
+                 a.nF, lv.P, a.B, t);
+    CGNET_HIP(hipGetLastError());
     return CGNET_OK;
 }
 
@@ -108,14 +214,6 @@ const BackLevel& back_level(const BackSet& set, int B) {
     for (const BackLevel& lv : set.levels)
         if (B >= lv.least_B) return lv;
     return set.levels.back();
-}
-
-int launch_back_combine(const BackLevel& lv, const float* d_part, float* d_gF, int L, int nF, int B, hipStream_t s) {
-    const size_t n = (size_t)nF * B;
-    CGNET_LAUNCH(cg_backward_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const float2*)d_part, (float2*)d_gF,
-                 lv.d_combine, L, nF, lv.P, B);
-    CGNET_HIP(hipGetLastError());
-    return CGNET_OK;
 }
 
 int back_most_batch(const BackSet& set, int L, int nFF, int ntasks, const BackRule& rule) {
@@ -323,12 +421,14 @@ int launch_pack_coef_back(const BackSet& set, const float* d_CG, float* d_coef, 
 }
 
 int launch_back_memory(const BackSet& set, const BackLevel& lv, const float* d_F, const float* d_gFF, const float* d_coef,
-                       float* d_part, int nF, int nFF, int B, hipStream_t s) {
+                       float* d_part, float* d_gF, int L, int nF, int nFF, int B, hipStream_t s) {
     BackArgs a{};
     a.F = (const float2*)d_F; a.gFF = (const float2*)d_gFF;
     a.coef = d_coef; a.part = (float2*)d_part;
     a.nF = nF; a.nFF = nFF; a.B = B;
-    return launch_back(set, lv, 0, a, s);
+    BackTerms t{};
+    t.gFF = a.gFF; t.nFF = nFF;
+    return launch_back(set, lv, 0, a, t, d_gF, L, s);
 }
 
 // ---- layer source --------------------------------------------------------------------------------
@@ -422,7 +522,8 @@ int launch_pack_w_back(const BackLink& link, const float* d_W, const float* d_st
 }
 
 int launch_back_layer(const BackSet& set, const BackLink& link, const BackLevel& lv, const float* d_F, const float* d_gO,
-                      const float* d_Wp, const float* d_coef, float* d_Go, float* d_part, int nF, int B, hipStream_t s) {
+                      const float* d_Wp, const float* d_coef, float* d_Go, float* d_part, float* d_gF, int L, int nF, int B,
+                      hipStream_t s) {
     CGNET_REQUIRE(B <= 65535, CGNET_ERR_UNSUPPORTED, "B=%d above 65535", B);
     const int per_chunk = link.ndeg * 128 * link.pairs;
     CGNET_LAUNCH(pack_go_back_kernel, dim3((unsigned)(set.nchunks * link.ndeg), (unsigned)B), dim3(64), 0, s, (const float2*)d_gO,
@@ -432,7 +533,9 @@ int launch_back_layer(const BackSet& set, const BackLink& link, const BackLevel&
     a.F = (const float2*)d_F; a.Go = d_Go; a.W = d_Wp; a.gp = link.d_gp;
     a.coef = d_coef; a.part = (float2*)d_part;
     a.nF = nF; a.nGo = link.go_floats; a.go_chunk = per_chunk; a.go_degree = 128 * link.pairs; a.B = B;
-    return launch_back(set, lv, link.pairs, a, s);
+    BackTerms t{};
+    t.gO = (const float2*)d_gO; t.W = d_Wp; t.gp = link.d_gp; t.degs = link.d_degs; t.nO = link.nO; t.ndeg = link.ndeg; t.steps = link.pairs;
+    return launch_back(set, lv, link.pairs, a, t, d_gF, L, s);
 }
 
 }  // namespace cgnet

@@ -200,17 +200,6 @@ __device__ __forceinline__ void mem_ends(const BackWave& w, int M0, int nd, f32x
     CGNET_END;
 }
 
-// Zeros in the places of a chunk that stand for no value of a degree, no degree or no column.
-template <int KS>
-__device__ __forceinline__ void back_mask(const BackWave& w, int M0, int nd, bool column, f32x4 (&r)[KS][4]) {
-    CGNET_EACH(4 * KS, k)
-        const int l = w.p->l[k], M = M0 + 2 * w.kk;
-        const bool in = column && k < nd, lo = in && abs(M) <= l, hi = in && abs(M + 1) <= l;
-        const f32x4 z = r[k / 4][k % 4];
-        r[k / 4][k % 4] = (f32x4){lo ? z[0] : 0.f, lo ? z[1] : 0.f, hi ? z[2] : 0.f, hi ? z[3] : 0.f};
-    CGNET_END;
-}
-
 template <int KS>
 __device__ __forceinline__ void turn_all(int nd, f32x4 (&r)[KS][4]) {
     CGNET_EACH(KS, ks)
@@ -229,10 +218,9 @@ struct BackAcc {
 
 // A chunk of eight M with at most KC groups of degrees.  AHEAD (memory source): the loads of the chunk at next_M0 with next_nd degrees
 // go out between the steps, behind the coefficients of the step after, so that no wait for those is one for all of them.
-// MASKED: rows of H whose m1 or m2 is no value of its degree are zero whatever G holds.
-template <int KS, int NT, int KC, bool AHEAD, bool MASKED>
+template <int KS, int NT, int KC, bool AHEAD>
 __device__ __forceinline__ void back_chunk(BackWave& w, BackAcc<NT>& A, const f32x4 (&G)[KS][4], int steps8, int tiles8,
-                                           f32x4 (&next)[KS][4], int M0, int next_M0, int next_nd) {
+                                           f32x4 (&next)[KS][4], int next_M0, int next_nd) {
     float cf[2][KC][NT];
     CGNET_EACH(KC, ks) CGNET_EACH(NT, rt) cf[0][ks][rt] = (w.cp + (ks * NT + rt) * 64)[w.lane]; CGNET_END; CGNET_END;
     lds_order();                                                   // keeps the loads here and not where they are used
@@ -266,14 +254,6 @@ __device__ __forceinline__ void back_chunk(BackWave& w, BackAcc<NT>& A, const f3
                         hi = mfma4(cf[now][k + 1][rt], G[k + 1][x / 2][2 * now + 1], hi);
                     }
                 CGNET_END;
-                if constexpr (MASKED) {
-                    CGNET_EACH(4, v)
-                        const int m = 16 * rt + 4 * w.kk + v, l2 = w.p->l2;
-                        const bool in = m <= 2 * l2 && abs(M0 + x + l2 - m) <= w.p->l1;
-                        hr[v] = in ? hr[v] : 0.f;
-                        hi[v] = in ? hi[v] : 0.f;
-                    CGNET_END;
-                }
                 CGNET_EACH(4, v)
                     constexpr int s = (x - v) & 3;
                     A.a2r[rt][v] = fmaf(hr[v], A.f1[rt][s].x, A.a2r[rt][v]);
@@ -296,14 +276,8 @@ __device__ __forceinline__ void back_chunk(BackWave& w, BackAcc<NT>& A, const f3
     w.s_at += 64u * kBackPitch;
 }
 
-__device__ __forceinline__ bool not_finite(float2 z) {
-    return (__float_as_uint(z.x) & 0x7f800000u) == 0x7f800000u || (__float_as_uint(z.y) & 0x7f800000u) == 0x7f800000u;
-}
-
-// Returns whether an entry of the unit's gradients is not finite.
-template <int KS, int NT, int PAIRS, bool MASKED>
-__device__ __forceinline__ bool back_pass(const BackArgs& a, pair_p p, const BackUnit& u, int b, float* lds, int lane) {
-    bool odd = false;
+template <int KS, int NT, int PAIRS>
+__device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const BackUnit& u, int b, float* lds, int lane) {
     const int j = lane & 15, kk = lane >> 4;
     const int l1 = p->l1, l2 = p->l2, M1 = 2 * l1 + 1, M2 = 2 * l2 + 1, tau2 = p->tau2, nrows = p->nrows;
     const int rows = back_rows(p->nch, NT), pitch = back_row_pitch(rows);
@@ -378,7 +352,7 @@ __device__ __forceinline__ bool back_pass(const BackArgs& a, pair_p p, const Bac
         // memory source: a lane past the last channel repeats the last row's of its t2
         if constexpr (PAIRS == 0) w.chan = min(t1, p->tau1 - 1) * tau2 + (t1 < p->tau1 ? c0 + jj - t1 * tau2 : t2);
         // all loads of a chunk go out during the one before it where there are registers for them
-        constexpr bool AHEAD = PAIRS == 0 && KS + NT <= 6 && !MASKED;
+        constexpr bool AHEAD = PAIRS == 0 && KS + NT <= 6;
         const bool ends = (p->ends & 1 && c0 == 0) || (p->ends & 2 && c0 + ncol == C);
         f32x4 next[KS][4];
         if constexpr (AHEAD) {
@@ -397,11 +371,10 @@ __device__ __forceinline__ bool back_pass(const BackArgs& a, pair_p p, const Bac
                 CGNET_END;
                 if (ends) mem_ends<KS>(w, Mc, nd, G);
             }
-            if constexpr (MASKED) back_mask<KS>(w, Mc, nd, jj < ncol, G);
             turn_all<KS>(nd, G);
-            if (!MASKED && nd <= 4) back_chunk<KS, NT, 1, AHEAD, MASKED>(w, A, G, steps8, tiles8, next, Mc, next_M0, next_nd);
-            else if (KS == 2 || (!MASKED && nd <= 8)) back_chunk<KS, NT, 2, AHEAD, MASKED>(w, A, G, steps8, tiles8, next, Mc, next_M0, next_nd);
-            else back_chunk<KS, NT, KS, AHEAD, MASKED>(w, A, G, steps8, tiles8, next, Mc, next_M0, next_nd);
+            if (nd <= 4) back_chunk<KS, NT, 1, AHEAD>(w, A, G, steps8, tiles8, next, next_M0, next_nd);
+            else if (KS == 2 || nd <= 8) back_chunk<KS, NT, 2, AHEAD>(w, A, G, steps8, tiles8, next, next_M0, next_nd);
+            else back_chunk<KS, NT, KS, AHEAD>(w, A, G, steps8, tiles8, next, next_M0, next_nd);
         }
         // the three sums that have not seen their last row
         CGNET_EACH(3, x)
@@ -425,7 +398,6 @@ __device__ __forceinline__ bool back_pass(const BackArgs& a, pair_p p, const Bac
                 s.y += col[t].y;
             }
             p1[e] = s;
-            odd |= not_finite(s);
         }
         lds_order();
         {
@@ -453,24 +425,7 @@ __device__ __forceinline__ bool back_pass(const BackArgs& a, pair_p p, const Bac
                 s.y += from[r * tau2].y;
             }
         p2[e] = s;
-        odd |= not_finite(s);
     }
-    return __any(odd);
-}
-
-// Coefficients of places that stand for nothing are zero, and zero times infinity is not: a unit that leaves entries that are not
-// finite is done again with those places masked, so that such an entry of G reaches what depends on it and nothing else.
-// (Masking in every pass would add two instructions to each eight of the vector half.  The second pass as a copy off the hot path,
-// fed by values the compiler cannot follow, leaves the first as it was: lmax 11, 12 channels, B = 100, training step 1044 -> 1046 us, lmax
-// 15 stand-alone 2000 -> 2000; with a switch in one body, or a copy placed in line, 91 .. 126 more registers spilled, 1 .. 2 %.)
-template <int KS, int NT, int PAIRS>
-__device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const BackUnit& u, int b, float* lds, int lane) {
-    if (__builtin_expect(!back_pass<KS, NT, PAIRS, false>(a, p, u, b, lds, lane), 1)) return;
-    // copies the compiler knows nothing of: nothing is kept for this through the pass before
-    uint64_t p1 = (uint64_t)(uintptr_t)p;
-    BackUnit u1 = u;
-    asm volatile("" : "+s"(p1), "+s"(u1.tile0), "+s"(u1.ntiles), "+s"(u1.p1off), "+s"(u1.p2off), "+s"(b));
-    back_pass<KS, NT, PAIRS, true>(a, (pair_p)(uintptr_t)p1, u1, b, lds, opaque(lane));
 }
 
 template <int KS, int NTMAX, int PAIRS>

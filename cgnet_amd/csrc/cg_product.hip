@@ -2808,8 +2808,7 @@ extern "C" int cgnet_sparse_backward(const cgnet_cg_plan* plan, const float* d_F
         float* part = (float*)d_workspace;
         float* coef = (float*)((char*)d_workspace + align_up(sizeof(float) * 2 * (size_t)lv.P * B, 256));
         if (int rc = launch_pack_coef_back(plan->back, d_CG, coef, s)) return rc;
-        if (int rc = launch_back_memory(plan->back, lv, d_F, d_gFF, coef, part, plan->nF, plan->nFF, B, s)) return rc;
-        return launch_back_combine(lv, part, d_gF, plan->L, plan->nF, B, s);
+        return launch_back_memory(plan->back, lv, d_F, d_gFF, coef, part, d_gF, plan->L, plan->nF, plan->nFF, B, s);
     }
     if (plan->bwd_fast) {
         float2* part1 = (float2*)d_workspace;

@@ -89,17 +89,17 @@ constexpr BackRule kBackRuleHybrid = {1.8, 37., 0., 0.041, 13., 8., 0.21};
 constexpr BackRule kBackRuleLayer = {1.2, 46., 0., 0.059, 51., 13., 0.04};
 int back_most_batch(const BackSet& set, int L, int nFF, int ntasks, const BackRule& rule);
 int launch_pack_coef_back(const BackSet& set, const float* d_CG, float* d_coef, hipStream_t s);
-// d_part: lv.P * B complex entries, added up by launch_back_combine
+// d_part: lv.P * B complex entries for the partial gradients, which are added up to d_gF
 int launch_back_memory(const BackSet& set, const BackLevel& lv, const float* d_F, const float* d_gFF, const float* d_coef,
-                       float* d_part, int nF, int nFF, int B, hipStream_t s);
+                       float* d_part, float* d_gF, int L, int nF, int nFF, int B, hipStream_t s);
 // The same with the gradient of the product made in registers from packed weights and gO.  link->ok says whether the pair of
 // plans is taken; when it is not, the return code is CGNET_ERR_UNSUPPORTED and cgnet_last_error() names the reason.
 int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* link);
 void free_back_link(BackLink* link);
 int launch_pack_w_back(const BackLink& link, const float* d_W, const float* d_stds, float eps, float* d_Wp, hipStream_t s);
 int launch_back_layer(const BackSet& set, const BackLink& link, const BackLevel& lv, const float* d_F, const float* d_gO,
-                      const float* d_Wp, const float* d_coef, float* d_Go, float* d_part, int nF, int B, hipStream_t s);
-int launch_back_combine(const BackLevel& lv, const float* d_part, float* d_gF, int L, int nF, int B, hipStream_t s);
+                      const float* d_Wp, const float* d_coef, float* d_Go, float* d_part, float* d_gF, int L, int nF, int B,
+                      hipStream_t s);
 
 // ---- fused inference forward (cg_product.hip)
 int build_fwd_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, FwdLink* link);

@@ -544,10 +544,8 @@ extern "C" int cgnet_CGBN_backward_fused(const cgnet_layer_plan* plan, const flo
         return launch_fused_backward(cg, plan->fused, d_gO, Wb, F, coef, (float*)(ws + ba.Go), (float*)(ws + ba.own.part1),
                                      (float*)(ws + ba.own.part2), d_gF, B, s);
     const BackLevel& lv = back_level(cg->back, B);
-    if (int rc = launch_back_layer(cg->back, plan->link, lv, F, d_gO, Wb, coef, (float*)(ws + ba.Go), (float*)(ws + ba.part),
-                                   cg->nF, B, s))
-        return rc;
-    return launch_back_combine(lv, (const float*)(ws + ba.part), d_gF, cg->L, cg->nF, B, s);
+    return launch_back_layer(cg->back, plan->link, lv, F, d_gO, Wb, coef, (float*)(ws + ba.Go), (float*)(ws + ba.part), d_gF, cg->L,
+                             cg->nF, B, s);
 }
 
 // ---- compact product tensor: sizes, weight gradient --------------------------------------------------

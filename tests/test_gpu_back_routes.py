@@ -235,4 +235,8 @@ def test_entries_that_are_not_finite_reach_what_depends_on_them(dev, lmax, taus,
             hit = torch.zeros(3, plan.nF, dtype=torch.bool)
             hit[1] = _reached(plan, l, m, channel if of_channel else None)
             assert torch.equal((~torch.isfinite(got)).any(-1).cpu(), hit), (of_channel, l, m, channel)
-            assert torch.equal(got[~hit.to(dev)], want[~hit.to(dev)])
+            assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2])
+            # entries that a zero times infinity had reached are added up again, term by term: some thousand products in another
+            # order, an error that grows like the root of the terms, and the largest entry a few times their root mean square
+            rest = ~hit[1].to(dev)
+            assert (got[1] - want[1])[rest].abs().sum() == 0 or (got[1] - want[1])[rest].abs().max() <= 2e-5 * want.abs().max()
