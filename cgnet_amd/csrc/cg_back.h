@@ -84,11 +84,12 @@ struct BackLink {
     unsigned char* d_tables = nullptr;
     BackGenPair* d_gp = nullptr;
     int2* d_degs = nullptr;        // per degree: cumO, t_O
+    int* d_reach = nullptr;        // per (degree, output degree): the largest degree of the other fragment, -1: no such pair
     BackGenW* d_gens = nullptr;
     int ngens = 0, ndeg = 0;
     int pairs = 0;                 // pairs of steps of the degree with most outputs
     size_t w_floats = 0;           // packed weights
-    int go_floats = 0;             // packed gO of a sample
+    int go_floats = 0;             // packed gO of a sample, with the flags behind it
     int nO = 0;                    // complex entries of one sample's layer output
     int most_B = 0;                // the largest batch it is taken for where there is another route
 };

@@ -20,8 +20,13 @@ pack_coef_back_kernel(const float* __restrict__ CG, const BackPair* __restrict__
     pack_coef_back_block(CG, pairs, map[blockIdx.x], grid0, coef);
 }
 
+__device__ __forceinline__ bool finite(float2 z) {
+    return (__float_as_uint(z.x) & 0x7f800000u) != 0x7f800000u && (__float_as_uint(z.y) & 0x7f800000u) != 0x7f800000u;
+}
+
 // Packed gO of the layer source: [chunk of eight M][degree][step][lane (k, (M, re / im))], k = (channel, re / im); zero past the
-// degree's channels and values.  A work-group takes a (chunk, degree) of a sample.  degs: per degree cumO, t_O.
+// degree's channels and values, and in the place of entries that are not finite; behind it a flag per (chunk, degree): whether it has
+// such entries.  A work-group takes a (chunk, degree) of a sample.  degs: per degree cumO, t_O.
 __global__ void __launch_bounds__(64)
 pack_go_back_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs, float* __restrict__ Go, int ndeg, int pairs,
                     int grid0, int nO, int nGo) {
@@ -30,142 +35,128 @@ pack_go_back_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs
     const int lane = threadIdx.x, i = lane & 15, kk = lane >> 4;
     const int x = grid0 + 8 * c + (i >> 1) + l, r = i & 1;
     const float2* src = gO + (size_t)blockIdx.y * nO + d.x;
-    float* dst = Go + (size_t)blockIdx.y * nGo + (size_t)blockIdx.x * 128 * pairs + lane;
+    float* const sample = Go + (size_t)blockIdx.y * nGo;
+    float* dst = sample + (size_t)blockIdx.x * 128 * pairs + lane;
+    bool odd = false;
     for (int s = 0; s < 2 * pairs; ++s) {
         const int k = 4 * s + kk, to = k >> 1, sel = k & 1;
         float v = 0.f;
         if (to < d.y && x >= 0 && x <= 2 * l) {
             const float2 z = src[to * (2 * l + 1) + x];
-            v = (r == sel) ? (r ? -z.x : z.x) : z.y;
+            if (finite(z)) v = (r == sel) ? (r ? -z.x : z.x) : z.y;
+            else odd = true;
         }
         dst[64 * s] = v;
     }
+    odd = __any(odd);
+    if (lane == 0) reinterpret_cast<int*>(sample)[(size_t)gridDim.x * 128 * pairs + blockIdx.x] = odd;
 }
 
-// What an entry of the input gradient is a sum of, straight from the operands of the pair kernel.
+// What cg_backward_rows_kernel looks at where something is not finite.
 struct BackTerms {
-    const float2 *F, *gFF, *gO;    // gFF: memory source, else gO
-    const float* W;                // layer source: packed weights
-    const BackGenPair* gp;
-    const int2* degs;
+    const BackPair* pairs;         // memory source
+    const float2 *F, *gFF;
     const float* coef;
-    const BackPair* pairs;
-    int npairs, nFF, nO, ndeg, steps, grid0;   // steps: pairs of steps over the output channels
+    const float2* gO;              // layer source
+    const int* odd;                // ... the flags of pack_go_back_kernel
+    const int2* degs;
+    const int* reach;              // ... per (degree l, degree d of gO): the largest degree of a fragment between them, -1: none
+    int nFF, nO, nGo, nodd, ndeg, grid0;
 };
 
-__device__ __forceinline__ bool finite(float2 z) {
-    return (__float_as_uint(z.x) & 0x7f800000u) != 0x7f800000u && (__float_as_uint(z.y) & 0x7f800000u) != 0x7f800000u;
-}
-
-// G of (pair k, channel c), its degree q, value M.
-__device__ float2 back_gradient(const BackTerms& a, const BackPair& p, int k, int c, int q, int M, int b) {
-    const int l = p.l[q];
-    if (a.gFF) return a.gFF[(size_t)b * a.nFF + p.offFF[q] + c * (2 * l + 1) + M + l];
-    const int tile = c / p.ncol, j = c - tile * p.ncol;
-    const float* w = a.W + a.gp[k].w + (size_t)tile * a.gp[k].wtile + 512 * a.steps * (q >> 2) + 256 * ((q >> 1) & 1) + 2 * (q & 1) + 4 * j;
-    const float2* g = a.gO + (size_t)b * a.nO + a.degs[l].x + M + l;
+// Entry m of row t of a degree: its share from some of a pair's tiles, term by term.  which: pair and whether the degree is the pair's
+// l2; tiles: the first, how many << 16.
+__device__ float2 back_share(const BackTerms& a, int b, int nF, int t, int m, int which, int tiles) {
+    const BackPair& p = a.pairs[which >> 1];
+    const bool second = which & 1;
+    const int n = second ? p.tau1 : p.tau2, lo = second ? p.l1 : p.l2;
+    const float2* other = a.F + (size_t)b * nF + (second ? p.offF1 : p.offF2);
+    const float2* G = a.gFF + (size_t)b * a.nFF;
     float2 s = make_float2(0.f, 0.f);
-    for (int to = 0; to < a.degs[l].y; ++to) {
-        // places of the real and the imaginary part: operand rows 2 to, 2 to + 1 of steps of four
-        const float* at = w + 512 * (to >> 2) + ((to >> 1) & 1) + 128 * (to & 1);
-        const float x = at[0], y = at[64];
-        const float2 z = g[to * (2 * l + 1)];
-        s.x += z.x * x + z.y * y;
-        s.y += z.y * x - z.x * y;
+    for (int o = 0; o < n; ++o) {
+        const int c = second ? o * p.tau2 + t : t * p.tau2 + o, k = c / p.ncol - (tiles & 0xffff);
+        if (k < 0 || k >= (tiles >> 16) * p.tstep || k % p.tstep) continue;
+        for (int mo = max(-lo, -p.l[0] - m); mo <= min(lo, p.l[0] - m); ++mo) {
+            const int M = m + mo, m2 = p.l2 + (second ? m : mo);
+            const float* coef = a.coef + p.coef + ((M - a.grid0 - 8 * p.c0) * p.nks * p.nt + (m2 >> 4)) * 64 + (m2 & 15);
+            float2 h = make_float2(0.f, 0.f);
+#pragma unroll 4
+            for (int q = 0; q < p.nl; ++q) {
+                const int l = p.l[q];
+                if (abs(M) > l) break;
+                const float2 g = G[p.offFF[q] + c * (2 * l + 1) + M + l];
+                const float v = coef[(q >> 2) * p.nt * 64 + 16 * (q & 3)];
+                h.x += v * g.x;
+                h.y += v * g.y;
+            }
+            const float2 z = other[o * (2 * lo + 1) + lo + mo];
+            s.x += h.x * z.x + h.y * z.y;
+            s.y += h.y * z.x - h.x * z.y;
+            if (!finite(s)) return s;                              // and stays so
+        }
     }
     return s;
 }
 
-// f(pair, its number, the other degree's channels, degree and offset in F, whether degree l is the pair's l2) for all pairs that hold
-// degree l, until it returns true.
-template <typename F>
-__device__ __forceinline__ bool any_pair(const BackTerms& a, int l, F&& f) {
-    for (int k = 0; k < a.npairs; ++k) {
-        const BackPair& p = a.pairs[k];
-        if (p.l1 == l && f(p, k, p.tau2, p.l2, p.offF2, false)) return true;
-        if (p.l2 == l && f(p, k, p.tau1, p.l1, p.offF1, true)) return true;
+// Whether an entry of the sample's gO that is not finite is in the gradient of entry m of degree l: it is in G of every channel.
+__device__ bool back_reached(const BackTerms& a, int b, int l, int m) {
+    for (int k = 0; k < a.nodd; ++k) {
+        if (!a.odd[(size_t)b * a.nGo + k]) continue;
+        const int d = k % a.ndeg, M0 = a.grid0 + 8 * (k / a.ndeg), far = a.reach[l * a.ndeg + d];
+        const float2* g = a.gO + (size_t)b * a.nO + a.degs[d].x + d;
+        for (int M = max(max(-d, M0), m - far); M <= min(min(d, M0 + 7), m + far); ++M)
+            for (int to = 0; to < a.degs[d].y; ++to)
+                if (!finite(g[to * (2 * d + 1) + M])) return true;
     }
     return false;
 }
 
-// Entry m of row t of degree l, term by term; `sum` if a term is not finite.
-__device__ float2 back_entry(const BackTerms& a, int b, int nF, int l, int t, int m, float2 sum) {
-    const float2* const Fb = a.F + (size_t)b * nF;
-    // what makes most entries of a sample not finite is looked at first: (the layer) an entry of gO, which is in every channel's G, or a
-    // fragment
-    for (int d = 0; d < a.ndeg && !a.gFF; ++d) {
-        const float2* g = a.gO + (size_t)b * a.nO + a.degs[d].x;
-        for (int e = 0; e < a.degs[d].y * (2 * d + 1); ++e) {
-            if (finite(g[e])) continue;
-            const int M = e % (2 * d + 1) - d;
-            if (any_pair(a, l, [&](const BackPair& p, int, int, int lo, int, bool) {
-                    for (int q = 0; q < p.nl; ++q)
-                        if (p.l[q] == d) return abs(M - m) <= lo;
-                    return false;
-                }))
-                return sum;
-        }
-    }
-    if (any_pair(a, l, [&](const BackPair& p, int, int n, int lo, int off, bool) {
-            for (int o = 0; o < n; ++o)
-                for (int mo = max(-lo, -p.l[0] - m); mo <= min(lo, p.l[0] - m); ++mo)
-                    if (!finite(Fb[off + o * (2 * lo + 1) + lo + mo])) return true;
-            return false;
-        }))
-        return sum;
-    float2 s = make_float2(0.f, 0.f);
-    if (any_pair(a, l, [&](const BackPair& p, int k, int n, int lo, int off, bool second) {
-            for (int o = 0; o < n; ++o)
-                for (int mo = max(-lo, -p.l[0] - m); mo <= min(lo, p.l[0] - m); ++mo) {
-                    const int M = m + mo, m2 = p.l2 + (second ? m : mo), c = second ? o * p.tau2 + t : t * p.tau2 + o;
-                    const float* coef = a.coef + p.coef + ((M - a.grid0 - 8 * p.c0) * p.nks * p.nt + (m2 >> 4)) * 64 + (m2 & 15);
-                    float2 h = make_float2(0.f, 0.f);
-                    for (int q = 0; q < p.nl && abs(M) <= p.l[q]; ++q) {
-                        const float2 g = back_gradient(a, p, k, c, q, M, b);
-                        if (!finite(g)) return true;
-                        const float v = coef[(q >> 2) * p.nt * 64 + 16 * (q & 3)];
-                        h.x += v * g.x;
-                        h.y += v * g.y;
-                    }
-                    const float2 z = Fb[off + o * (2 * lo + 1) + lo + mo];
-                    s.x += h.x * z.x + h.y * z.y;
-                    s.y += h.y * z.x - h.x * z.y;
-                }
-            return false;
-        }))
-        return sum;
-    return s;
-}
-
 // Input gradient from the units' partial ones: a row's shares added in the order of its list.
 // The pair kernel multiplies places that stand for no value of m, no degree or no channel by zero coefficients, and zero times
-// infinity is no zero: a sum that is not finite is looked at term by term, so that an entry of G that is not finite reaches what
-// depends on it and nothing else.  (Masks in the pair kernel itself, even as a second pass off its hot path, cost it 1 .. 6 %: more
-// registers to spill, and a check per unit.  Here finite gradients cost nothing: lmax 11, 12 channels, B = 100 14 us, as without; 43 us where
-// all of gO is NaN, 46 with one infinity in each sample; lmax 10, 4 channels, with entries to add up again in every sample, 8 -> 1370.)
-// meta: [L+2] cumF | [L+2] first row of a degree | [rows + 1] list begin | offsets of the shares
+// infinity is no zero.  An entry of the gradient that comes in and is not finite still reaches what depends on it and nothing else: from
+// memory, a share that is not finite is added up again term by term; the layer's gO is packed without such entries, and what depends
+// on them is made NaN here.  (Masks in the pair kernel itself, even as a second pass off its hot path, cost it 1 .. 6 %: more registers
+// to spill, and a check per unit.)  Whole backward at lmax 20, 16 channels, B = 8: inside the layer 0.8 ms whatever gO holds; from memory
+// 0.7 ms where all is finite or nothing is, 2.8 with one infinity in each sample, 9.4 where some sums of every row are too large.
+// meta: [L+2] cumF | [L+2] first row of a degree | [rows + 1] list begin | offsets of the shares | which, tiles of back_share
 __global__ void __launch_bounds__(256)
 cg_backward_rows_kernel(const float2* __restrict__ part, float2* __restrict__ gF, const int* __restrict__ meta, int L, int nF, int P,
                         int B, BackTerms terms) {
     __shared__ int s_tab[kMaxLookup];
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t first = (size_t)blockIdx.x * blockDim.x, idx = first + threadIdx.x;
     const int b = (int)(idx / nF), e = (int)(idx % nF);
     const int* cum_rows = meta + (L + 2);
     const int* begin = cum_rows + (L + 2);
     const int* at = begin + cum_rows[L + 1] + 1;
+    int odd = 0;
+    if (terms.gO) {                                                // samples of the work-group with entries that are not finite
+        const int b0 = (int)(first / nF), n = (min(B - 1, (int)((first + blockDim.x - 1) / nF)) - b0 + 1) * terms.nodd;
+        for (int k = threadIdx.x; k < n; k += blockDim.x) odd |= terms.odd[(size_t)(b0 + k / terms.nodd) * terms.nGo + k % terms.nodd];
+        odd = __syncthreads_or(odd);
+    }
     const int l = lookup_in_group(L + 1, e, [&](int k) { return meta[k]; }, s_tab);
     if (idx >= (size_t)B * nF) return;
     const int M = 2 * l + 1, rel = e - s_tab[l], t = rel / M, x = rel - t * M;
-    const int row = cum_rows[l] + t;
+    const int row = cum_rows[l] + t, k0 = begin[row], k1 = begin[row + 1];
     const float2* from = part + (size_t)b * P + x;
     float2 s = make_float2(0.f, 0.f);
 #pragma unroll 8
-    for (int k = begin[row]; k < begin[row + 1]; ++k) {
+    for (int k = k0; k < k1; ++k) {
         const float2 v = from[at[k]];
         s.x += v.x;
         s.y += v.y;
     }
-    if (__builtin_expect(!finite(s), 0)) s = back_entry(terms, b, nF, l, t, x - l, s);
+    if (terms.gFF && __builtin_expect(!finite(s), 0)) {
+        const int* which = at + begin[cum_rows[L + 1]];
+        s = make_float2(0.f, 0.f);
+        for (int k = k0; k < k1 && finite(s); ++k) {
+            float2 v = from[at[k]];
+            if (!finite(v)) v = back_share(terms, b, nF, t, x - l, which[2 * k], which[2 * k + 1]);
+            s.x += v.x;
+            s.y += v.y;
+        }
+    }
+    if (__builtin_expect(odd, 0) && back_reached(terms, b, l, x - l)) s = make_float2(__builtin_nanf(""), __builtin_nanf(""));
     gF[idx] = s;
 }
 
@@ -200,7 +191,7 @@ int launch_back(const BackSet& set, const BackLevel& lv, int pairs, BackArgs a, 
     auto* launch = set.variant == 0 ? back_launch_0 : set.variant == 1 ? back_launch_1 : set.variant == 2 ? back_launch_2 : back_launch_3;
     launch(pairs, grid, set.lds, s, a);
     CGNET_HIP(hipGetLastError());
-    t.F = a.F; t.coef = a.coef; t.pairs = set.d_pairs; t.npairs = (int)set.pairs.size(); t.grid0 = set.grid0;
+    t.pairs = set.d_pairs; t.grid0 = set.grid0;
     const size_t n = (size_t)a.nF * a.B;
     CGNET_LAUNCH(cg_backward_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.part, (float2*)d_gF, lv.d_combine, L,
                  a.nF, lv.P, a.B, t);
@@ -340,7 +331,7 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         lv.least_B = n == 1 << 30 ? 1 : (5120 + n - 1) / n;
         const double target = n == 1 << 30 ? 0. : all / n;
         std::vector<std::pair<double, BackUnit>> units;
-        std::vector<int2> shares;                                   // (row of a degree, where a share of it lies)
+        std::vector<int4> shares;                                   // (row of a degree, where a share of it lies, which, tiles of back_share)
         int at = 0;
         for (size_t k = 0; k < out->pairs.size(); ++k) {
             const BackPair& p = out->pairs[k];
@@ -354,11 +345,13 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
                     for (int t = 0; t < n; ++t) {
                         const int c0 = (u.tile0 + t * p.tstep) * p.ncol, c1 = std::min(p.tau1 * p.tau2, c0 + p.ncol);
                         for (int r = c0 / p.tau2; r <= (c1 - 1) / p.tau2; ++r)
-                            shares.push_back(make_int2(cum_rows[p.l1] + r, at + (t * p.nrows + r - c0 / p.tau2) * M1));
+                            shares.push_back(make_int4(cum_rows[p.l1] + r, at + (t * p.nrows + r - c0 / p.tau2) * M1, 2 * (int)k,
+                                                       (u.tile0 + t * p.tstep) | 1 << 16));
                     }
                     at += n * p.nrows * M1;
                     u.p2off = at;
-                    for (int r = 0; r < p.tau2; ++r) shares.push_back(make_int2(cum_rows[p.l2] + r, at + r * M2));
+                    for (int r = 0; r < p.tau2; ++r)
+                        shares.push_back(make_int4(cum_rows[p.l2] + r, at + r * M2, 2 * (int)k + 1, u.tile0 | n << 16));
                     at += p.tau2 * M2;
                     units.push_back({tile_cost[k] * n, u});
                 }
@@ -367,16 +360,22 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         std::stable_sort(units.begin(), units.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
         for (const auto& x : units) lv.units.push_back(x.second);
         lv.P = at;
-        // meta of cg_backward_rows_kernel: [L+2] cumF | [L+2] first row of a degree | [rows + 1] list begin | offsets
+        // meta of cg_backward_rows_kernel
         std::vector<int> meta(cumF.begin(), cumF.end());
         meta.insert(meta.end(), cum_rows.begin(), cum_rows.end());
         const size_t head = meta.size(), nrows = cum_rows[L + 1];
-        meta.resize(head + nrows + 1 + shares.size());
+        meta.resize(head + nrows + 1 + 3 * shares.size());
         int* begin = meta.data() + head;                            // (counted one place on, then summed)
-        for (const int2& x : shares) ++begin[x.x + 1];
+        for (const int4& x : shares) ++begin[x.x + 1];
         for (size_t r = 0; r < nrows; ++r) begin[r + 1] += begin[r];
         std::vector<int> next(begin, begin + nrows);
-        for (const int2& x : shares) begin[nrows + 1 + next[x.x]++] = x.y;
+        int *offset = begin + nrows + 1, *which = offset + shares.size();
+        for (const int4& x : shares) {
+            const int to = next[x.x]++;
+            offset[to] = x.y;
+            which[2 * to] = x.z;
+            which[2 * to + 1] = x.w;
+        }
         bool finest = true;
         for (const BackUnit& u : lv.units) finest &= u.ntiles == 1;
         out->levels.push_back(lv);
@@ -427,7 +426,7 @@ int launch_back_memory(const BackSet& set, const BackLevel& lv, const float* d_F
     a.coef = d_coef; a.part = (float2*)d_part;
     a.nF = nF; a.nFF = nFF; a.B = B;
     BackTerms t{};
-    t.gFF = a.gFF; t.nFF = nFF;
+    t.F = a.F; t.gFF = a.gFF; t.nFF = nFF; t.coef = d_coef;
     return launch_back(set, lv, 0, a, t, d_gF, L, s);
 }
 
@@ -457,7 +456,14 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
         degs[l] = make_int2(info[l].cumO, info[l].tO);
         link->pairs = std::max(link->pairs, std::max(1, (info[l].tO + 3) / 4));
     }
-    link->go_floats = set.nchunks * (p->L + 1) * 128 * link->pairs;
+    link->go_floats = set.nchunks * (p->L + 1) * 128 * link->pairs + (int)align_up(set.nchunks * (p->L + 1), 64);
+    std::vector<int> reach((p->L + 1) * (p->L + 1), -1);
+    for (const BackPair& b : set.pairs)
+        for (int q = 0; q < b.nl; ++q) {
+            int &r1 = reach[b.l1 * (p->L + 1) + b.l[q]], &r2 = reach[b.l2 * (p->L + 1) + b.l[q]];
+            r1 = std::max(r1, b.l2);
+            r2 = std::max(r2, b.l1);
+        }
     std::vector<BackGenPair> gps(set.pairs.size());
     std::vector<BackGenW> gens;
     size_t at = 0;
@@ -491,11 +497,12 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
     size_t bytes = 0;
     auto place = [&](size_t n) { const size_t o = bytes; bytes += align_up(n, 256); return o; };
     const size_t at_gp = place(sizeof(BackGenPair) * gps.size()), at_gd = place(sizeof(int2) * degs.size());
-    const size_t at_gw = place(sizeof(BackGenW) * gens.size());
+    const size_t at_gw = place(sizeof(BackGenW) * gens.size()), at_reach = place(sizeof(int) * reach.size());
     const std::unique_ptr<unsigned char[]> host(new unsigned char[bytes]());
     memcpy(host.get() + at_gp, gps.data(), sizeof(BackGenPair) * gps.size());
     memcpy(host.get() + at_gd, degs.data(), sizeof(int2) * degs.size());
     memcpy(host.get() + at_gw, gens.data(), sizeof(BackGenW) * gens.size());
+    memcpy(host.get() + at_reach, reach.data(), sizeof(int) * reach.size());
     CGNET_HIP(hipMalloc((void**)&link->d_tables, bytes));
     if (hipMemcpy(link->d_tables, host.get(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
         free_back_link(link);
@@ -504,6 +511,7 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
     }
     link->d_gp = reinterpret_cast<BackGenPair*>(link->d_tables + at_gp);
     link->d_degs = reinterpret_cast<int2*>(link->d_tables + at_gd);
+    link->d_reach = reinterpret_cast<int*>(link->d_tables + at_reach);
     link->d_gens = reinterpret_cast<BackGenW*>(link->d_tables + at_gw);
     link->ndeg = p->L + 1;
     link->most_B = p->bwd_hybrid ? back_most_batch(set, p->L, p->nFF, (int)p->bwd_utasks.size(), kBackRuleLayer) : INT32_MAX;
@@ -534,7 +542,8 @@ int launch_back_layer(const BackSet& set, const BackLink& link, const BackLevel&
     a.coef = d_coef; a.part = (float2*)d_part;
     a.nF = nF; a.nGo = link.go_floats; a.go_chunk = per_chunk; a.go_degree = 128 * link.pairs; a.B = B;
     BackTerms t{};
-    t.gO = (const float2*)d_gO; t.W = d_Wp; t.gp = link.d_gp; t.degs = link.d_degs; t.nO = link.nO; t.ndeg = link.ndeg; t.steps = link.pairs;
+    t.gO = (const float2*)d_gO; t.degs = link.d_degs; t.reach = link.d_reach; t.nO = link.nO; t.ndeg = link.ndeg;
+    t.odd = reinterpret_cast<const int*>(d_Go) + (size_t)set.nchunks * per_chunk; t.nodd = set.nchunks * link.ndeg; t.nGo = link.go_floats;
     return launch_back(set, lv, link.pairs, a, t, d_gF, L, s);
 }
 
