@@ -123,21 +123,17 @@ __global__ void __launch_bounds__(256)
 cg_backward_rows_kernel(const float2* __restrict__ part, float2* __restrict__ gF, const int* __restrict__ meta, int L, int nF, int P,
                         int B, BackTerms terms) {
     __shared__ int s_tab[kMaxLookup];
-    const size_t first = (size_t)blockIdx.x * blockDim.x, idx = first + threadIdx.x;
+    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int b = (int)(idx / nF), e = (int)(idx % nF);
     const int* cum_rows = meta + (L + 2);
     const int* begin = cum_rows + (L + 2);
     const int* at = begin + cum_rows[L + 1] + 1;
-    int odd = 0;
-    if (terms.gO) {                                                // samples of the work-group with entries that are not finite
-        const int b0 = (int)(first / nF), n = (min(B - 1, (int)((first + blockDim.x - 1) / nF)) - b0 + 1) * terms.nodd;
-        for (int k = threadIdx.x; k < n; k += blockDim.x) odd |= terms.odd[(size_t)(b0 + k / terms.nodd) * terms.nGo + k % terms.nodd];
-        odd = __syncthreads_or(odd);
-    }
+    const int lane = threadIdx.x & 63, b0 = __builtin_amdgcn_readfirstlane(b), b1 = min(__builtin_amdgcn_readlane(b, 63), B - 1);
+    // flags of the wave's samples: the first ones are fetched here and looked at behind the sums
+    int odd = b0 < B && lane < terms.nodd ? terms.odd[(size_t)b0 * terms.nGo + lane] : 0;
     const int l = lookup_in_group(L + 1, e, [&](int k) { return meta[k]; }, s_tab);
-    if (idx >= (size_t)B * nF) return;
     const int M = 2 * l + 1, rel = e - s_tab[l], t = rel / M, x = rel - t * M;
-    const int row = cum_rows[l] + t, k0 = begin[row], k1 = begin[row + 1];
+    const int row = cum_rows[l] + t, k0 = begin[row], k1 = b < B ? begin[row + 1] : k0;     // (lanes past the end fetch flags)
     const float2* from = part + (size_t)b * P + x;
     float2 s = make_float2(0.f, 0.f);
 #pragma unroll 8
@@ -156,8 +152,12 @@ cg_backward_rows_kernel(const float2* __restrict__ part, float2* __restrict__ gF
             s.y += v.y;
         }
     }
-    if (__builtin_expect(odd, 0) && back_reached(terms, b, l, x - l)) s = make_float2(__builtin_nanf(""), __builtin_nanf(""));
-    gF[idx] = s;
+    if (terms.nodd) {
+        for (int bb = b0; bb <= b1; ++bb)
+            for (int k = lane + (bb == b0 ? 64 : 0); k < terms.nodd; k += 64) odd |= terms.odd[(size_t)bb * terms.nGo + k];
+        if (__builtin_expect(__any(odd), 0) && b < B && back_reached(terms, b, l, x - l)) s = make_float2(__builtin_nanf(""), __builtin_nanf(""));
+    }
+    if (b < B) gF[idx] = s;
 }
 
 // Packed weights of the layer source, one work-group of four waves per (pair, degree).
