@@ -68,14 +68,14 @@ SQ_PROFILE = os.path.join("profiles", "cg_layer_L11_tau12_B100_sq_counters_pmc.t
 
 def profiled_issue(kernel, avg_launch_ms):
     """SIMD issue time of `kernel` from the committed SQ counter summary: vector and matrix instructions take turns
-    on a SIMD of this GPU (2.7 cycles per vector instruction, 32 per v_mfma_f32_16x16x4_f32; measured, see the
-    summary's header), so (2.7 N_vector + 32 N_matrix) / (1024 SIMDs x clock) bounds the kernel from below."""
+    on a SIMD of this GPU but for a tenth (4 cycles per vector instruction, 32 per v_mfma_f32_16x16x4_f32; measured, see the
+    summary's header), so (4 N_vector + 32 N_matrix) / (1024 SIMDs x clock) is what they take one after the other."""
     try:
         for line in open(os.path.join(ROOT, SQ_PROFILE)):
             f = line.split()
             if len(f) >= 7 and f[0].split("<")[0] == kernel:
                 mhz, n_valu, n_mfma = float(f[2]), float(f[3]), float(f[6])
-                bound_ms = (2.7 * (n_valu - n_mfma) + 32.0 * n_mfma) / (1024 * mhz * 1e6) * 1e3
+                bound_ms = (4.0 * (n_valu - n_mfma) + 32.0 * n_mfma) / (1024 * mhz * 1e6) * 1e3
                 return {"bound_ms": round(bound_ms, 4), "frac": round(bound_ms / avg_launch_ms, 3), "clock_MHz": mhz,
                         "vector_instructions": n_valu - n_mfma, "matrix_instructions": n_mfma,
                         "source": SQ_PROFILE + " (counters of an earlier run, not of this one)"}

@@ -172,8 +172,8 @@ constexpr int kVariantL[kVariants] = {7, 11, 15, kBackMaxL};
 // Groups of four output degrees: the smallest number that holds all of a pair, up to lmax 15.  Above it that took 256 registers, 177
 // of them spilled, at six groups; a pair of more than sixteen degrees is cut, its smaller ones make a pair of their own that spans few M
 // (layer, lmax 20, 16 channels, B = 32: 2.39 -> 2.18 ms, five groups 2.28, three 2.27; from memory at B = 16: 1.54 -> 1.14 ms).  Where
-// all fit, cutting only repeats the vector half (lmax 11, 12 channels, B = 100: 424 us, cut at two groups 452; lmax 15, 16 channels,
-// B = 64: 1.52 ms, cut at three groups 1.64).
+// all fit, cutting only repeats the vector half (lmax 11, 12 channels, B = 100, cut at two groups: 1.07 times as long; lmax 15, 16 channels,
+// B = 64, cut at three: 1.08).
 constexpr int kVariantKS[kVariants] = {2, 3, 4, 4};
 
 const void* variant_kernel(int v, int pairs) {

@@ -24,13 +24,14 @@
 //
 // Bounded by issue where enough waves run: a vector multiply-add holds a SIMD for four cycles, a matrix instruction for 32, and the two
 // take turns.  lmax 11, 12 channels, B = 100, inside the layer: 8.6e7 vector and 1.1e7 matrix instructions, 75 % of the cycles of
-// 1024 SIMDs; three waves a SIMD (168 registers; from lmax 12 on two, 256).  Without the loads of packed gO and weights it takes
-// 345 us, without the vector half 414 of then 494: the loads come out of L1, which gives 64 bytes a cycle to loads of 4 or 16 bytes a
-// lane and half of that to 8 bytes, and out of L2, for which the work-groups of a sample stay on one XCD.  Adding the sums in LDS with
-// ds_add_f32 is no alternative to read and write: 18 times slower (measured alone).
-// Against the kernels that work triple by triple (whole input gradient, us): lmax 11, 12 channels, B = 100, layer 561 -> 450; lmax 20,
-// 16 channels, B = 32, layer 3960 -> 2290; lmax 15, 16 channels, B = 64, stand-alone 1760 -> 1420; lmax 10, 4 channels, B = 100,
-// stand-alone 116 -> 66, layer (two kernels before) 155 -> 66.
+// 1024 SIMDs; three waves a SIMD.  That takes 168 registers and spills 41 more to 148 bytes of scratch a lane (41 .. 45 whatever the
+// output channels; from lmax 16 on 256 registers, 25 .. 35 spilled; none at lmax 12..15, 216 .. 254 registers, two waves): the
+// kernel writes 161 MB there, of which 36 are partial gradients.  The loads of packed gO and weights come out of L1, which gives 64 bytes a
+// cycle to loads of 4 or 16 bytes a lane and half of that to 8 bytes, and out of L2, for which the work-groups of a sample stay on one
+// XCD.  Adding the sums in LDS with ds_add_f32 is no alternative to read and write: 18 times slower (measured alone).
+// Against the kernels that work triple by triple, us (whole call, operands packed by itself): lmax 11, 12 channels, B = 100, layer
+// 568 -> 427 (this kernel 391); lmax 20, 16 channels, B = 32, layer 4021 -> 2247; lmax 15, 16 channels, B = 64, stand-alone
+// 1623 -> 1361; lmax 10, 4 channels, B = 100, stand-alone 106 -> 59.
 #pragma once
 #include <utility>
 

@@ -563,7 +563,7 @@ def test_layer_forward_backward(dev, lmax, tin, tout, bsz, sparse, bn, fused):
 
 def test_layer_config5_shape(dev):
     """One 16 -> 16 channel layer of benchmark configuration 5 (L=20, default triples), B=1, one training step:
-    the three-tile matrix-core backward, the two-class forward launch and the stream join that shape takes."""
+    the three row tiles and the cut pairs of the backward, and the two-class forward launch that shape takes."""
     lmax, tau = 20, [16] * 21
     mod, ora, twin, w64 = build_layer_pair(dev, lmax, tau, tau, False, True, seed=20)
     x64 = rand_straight(tau, 1, seed=22)
