@@ -129,8 +129,10 @@ cg_backward_rows_kernel(const float2* __restrict__ part, float2* __restrict__ gF
     const int* begin = cum_rows + (L + 2);
     const int* at = begin + cum_rows[L + 1] + 1;
     const int lane = threadIdx.x & 63, b0 = __builtin_amdgcn_readfirstlane(b), b1 = min(__builtin_amdgcn_readlane(b, 63), B - 1);
-    // flags of the wave's samples: the first ones are fetched here and looked at behind the sums
-    int odd = b0 < B && lane < terms.nodd ? terms.odd[(size_t)b0 * terms.nGo + lane] : 0;
+    // flags of the wave's samples: the first 64 are fetched here and looked at behind the sums
+    const int nodd = terms.nodd, flags = (b1 - b0 + 1) * nodd;
+    auto flag = [&](int k) { return terms.odd[(size_t)(b0 + k / nodd) * terms.nGo + k % nodd]; };
+    int odd = lane < flags ? flag(lane) : 0;
     const int l = lookup_in_group(L + 1, e, [&](int k) { return meta[k]; }, s_tab);
     const int M = 2 * l + 1, rel = e - s_tab[l], t = rel / M, x = rel - t * M;
     const int row = cum_rows[l] + t, k0 = begin[row], k1 = b < B ? begin[row + 1] : k0;     // (lanes past the end fetch flags)
@@ -152,9 +154,8 @@ cg_backward_rows_kernel(const float2* __restrict__ part, float2* __restrict__ gF
             s.y += v.y;
         }
     }
-    if (terms.nodd) {
-        for (int bb = b0; bb <= b1; ++bb)
-            for (int k = lane + (bb == b0 ? 64 : 0); k < terms.nodd; k += 64) odd |= terms.odd[(size_t)bb * terms.nGo + k];
+    if (nodd) {
+        for (int k = lane + 64; k < flags; k += 64) odd |= flag(k);
         if (__builtin_expect(__any(odd), 0) && b < B && back_reached(terms, b, l, x - l)) s = make_float2(__builtin_nanf(""), __builtin_nanf(""));
     }
     if (b < B) gF[idx] = s;
