@@ -2,7 +2,7 @@
 #pragma once
 #include <vector>
 
-#include "common.h"
+#include "split.h"
 
 namespace cgnet {
 
@@ -34,6 +34,7 @@ struct BackPair {
     int inv_tau2, inv_M1, inv_M2;  // ceil(2^16 / tau2), ceil(2^20 / (2 l1 + 1)), ceil(2^20 / (2 l2 + 1))
     int ends;                      // bit 0 / 1: the first / last channel of a degree is the first / last of a sample's product
     int nbuf;                      // buffers of F1 rows
+    unsigned l8[kBackNL / 4];      // the output degrees again, a byte each
 };
 
 // One wave's share of a pair: tiles tile0, tile0 + tstep, ...  Its partial gradients inside a sample's: nrows rows of degree l1 per
@@ -74,10 +75,14 @@ struct BackGenPair {
 struct BackGenW {                  // of a (pair, degree): what packing its weights needs to know
     int chan0, nch;                // the triple's channels inside degree l: first, count
     int tO, cumW, K, cumT;         // degree l: output channels, complex offset of its weights, mid channels, first of them among all
-    int pairs, at;                 // pairs of steps, float offset of the first tile's first pair
+    int source, at;                // BackLink::source, float offset of the first tile's operands
     int ncol, ntiles, wtile;       // columns of a tile, tiles, floats from one tile to the next
-    int pad;
+    int scale;                     // kBackSplit: float offset of the first tile's scales
 };
+
+// Where the kernel's gradient of the product comes from: memory; packed gO and weights, multiplied in one to four pairs of steps (of
+// four output channels) of v_mfma_f32_16x16x4_f32, or as halves (split.h).
+constexpr int kBackMemory = 0, kBackSplit = 5;
 
 struct BackLink {
     bool ok = false;
@@ -87,9 +92,10 @@ struct BackLink {
     int* d_reach = nullptr;        // per (degree, output degree): the largest degree of the other fragment, -1: no such pair
     BackGenW* d_gens = nullptr;
     int ngens = 0, ndeg = 0;
-    int pairs = 0;                 // pairs of steps of the degree with most outputs
+    int source = 0;                // by the degree with most outputs, halves where the one with fewest allows it
     size_t w_floats = 0;           // packed weights
-    int go_floats = 0;             // packed gO of a sample, with the flags behind it
+    int go_degree = 0, go_floats = 0;      // packed gO of a degree, of a sample with the scales and flags behind it
+    int lanes = 64;                // lanes that hold places of output channels
     int nO = 0;                    // complex entries of one sample's layer output
     int most_B = 0;                // the largest batch it is taken for where there is another route
 };
@@ -115,9 +121,10 @@ __device__ __forceinline__ void pack_coef_back_block(const float* __restrict__ C
     }
 }
 
-// The weights of a (pair, degree) as right operands, tiles wave, wave + 4, ...: per tile and group of four degrees
-// [pair of steps][pair of degrees][lane (k, column)][degree][step], k = (output channel, re / im): W / max(eps, std) of the column's
-// channel, zero past t_O and past the tile's channels.
+// The weights of a (pair, degree) as right operands, tiles wave, wave + 4, ...: W / max(eps, std) of the column's channel, zero past t_O
+// and past the tile's channels.  As halves: per tile [degree][piece][lane (k, column)] of eight k = (output channel, re / im), then
+// [degree][column] scales.  For fp32 steps: per tile and group of four degrees
+// [pair of steps][pair of degrees][lane (k, column)][degree][step].
 __device__ __forceinline__ void pack_w_back_wave(const float2* __restrict__ W, const float* __restrict__ stds, float eps,
                                                  const BackGenW& g, int wave, int lane, float* __restrict__ Wp) {
     const int j = lane & 15, kk = lane >> 4;
@@ -127,7 +134,28 @@ __device__ __forceinline__ void pack_w_back_wave(const float2* __restrict__ W, c
         const int c = g.chan0 + cl;
         const float r = (on && stds) ? fmaxf(eps, stds[g.cumT + c]) : 1.f;
         float* dst = Wp + g.at + (size_t)tile * g.wtile + 4 * lane;
-        for (int s = 0; s < g.pairs; ++s) {
+        if (g.source == kBackSplit) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int to = 4 * kk + e;
+                float2 w = make_float2(0.f, 0.f);
+                if (on && to < g.tO) {
+                    w = W[g.cumW + (size_t)to * g.K + c];
+                    if (stds) w = make_float2(w.x / r, w.y / r);
+                }
+                v[2 * e] = w.x;
+                v[2 * e + 1] = w.y;
+            }
+            const int e = split_exponent(split_largest(v));
+            halfx8 p[2];
+            split8(v, e, p);
+            *reinterpret_cast<halfx8*>(dst) = p[0];
+            *reinterpret_cast<halfx8*>(dst + 256) = p[1];
+            if (kk == 0) Wp[g.scale + (size_t)tile * g.wtile + j] = split_scale(e);
+            continue;
+        }
+        for (int s = 0; s < g.source; ++s) {
             float v[2];
 #pragma unroll
             for (int e = 0; e < 2; ++e) {

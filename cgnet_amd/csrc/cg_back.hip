@@ -24,32 +24,57 @@ __device__ __forceinline__ bool finite(float2 z) {
     return (__float_as_uint(z.x) & 0x7f800000u) != 0x7f800000u && (__float_as_uint(z.y) & 0x7f800000u) != 0x7f800000u;
 }
 
-// Packed gO of the layer source: [chunk of eight M][degree][step][lane (k, (M, re / im))], k = (channel, re / im); zero past the
-// degree's channels and values, and in the place of entries that are not finite; behind it a flag per (chunk, degree): whether it has
-// such entries.  A work-group takes a (chunk, degree) of a sample.  degs: per degree cumO, t_O.
+// Packed gO of the layer source, k = (channel, re / im); zero past the degree's channels and values, and in the place of entries that are
+// not finite; behind it a flag per (chunk of eight M, degree): whether it has such entries.  A work-group takes a (chunk, degree) of a
+// sample.  degs: per degree cumO, t_O.
+// For fp32 steps: [chunk][degree][step][lane (k, (M, re / im))].  As halves: [degree][chunk][piece][lane (k, (M, re / im))] of eight k, then
+// [degree][chunk][M] scales.
 __global__ void __launch_bounds__(64)
-pack_go_back_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs, float* __restrict__ Go, int ndeg, int pairs,
-                    int grid0, int nO, int nGo) {
-    const int l = (int)blockIdx.x % ndeg, c = (int)blockIdx.x / ndeg;
+pack_go_back_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs, float* __restrict__ Go, int ndeg, int source, int grid0,
+                    int nO, int nGo) {
+    const int l = (int)blockIdx.x % ndeg, c = (int)blockIdx.x / ndeg, nchunks = (int)gridDim.x / ndeg;
     const int2 d = degs[l];
     const int lane = threadIdx.x, i = lane & 15, kk = lane >> 4;
     const int x = grid0 + 8 * c + (i >> 1) + l, r = i & 1;
     const float2* src = gO + (size_t)blockIdx.y * nO + d.x;
     float* const sample = Go + (size_t)blockIdx.y * nGo;
-    float* dst = sample + (size_t)blockIdx.x * 128 * pairs + lane;
     bool odd = false;
-    for (int s = 0; s < 2 * pairs; ++s) {
-        const int k = 4 * s + kk, to = k >> 1, sel = k & 1;
-        float v = 0.f;
-        if (to < d.y && x >= 0 && x <= 2 * l) {
-            const float2 z = src[to * (2 * l + 1) + x];
-            if (finite(z)) v = (r == sel) ? (r ? -z.x : z.x) : z.y;
-            else odd = true;
+    auto entry = [&](int to) {
+        if (to >= d.y || x < 0 || x > 2 * l) return make_float2(0.f, 0.f);
+        const float2 z = src[to * (2 * l + 1) + x];
+        if (finite(z)) return z;
+        odd = true;
+        return make_float2(0.f, 0.f);
+    };
+    size_t flags;
+    if (source == kBackSplit) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float2 z = entry(4 * kk + e);
+            v[2 * e] = r ? z.y : z.x;
+            v[2 * e + 1] = r ? -z.x : z.y;
         }
-        dst[64 * s] = v;
+        const int e = split_exponent(split_largest(v));
+        halfx8 p[2];
+        split8(v, e, p);
+        const size_t at = (size_t)(l * nchunks + c), scales = (size_t)gridDim.x * 512;
+        halfx8* dst = reinterpret_cast<halfx8*>(sample + 512 * at) + lane;
+        dst[0] = p[0];
+        dst[64] = p[1];
+        if (kk == 0 && r == 0) sample[scales + 8 * at + (i >> 1)] = split_scale(e);
+        flags = scales + 8 * (size_t)gridDim.x;
+    } else {
+        float* dst = sample + (size_t)blockIdx.x * 128 * source + lane;
+        for (int s = 0; s < 2 * source; ++s) {
+            const int k = 4 * s + kk, sel = k & 1;
+            const float2 z = entry(k >> 1);
+            dst[64 * s] = (r == sel) ? (r ? -z.x : z.x) : z.y;
+        }
+        flags = (size_t)gridDim.x * 128 * source;
     }
     odd = __any(odd);
-    if (lane == 0) reinterpret_cast<int*>(sample)[(size_t)gridDim.x * 128 * pairs + blockIdx.x] = odd;
+    if (lane == 0) reinterpret_cast<int*>(sample)[flags + blockIdx.x] = odd;
 }
 
 // What cg_backward_rows_kernel looks at where something is not finite.
@@ -177,12 +202,12 @@ constexpr int kVariantL[kVariants] = {7, 11, 15, kBackMaxL};
 // B = 64, cut at three: 1.08).
 constexpr int kVariantKS[kVariants] = {2, 3, 4, 4};
 
-const void* variant_kernel(int v, int pairs) {
-    return v == 0 ? back_kernel_0(pairs) : v == 1 ? back_kernel_1(pairs) : v == 2 ? back_kernel_2(pairs) : back_kernel_3(pairs);
+const void* variant_kernel(int v, int source) {
+    return v == 0 ? back_kernel_0(source) : v == 1 ? back_kernel_1(source) : v == 2 ? back_kernel_2(source) : back_kernel_3(source);
 }
 
-int launch_back(const BackSet& set, const BackLevel& lv, int pairs, BackArgs a, BackTerms t, float* d_gF, int L, hipStream_t s) {
-    a.pairs = set.d_pairs; a.units = lv.d_units; a.P = lv.P; a.grid0 = set.grid0;
+int launch_back(const BackSet& set, const BackLevel& lv, int source, BackArgs a, BackTerms t, float* d_gF, int L, hipStream_t s) {
+    a.pairs = set.d_pairs; a.units = lv.d_units; a.P = lv.P; a.grid0 = set.grid0; a.nchunks = set.nchunks;
     a.lds_wave = (int)(set.lds / (4 * kBackWaves));
     a.nunits = (int)lv.units.size();
     const int quads = (a.B + kBackWaves - 1) / kBackWaves;
@@ -190,7 +215,7 @@ int launch_back(const BackSet& set, const BackLevel& lv, int pairs, BackArgs a, 
                   a.nunits, quads);
     const dim3 grid((unsigned)(a.nunits * quads));
     auto* launch = set.variant == 0 ? back_launch_0 : set.variant == 1 ? back_launch_1 : set.variant == 2 ? back_launch_2 : back_launch_3;
-    launch(pairs, grid, set.lds, s, a);
+    launch(source, grid, set.lds, s, a);
     CGNET_HIP(hipGetLastError());
     t.pairs = set.d_pairs; t.grid0 = set.grid0;
     const size_t n = (size_t)a.nF * a.B;
@@ -283,6 +308,7 @@ int build_back_set(const std::vector<PairTriple>& triples, const std::vector<int
         for (int q = 0; q < p.nl; ++q) {
             const PairTriple& t = triples[order[from + q][4]];
             p.l[q] = t.l;
+            p.l8[q >> 2] |= (unsigned)t.l << (8 * (q & 3));
             p.cg[q] = t.cg;
             p.offFF[q] = t.offFF;
             if (p.offFF[q] == 0) p.ends |= 1;
@@ -428,7 +454,7 @@ int launch_back_memory(const BackSet& set, const BackLevel& lv, const float* d_F
     a.nF = nF; a.nFF = nFF; a.B = B;
     BackTerms t{};
     t.F = a.F; t.gFF = a.gFF; t.nFF = nFF; t.coef = d_coef;
-    return launch_back(set, lv, 0, a, t, d_gF, L, s);
+    return launch_back(set, lv, kBackMemory, a, t, d_gF, L, s);
 }
 
 // ---- layer source --------------------------------------------------------------------------------
@@ -451,13 +477,17 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
                   "the fused backward needs lmax <= %d and at most %d channels in every input degree", kBackMaxL, kBackMaxTau);
     CGNET_REQUIRE(wmm_gradff_operand_ok(w), CGNET_ERR_UNSUPPORTED, "the fused backward needs t_O <= 16 in every degree");
     link->nO = info[p->L].cumO + info[p->L].tO * (2 * p->L + 1);
-    // every degree takes the pairs of steps (four output channels each) of the one with most outputs
+    int most = 0;
     std::vector<int2> degs(p->L + 1);
     for (int l = 0; l <= p->L; ++l) {
         degs[l] = make_int2(info[l].cumO, info[l].tO);
-        link->pairs = std::max(link->pairs, std::max(1, (info[l].tO + 3) / 4));
+        most = std::max(most, info[l].tO);
     }
-    link->go_floats = set.nchunks * (p->L + 1) * 128 * link->pairs + (int)align_up(set.nchunks * (p->L + 1), 64);
+    const bool split = split_taken(p->L, [&](int l) { return info[l].tO; });
+    link->source = split ? kBackSplit : std::max(1, (most + 3) / 4);
+    link->lanes = split ? 16 * ((most + 3) / 4) : 64;
+    link->go_degree = split ? set.nchunks * 512 : 128 * link->source;
+    link->go_floats = set.nchunks * (p->L + 1) * (split ? 512 + 8 : 128 * link->source) + (int)align_up(set.nchunks * (p->L + 1), 64);
     std::vector<int> reach((p->L + 1) * (p->L + 1), -1);
     for (const BackPair& b : set.pairs)
         for (int q = 0; q < b.nl; ++q) {
@@ -473,27 +503,25 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
         BackGenPair& g = gps[k];
         g = BackGenPair{};
         g.w = (int)at;
-        for (int grp = 0; grp < b.nks; ++grp) {
-            const int n = std::min(4, b.nl - 4 * grp);
-            for (int q = 0; q < n; ++q) {
-                const int l = b.l[4 * grp + q];
-                BackGenW e{};
-                e.chan0 = (b.offFF[4 * grp + q] - p->cumFF[l]) / (2 * l + 1);
-                e.nch = b.tau1 * b.tau2;
-                e.tO = info[l].tO; e.cumW = info[l].cumW; e.K = info[l].K; e.cumT = info[l].cumT;
-                e.pairs = link->pairs;
-                e.at = (int)at + g.wtile + 256 * (q / 2) + 2 * (q & 1);
-                e.ncol = b.ncol;
-                e.ntiles = b.ntiles;
-                gens.push_back(e);
-            }
-            g.wtile += 512 * link->pairs;
+        g.wtile = split ? b.nl * (512 + 16) : b.nks * 512 * link->source;
+        for (int q = 0; q < b.nl; ++q) {
+            const int l = b.l[q];
+            BackGenW e{};
+            e.chan0 = (b.offFF[q] - p->cumFF[l]) / (2 * l + 1);
+            e.nch = b.tau1 * b.tau2;
+            e.tO = info[l].tO; e.cumW = info[l].cumW; e.K = info[l].K; e.cumT = info[l].cumT;
+            e.source = link->source;
+            e.at = (int)at + (split ? 512 * q : (q / 4) * 512 * link->source + 256 * (q / 2 % 2) + 2 * (q & 1));
+            e.scale = (int)at + 512 * b.nl + 16 * q;
+            e.ncol = b.ncol;
+            e.ntiles = b.ntiles;
+            e.wtile = g.wtile;
+            gens.push_back(e);
         }
-        for (size_t i = gens.size() - b.nl; i < gens.size(); ++i) gens[i].wtile = g.wtile;
         at += (size_t)g.wtile * b.ntiles;
         CGNET_REQUIRE(at < (1u << 30), CGNET_ERR_UNSUPPORTED, "packed weights of the fused backward exceed 2^30 floats");
     }
-    link->w_floats = at;
+    link->w_floats = at + 2 * 512;         // fetches run ahead of a tile's degrees
     link->ngens = (int)gens.size();
     size_t bytes = 0;
     auto place = [&](size_t n) { const size_t o = bytes; bytes += align_up(n, 256); return o; };
@@ -516,7 +544,7 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
     link->d_gens = reinterpret_cast<BackGenW*>(link->d_tables + at_gw);
     link->ndeg = p->L + 1;
     link->most_B = p->bwd_hybrid ? back_most_batch(set, p->L, p->nFF, (int)p->bwd_utasks.size(), kBackRuleLayer) : INT32_MAX;
-    if (int rc = raise_dynamic_lds(variant_kernel(set.variant, link->pairs), set.lds)) {
+    if (int rc = raise_dynamic_lds(variant_kernel(set.variant, link->source), set.lds)) {
         free_back_link(link);
         return rc;
     }
@@ -534,18 +562,20 @@ int launch_back_layer(const BackSet& set, const BackLink& link, const BackLevel&
                       const float* d_Wp, const float* d_coef, float* d_Go, float* d_part, float* d_gF, int L, int nF, int B,
                       hipStream_t s) {
     CGNET_REQUIRE(B <= 65535, CGNET_ERR_UNSUPPORTED, "B=%d above 65535", B);
-    const int per_chunk = link.ndeg * 128 * link.pairs;
+    const bool split = link.source == kBackSplit;
+    const int places = set.nchunks * link.ndeg;
     CGNET_LAUNCH(pack_go_back_kernel, dim3((unsigned)(set.nchunks * link.ndeg), (unsigned)B), dim3(64), 0, s, (const float2*)d_gO,
-                 link.d_degs, d_Go, link.ndeg, link.pairs, set.grid0, link.nO, link.go_floats);
+                 link.d_degs, d_Go, link.ndeg, link.source, set.grid0, link.nO, link.go_floats);
     CGNET_HIP(hipGetLastError());
     BackArgs a{};
     a.F = (const float2*)d_F; a.Go = d_Go; a.W = d_Wp; a.gp = link.d_gp;
     a.coef = d_coef; a.part = (float2*)d_part;
-    a.nF = nF; a.nGo = link.go_floats; a.go_chunk = per_chunk; a.go_degree = 128 * link.pairs; a.B = B;
+    a.nF = nF; a.nGo = link.go_floats; a.go_degree = link.go_degree; a.go_chunk = split ? 512 : link.ndeg * link.go_degree;
+    a.go_scales = 512 * places; a.lanes = link.lanes; a.B = B;
     BackTerms t{};
     t.gO = (const float2*)d_gO; t.degs = link.d_degs; t.reach = link.d_reach; t.nO = link.nO; t.ndeg = link.ndeg;
-    t.odd = reinterpret_cast<const int*>(d_Go) + (size_t)set.nchunks * per_chunk; t.nodd = set.nchunks * link.ndeg; t.nGo = link.go_floats;
-    return launch_back(set, lv, link.pairs, a, t, d_gF, L, s);
+    t.odd = reinterpret_cast<const int*>(d_Go) + (size_t)places * (split ? 512 + 8 : 128 * link.source); t.nodd = places; t.nGo = link.go_floats;
+    return launch_back(set, lv, link.source, a, t, d_gF, L, s);
 }
 
 }  // namespace cgnet

@@ -14,7 +14,7 @@ struct BackArgs {
     const BackPair* pairs;
     const BackUnit* units;
     float2* part;
-    int nF, nFF, go_chunk, go_degree, nGo, P, grid0, B, nunits, lds_wave;
+    int nF, nFF, go_chunk, go_degree, go_scales, lanes, nchunks, nGo, P, grid0, B, nunits, lds_wave;
 };
 
 // LDS of a wave (floats): sums [rows][kBackPitch] complex | a row of zeros | nbuf buffers of nrows rows of degree l1 between zeros (two
@@ -31,10 +31,10 @@ __host__ __device__ inline int back_lds_floats(int nch, int nt, int nrows, int n
     return (2 * (rows * kBackPitch - kBackSpare + (nbuf * nrows + 1) * back_row_pitch(rows) - 1) + 3) & ~3;
 }
 
-// a variant's kernel for the layer source with so many pairs of steps (0: memory source), and its launch
+// a variant's kernel for a source of the product's gradient (cg_back.h), and its launch
 #define CGNET_BACK_DECLARE(V)              \
-    const void* back_kernel_##V(int pairs); \
-    void back_launch_##V(int pairs, dim3 grid, size_t lds, hipStream_t s, const BackArgs& a);
+    const void* back_kernel_##V(int source); \
+    void back_launch_##V(int source, dim3 grid, size_t lds, hipStream_t s, const BackArgs& a);
 CGNET_BACK_DECLARE(0)
 CGNET_BACK_DECLARE(1)
 CGNET_BACK_DECLARE(2)

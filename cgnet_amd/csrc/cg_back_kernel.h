@@ -20,7 +20,8 @@
 // degree; four lane-group swaps per register set of four degrees turn it into right operands (lane group = degree).  It is read
 // from memory (the stand-alone operator: sixteen segments of 64 bytes per load instruction) or, inside the layer, made from
 // packed gO and packed weights by matrix instructions in the order of wmm_gradff_mfma_kernel, so that both sources hold the
-// same values to the bit.
+// same values to the bit; where every degree has nine output channels or more, as halves (split.h; lmax 20, 16 channels, B = 32:
+// 2180 -> 1940 us; lmax 11, 12 channels, B = 100: 392 -> 384).
 //
 // Bounded by issue where enough waves run: a vector multiply-add holds a SIMD for four cycles, a matrix instruction for 32, and the two
 // take turns.  lmax 11, 12 channels, B = 100, inside the layer: 8.6e7 vector and 1.1e7 matrix instructions, 75 % of the cycles of
@@ -72,6 +73,13 @@ __device__ __forceinline__ int opaque(int v) {
     return v;
 }
 
+// a pointer that is the same in all lanes, in scalar registers
+__device__ __forceinline__ const float* uniform(const float* p) {
+    const unsigned long long v = (unsigned long long)(uintptr_t)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (const float*)(uintptr_t)((unsigned long long)hi << 32 | lo);
+}
+
 // Four registers, lane groups of sixteen = four rows: register q, row a -> register a, row q.
 __device__ __forceinline__ void swap32(float& x, float& y) {
     const auto z = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
@@ -104,10 +112,13 @@ struct BackWave {
     pair_p p;
     const float* w;                // layer source: the tile's packed weights, the sample's packed gO
     const float* go;
+    const float* go_scales;
     const float2* gff;             // memory source: the sample's gFF
     const float* cp;               // coefficients of the current M
     int cstride;
     int w_group, go_chunk, go_degree;          // floats of a group of packed weights, of a chunk of packed gO, of a degree in it
+    unsigned l8[kBackNL / 4];      // output degrees, a byte each: a table in memory would cost a wait before every fetch
+    int lanes;                     // lanes that hold places of output channels
     int chan;                      // memory source: the lane's channel among those of the pair
     int last;                      // ... the last place in a sample with an entry behind it
     int lane, kk;
@@ -177,6 +188,38 @@ __device__ __forceinline__ void back_make(const BackWave& w, int chunk, int nd, 
             }
         CGNET_END;
     }
+}
+
+// The same from operands in halves.
+struct SplitOps { halfx8 a[2], b[2]; v2f sa; float sb; };
+
+template <int KS>
+__device__ __forceinline__ void back_make_split(const BackWave& w, int chunk, int nd, int nchunks, int nl, f32x4 (&r)[KS][4]) {
+    // The operands of a degree are fetched while those of the one before it are multiplied (places past the last degree: whatever
+    // lies there).
+    SplitOps ops[2] = {};
+    const bool on = w.lane < w.lanes;                              // places past the output channels stay zero
+    const float *go = w.go + 512 * chunk, *sa = w.go_scales + 8 * chunk, *wt = uniform(w.w);
+    auto load = [&](auto k, SplitOps& o) __attribute__((always_inline)) {
+        const unsigned l = (w.l8[k / 4] >> (8 * (k % 4))) & 255u;
+        if (on) {
+            CGNET_EACH(2, i) o.b[i] = reinterpret_cast<const halfx8*>(wt + 512 * k)[64 * i + w.lane]; CGNET_END;
+            CGNET_EACH(2, i) o.a[i] = reinterpret_cast<const halfx8*>(go + l * (unsigned)w.go_degree)[64 * i + w.lane]; CGNET_END;
+        }
+        o.sa = *reinterpret_cast<const v2f*>(sa + 8 * (l * (unsigned)nchunks) + 2 * w.kk);
+        o.sb = (wt + 512 * nl + 16 * k)[w.lane & 15];
+    };
+    load(std::integral_constant<int, 0>(), ops[0]);
+    CGNET_EACH(4 * KS, q)
+        if (q < nd) {
+            if constexpr (q + 1 < 4 * KS) load(std::integral_constant<int, q + 1>(), ops[1 - (q & 1)]);
+            __builtin_amdgcn_sched_barrier(0);
+            const SplitOps& o = ops[q & 1];
+            const f32x4 z = split_product(o.a, o.b);
+            const float s0 = o.sa.x * o.sb, s1 = o.sa.y * o.sb;
+            r[q / 4][q % 4] = (f32x4){z[0] * s0, z[1] * s0, z[2] * s1, z[3] * s1};
+        }
+    CGNET_END;
 }
 
 // Memory source: entries M0 + 2 kk, M0 + 2 kk + 1 of the lane's channel, degree k of the pair.  Where one of them is no value of the
@@ -277,7 +320,7 @@ __device__ __forceinline__ void back_chunk(BackWave& w, BackAcc<NT>& A, const f3
     w.s_at += 64u * kBackPitch;
 }
 
-template <int KS, int NT, int PAIRS>
+template <int KS, int NT, int SOURCE>
 __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const BackUnit& u, int b, float* lds, int lane) {
     const int j = lane & 15, kk = lane >> 4;
     const int l1 = p->l1, l2 = p->l2, M1 = 2 * l1 + 1, M2 = 2 * l2 + 1, tau2 = p->tau2, nrows = p->nrows;
@@ -323,12 +366,15 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
     CGNET_EACH(KS, ks) CGNET_EACH(4, q) G[ks][q] = (f32x4){0.f, 0.f, 0.f, 0.f}; CGNET_END; CGNET_END;
     BackWave w;
     w.p = p;
-    const gen_pair_p g = (gen_pair_p)(uintptr_t)(PAIRS > 0 ? a.gp + u.pair : nullptr);
-    w.w_group = 512 * PAIRS;
+    const gen_pair_p g = (gen_pair_p)(uintptr_t)(SOURCE != kBackMemory ? a.gp + u.pair : nullptr);
+    w.w_group = 512 * SOURCE;
+    w.go_scales = SOURCE == kBackSplit ? a.Go + (size_t)b * a.nGo + a.go_scales : nullptr;
+    w.lanes = a.lanes;
+    CGNET_EACH(kBackNL / 4, q) w.l8[q] = p->l8[q]; CGNET_END;
     w.go_chunk = a.go_chunk;
     w.go_degree = a.go_degree;
-    w.go = PAIRS > 0 ? a.Go + (size_t)b * a.nGo : nullptr;
-    w.gff = PAIRS > 0 ? nullptr : a.gFF + (size_t)b * a.nFF;
+    w.go = SOURCE != kBackMemory ? a.Go + (size_t)b * a.nGo : nullptr;
+    w.gff = SOURCE != kBackMemory ? nullptr : a.gFF + (size_t)b * a.nFF;
     w.cstride = p->nks * NT * 64;
     w.last = a.nFF - 2;
     w.lane = lane;
@@ -349,11 +395,11 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
             A.f1[rt][3 - v] = lds_get(w.f_at, 16 * (NT - 1 - rt) + 2 - v);
             A.s1r[rt][3 - v] = A.s1i[rt][3 - v] = 0.f;
         CGNET_END; CGNET_END;
-        w.w = PAIRS > 0 ? a.W + (g->w + tile * g->wtile) : nullptr;
+        w.w = SOURCE != kBackMemory ? a.W + (g->w + tile * g->wtile) : nullptr;
         // memory source: a lane past the last channel repeats the last row's of its t2
-        if constexpr (PAIRS == 0) w.chan = min(t1, p->tau1 - 1) * tau2 + (t1 < p->tau1 ? c0 + jj - t1 * tau2 : t2);
+        if constexpr (SOURCE == kBackMemory) w.chan = min(t1, p->tau1 - 1) * tau2 + (t1 < p->tau1 ? c0 + jj - t1 * tau2 : t2);
         // all loads of a chunk go out during the one before it where there are registers for them
-        constexpr bool AHEAD = PAIRS == 0 && KS + NT <= 6;
+        constexpr bool AHEAD = SOURCE == kBackMemory && KS + NT <= 6;
         const bool ends = (p->ends & 1 && c0 == 0) || (p->ends & 2 && c0 + ncol == C);
         f32x4 next[KS][4];
         if constexpr (AHEAD) {
@@ -363,8 +409,10 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
         for (int c = 0; c < p->nch; ++c) {
             const int steps8 = p->steps[c], tiles8 = p->tiles[c], nd = p->degs[c];
             const int Mc = M0 + 8 * c, c1 = min(c + 1, p->nch - 1), next_M0 = M0 + 8 * c1, next_nd = p->degs[c1];
-            if constexpr (PAIRS > 0) {
-                back_make<PAIRS, KS>(w, p->c0 + c, nd, G);
+            if constexpr (SOURCE == kBackSplit) {
+                back_make_split<KS>(w, p->c0 + c, nd, a.nchunks, p->nl, G);
+            } else if constexpr (SOURCE > 0) {
+                back_make<SOURCE, KS>(w, p->c0 + c, nd, G);
             } else {
                 CGNET_EACH(4 * KS, q)
                     if constexpr (AHEAD) G[q / 4][q % 4] = next[q / 4][q % 4];
@@ -429,8 +477,8 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
     }
 }
 
-template <int KS, int NTMAX, int PAIRS>
-__global__ void __launch_bounds__(kBackThreads, PAIRS == 0 ? (NTMAX == 1 ? 3 : 2) : NTMAX == 1 ? 4 : KS + NTMAX <= 5 ? 3 : 2)
+template <int KS, int NTMAX, int SOURCE>
+__global__ void __launch_bounds__(kBackThreads, SOURCE == kBackMemory ? (NTMAX == 1 ? 3 : 2) : NTMAX == 1 ? 4 : KS + NTMAX <= 5 ? 3 : 2)
 cg_backward_pair_kernel(BackArgs a) {
     extern __shared__ __align__(16) float back_lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -445,40 +493,42 @@ cg_backward_pair_kernel(BackArgs a) {
     const BackUnit u = {up4[0], up4[1], up4[2], up4[3], up4[4]};
     const pair_p p = (pair_p)(uintptr_t)(a.pairs + u.pair);
     float* lds = back_lds + wave * a.lds_wave;
-    if (NTMAX == 1 || p->nt == 1) back_unit<KS, 1, PAIRS>(a, p, u, b, lds, lane);
-    else if (NTMAX == 2 || p->nt == 2) back_unit<KS, NTMAX >= 2 ? 2 : 1, PAIRS>(a, p, u, b, lds, lane);
-    else back_unit<KS, NTMAX, PAIRS>(a, p, u, b, lds, lane);
+    if (NTMAX == 1 || p->nt == 1) back_unit<KS, 1, SOURCE>(a, p, u, b, lds, lane);
+    else if (NTMAX == 2 || p->nt == 2) back_unit<KS, NTMAX >= 2 ? 2 : 1, SOURCE>(a, p, u, b, lds, lane);
+    else back_unit<KS, NTMAX, SOURCE>(a, p, u, b, lds, lane);
 }
 
 template <int KS, int NT>
-const void* back_kernel(int pairs) {
-    return pairs == 0   ? (const void*)cg_backward_pair_kernel<KS, NT, 0>
-           : pairs == 1 ? (const void*)cg_backward_pair_kernel<KS, NT, 1>
-           : pairs == 2 ? (const void*)cg_backward_pair_kernel<KS, NT, 2>
-           : pairs == 3 ? (const void*)cg_backward_pair_kernel<KS, NT, 3>
-                        : (const void*)cg_backward_pair_kernel<KS, NT, 4>;
+const void* back_kernel(int source) {
+    return source == 0   ? (const void*)cg_backward_pair_kernel<KS, NT, 0>
+           : source == 1 ? (const void*)cg_backward_pair_kernel<KS, NT, 1>
+           : source == 2 ? (const void*)cg_backward_pair_kernel<KS, NT, 2>
+           : source == 3 ? (const void*)cg_backward_pair_kernel<KS, NT, 3>
+           : source == 4 ? (const void*)cg_backward_pair_kernel<KS, NT, 4>
+                         : (const void*)cg_backward_pair_kernel<KS, NT, kBackSplit>;
 }
 
 template <int KS, int NT>
-void back_launch(int pairs, dim3 grid, size_t lds, hipStream_t s, const BackArgs& a) {
+void back_launch(int source, dim3 grid, size_t lds, hipStream_t s, const BackArgs& a) {
     auto launch = [&](auto* cg_backward_pair_kernel) {
         CGNET_LAUNCH(cg_backward_pair_kernel, grid, dim3(kBackThreads), lds, s, a);
     };
-    switch (pairs) {
+    switch (source) {
         case 0: launch(&cg_backward_pair_kernel<KS, NT, 0>); break;
         case 1: launch(&cg_backward_pair_kernel<KS, NT, 1>); break;
         case 2: launch(&cg_backward_pair_kernel<KS, NT, 2>); break;
         case 3: launch(&cg_backward_pair_kernel<KS, NT, 3>); break;
-        default: launch(&cg_backward_pair_kernel<KS, NT, 4>); break;
+        case 4: launch(&cg_backward_pair_kernel<KS, NT, 4>); break;
+        default: launch(&cg_backward_pair_kernel<KS, NT, kBackSplit>); break;
     }
 }
 
 }  // namespace
 
 #define CGNET_BACK_VARIANT(V, KS, NT)                                                                              \
-    const void* back_kernel_##V(int pairs) { return back_kernel<KS, NT>(pairs); }                                  \
-    void back_launch_##V(int pairs, dim3 grid, size_t lds, hipStream_t s, const BackArgs& a) {                     \
-        back_launch<KS, NT>(pairs, grid, lds, s, a);                                                               \
+    const void* back_kernel_##V(int source) { return back_kernel<KS, NT>(source); }                                  \
+    void back_launch_##V(int source, dim3 grid, size_t lds, hipStream_t s, const BackArgs& a) {                     \
+        back_launch<KS, NT>(source, grid, lds, s, a);                                                               \
     }
 
 }  // namespace cgnet

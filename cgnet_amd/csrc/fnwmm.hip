@@ -15,6 +15,7 @@
 //   grad W  : the contraction runs over (b, m, re/im); lane (kk, i) reads complex entries
 //             8*blk + 2*kk, +1 of channel row i and feeds four k-steps.
 #include <algorithm>
+#include <cstdlib>
 #include <cstring>
 #include <iterator>
 #include <memory>
@@ -22,6 +23,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "split.h"
 
 namespace cgnet {
 namespace {
@@ -579,6 +581,37 @@ pack_w_gradff_kernel(const float2* __restrict__ W, const float* __restrict__ std
     *reinterpret_cast<float4*>(dst + 16) = make_float4(im[0], im[1], im[2], im[3]);
 }
 
+// The same as halves (split.h), a wave per tile of 16 channels: [piece][lane (k, channel)] of eight k, then the channels' scales.
+constexpr int kGffSplitBlocks = 9;             // blocks of 64 floats of a tile
+__global__ void __launch_bounds__(64)
+pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict__ stds, float eps, const WmmDeg* __restrict__ degs,
+                           int ndeg, float* __restrict__ Ap) {
+    __shared__ int s_tab[kMaxLookup];
+    const int blk = blockIdx.x * kGffSplitBlocks;
+    const WmmDeg d = degs[lookup_in_group(ndeg, blk, [&](int k) { return degs[k].ap_base; }, s_tab)];
+    const int lane = threadIdx.x, i = lane & 15, kk = lane >> 4, c = (blk - d.ap_base) / kGffSplitBlocks * 16 + i;
+    const float r = stds && c < d.K ? fmaxf(eps, stds[d.cumT + c]) : 1.f;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int to = 4 * kk + e;
+        float2 w = make_float2(0.f, 0.f);
+        if (to < d.tO && c < d.K) {
+            w = W[d.cumW + (size_t)to * d.K + c];
+            if (stds) w = make_float2(w.x / r, w.y / r);
+        }
+        v[2 * e] = w.x;
+        v[2 * e + 1] = w.y;
+    }
+    const int e = split_exponent(split_largest(v));
+    halfx8 p[2];
+    split8(v, e, p);
+    float* dst = Ap + (size_t)blk * 64;
+    reinterpret_cast<halfx8*>(dst)[lane] = p[0];
+    reinterpret_cast<halfx8*>(dst)[64 + lane] = p[1];
+    dst[512 + lane] = split_scale(e);
+}
+
 // Gradient with respect to FF on the matrix cores (t_O <= 16): gFF[c, (m, re/im)] = sum_k A[c, k] * B[k, (m, re/im)]
 // with k = (to, re/im).  A work-group is one wave (no barrier): it owns the up to 64 channels of its
 // unit as tiles of 16, keeps their A operands in registers and walks over the samples of its group.
@@ -588,10 +621,72 @@ pack_w_gradff_kernel(const float2* __restrict__ W, const float* __restrict__ std
 // NT = column tiles worked on together; ONE: these are all column tiles of the degree, so the B
 // operands are built once per sample and shared by the channel tiles.
 constexpr int kGffSub = 4;     // channel tiles per wave
+// lmax 11, 12 channels, B=50 (383 MB of gFF): fp32 steps 103 us, halves 82.
 // Waves wanted (at least eight groups of samples are made in any case), samples a wave keeps at least: it loads its operand
 // once.  lmax 10, layers of 12..3 channels, B=100 (112 units), us: 8 groups 151, 2048 waves 95, 4096 waves 84, 8192 waves 87.
 // Both gradients together, over the shapes named at kFwdSlices: 0.80 of the time, none slower by more than 5 %.
 constexpr int kGffFill = 4096, kGffMin = 2;
+// What a wave multiplies.  NKS steps of fp32: a tile's weights, a column tile's gO.
+template <int NKS>
+struct GffOps {
+    struct Left { float a[NKS]; };
+    struct Right { float b[NKS]; };
+    static __device__ __forceinline__ void load(const float* tile, int lane, Left& o) {
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) o.a[ks] = tile[64 * ks + lane];
+    }
+    // rows past t_O are those of the last channel, times zero weights; k = 4 ks + kk -> channel 2 ks + (kk >> 1), re / im kk & 1
+    static __device__ __forceinline__ void build(const float2* g, int M, int tO, int kk, int r, Right& o) {
+        const int to_lane = kk >> 1, sel = kk & 1;
+        const float cx = (r == sel) ? (r ? -1.f : 1.f) : 0.f, cy = (r == sel) ? 0.f : 1.f;   // B = cx * re + cy * im
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const float2 z = g[min(2 * ks + to_lane, tO - 1) * M];
+            o.b[ks] = fmaf(z.x, cx, z.y * cy);
+        }
+    }
+    static __device__ __forceinline__ f32x4 product(const Left& l, const Right& r) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) acc = mfma4(l.a[ks], r.b[ks], acc);
+        return acc;
+    }
+};
+// Halves: the operand of gO is split here, once for all channel tiles of the wave.
+template <>
+struct GffOps<kGffSplitBlocks> {
+    struct Left { halfx8 a[2]; f32x4 scale; };
+    struct Right { halfx8 b[2]; float scale; };
+    static __device__ __forceinline__ void load(const float* tile, int lane, Left& o) {
+        const halfx8* p = reinterpret_cast<const halfx8*>(tile);
+        o.a[0] = p[lane];
+        o.a[1] = p[64 + lane];
+        o.scale = *reinterpret_cast<const f32x4*>(tile + 512 + 4 * (lane >> 4));
+    }
+    static __device__ __forceinline__ void build(const float2* g, int M, int tO, int kk, int r, Right& o) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int to = 4 * kk + e;
+            float2 z = g[min(to, tO - 1) * M];
+            if (to >= tO) z = make_float2(0.f, 0.f);               // no part in the scale
+            v[2 * e] = r ? z.y : z.x;
+            v[2 * e + 1] = r ? -z.x : z.y;
+        }
+        const int e = split_exponent(split_largest(v));
+        split8(v, e, o.b);
+        o.scale = split_scale(e);
+    }
+    static __device__ __forceinline__ f32x4 product(const Left& l, const Right& r) {
+        f32x4 z = {0.f, 0.f, 0.f, 0.f};                            // (the products of split_product, operands exchanged: the same bits)
+        z = mfma_half(l.a[1], r.b[1], z);
+        z = mfma_half(l.a[0], r.b[1], z);
+        z = mfma_half(l.a[1], r.b[0], z);
+        z = mfma_half(l.a[0], r.b[0], z);
+        return (f32x4){z[0] * (l.scale[0] * r.scale), z[1] * (l.scale[1] * r.scale), z[2] * (l.scale[2] * r.scale),
+                       z[3] * (l.scale[3] * r.scale)};
+    }
+};
 template <int NKS, int NT, bool ONE>
 __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, const float* __restrict__ Ap,
                                                 float2* __restrict__ gFF, const WmmDeg& d, const WmmChanUnit& u, int B,
@@ -601,17 +696,13 @@ __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, c
     unsigned char* gobuf = mine + out_bytes;                                  // [2][go_bytes]
     const int i = lane & 15, kk = lane >> 4;
     const int M = d.M, tO = d.tO;
-    constexpr int nks = NKS;
     const int nsub = (u.nc + 15) >> 4;
-    float a[kGffSub][NKS];
+    using Ops = GffOps<NKS>;
+    typename Ops::Left a[kGffSub];
 #pragma unroll
     for (int sub = 0; sub < kGffSub; ++sub)
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks)
-            a[sub][ks] = sub < nsub ? Ap[((size_t)d.ap_base + (size_t)((u.c0 >> 4) + sub) * nks + ks) * 64 + lane] : 0.f;
-    // k = 4*ks + kk  ->  to = 2*ks + (kk >> 1), re/im = kk & 1;  column 16*ct + i -> m = 8*ct + (i >> 1), re/im = i & 1
-    const int to_lane = kk >> 1, sel = kk & 1, r = i & 1;
-    const float cx = (r == sel) ? (r ? -1.f : 1.f) : 0.f, cy = (r == sel) ? 0.f : 1.f;   // B = cx * re + cy * im
+        if (sub < nsub) Ops::load(Ap + ((size_t)d.ap_base + (size_t)((u.c0 >> 4) + sub) * NKS) * 64, lane, a[sub]);
+    const int r = i & 1;                          // column 16*ct + i -> m = 8*ct + (i >> 1), re/im = i & 1
     const int nct = (2 * M + 15) >> 4;
     const int n_go = tO * M;                      // complex entries of the gO rows
     const int b_begin = group * samples_per_group, b_end = min(B, b_begin + samples_per_group);
@@ -659,20 +750,11 @@ __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, c
         wait_vmcnt(b == b_begin ? 0 : later_stores + (b - 2 >= b_begin ? last_stores : 0));   // gO rows of sample b landed
         if (b + 1 < b_end) issue(b + 1, par ^ 1);
         const float2* g = reinterpret_cast<const float2*>(gobuf + (size_t)par * go_bytes);
-        float bv[NKS][NT];
+        typename Ops::Right bv[NT];
         auto build_b = [&](int ct0) {
-            int mofs[NT];
 #pragma unroll
-            for (int t = 0; t < NT; ++t) mofs[t] = min(8 * (ct0 + t) + (i >> 1), M - 1);   // clamped: extra columns are not stored
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-                const int to = min(2 * ks + to_lane, tO - 1);                 // clamped: rows past t_O carry zero weights
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const float2 z = g[to * M + mofs[t]];
-                    bv[ks][t] = fmaf(z.x, cx, z.y * cy);
-                }
-            }
+            for (int t = 0; t < NT; ++t)          // clamped: extra columns are not stored
+                Ops::build(g + min(8 * (ct0 + t) + (i >> 1), M - 1), M, tO, kk, r, bv[t]);
         };
         if (ONE) build_b(0);
 #pragma unroll
@@ -685,11 +767,7 @@ __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, c
                     if (!ONE) build_b(ct0);
                     f32x4 acc[NT];
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-                        for (int t = 0; t < NT; ++t) acc[t] = mfma4(a[sub][ks], bv[ks][t], acc[t]);
+                    for (int t = 0; t < NT; ++t) acc[t] = Ops::product(a[sub], bv[t]);
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
                         const int col = (ct0 + t) * 16 + i;
@@ -726,12 +804,7 @@ wmm_gradff_mfma_kernel(const float2* __restrict__ gO, const float* __restrict__ 
     const int nct = (2 * d.M + 15) >> 4;
     switch (d.nks_b) {
         CGNET_GFF(1) CGNET_GFF(2) CGNET_GFF(3) CGNET_GFF(4) CGNET_GFF(5) CGNET_GFF(6) CGNET_GFF(7)
-        default:
-            if (nct == 1) wmm_gradff_wave<8, 1, true>(CGNET_GFF_ARGS);
-            else if (nct == 2) wmm_gradff_wave<8, 2, true>(CGNET_GFF_ARGS);
-            else if (nct == 3) wmm_gradff_wave<8, 3, true>(CGNET_GFF_ARGS);
-            else wmm_gradff_wave<8, 3, false>(CGNET_GFF_ARGS);
-            break;
+        CGNET_GFF(8) CGNET_GFF(kGffSplitBlocks)
     }
 #undef CGNET_GFF_ARGS
 #undef CGNET_GFF
@@ -796,6 +869,9 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
     p->L = L;
     long long cFF = 0, cO = 0, cW = 0, cT = 0;
     int wp = 0;
+    // CGNET_BWD_PAIRS=0 (as in cgnet_cg_plan_create) keeps the fp32 steps in which the layer's kernel by triples makes the same gradient
+    const char* by_pairs = getenv("CGNET_BWD_PAIRS");
+    p->gff_split = split_taken(L, [&](int l) { return h_t_O[l]; }) && !(by_pairs && by_pairs[0] == '0');
     for (int l = 0; l <= L; ++l) {
         const int K = h_t_FF[l], tO = h_t_O[l], M = 2 * l + 1;
         CGNET_REQUIRE(K >= 0 && tO >= 0, CGNET_ERR_ARG, "negative channel count at degree %d", l);
@@ -818,7 +894,7 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
         }
         d.G = bestG;
         d.NC = bestNC;
-        d.nks_b = std::max(1, (2 * tO + 3) / 4);
+        d.nks_b = p->gff_split ? kGffSplitBlocks : std::max(1, (2 * tO + 3) / 4);
         d.ap_base = p->ap_blocks;
         p->ap_blocks += ((K + 15) / 16) * d.nks_b;
         if (tO > 16) p->gff_mfma = false;
@@ -1174,8 +1250,12 @@ extern "C" int cgnet_FN_WMM_backward(const cgnet_wmm_plan* plan, const float* d_
         if (plan->gff_mfma && plan->nW > 0 && plan->nO > 0) {
             float* Ap = (float*)d_workspace;
             const int total = plan->ap_blocks * 8;    // one thread per four weights
-            CGNET_LAUNCH(pack_w_gradff_kernel, dim3((total + 255) / 256), dim3(256), 0, s, (const float2*)d_W,
-                         bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap, plan->ap_blocks);
+            if (plan->gff_split)
+                CGNET_LAUNCH(pack_w_gradff_split_kernel, dim3(plan->ap_blocks / kGffSplitBlocks), dim3(64), 0, s, (const float2*)d_W,
+                             bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap);
+            else
+                CGNET_LAUNCH(pack_w_gradff_kernel, dim3((total + 255) / 256), dim3(256), 0, s, (const float2*)d_W,
+                             bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap, plan->ap_blocks);
             CGNET_HIP(hipGetLastError());
             const int units = (int)plan->gw_units_rc0.size();
             const int groups = std::max(std::min(B, 8), std::min((kGffFill + units - 1) / units, (B + kGffMin - 1) / kGffMin));

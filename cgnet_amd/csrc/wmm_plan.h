@@ -16,7 +16,7 @@ struct WmmDeg {
     int nrc;           // row chunks of 16 output channels
     int wp_base;       // first 64-float block of the degree in the packed weights
     int G, NC;         // forward: samples per work-group, 32-column chunks per wave
-    int nks_b;         // gradient wrt FF: k-steps of 4 over the 2*tO real rows (re, im interleaved)
+    int nks_b;         // gradient wrt FF: k-steps of 4 over the 2*tO real rows (re, im interleaved), or kGffSplitBlocks
     int ap_base;       // first 64-float block of the degree in the packed conj(W)/div operand
 };
 
@@ -40,6 +40,7 @@ struct cgnet_wmm_plan {
     int wp_blocks = 0;     // 64-float blocks of the packed forward weights
     int ap_blocks = 0;     // 64-float blocks of the packed operand of the FF-gradient kernel
     bool gff_mfma = true;  // every degree has t_O <= 16 (the operand then fits eight registers)
+    bool gff_split = false;// products of halves (split.h)
     int gw_ff_cap = 2, gw_go_cap = 2;   // LDS capacities (complex entries) of one stage of the weight-gradient kernel
     int maxK = 0;          // channels of the largest degree with outputs
     int fwd_stage_cap = 16;             // LDS bytes of one stage of one wave of the forward kernel
