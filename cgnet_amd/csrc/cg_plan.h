@@ -149,7 +149,6 @@ struct FwdMixTask {
 };
 
 struct FwdLaunch {
-    int T;                    // column tiles of 16 values of m of the launch's tasks
     int sel0, n;              // its tasks: entries [sel0, sel0 + n) of FwdLink::d_sel
     size_t lds;               // LDS bytes of a work-group
 };
