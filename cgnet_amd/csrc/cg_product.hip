@@ -18,7 +18,6 @@
 // and combines with a fixed DPP tree, so the result does not depend on scheduling.  Groups
 // write partial gradients that a second kernel adds in a fixed order.
 #include <algorithm>
-#include <cfloat>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -27,7 +26,6 @@
 #include <vector>
 
 #include "internal.h"
-#include "split.h"
 
 namespace cgnet {
 namespace {
@@ -319,13 +317,11 @@ __host__ __device__ inline size_t fwd_task_lds_mm(const CgTask& t) {
 // One sample of a task: the waves take the values of m in turn (from the middle outwards, so that every wave gets
 // long and short ones); for one m the accumulator D[t1][t2] gathers the steps of four m2.
 // STATS: the lane also adds |z| and |z|^2 of its four results (channels (4 kk + v, i)) to its own sums.
-// LARGEST: `largest` is the largest modulus of a part of the lane's results (of the results of others where it stores none).
-template <bool STATS, bool LARGEST = false>
+template <bool STATS>
 __device__ __forceinline__ void fwd_mm_sample(const CgTask& t, const float* __restrict__ cg, int P,
                                               const float2* __restrict__ f1, const float2* __restrict__ f2,
                                               float2* __restrict__ out, int wave, int nwaves, int lane,
-                                              double (&s1)[4], double (&s2)[4], float* largest = nullptr) {
-    float top = 0.f;
+                                              double (&s1)[4], double (&s2)[4]) {
     const int l = t.l, l1 = t.l1, l2 = t.l2;
     const int M = 2 * l + 1, M1 = 2 * l1 + 1, M2 = 2 * l2 + 1;
     const int rows = t.rows, tau2 = t.tau2;
@@ -379,10 +375,6 @@ __device__ __forceinline__ void fwd_mm_sample(const CgTask& t, const float* __re
             dre = mfma4(nai, fb.y, dre);
             dim = mfma4(ai, fb.x, dim);
         }
-        if (LARGEST) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) top = fmaxf(fmaxf(top, fabsf(dre[v])), fabsf(dim[v]));
-        }
         if (i < tau2) {
             // re and im go out as two 4-byte writes (one two-address LDS instruction): an 8-byte write would first
             // copy the pair into adjacent registers
@@ -405,7 +397,6 @@ __device__ __forceinline__ void fwd_mm_sample(const CgTask& t, const float* __re
             }
         }
     }
-    if (LARGEST) *largest = top;
 }
 
 constexpr int kFwdMmThreads = 512;
@@ -512,51 +503,28 @@ cg_forward_mm_kernel(const float2* __restrict__ F, float2* __restrict__ FF, cons
     }
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-
 // ---- inference forward of the whole layer: the product tile is mixed while it lies in LDS -------------------------
 // cg_forward_mm_kernel whose tile never leaves for memory: when a sample's tile of a task is complete, the eight waves
 // multiply it with the task's slice of the weights, O_part[to, m] = sum over the tile's channels c of
 // (W[to, c] / div[c]) FF[c, m], on the matrix cores (rows = the up to 16 output channels, columns = one or two tiles of 16
-// values of m with re / im of a column in one lane, reduction over the channels in steps of 32), and what leaves
+// values of m with re / im of a column in one lane, reduction over the channels in steps of four), and what leaves
 // is the task's t_O x (2l+1) partial output, a twelfth of the tile.  cgbn_forward_reduce_kernel adds the partial
 // outputs of a degree's tasks in channel order.  A wave has a role (column tile, share of the reduction steps) and
-// keeps its share of the weights in registers for all samples of the group; the shares meet in LDS and are added while the
-// next sample's fragments are multiplied.  Statistics cannot be taken on this route (the mixing needs the stds of the whole
+// keeps its share of the packed weights in registers for all samples of the group; the shares meet in LDS and are added while
+// the next sample's fragments are multiplied.  Statistics cannot be taken on this route (the mixing needs the stds of the whole
 // batch before the first tile): it serves evaluation mode and layers without fragment norm.
-// The mixing takes products of halves (split.h): the weights of a wave's share are split once for all samples, the tile's entries as they
-// are read, both scaled by the largest of all (an entry keeps its full precision down to 2^-16 of it); the product's waves find the tile's
-// largest modulus among their accumulators.  A tile that is not finite is mixed by the fp32 instructions.
-// lmax 11, 12 channels, B = 100, evaluation step: fp32 instructions for the mixing as well 408 us, halves 364, and one launch for
-// tasks of one and of two column tiles, seven shares instead of four where there is one, 354.  Three work-groups a compute unit (80 registers):
-// one spilled register is reloaded behind the next sample's copies and costs more than it holds (31 spilled: 395 us).  What bounds it now:
-// the product's fp32 matrix instructions and the vector instructions, in turn (78 % of the cycles before the last step).
-constexpr int kMixChannels = 32;               // channels of a step
-constexpr int kMixMaxSteps = 2;                // steps of one wave (64 channels)
-__host__ __device__ constexpr int mix_shares(int T) { return T == 1 ? 7 : 4; }   // of the steps of a column tile, at most
+// The mixing stays on the fp32 instructions.  The entries of a tile and the weights of a share may lie any number of powers of two apart
+// (a channel of small entries has large weights / std), and 16-bit operands would have to hold them all: three bfloat16 pieces, which do,
+// want 48 registers for the weights of a share (lmax 11, 12 channels, B = 100, evaluation step: 481 us at three work-groups a compute
+// unit with 45 registers spilled, 446 at two); two scaled f16 pieces (352) lose what lies 2^16 and more below the largest of the tile, and
+// showing for each sample that nothing did leaves 375, and 576 where it cannot be shown.  Fp32: a launch for each number of column
+// tiles and a barrier behind the shares 408, one launch and the shares added while the next sample runs 398.
+// What bounds it: the fp32 matrix instructions of product and mixing and the vector instructions, which take turns.
+constexpr int kMixMaxK = 16;                   // reduction steps of one wave (64 channels)
+constexpr int kMixShares = 4;                  // shares of the reduction steps of a column tile: one wave per SIMD
 constexpr size_t kMixShareBytes = 2048;        // a share's 16 x 16 complex partial sums
-constexpr size_t kMixTopBytes = 128;           // largest moduli: eight waves x four groups of sixteen lanes
 
-__host__ __device__ constexpr size_t mix_red_bytes(int T) { return (size_t)T * (mix_shares(T) - 1) * kMixShareBytes + kMixTopBytes; }
-
-// largest of a row of sixteen lanes, in all of them
-__device__ __forceinline__ float row_largest(float v) {
-    v = fmaxf(v, dpp_move<0xB1>(v));
-    v = fmaxf(v, dpp_move<0x4E>(v));
-    v = fmaxf(v, dpp_move<0x141>(v));
-    return fmaxf(v, dpp_move<0x140>(v));
-}
-__device__ __forceinline__ float read_lane(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
-
-// The lane's eight entries of a step, four channels apart: re (part 0) or im (1).  Channels past the tile's last repeat it (their
-// weights are zero).  (A second body without the comparison for steps that are whole: 365 -> 374 us at lmax 11, 12 channels, B = 100.)
-__device__ __forceinline__ void mix_read(unsigned at, unsigned step, unsigned last, int part, float (&x)[8]) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j, at += step) x[j] = lds_f(min(at, last))[part];
-}
+__host__ __device__ constexpr size_t mix_red_bytes(int T) { return (size_t)T * (kMixShares - 1) * kMixShareBytes; }
 
 __global__ void __launch_bounds__(kFwdMmThreads, 6)
 cgbn_forward_fused_kernel(const float2* __restrict__ F, const float* __restrict__ CG, const CgTask* __restrict__ tasks,
@@ -580,7 +548,6 @@ cgbn_forward_fused_kernel(const float2* __restrict__ F, const float* __restrict_
     float* cg = reinterpret_cast<float*>(frag + 2 * frag_bytes + out_bytes);
     const int T = (M + 15) >> 4;                                   // column tiles of 16 values of m: 1 or 2
     float4* red = reinterpret_cast<float4*>(smem + lds_bytes - mix_red_bytes(T));   // [share - 1][column tile][2][64]
-    float* tops = reinterpret_cast<float*>(smem + lds_bytes - kMixTopBytes);        // [wave][4]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     {
@@ -605,40 +572,16 @@ cgbn_forward_fused_kernel(const float2* __restrict__ F, const float* __restrict_
         const int m1 = (r - t.l) - (c - t.l2);
         cg[r * P + c] = (m1 >= -t.l1 && m1 <= t.l1) ? CG[t.cg_off + e] : 0.f;
     }
-    // Role of the wave in the mixing: column tile tcol, share kh of the steps.  As many shares as there are steps, so that the waves of a
-    // tile hold one step each where the waves suffice (two at most); the others only take part in the product.
-    const int nst = (g.nks + 7) >> 3, shares = min(nst, mix_shares(T));
+    // Role of the wave in the mixing: column tile tcol, share kh of the reduction steps.  Four shares put one wave of
+    // a column tile on every SIMD; with one column tile the other four waves only take part in the product.
     const int tcol = T == 1 ? 0 : wave & 1, kh = T == 1 ? wave : wave >> 1;
-    const bool mixing = kh < shares;
-    const int st0 = mixing ? (kh * nst) / shares : 0, st1 = mixing ? ((kh + 1) * nst) / shares : 0;
-    const int ks0 = 8 * st0, cnt = st1 - st0;                      // <= kMixMaxSteps (the plan checks)
-    // the lane's eight weights of a step: channels 4 j + kk, j = 0 .. 7 (zero behind the task's last)
-    const float2* wmine = reinterpret_cast<const float2*>(Af + g.aoff) + (size_t)ks0 * 64;
-    halfx8 wre[kMixMaxSteps][2], wim[kMixMaxSteps][2];
-    int we;
-    bool wfinite;
-    {
-        float re[kMixMaxSteps][8], im[kMixMaxSteps][8], top = 0.f;
+    const bool mixing = kh < kMixShares && g.nks > 0;
+    const int ks0 = mixing ? (kh * g.nks) / kMixShares : 0, ks1 = mixing ? ((kh + 1) * g.nks) / kMixShares : 0;
+    const int cnt = ks1 - ks0;                                     // <= kMixMaxK (the plan checks)
+    float2 a[kMixMaxK];
 #pragma unroll
-        for (int st = 0; st < kMixMaxSteps; ++st)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const bool on = st < cnt && ks0 + 8 * st + j < g.nks;
-                const float2 v = on ? wmine[(8 * st + j) * 64 + lane] : make_float2(0.f, 0.f);
-                re[st][j] = v.x;
-                im[st][j] = v.y;
-                top = fmaxf(fmaxf(top, fabsf(v.x)), fabsf(v.y));
-            }
-        top = row_largest(top);
-        top = fmaxf(fmaxf(read_lane(top, 0), read_lane(top, 16)), fmaxf(read_lane(top, 32), read_lane(top, 48)));
-        wfinite = top <= FLT_MAX;
-        we = __builtin_amdgcn_readfirstlane(split_exponent(top));
-#pragma unroll
-        for (int st = 0; st < kMixMaxSteps; ++st) {
-            split8(re[st], we, wre[st]);
-            split8(im[st], we, wim[st]);
-        }
-    }
+    for (int j = 0; j < kMixMaxK; ++j)
+        a[j] = j < cnt ? reinterpret_cast<const float2*>(Af + g.aoff)[(size_t)(ks0 + j) * 64 + lane] : make_float2(0.f, 0.f);
     const int i = lane & 15, kk = lane >> 4;
     const int col = 16 * tcol + i;
     const unsigned pb_last = lds_addr(out + (nch - 1) * M + min(col, M - 1));
@@ -650,7 +593,7 @@ cgbn_forward_fused_kernel(const float2* __restrict__ F, const float* __restrict_
     // Partial output of a sample whose shares have been written: the wave that holds share 0 of its column tile adds the others in order.
     auto finish = [&](int b) {
         if (kh != 0 || g.tO == 0) return;
-        for (int k = 1; k < shares; ++k) {
+        for (int k = 1; k < kMixShares; ++k) {
             const f32x4* theirs = reinterpret_cast<const f32x4*>(red + ((k - 1) * T + tcol) * 128);
             re += theirs[lane];
             im += theirs[64 + lane];
@@ -672,55 +615,24 @@ cgbn_forward_fused_kernel(const float2* __restrict__ F, const float* __restrict_
         if (b > b0) finish(b - 1);
         const float2* f1 = reinterpret_cast<const float2*>(frag + par * frag_bytes);
         const float2* f2 = reinterpret_cast<const float2*>(frag + par * frag_bytes + f1_bytes);
-        float top;
-        fwd_mm_sample<false, true>(t, cg, P, f1, f2, out, wave, kFwdMmThreads / 64, lane, dummy1, dummy2, &top);
-        top = row_largest(top);
-        if (i == 0) tops[4 * wave + kk] = top;
+        fwd_mm_sample<false>(t, cg, P, f1, f2, out, wave, kFwdMmThreads / 64, lane, dummy1, dummy2);
         lds_barrier();         // the tile is complete
-        re = im = (f32x4){0.f, 0.f, 0.f, 0.f};
         if (mixing) {
-            top = row_largest(tops[lane & 31]);
-            top = fmaxf(read_lane(top, 0), read_lane(top, 16));
+            f32x4 yr = {0.f, 0.f, 0.f, 0.f}, yi = yr;
+            re = im = yr;
             unsigned pb = opaque(pb_first);
-            if (wfinite && top <= FLT_MAX) {
-                const int e = __builtin_amdgcn_readfirstlane(split_exponent(top));
-                const float scale = read_lane(split_scale(-e), 0);
 #pragma unroll
-                for (int st = 0; st < kMixMaxSteps; ++st) {
-                    if (st < cnt) {
-                        // re, then im: one of the two in registers at a time
-                        float x[8];
-                        halfx8 p[2];
-                        mix_read(pb, pb_step, pb_last, 0, x);
-                        split8_scaled(x, scale, p);
-                        re = split_product(wre[st], p, re);
-                        im = split_product(wim[st], p, im);
-                        __builtin_amdgcn_sched_barrier(0);
-                        mix_read(pb, pb_step, pb_last, 1, x);
-                        split8_scaled(x, scale, p);
-                        im = split_product(wre[st], p, im);
-                        p[0] = -p[0];
-                        p[1] = -p[1];
-                        re = split_product(wim[st], p, re);
-                        pb += 8 * pb_step;
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                }
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    re[v] = __builtin_amdgcn_ldexpf(re[v], -e - we);
-                    im[v] = __builtin_amdgcn_ldexpf(im[v], -e - we);
-                }
-            } else {
-                for (int ks = ks0; ks < min(8 * st1, g.nks); ++ks) {
-                    const float2 a = wmine[(ks - ks0) * 64 + (int)opaque(lane)], v = lds_c(min(pb, pb_last), 0);
+            for (int j = 0; j < kMixMaxK; ++j)
+                if (j < cnt) {
+                    const float2 v = lds_c(min(pb, pb_last), 0);   // channels past the tile's last meet zero weights
                     pb += pb_step;
-                    re = mfma4(a.x, v.x, re);
-                    re = mfma4(-a.y, v.y, re);
-                    im = mfma4(a.x, v.y, im);
-                    im = mfma4(a.y, v.x, im);
+                    re = mfma4(a[j].x, v.x, re);
+                    im = mfma4(a[j].x, v.y, im);
+                    yr = mfma4(a[j].y, v.x, yr);
+                    yi = mfma4(a[j].y, v.y, yi);
                 }
-            }
+            re -= yi;
+            im += yr;
         }
         if (mixing && kh > 0) {
             float4* mine = red + ((kh - 1) * T + tcol) * 128;
@@ -769,6 +681,11 @@ stats_reduce_kernel(const double* __restrict__ part, double* __restrict__ sums, 
 }
 
 // ----------------------------------------------------------------------------------- backward
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
 // Sum over aligned groups of RW consecutive lanes; every lane of the group receives the sum.
 // Must be executed by all lanes of the wave.
 template <int RW>
@@ -3170,7 +3087,7 @@ int build_fwd_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, FwdLink* lin
         const CgTask& t = p->fwd_tasks[k];
         const WmmDegInfo& d = info[t.l];
         const int nch = t.rows * t.tau2, M = 2 * t.l + 1;
-        CGNET_REQUIRE(nch <= mix_shares(2) * kMixMaxSteps * kMixChannels, CGNET_ERR_UNSUPPORTED, "a product tile of %d channels exceeds the mixing registers", nch);
+        CGNET_REQUIRE(nch <= 4 * kMixMaxK * kMixShares, CGNET_ERR_UNSUPPORTED, "a product tile of %d channels exceeds the mixing registers", nch);
         FwdMixTask g{};
         g.aoff = (int)aoff;
         g.nks = d.tO > 0 ? (nch + 3) / 4 : 0;
@@ -3221,7 +3138,7 @@ int build_fwd_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, FwdLink* lin
             sel.push_back(i);
         }
         fl.n = (int)sel.size() - fl.sel0;
-        fl.lds = p->fwd_class_lds[k] + std::max(mix_red_bytes(1), mix_red_bytes(T));
+        fl.lds = p->fwd_class_lds[k] + mix_red_bytes(T);
         if (fl.n == 0) continue;
         lds_max = std::max(lds_max, fl.lds);
         tmp.launches.push_back(fl);

@@ -66,25 +66,6 @@ __device__ __forceinline__ void split8(const float (&x)[8], int e, halfx8 (&p)[2
         p[1][q] = (_Float16)(s - (float)p[0][q]);
     }
 }
-// As split8, by an exponent's scale; the rest of an entry is one mixed fma, s - (float)h, exact: fewer registers than the second
-// conversion, conversion back and subtraction that the arithmetic becomes.
-__device__ __forceinline__ void split8_scaled(const float (&x)[8], float scale, halfx8 (&p)[2]) {
-    typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 h, l;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const f32x2 s = {x[2 * q] * scale, x[2 * q + 1] * scale};
-        h[q] = __builtin_bit_cast(unsigned, __builtin_convertvector(s, halfx2));
-        f32x2 r;
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r.x) : "v"(h[q]), "v"(s.x));
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r.y) : "v"(h[q]), "v"(s.y));
-        l[q] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, halfx2));
-    }
-    p[0] = __builtin_bit_cast(halfx8, h);
-    p[1] = __builtin_bit_cast(halfx8, l);
-}
 #endif
 
 }  // namespace cgnet
