@@ -77,12 +77,12 @@ struct BackGenW {                  // of a (pair, degree): what packing its weig
     int tO, cumW, K, cumT;         // degree l: output channels, complex offset of its weights, mid channels, first of them among all
     int source, at;                // BackLink::source, float offset of the first tile's operands
     int ncol, ntiles, wtile;       // columns of a tile, tiles, floats from one tile to the next
-    int scale;                     // kBackSplit: float offset of the first tile's scales
 };
 
 // Where the kernel's gradient of the product comes from: memory; packed gO and weights, multiplied in one to four pairs of steps (of
-// four output channels) of v_mfma_f32_16x16x4_f32, or as halves (split.h).
+// four output channels) of v_mfma_f32_16x16x4_f32, or as pieces (split.h: floats of an operand, of the scales of a chunk of eight M).
 constexpr int kBackMemory = 0, kBackSplit = 5;
+constexpr int kBackOperand = 256 * kPieces, kBackScales = 8;
 
 struct BackLink {
     bool ok = false;
@@ -92,9 +92,9 @@ struct BackLink {
     int* d_reach = nullptr;        // per (degree, output degree): the largest degree of the other fragment, -1: no such pair
     BackGenW* d_gens = nullptr;
     int ngens = 0, ndeg = 0;
-    int source = 0;                // by the degree with most outputs, halves where the one with fewest allows it
+    int source = 0;                // by the degree with most outputs, pieces where the one with fewest allows it
     size_t w_floats = 0;           // packed weights
-    int go_degree = 0, go_floats = 0;      // packed gO of a degree, of a sample with the scales and flags behind it
+    int go_degree = 0, go_flags = 0, go_floats = 0;    // packed gO of a degree, of a sample up to its flags, with scales and flags
     int lanes = 64;                // lanes that hold places of output channels
     int nO = 0;                    // complex entries of one sample's layer output
     int most_B = 0;                // the largest batch it is taken for where there is another route
@@ -122,8 +122,8 @@ __device__ __forceinline__ void pack_coef_back_block(const float* __restrict__ C
 }
 
 // The weights of a (pair, degree) as right operands, tiles wave, wave + 4, ...: W / max(eps, std) of the column's channel, zero past t_O
-// and past the tile's channels.  As halves: per tile [degree][piece][lane (k, column)] of eight k = (output channel, re / im), then
-// [degree][column] scales.  For fp32 steps: per tile and group of four degrees
+// and past the tile's channels.  As pieces: per tile [degree][piece][lane (k, column)] of eight k = (output channel, re / im).  For fp32
+// steps: per tile and group of four degrees
 // [pair of steps][pair of degrees][lane (k, column)][degree][step].
 __device__ __forceinline__ void pack_w_back_wave(const float2* __restrict__ W, const float* __restrict__ stds, float eps,
                                                  const BackGenW& g, int wave, int lane, float* __restrict__ Wp) {
@@ -147,12 +147,10 @@ __device__ __forceinline__ void pack_w_back_wave(const float2* __restrict__ W, c
                 v[2 * e] = w.x;
                 v[2 * e + 1] = w.y;
             }
-            const int e = split_exponent(split_largest(v));
-            halfx8 p[2];
-            split8(v, e, p);
-            *reinterpret_cast<halfx8*>(dst) = p[0];
-            *reinterpret_cast<halfx8*>(dst + 256) = p[1];
-            if (kk == 0) Wp[g.scale + (size_t)tile * g.wtile + j] = split_scale(e);
+            bf16x8 p[kPieces];
+            split8_weights(v, p);
+#pragma unroll
+            for (int k = 0; k < kPieces; ++k) *reinterpret_cast<bf16x8*>(dst + 256 * k) = p[k];
             continue;
         }
         for (int s = 0; s < g.source; ++s) {

@@ -25,56 +25,85 @@ __device__ __forceinline__ bool finite(float2 z) {
 }
 
 // Packed gO of the layer source, k = (channel, re / im); zero past the degree's channels and values, and in the place of entries that are
-// not finite; behind it a flag per (chunk of eight M, degree): whether it has such entries.  A work-group takes a (chunk, degree) of a
-// sample.  degs: per degree cumO, t_O.
-// For fp32 steps: [chunk][degree][step][lane (k, (M, re / im))].  As halves: [degree][chunk][piece][lane (k, (M, re / im))] of eight k, then
-// [degree][chunk][M] scales.
-__global__ void __launch_bounds__(64)
-pack_go_back_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs, float* __restrict__ Go, int ndeg, int source, int grid0,
-                    int nO, int nGo) {
-    const int l = (int)blockIdx.x % ndeg, c = (int)blockIdx.x / ndeg, nchunks = (int)gridDim.x / ndeg;
-    const int2 d = degs[l];
-    const int lane = threadIdx.x, i = lane & 15, kk = lane >> 4;
-    const int x = grid0 + 8 * c + (i >> 1) + l, r = i & 1;
-    const float2* src = gO + (size_t)blockIdx.y * nO + d.x;
-    float* const sample = Go + (size_t)blockIdx.y * nGo;
+// not finite; behind it a flag per (chunk of eight M, degree): whether it has such entries.  degs: per degree cumO, t_O.
+struct GoEntries {
+    const float2* src;
+    int l, tO, x;
     bool odd = false;
-    auto entry = [&](int to) {
-        if (to >= d.y || x < 0 || x > 2 * l) return make_float2(0.f, 0.f);
+    __device__ __forceinline__ GoEntries(const float2* gO, int2 d, int l, int M) : src(gO + d.x), l(l), tO(d.y), x(M + l) {}
+    __device__ __forceinline__ float2 operator()(int to) {
+        if (to >= tO || x < 0 || x > 2 * l) return make_float2(0.f, 0.f);
         const float2 z = src[to * (2 * l + 1) + x];
         if (finite(z)) return z;
         odd = true;
         return make_float2(0.f, 0.f);
-    };
-    size_t flags;
-    if (source == kBackSplit) {
-        float v[8];
+    }
+};
+
+// For fp32 steps: [chunk][degree][step][lane (k, (M, re / im))].  A work-group takes a (chunk, degree) of a sample.
+__global__ void __launch_bounds__(64)
+pack_go_back_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs, float* __restrict__ Go, int ndeg, int pairs, int grid0,
+                    int nO, int nGo) {
+    const int l = (int)blockIdx.x % ndeg, c = (int)blockIdx.x / ndeg;
+    const int lane = threadIdx.x, i = lane & 15, kk = lane >> 4, r = i & 1;
+    GoEntries entry(gO + (size_t)blockIdx.y * nO, degs[l], l, grid0 + 8 * c + (i >> 1));
+    float* const sample = Go + (size_t)blockIdx.y * nGo;
+    float* dst = sample + (size_t)blockIdx.x * 128 * pairs + lane;
+    for (int s = 0; s < 2 * pairs; ++s) {
+        const int k = 4 * s + kk, sel = k & 1;
+        const float2 z = entry(k >> 1);
+        dst[64 * s] = (r == sel) ? (r ? -z.x : z.x) : z.y;
+    }
+    const int odd = __any(entry.odd);
+    if (lane == 0) reinterpret_cast<int*>(sample)[(size_t)gridDim.x * 128 * pairs + blockIdx.x] = odd;
+}
+
+// As pieces: [degree][chunk][piece][lane (k, (M, re / im))] of eight k, then [chunk][M] scales: the degrees share one, so that the pair
+// kernel holds it for a chunk (a scale for each degree: 74 instead of 46 registers spilled at lmax 8..11, layer of 12 channels at lmax 11,
+// B = 100: 1199 us a step instead of 1029).  A work-group takes a chunk of a sample, its waves the degrees in turn.
+constexpr int kPackGoWaves = 8;
+__global__ void __launch_bounds__(64 * kPackGoWaves)
+pack_go_back_split_kernel(const float2* __restrict__ gO, const int2* __restrict__ degs, float* __restrict__ Go, int ndeg, int grid0, int nO,
+                          int nGo) {
+    __shared__ float s_top[kPackGoWaves][16];
+    const int c = (int)blockIdx.x, nchunks = (int)gridDim.x, places = nchunks * ndeg;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, kk = lane >> 4, r = i & 1;
+    float* const sample = Go + (size_t)blockIdx.y * nGo;
+    int* const flags = reinterpret_cast<int*>(sample) + kBackOperand * places + kBackScales * nchunks + c * ndeg;
+    constexpr int kMost = (kBackMaxL + kPackGoWaves) / kPackGoWaves;       // degrees of a wave
+    float v[kMost][8], top = 0.f;
+#pragma unroll
+    for (int n = 0; n < kMost; ++n) {
+        const int l = wave + n * kPackGoWaves;
+        if (l >= ndeg) break;
+        GoEntries entry(gO + (size_t)blockIdx.y * nO, degs[l], l, grid0 + 8 * c + (i >> 1));
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const float2 z = entry(4 * kk + e);
-            v[2 * e] = r ? z.y : z.x;
-            v[2 * e + 1] = r ? -z.x : z.y;
+            v[n][2 * e] = r ? z.y : z.x;
+            v[n][2 * e + 1] = r ? -z.x : z.y;
         }
-        const int e = split_exponent(split_largest(v));
-        halfx8 p[2];
-        split8(v, e, p);
-        const size_t at = (size_t)(l * nchunks + c), scales = (size_t)gridDim.x * 512;
-        halfx8* dst = reinterpret_cast<halfx8*>(sample + 512 * at) + lane;
-        dst[0] = p[0];
-        dst[64] = p[1];
-        if (kk == 0 && r == 0) sample[scales + 8 * at + (i >> 1)] = split_scale(e);
-        flags = scales + 8 * (size_t)gridDim.x;
-    } else {
-        float* dst = sample + (size_t)blockIdx.x * 128 * source + lane;
-        for (int s = 0; s < 2 * source; ++s) {
-            const int k = 4 * s + kk, sel = k & 1;
-            const float2 z = entry(k >> 1);
-            dst[64 * s] = (r == sel) ? (r ? -z.x : z.x) : z.y;
-        }
-        flags = (size_t)gridDim.x * 128 * source;
+        top = fmaxf(top, split_largest(v[n]));
+        const int odd = __any(entry.odd);
+        if (lane == 0) flags[l] = odd;
     }
-    odd = __any(odd);
-    if (lane == 0) reinterpret_cast<int*>(sample)[flags + blockIdx.x] = odd;
+    if (lane < 16) s_top[wave][lane] = top;                        // (the same for both columns of an M)
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kPackGoWaves; ++w) top = fmaxf(top, s_top[w][i]);
+    const int e = split_exponent(top);
+    if (wave == 0 && lane < 16 && r == 0) sample[kBackOperand * places + kBackScales * c + (i >> 1)] = split_scale(-e);
+    const float scale = split_scale(e);
+#pragma unroll
+    for (int n = 0; n < kMost; ++n) {
+        const int l = wave + n * kPackGoWaves;
+        if (l >= ndeg) break;
+        bf16x8 p[kPieces];
+        split8(v[n], scale, p);
+        bf16x8* dst = reinterpret_cast<bf16x8*>(sample + (size_t)kBackOperand * (l * nchunks + c)) + lane;
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) dst[64 * k] = p[k];
+    }
 }
 
 // What cg_backward_rows_kernel looks at where something is not finite.
@@ -207,7 +236,7 @@ const void* variant_kernel(int v, int source) {
 }
 
 int launch_back(const BackSet& set, const BackLevel& lv, int source, BackArgs a, BackTerms t, float* d_gF, int L, hipStream_t s) {
-    a.pairs = set.d_pairs; a.units = lv.d_units; a.P = lv.P; a.grid0 = set.grid0; a.nchunks = set.nchunks;
+    a.pairs = set.d_pairs; a.units = lv.d_units; a.P = lv.P; a.grid0 = set.grid0;
     a.lds_wave = (int)(set.lds / (4 * kBackWaves));
     a.nunits = (int)lv.units.size();
     const int quads = (a.B + kBackWaves - 1) / kBackWaves;
@@ -486,8 +515,10 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
     const bool split = split_taken(p->L, [&](int l) { return info[l].tO; });
     link->source = split ? kBackSplit : std::max(1, (most + 3) / 4);
     link->lanes = split ? 16 * ((most + 3) / 4) : 64;
-    link->go_degree = split ? set.nchunks * 512 : 128 * link->source;
-    link->go_floats = set.nchunks * (p->L + 1) * (split ? 512 + 8 : 128 * link->source) + (int)align_up(set.nchunks * (p->L + 1), 64);
+    const int places = set.nchunks * (p->L + 1);
+    link->go_degree = split ? set.nchunks * kBackOperand : 128 * link->source;
+    link->go_flags = split ? places * kBackOperand + set.nchunks * kBackScales : places * 128 * link->source;
+    link->go_floats = (int)align_up(link->go_flags + places, 64);
     std::vector<int> reach((p->L + 1) * (p->L + 1), -1);
     for (const BackPair& b : set.pairs)
         for (int q = 0; q < b.nl; ++q) {
@@ -503,7 +534,7 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
         BackGenPair& g = gps[k];
         g = BackGenPair{};
         g.w = (int)at;
-        g.wtile = split ? b.nl * (512 + 16) : b.nks * 512 * link->source;
+        g.wtile = split ? b.nl * kBackOperand : b.nks * 512 * link->source;
         for (int q = 0; q < b.nl; ++q) {
             const int l = b.l[q];
             BackGenW e{};
@@ -511,8 +542,7 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
             e.nch = b.tau1 * b.tau2;
             e.tO = info[l].tO; e.cumW = info[l].cumW; e.K = info[l].K; e.cumT = info[l].cumT;
             e.source = link->source;
-            e.at = (int)at + (split ? 512 * q : (q / 4) * 512 * link->source + 256 * (q / 2 % 2) + 2 * (q & 1));
-            e.scale = (int)at + 512 * b.nl + 16 * q;
+            e.at = (int)at + (split ? kBackOperand * q : (q / 4) * 512 * link->source + 256 * (q / 2 % 2) + 2 * (q & 1));
             e.ncol = b.ncol;
             e.ntiles = b.ntiles;
             e.wtile = g.wtile;
@@ -521,7 +551,7 @@ int build_back_link(const cgnet_cg_plan* p, const cgnet_wmm_plan* w, BackLink* l
         at += (size_t)g.wtile * b.ntiles;
         CGNET_REQUIRE(at < (1u << 30), CGNET_ERR_UNSUPPORTED, "packed weights of the fused backward exceed 2^30 floats");
     }
-    link->w_floats = at + 2 * 512;         // fetches run ahead of a tile's degrees
+    link->w_floats = at + 2 * kBackOperand;         // fetches run ahead of a tile's degrees
     link->ngens = (int)gens.size();
     size_t bytes = 0;
     auto place = [&](size_t n) { const size_t o = bytes; bytes += align_up(n, 256); return o; };
@@ -564,17 +594,21 @@ int launch_back_layer(const BackSet& set, const BackLink& link, const BackLevel&
     CGNET_REQUIRE(B <= 65535, CGNET_ERR_UNSUPPORTED, "B=%d above 65535", B);
     const bool split = link.source == kBackSplit;
     const int places = set.nchunks * link.ndeg;
-    CGNET_LAUNCH(pack_go_back_kernel, dim3((unsigned)(set.nchunks * link.ndeg), (unsigned)B), dim3(64), 0, s, (const float2*)d_gO,
-                 link.d_degs, d_Go, link.ndeg, link.source, set.grid0, link.nO, link.go_floats);
+    if (split)
+        CGNET_LAUNCH(pack_go_back_split_kernel, dim3((unsigned)set.nchunks, (unsigned)B), dim3(64 * kPackGoWaves), 0, s, (const float2*)d_gO,
+                     link.d_degs, d_Go, link.ndeg, set.grid0, link.nO, link.go_floats);
+    else
+        CGNET_LAUNCH(pack_go_back_kernel, dim3((unsigned)(set.nchunks * link.ndeg), (unsigned)B), dim3(64), 0, s, (const float2*)d_gO,
+                     link.d_degs, d_Go, link.ndeg, link.source, set.grid0, link.nO, link.go_floats);
     CGNET_HIP(hipGetLastError());
     BackArgs a{};
     a.F = (const float2*)d_F; a.Go = d_Go; a.W = d_Wp; a.gp = link.d_gp;
     a.coef = d_coef; a.part = (float2*)d_part;
-    a.nF = nF; a.nGo = link.go_floats; a.go_degree = link.go_degree; a.go_chunk = split ? 512 : link.ndeg * link.go_degree;
-    a.go_scales = 512 * places; a.lanes = link.lanes; a.B = B;
+    a.nF = nF; a.nGo = link.go_floats; a.go_degree = link.go_degree; a.go_chunk = split ? kBackOperand : link.ndeg * link.go_degree;
+    a.go_scales = kBackOperand * places; a.lanes = link.lanes; a.B = B;
     BackTerms t{};
     t.gO = (const float2*)d_gO; t.degs = link.d_degs; t.reach = link.d_reach; t.nO = link.nO; t.ndeg = link.ndeg;
-    t.odd = reinterpret_cast<const int*>(d_Go) + (size_t)places * (split ? 512 + 8 : 128 * link.source); t.nodd = places; t.nGo = link.go_floats;
+    t.odd = reinterpret_cast<const int*>(d_Go) + link.go_flags; t.nodd = places; t.nGo = link.go_floats;
     return launch_back(set, lv, link.source, a, t, d_gF, L, s);
 }
 

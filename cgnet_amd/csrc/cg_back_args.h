@@ -14,7 +14,7 @@ struct BackArgs {
     const BackPair* pairs;
     const BackUnit* units;
     float2* part;
-    int nF, nFF, go_chunk, go_degree, go_scales, lanes, nchunks, nGo, P, grid0, B, nunits, lds_wave;
+    int nF, nFF, go_chunk, go_degree, go_scales, lanes, nGo, P, grid0, B, nunits, lds_wave;
 };
 
 // LDS of a wave (floats): sums [rows][kBackPitch] complex | a row of zeros | nbuf buffers of nrows rows of degree l1 between zeros (two

@@ -20,8 +20,7 @@
 // degree; four lane-group swaps per register set of four degrees turn it into right operands (lane group = degree).  It is read
 // from memory (the stand-alone operator: sixteen segments of 64 bytes per load instruction) or, inside the layer, made from
 // packed gO and packed weights by matrix instructions in the order of wmm_gradff_mfma_kernel, so that both sources hold the
-// same values to the bit; where every degree has nine output channels or more, as halves (split.h; lmax 20, 16 channels, B = 32:
-// 2180 -> 1940 us; lmax 11, 12 channels, B = 100: 392 -> 384).
+// same values to the bit; where every degree has nine output channels or more, in bfloat16 pieces (split.h).
 //
 // Bounded by issue where enough waves run: a vector multiply-add holds a SIMD for four cycles, a matrix instruction for 32, and the two
 // take turns.  lmax 11, 12 channels, B = 100, inside the layer: 8.6e7 vector and 1.1e7 matrix instructions, 75 % of the cycles of
@@ -190,24 +189,23 @@ __device__ __forceinline__ void back_make(const BackWave& w, int chunk, int nd, 
     }
 }
 
-// The same from operands in halves.
-struct SplitOps { halfx8 a[2], b[2]; v2f sa; float sb; };
+// The same from operands in pieces.
+struct SplitOps { bf16x8 a[kPieces], b[kPieces]; };
 
 template <int KS>
-__device__ __forceinline__ void back_make_split(const BackWave& w, int chunk, int nd, int nchunks, int nl, f32x4 (&r)[KS][4]) {
+__device__ __forceinline__ void back_make_split(const BackWave& w, int chunk, int nd, f32x4 (&r)[KS][4]) {
     // The operands of a degree are fetched while those of the one before it are multiplied (places past the last degree: whatever
     // lies there).
     SplitOps ops[2] = {};
     const bool on = w.lane < w.lanes;                              // places past the output channels stay zero
-    const float *go = w.go + 512 * chunk, *sa = w.go_scales + 8 * chunk, *wt = uniform(w.w);
+    const float *go = w.go + kBackOperand * chunk, *wt = uniform(w.w);
+    const v2f scale = *reinterpret_cast<const v2f*>(w.go_scales + kBackScales * chunk + 2 * w.kk);
     auto load = [&](auto k, SplitOps& o) __attribute__((always_inline)) {
         const unsigned l = (w.l8[k / 4] >> (8 * (k % 4))) & 255u;
         if (on) {
-            CGNET_EACH(2, i) o.b[i] = reinterpret_cast<const halfx8*>(wt + 512 * k)[64 * i + w.lane]; CGNET_END;
-            CGNET_EACH(2, i) o.a[i] = reinterpret_cast<const halfx8*>(go + l * (unsigned)w.go_degree)[64 * i + w.lane]; CGNET_END;
+            CGNET_EACH(kPieces, i) o.b[i] = reinterpret_cast<const bf16x8*>(wt + kBackOperand * k)[64 * i + w.lane]; CGNET_END;
+            CGNET_EACH(kPieces, i) o.a[i] = reinterpret_cast<const bf16x8*>(go + l * (unsigned)w.go_degree)[64 * i + w.lane]; CGNET_END;
         }
-        o.sa = *reinterpret_cast<const v2f*>(sa + 8 * (l * (unsigned)nchunks) + 2 * w.kk);
-        o.sb = (wt + 512 * nl + 16 * k)[w.lane & 15];
     };
     load(std::integral_constant<int, 0>(), ops[0]);
     CGNET_EACH(4 * KS, q)
@@ -216,8 +214,7 @@ __device__ __forceinline__ void back_make_split(const BackWave& w, int chunk, in
             __builtin_amdgcn_sched_barrier(0);
             const SplitOps& o = ops[q & 1];
             const f32x4 z = split_product(o.a, o.b);
-            const float s0 = o.sa.x * o.sb, s1 = o.sa.y * o.sb;
-            r[q / 4][q % 4] = (f32x4){z[0] * s0, z[1] * s0, z[2] * s1, z[3] * s1};
+            r[q / 4][q % 4] = (f32x4){z[0] * scale.x, z[1] * scale.x, z[2] * scale.y, z[3] * scale.y};
         }
     CGNET_END;
 }
@@ -410,7 +407,7 @@ __device__ __forceinline__ void back_unit(const BackArgs& a, pair_p p, const Bac
             const int steps8 = p->steps[c], tiles8 = p->tiles[c], nd = p->degs[c];
             const int Mc = M0 + 8 * c, c1 = min(c + 1, p->nch - 1), next_M0 = M0 + 8 * c1, next_nd = p->degs[c1];
             if constexpr (SOURCE == kBackSplit) {
-                back_make_split<KS>(w, p->c0 + c, nd, a.nchunks, p->nl, G);
+                back_make_split<KS>(w, p->c0 + c, nd, G);
             } else if constexpr (SOURCE > 0) {
                 back_make<SOURCE, KS>(w, p->c0 + c, nd, G);
             } else {

@@ -581,8 +581,8 @@ pack_w_gradff_kernel(const float2* __restrict__ W, const float* __restrict__ std
     *reinterpret_cast<float4*>(dst + 16) = make_float4(im[0], im[1], im[2], im[3]);
 }
 
-// The same as halves (split.h), a wave per tile of 16 channels: [piece][lane (k, channel)] of eight k, then the channels' scales.
-constexpr int kGffSplitBlocks = 9;             // blocks of 64 floats of a tile
+// The same as pieces (split.h), a wave per tile of 16 channels: [piece][lane (k, channel)] of eight k.
+constexpr int kGffSplitBlocks = 4 * kPieces;   // blocks of 64 floats of a tile
 __global__ void __launch_bounds__(64)
 pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict__ stds, float eps, const WmmDeg* __restrict__ degs,
                            int ndeg, float* __restrict__ Ap) {
@@ -603,13 +603,10 @@ pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict
         v[2 * e] = w.x;
         v[2 * e + 1] = w.y;
     }
-    const int e = split_exponent(split_largest(v));
-    halfx8 p[2];
-    split8(v, e, p);
-    float* dst = Ap + (size_t)blk * 64;
-    reinterpret_cast<halfx8*>(dst)[lane] = p[0];
-    reinterpret_cast<halfx8*>(dst)[64 + lane] = p[1];
-    dst[512 + lane] = split_scale(e);
+    bf16x8 p[kPieces];
+    split8_weights(v, p);
+#pragma unroll
+    for (int k = 0; k < kPieces; ++k) reinterpret_cast<bf16x8*>(Ap + (size_t)blk * 64)[64 * k + lane] = p[k];
 }
 
 // Gradient with respect to FF on the matrix cores (t_O <= 16): gFF[c, (m, re/im)] = sum_k A[c, k] * B[k, (m, re/im)]
@@ -621,7 +618,7 @@ pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict
 // NT = column tiles worked on together; ONE: these are all column tiles of the degree, so the B
 // operands are built once per sample and shared by the channel tiles.
 constexpr int kGffSub = 4;     // channel tiles per wave
-// lmax 11, 12 channels, B=50 (383 MB of gFF): fp32 steps 103 us, halves 82.
+// lmax 11, 12 channels, B=50 (383 MB of gFF): fp32 steps 100 us, pieces 84.
 // Waves wanted (at least eight groups of samples are made in any case), samples a wave keeps at least: it loads its operand
 // once.  lmax 10, layers of 12..3 channels, B=100 (112 units), us: 8 groups 151, 2048 waves 95, 4096 waves 84, 8192 waves 87.
 // Both gradients together, over the shapes named at kFwdSlices: 0.80 of the time, none slower by more than 5 %.
@@ -652,16 +649,14 @@ struct GffOps {
         return acc;
     }
 };
-// Halves: the operand of gO is split here, once for all channel tiles of the wave.
+// Pieces: the operand of gO is split here, once for all channel tiles of the wave.
 template <>
 struct GffOps<kGffSplitBlocks> {
-    struct Left { halfx8 a[2]; f32x4 scale; };
-    struct Right { halfx8 b[2]; float scale; };
+    struct Left { bf16x8 a[kPieces]; };
+    struct Right { bf16x8 b[kPieces]; float scale; };
     static __device__ __forceinline__ void load(const float* tile, int lane, Left& o) {
-        const halfx8* p = reinterpret_cast<const halfx8*>(tile);
-        o.a[0] = p[lane];
-        o.a[1] = p[64 + lane];
-        o.scale = *reinterpret_cast<const f32x4*>(tile + 512 + 4 * (lane >> 4));
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) o.a[k] = reinterpret_cast<const bf16x8*>(tile)[64 * k + lane];
     }
     static __device__ __forceinline__ void build(const float2* g, int M, int tO, int kk, int r, Right& o) {
         float v[8];
@@ -674,17 +669,17 @@ struct GffOps<kGffSplitBlocks> {
             v[2 * e + 1] = r ? -z.x : z.y;
         }
         const int e = split_exponent(split_largest(v));
-        split8(v, e, o.b);
-        o.scale = split_scale(e);
+        split8(v, split_scale(e), o.b);
+        o.scale = split_scale(-e);
     }
     static __device__ __forceinline__ f32x4 product(const Left& l, const Right& r) {
         f32x4 z = {0.f, 0.f, 0.f, 0.f};                            // (the products of split_product, operands exchanged: the same bits)
-        z = mfma_half(l.a[1], r.b[1], z);
-        z = mfma_half(l.a[0], r.b[1], z);
-        z = mfma_half(l.a[1], r.b[0], z);
-        z = mfma_half(l.a[0], r.b[0], z);
-        return (f32x4){z[0] * (l.scale[0] * r.scale), z[1] * (l.scale[1] * r.scale), z[2] * (l.scale[2] * r.scale),
-                       z[3] * (l.scale[3] * r.scale)};
+        z = mfma_piece(l.a[0], r.b[2], z);
+        z = mfma_piece(l.a[2], r.b[0], z);
+        z = mfma_piece(l.a[1], r.b[1], z);
+        z = mfma_piece(l.a[0], r.b[1], z);
+        z = mfma_piece(l.a[1], r.b[0], z);
+        return mfma_piece(l.a[0], r.b[0], z) * r.scale;
     }
 };
 template <int NKS, int NT, bool ONE>

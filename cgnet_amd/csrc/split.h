@@ -1,26 +1,29 @@
-// Products of fp32 operands on the half-precision matrix instructions.
+// Products of fp32 operands on the 16-bit matrix instructions.
 //
 // v_mfma_f32_16x16x4_f32 holds a SIMD's vector ALUs for its 32 cycles: it and vector instructions take turns.
-// v_mfma_f32_16x16x32_f16 takes 16 cycles for eight times the terms and runs beside vector instructions of other waves.  (Probe, eight
-// waves a compute unit, half of them vector and half matrix, us: vector half alone 177, fp32 matrix half alone 216, both 383; the same
-// with 16-bit matrix instructions 177, 234, 248.)
+// v_mfma_f32_16x16x32_bf16 takes 16 cycles for eight times the terms and runs beside vector instructions of other waves.
 //
-// The left operand's rows and the right operand's columns are scaled by powers of two to a largest entry in [2^14, 2^15), and an entry is
-// the sum of two halves h + l (11 + 11 bits and l's sign, the rest rounded off: at most 2^-23 of the entry's leading place or 2^-39 of the
-// row's largest entry).  The four products ll + lh + hl + hh are exact and summed in fp32, and the result is scaled back.  Sums of 32
-// products of normal numbers against 64 bits, rms error over rms: eight chained fp32 instructions 1.03e-7, this 0.77e-7 (0.88e-7 without
-// ll); factors spread log-normally by e^2: 1.11e-7 and 0.66e-7.  The error hardly depends on the number of products, that of the fp32
-// chain grows with its root: up to eight (complex) channels the fp32 instructions stay, which are also few then.  Three bfloat16 pieces
-// in six products (0.38e-7, no scaling) take half as many bytes again for no less time: lmax 20, 16 channels, B = 32, three layers:
-// fp32 6540 us, bfloat16 5660 .. 5830, halves 5840; lmax 11, 12 channels, B = 100: 392, 380, 384.
+// An operand is the sum of three bfloat16 pieces h + m + l, which hold its 24 bits, and six of the nine products (ml, lm and ll, together
+// at most 2^-23 of the product and mostly far less, are left out) are summed in fp32.  bfloat16 has the exponents of fp32: an entry keeps its
+// bits whatever lies beside it, down to 2^-110 (below, an absolute error of 2^-134).  gO, whose size follows the loss, is scaled by a power
+// of two where its largest entry is below 2^-16, to [2^-17, 2^-16): entries down to 2^-93 of that one keep their bits, and products with
+// weights of any size stay in range until the result is scaled back.
+// gFF against 64 bits (rms, lmax 11, whether or not the output channels are spread over six decades): 9 channels 7.8e-8 by fp32 instructions,
+// 3.5e-8 by pieces, 12 channels 8.9e-8 and 3.6e-8, 16 channels 10.2e-8 and 3.8e-8.
+// Backward by pairs (cg_back_kernel.h), fp32 instructions -> pieces, us: lmax 11, 12 channels, B = 100: 390 -> 377; lmax 20, 16 channels,
+// B = 32: 2136 -> 1976; gFF alone, lmax 11, 12 channels, B = 50: 100 -> 84.  Two f16 pieces with a scale for each row and column took 381,
+// 1921 and 79, but lost what lay 2^16 and more below the largest of its row or column: output channels spread over ten decades, with
+// weights and gO that balance each other, came back with an error of 3e-3.
 #pragma once
 #include "common.h"
 
 namespace cgnet {
 
-// The 32 places of a product are (output channel, re / im).  Whether halves take the place of fp32 for output channels `t` of the degrees
-// 0 .. L: every degree that has any has at least nine.  (gFF against 64 bits, rms, fp32 and halves: 9 channels 8.2e-8 and 8.0e-8, 12
-// 9.3e-8 and 7.9e-8, 16 10.6e-8 and 8.1e-8, but 12, 7, 6, 5, 4 ... 3 channels 6.0e-8 and 7.5e-8.)
+// The 32 places of a product are (output channel, re / im).  Whether pieces take the place of fp32 for output channels `t` of the degrees
+// 0 .. L: every degree that has any has at least nine.  Up to eight the fp32 instructions are four at most, and a third of the operands to
+// load.  Whole step, B = 100, lmax 11, fp32 -> pieces, us: layer of 5 channels 278 -> 292, 8 channels 624 -> 650, 9 channels 796 -> 795;
+// mixing alone, 8 channels 372 -> 379, 9 channels 505 -> 505.
+constexpr int kPieces = 3;
 constexpr int kSplitFrom = 9, kSplitMax = 16;
 template <typename Count>
 bool split_taken(int L, Count&& t) {
@@ -33,16 +36,20 @@ bool split_taken(int L, Count&& t) {
 }
 
 #ifdef __HIPCC__
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ f32x4 mfma_half(halfx8 a, halfx8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+__device__ __forceinline__ f32x4 mfma_piece(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ f32x4 split_product(const halfx8 (&a)[2], const halfx8 (&b)[2], f32x4 c = {0.f, 0.f, 0.f, 0.f}) {
-    c = mfma_half(a[1], b[1], c);
-    c = mfma_half(a[1], b[0], c);
-    c = mfma_half(a[0], b[1], c);
-    return mfma_half(a[0], b[0], c);
+// a: gO, b: weights, small products first
+__device__ __forceinline__ f32x4 split_product(const bf16x8 (&a)[kPieces], const bf16x8 (&b)[kPieces]) {
+    f32x4 c = {0.f, 0.f, 0.f, 0.f};
+    c = mfma_piece(a[2], b[0], c);
+    c = mfma_piece(a[0], b[2], c);
+    c = mfma_piece(a[1], b[1], c);
+    c = mfma_piece(a[1], b[0], c);
+    c = mfma_piece(a[0], b[1], c);
+    return mfma_piece(a[0], b[0], c);
 }
 
 // largest modulus of the lane's numbers and of those in the lanes of the other three groups of sixteen
@@ -53,18 +60,47 @@ __device__ __forceinline__ float split_largest(const float (&x)[8]) {
     m = fmaxf(m, __shfl_xor(m, 16));
     return fmaxf(m, __shfl_xor(m, 32));
 }
-// The exponent an operand's row is scaled by (the result's scale: 2^-e).  Below 2^-110 a row keeps its absolute error.
+// The exponent gO is scaled by; its power of two and the one that scales back are normal numbers.  (A lone zero: any.)
 __device__ __forceinline__ int split_exponent(float largest) {
-    return 15 - max(-110, __builtin_amdgcn_frexp_expf(largest));
+    return min(max(-16 - __builtin_amdgcn_frexp_expf(largest), 0), 126);
 }
-__device__ __forceinline__ float split_scale(int e) { return __builtin_amdgcn_ldexpf(1.f, -e); }
-__device__ __forceinline__ void split8(const float (&x)[8], int e, halfx8 (&p)[2]) {
+__device__ __forceinline__ float split_scale(int e) { return __builtin_amdgcn_ldexpf(1.f, e); }
+
+__device__ __forceinline__ void split8(const float (&x)[8], float scale, bf16x8 (&p)[kPieces]) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 u[kPieces];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        const float s = __builtin_amdgcn_ldexpf(x[q], e);
-        p[0][q] = (_Float16)s;
-        p[1][q] = (_Float16)(s - (float)p[0][q]);
+    for (int q = 0; q < 4; ++q) {
+        f32x2 r = {x[2 * q] * scale, x[2 * q + 1] * scale};
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) {
+            const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+            u[k][q] = h;
+            r.x -= __uint_as_float(h << 16);                       // exact
+            r.y -= __uint_as_float(h & 0xffff0000u);
+        }
     }
+#pragma unroll
+    for (int k = 0; k < kPieces; ++k) p[k] = __builtin_bit_cast(bf16x8, u[k]);
+}
+// Weights, unscaled.  One that would round to infinity has its first piece cut off instead; one that is not finite has no other pieces.
+__device__ __forceinline__ void split8_weights(const float (&x)[8], bf16x8 (&p)[kPieces]) {
+    float y[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) y[q] = fabsf(x[q]) >= 0x1p127f ? 0.f : x[q];
+    split8(y, 1.f, p);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+        if (!(fabsf(x[q]) < 0x1p127f)) {
+            const float h = __uint_as_float(__float_as_uint(x[q]) & 0xffff0000u), r = x[q] - h;
+            const float m = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
+            const bool finite = fabsf(x[q]) <= 0x1.fffffep127f;
+            p[0][q] = finite ? (__bf16)h : (__bf16)x[q];
+            p[1][q] = finite ? (__bf16)m : (__bf16)0.f;
+            p[2][q] = finite ? (__bf16)(r - m) : (__bf16)0.f;
+        }
 }
 #endif
 

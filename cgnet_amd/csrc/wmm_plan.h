@@ -40,7 +40,7 @@ struct cgnet_wmm_plan {
     int wp_blocks = 0;     // 64-float blocks of the packed forward weights
     int ap_blocks = 0;     // 64-float blocks of the packed operand of the FF-gradient kernel
     bool gff_mfma = true;  // every degree has t_O <= 16 (the operand then fits eight registers)
-    bool gff_split = false;// products of halves (split.h)
+    bool gff_split = false;// products of pieces (split.h)
     int gw_ff_cap = 2, gw_go_cap = 2;   // LDS capacities (complex entries) of one stage of the weight-gradient kernel
     int maxK = 0;          // channels of the largest degree with outputs
     int fwd_stage_cap = 16;             // LDS bytes of one stage of one wave of the forward kernel
