@@ -62,7 +62,8 @@ __device__ __forceinline__ float split_largest(const float (&x)[8]) {
 }
 // The exponent gO is scaled by; its power of two and the one that scales back are normal numbers.  (A lone zero: any.)
 __device__ __forceinline__ int split_exponent(float largest) {
-    return min(max(-16 - __builtin_amdgcn_frexp_expf(largest), 0), 126);
+    const int f = __builtin_amdgcn_frexp_expf(largest);            // largest < 2^f
+    return min(max(-16 - f, min(0, 127 - f)), 126);                // (at f = 128 a first piece could round to infinity)
 }
 __device__ __forceinline__ float split_scale(int e) { return __builtin_amdgcn_ldexpf(1.f, e); }
 

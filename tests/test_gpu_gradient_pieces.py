@@ -107,6 +107,27 @@ def test_sizes_of_both_operands(dev, size_w, size_go):  # noqa: F811
     assert "pack_w_gradff_split_kernel" in _check(dev, w, go, torch.ones(60))
 
 
+def _draw(seed):
+    g = torch.Generator().manual_seed(seed)
+    sizes = [(33, 12), (16, 16), (80, 9), (17, 13)]
+    return ([torch.randn(n, k, 2, generator=g) for k, n in sizes],
+            [torch.randn(3, n, 2 * l + 1, 2, generator=g) for l, (_, n) in enumerate(sizes)])
+
+
+@pytest.mark.parametrize("which", ["gO", "weights"])
+def test_largest_numbers(dev, which):  # noqa: F811
+    """The largest fp32 number rounds to infinity as a bfloat16."""
+    w, go = _draw(8)
+    largest = torch.finfo(torch.float32).max
+    if which == "gO":
+        go[2][1, 3, 2, 1] = -largest
+        w[2] *= 0.01
+    else:
+        w[1][3, 4, 0] = largest
+        go[1] *= 0.01
+    _check(dev, w, go, torch.ones(146))
+
+
 @pytest.mark.parametrize("decades", [0, 10])
 @pytest.mark.parametrize("lmax,tin,tout,bsz,sparse", [
     (2, [3, 1, 2], [9, 9, 9], 1, False),
