@@ -86,7 +86,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], float scale, bf16x8 
 #pragma unroll
     for (int k = 0; k < kPieces; ++k) p[k] = __builtin_bit_cast(bf16x8, u[k]);
 }
-// Weights, unscaled.  One that would round to infinity has its first piece cut off instead; one that is not finite has no other pieces.
+// Weights, unscaled.  One that would round to infinity has its first piece cut off instead; one that is not finite has no other pieces
+// (inside the layer it makes NaN of every entry of G that it meets; the mixing alone looks for it first).
 __device__ __forceinline__ void split8_weights(const float (&x)[8], bf16x8 (&p)[kPieces]) {
     float y[8];
 #pragma unroll

@@ -114,6 +114,26 @@ def _draw(seed):
             [torch.randn(3, n, 2 * l + 1, 2, generator=g) for l, (_, n) in enumerate(sizes)])
 
 
+def test_infinite_weights(dev):  # noqa: F811
+    """A weight that is not finite gives what a chain of fp32 products gives, and nothing to other channels."""
+    w, go = _draw(7)
+    clean, _ = _gradient(dev, w, go, torch.ones(146))
+    w[1][3, 4, 0] = float("inf")
+    w[2][5, 70, 1] = -float("inf")
+    w[3][0, 16, 0] = float("nan")
+    got, names = _gradient(dev, w, go, torch.ones(146))
+    assert "pack_w_gradff_split_kernel" in names
+    signs = lambda t: torch.sign(t) * float("inf")  # noqa: E731
+    assert torch.equal(got[1][:, 4], signs(go[1][:, 3]))   # conj(inf) (x + i y) = inf x + i inf y
+    assert torch.equal(got[2][:, 70], signs(torch.stack([-go[2][:, 5, :, 1], go[2][:, 5, :, 0]], -1)))    # conj(-i inf) (x + i y)
+    assert torch.isnan(got[3][:, 16]).all()
+    for l, c in ((1, 4), (2, 70), (3, 16)):
+        got[l][:, c] = clean[l][:, c]
+    for a, b in zip(got, clean):                            # the other channels of the tile by the other instructions
+        assert (a - b).abs().max() <= 2e-6 * b.abs().max()
+    assert torch.equal(got[2][:, :64], clean[2][:, :64])    # the other tiles by the same
+
+
 @pytest.mark.parametrize("which", ["gO", "weights"])
 def test_largest_numbers(dev, which):  # noqa: F811
     """The largest fp32 number rounds to infinity as a bfloat16."""
