@@ -15,7 +15,6 @@
 //   grad W  : the contraction runs over (b, m, re/im); lane (kk, i) reads complex entries
 //             8*blk + 2*kk, +1 of channel row i and feeds four k-steps.
 #include <algorithm>
-#include <cfloat>
 #include <cstdlib>
 #include <cstring>
 #include <iterator>
@@ -582,12 +581,11 @@ pack_w_gradff_kernel(const float2* __restrict__ W, const float* __restrict__ std
     *reinterpret_cast<float4*>(dst + 16) = make_float4(im[0], im[1], im[2], im[3]);
 }
 
-// The same as pieces (split.h), a wave per tile of 16 channels: [piece][lane (k, channel)] of eight k; behind all tiles a flag each:
-// whether a weight is not finite.
+// The same as pieces (split.h), a wave per tile of 16 channels: [piece][lane (k, channel)] of eight k.
 constexpr int kGffSplitBlocks = 4 * kPieces;   // blocks of 64 floats of a tile
 __global__ void __launch_bounds__(64)
 pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict__ stds, float eps, const WmmDeg* __restrict__ degs,
-                           int ndeg, float* __restrict__ Ap, int* __restrict__ odd) {
+                           int ndeg, float* __restrict__ Ap) {
     __shared__ int s_tab[kMaxLookup];
     const int blk = blockIdx.x * kGffSplitBlocks;
     const WmmDeg d = degs[lookup_in_group(ndeg, blk, [&](int k) { return degs[k].ap_base; }, s_tab)];
@@ -609,11 +607,6 @@ pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict
     split8_weights(v, p);
 #pragma unroll
     for (int k = 0; k < kPieces; ++k) reinterpret_cast<bf16x8*>(Ap + (size_t)blk * 64)[64 * k + lane] = p[k];
-    bool off = false;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) off |= !(fabsf(v[q]) <= FLT_MAX);
-    off = __any(off);
-    if (lane == 0) odd[blockIdx.x] = off;
 }
 
 // Gradient with respect to FF on the matrix cores (t_O <= 16): gFF[c, (m, re/im)] = sum_k A[c, k] * B[k, (m, re/im)]
@@ -630,8 +623,6 @@ constexpr int kGffSub = 4;     // channel tiles per wave
 // once.  lmax 10, layers of 12..3 channels, B=100 (112 units), us: 8 groups 151, 2048 waves 95, 4096 waves 84, 8192 waves 87.
 // Both gradients together, over the shapes named at kFwdSlices: 0.80 of the time, none slower by more than 5 %.
 constexpr int kGffFill = 4096, kGffMin = 2;
-// the weights themselves
-struct GffWeights { const float2* W; const float* stds; float eps; const int* odd; };
 // What a wave multiplies.  NKS steps of fp32: a tile's weights, a column tile's gO.
 template <int NKS>
 struct GffOps {
@@ -640,20 +631,6 @@ struct GffOps {
     static __device__ __forceinline__ void load(const float* tile, int lane, Left& o) {
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) o.a[ks] = tile[64 * ks + lane];
-    }
-    // what pack_w_gradff_kernel would have put there for channel c
-    static __device__ __forceinline__ void load(const GffWeights& w, const WmmDeg& d, int c, int kk, Left& o) {
-        const float div = w.stds && c < d.K ? fmaxf(w.eps, w.stds[d.cumT + c]) : 1.f;
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const int to = 2 * ks + (kk >> 1);
-            o.a[ks] = 0.f;
-            if (to < d.tO && c < d.K) {
-                const float2 v = w.W[d.cumW + (size_t)to * d.K + c];
-                o.a[ks] = kk & 1 ? v.y : v.x;
-                if (w.stds) o.a[ks] = o.a[ks] / div;
-            }
-        }
     }
     // rows past t_O are those of the last channel, times zero weights; k = 4 ks + kk -> channel 2 ks + (kk >> 1), re / im kk & 1
     static __device__ __forceinline__ void build(const float2* g, int M, int tO, int kk, int r, Right& o) {
@@ -705,13 +682,11 @@ struct GffOps<kGffSplitBlocks> {
         return mfma_piece(l.a[0], r.b[0], z) * r.scale;
     }
 };
-// PACKED: the weights come from Ap, otherwise (NKS = 8) as they are: pieces of a weight that is not finite would meet those of gO as
-// inf - inf where a chain of fp32 products has an infinity.
-template <int NKS, int NT, bool ONE, bool PACKED = true>
+template <int NKS, int NT, bool ONE>
 __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, const float* __restrict__ Ap,
                                                 float2* __restrict__ gFF, const WmmDeg& d, const WmmChanUnit& u, int B,
                                                 int samples_per_group, int nFF, int nO, int out_bytes, int go_bytes,
-                                                unsigned char* mine, int lane, int group, const GffWeights& weights) {
+                                                unsigned char* mine, int lane, int group) {
     float* ol = reinterpret_cast<float*>(mine);                              // [16][2M]
     unsigned char* gobuf = mine + out_bytes;                                  // [2][go_bytes]
     const int i = lane & 15, kk = lane >> 4;
@@ -721,10 +696,7 @@ __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, c
     typename Ops::Left a[kGffSub];
 #pragma unroll
     for (int sub = 0; sub < kGffSub; ++sub)
-        if (sub < nsub) {
-            if constexpr (PACKED) Ops::load(Ap + ((size_t)d.ap_base + (size_t)((u.c0 >> 4) + sub) * NKS) * 64, lane, a[sub]);
-            else Ops::load(weights, d, u.c0 + 16 * sub + i, kk, a[sub]);
-        }
+        if (sub < nsub) Ops::load(Ap + ((size_t)d.ap_base + (size_t)((u.c0 >> 4) + sub) * NKS) * 64, lane, a[sub]);
     const int r = i & 1;                          // column 16*ct + i -> m = 8*ct + (i >> 1), re/im = i & 1
     const int nct = (2 * M + 15) >> 4;
     const int n_go = tO * M;                      // complex entries of the gO rows
@@ -810,36 +782,27 @@ __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, c
 __global__ void __launch_bounds__(64)
 wmm_gradff_mfma_kernel(const float2* __restrict__ gO, const float* __restrict__ Ap, float2* __restrict__ gFF,
                        const WmmDeg* __restrict__ degs, const WmmChanUnit* __restrict__ units, int B,
-                       int samples_per_group, int nFF, int nO, int out_bytes, int go_bytes, GffWeights weights) {
+                       int samples_per_group, int nFF, int nO, int out_bytes, int go_bytes) {
     extern __shared__ __align__(16) unsigned char smem[];
     const UnitPart up = part_major((B + samples_per_group - 1) / samples_per_group);
     const WmmChanUnit u = units[up.unit];
     const WmmDeg d = degs[u.deg];
     const int lane = threadIdx.x;
-#define CGNET_GFF_ARGS gO, Ap, gFF, d, u, B, samples_per_group, nFF, nO, out_bytes, go_bytes, smem, lane, up.part, weights
-#define CGNET_GFF(N_) CGNET_GFF_AS(N_, N_, true)
-#define CGNET_GFF_AS(CASE_, N_, PACKED_)                                                  \
-    case CASE_:                                                                           \
-        if (nct == 1) wmm_gradff_wave<N_, 1, true, PACKED_>(CGNET_GFF_ARGS);              \
-        else if (nct == 2) wmm_gradff_wave<N_, 2, true, PACKED_>(CGNET_GFF_ARGS);         \
-        else if (nct == 3) wmm_gradff_wave<N_, 3, true, PACKED_>(CGNET_GFF_ARGS);         \
-        else wmm_gradff_wave<N_, 3, false, PACKED_>(CGNET_GFF_ARGS);                      \
+#define CGNET_GFF_ARGS gO, Ap, gFF, d, u, B, samples_per_group, nFF, nO, out_bytes, go_bytes, smem, lane, up.part
+#define CGNET_GFF(N_)                                                                     \
+    case N_:                                                                              \
+        if (nct == 1) wmm_gradff_wave<N_, 1, true>(CGNET_GFF_ARGS);                       \
+        else if (nct == 2) wmm_gradff_wave<N_, 2, true>(CGNET_GFF_ARGS);                  \
+        else if (nct == 3) wmm_gradff_wave<N_, 3, true>(CGNET_GFF_ARGS);                  \
+        else wmm_gradff_wave<N_, 3, false>(CGNET_GFF_ARGS);                               \
         break;
     const int nct = (2 * d.M + 15) >> 4;
-    int form = d.nks_b;
-    if (form == kGffSplitBlocks) {
-        const int* odd = weights.odd + d.ap_base / kGffSplitBlocks + (u.c0 >> 4);
-        for (int k = 0; 16 * k < u.nc; ++k)
-            if (odd[k]) form = 0;
-    }
-    switch (form) {
-        CGNET_GFF_AS(0, 8, false)
+    switch (d.nks_b) {
         CGNET_GFF(1) CGNET_GFF(2) CGNET_GFF(3) CGNET_GFF(4) CGNET_GFF(5) CGNET_GFF(6) CGNET_GFF(7)
         CGNET_GFF(8) CGNET_GFF(kGffSplitBlocks)
     }
 #undef CGNET_GFF_ARGS
 #undef CGNET_GFF
-#undef CGNET_GFF_AS
 }
 
 __global__ void __launch_bounds__(256) fill_zero_kernel(float* p, size_t n) {
@@ -1233,7 +1196,7 @@ int wmm_gradw_raw(const cgnet_wmm_plan* plan, const float* d_gO, const float* d_
 }
 }  // namespace cgnet
 static size_t gff_operand_bytes(const cgnet_wmm_plan* plan) {
-    return plan->gff_mfma ? sizeof(float) * (64 * (size_t)plan->ap_blocks + (plan->gff_split ? plan->ap_blocks / kGffSplitBlocks : 0)) : sizeof(float) * 2 * (size_t)plan->nW;
+    return plan->gff_mfma ? sizeof(float) * 64 * (size_t)plan->ap_blocks : sizeof(float) * 2 * (size_t)plan->nW;
 }
 
 extern "C" size_t cgnet_FN_WMM_backward_workspace(const cgnet_wmm_plan* plan, int B) {
@@ -1281,11 +1244,10 @@ extern "C" int cgnet_FN_WMM_backward(const cgnet_wmm_plan* plan, const float* d_
         CGNET_REQUIRE(plan->nO == 0 || d_gO, CGNET_ERR_ARG, "d_gO is NULL");
         if (plan->gff_mfma && plan->nW > 0 && plan->nO > 0) {
             float* Ap = (float*)d_workspace;
-            int* odd = reinterpret_cast<int*>(Ap + 64 * (size_t)plan->ap_blocks);      // of pack_w_gradff_split_kernel
             const int total = plan->ap_blocks * 8;    // one thread per four weights
             if (plan->gff_split)
                 CGNET_LAUNCH(pack_w_gradff_split_kernel, dim3(plan->ap_blocks / kGffSplitBlocks), dim3(64), 0, s, (const float2*)d_W,
-                             bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap, odd);
+                             bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap);
             else
                 CGNET_LAUNCH(pack_w_gradff_kernel, dim3((total + 255) / 256), dim3(256), 0, s, (const float2*)d_W,
                              bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap, plan->ap_blocks);
@@ -1297,8 +1259,7 @@ extern "C" int cgnet_FN_WMM_backward(const cgnet_wmm_plan* plan, const float* d_
             const size_t lds = (size_t)out_bytes + 2 * (size_t)go_bytes;
             CGNET_LAUNCH(wmm_gradff_mfma_kernel, dim3(grid_1d(plan->gw_units_rc0.size(), (B + spg - 1) / spg)),
                          dim3(64), lds, s, (const float2*)d_gO, (const float*)Ap, (float2*)d_gFF, plan->d_degs,
-                         plan->d_gw_units_rc0, B, spg, plan->nFF, plan->nO, out_bytes, go_bytes,
-                         GffWeights{(const float2*)d_W, bn ? d_stds : nullptr, eps, odd});
+                         plan->d_gw_units_rc0, B, spg, plan->nFF, plan->nO, out_bytes, go_bytes);
             CGNET_HIP(hipGetLastError());
             if (!plan->gff_zero_units.empty()) {
                 // degrees that produce no output channels: the general kernel writes their zeros

@@ -86,8 +86,9 @@ __device__ __forceinline__ void split8(const float (&x)[8], float scale, bf16x8 
 #pragma unroll
     for (int k = 0; k < kPieces; ++k) p[k] = __builtin_bit_cast(bf16x8, u[k]);
 }
-// Weights, unscaled.  One that would round to infinity has its first piece cut off instead; one that is not finite has no other pieces
-// (inside the layer it makes NaN of every entry of G that it meets; the mixing alone looks for it first).
+// Weights, unscaled.  One that would round to infinity has its first piece cut off instead.  One that is not finite lies in the third
+// piece, which meets the first of gO alone, with its sign: pieces of either sign beside it would make inf - inf of what is an infinity in a
+// chain of fp32 products.
 __device__ __forceinline__ void split8_weights(const float (&x)[8], bf16x8 (&p)[kPieces]) {
     float y[8];
 #pragma unroll
@@ -99,9 +100,9 @@ __device__ __forceinline__ void split8_weights(const float (&x)[8], bf16x8 (&p)[
             const float h = __uint_as_float(__float_as_uint(x[q]) & 0xffff0000u), r = x[q] - h;
             const float m = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
             const bool finite = fabsf(x[q]) <= 0x1.fffffep127f;
-            p[0][q] = finite ? (__bf16)h : (__bf16)x[q];
-            p[1][q] = finite ? (__bf16)m : (__bf16)0.f;
-            p[2][q] = finite ? (__bf16)(r - m) : (__bf16)0.f;
+            p[0][q] = (__bf16)(finite ? h : 0.f);
+            p[1][q] = (__bf16)(finite ? m : 0.f);
+            p[2][q] = (__bf16)(finite ? r - m : x[q]);
         }
 }
 #endif

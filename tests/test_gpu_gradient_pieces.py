@@ -129,9 +129,7 @@ def test_infinite_weights(dev):  # noqa: F811
     assert torch.isnan(got[3][:, 16]).all()
     for l, c in ((1, 4), (2, 70), (3, 16)):
         got[l][:, c] = clean[l][:, c]
-    for a, b in zip(got, clean):                            # the other channels of the tile by the other instructions
-        assert (a - b).abs().max() <= 2e-6 * b.abs().max()
-    assert torch.equal(got[2][:, :64], clean[2][:, :64])    # the other tiles by the same
+    assert all(torch.equal(a, b) for a, b in zip(got, clean))
 
 
 @pytest.mark.parametrize("which", ["gO", "weights"])
