@@ -132,6 +132,29 @@ def test_infinite_weights(dev):  # noqa: F811
     assert all(torch.equal(a, b) for a, b in zip(got, clean))
 
 
+@pytest.mark.parametrize("lmax", [0, 2])
+def test_infinite_weight_in_a_layer(dev, lmax):  # noqa: F811
+    """The layer's kernel makes of it what the two kernels make: infinities where one degree is alone, and not finite is the same place."""
+    from cgnet_amd import CG_layers
+    taus = [9] * (lmax + 1)
+    mod = CG_layers.CGBN_cuda(lmax, taus, taus, device=dev)
+    mod.eval()
+    with torch.no_grad():
+        mod.bnWMM.W[5, 0] = float("inf")
+    go = torch.randn(2, 9 * (lmax + 1) ** 2, 2, generator=torch.Generator().manual_seed(1)).to(dev)
+    grads = []
+    for one_kernel in (False, True):
+        mod.fused_backward = one_kernel
+        x = rand_straight(taus, 2, seed=lmax).float().to(dev).requires_grad_(True)
+        mod(x, straight_output=True).backward(go)
+        grads.append(x.grad)
+    if lmax == 0:
+        assert torch.isinf(grads[1]).any()
+        assert torch.equal(grads[0].nan_to_num(3., 1e38, -1e38), grads[1].nan_to_num(3., 1e38, -1e38))
+    fine = torch.isfinite(grads[0])
+    assert torch.equal(fine, torch.isfinite(grads[1])) and torch.equal(grads[0][fine], grads[1][fine])
+
+
 @pytest.mark.parametrize("which", ["gO", "weights"])
 def test_largest_numbers(dev, which):  # noqa: F811
     """The largest fp32 number rounds to infinity as a bfloat16."""
