@@ -468,7 +468,7 @@ class CGBN_cuda(nn.Module):
         self.fused = True      # False: chain the two reference Functions (separate statistics pass)
         # With ``fused``: True takes the backward from grad_output to the input gradient in one kernel, without a
         # grad_FF tensor (B x nFF complex) in memory, where the shapes allow it
-        # (cgnet_CGBN_backward_fused_supported); False keeps the two-kernel backward.  Same gradients either way.
+        # (cgnet_CGBN_backward_fused_supported); False keeps the two-kernel backward.  Same gradients up to rounding.
         self.fused_backward = _FUSED_BACKWARD
         # With ``fused``: when no gradient is wanted and the statistics are not updated (evaluation mode, or no fragment
         # norm), True takes the forward without the product tensor FF (B x nFF complex) in memory, every tile of it mixed

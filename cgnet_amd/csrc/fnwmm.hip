@@ -864,7 +864,8 @@ extern "C" int cgnet_wmm_plan_create(cgnet_wmm_plan** plan, int L, const int* h_
     p->L = L;
     long long cFF = 0, cO = 0, cW = 0, cT = 0;
     int wp = 0;
-    // CGNET_BWD_PAIRS=0 (as in cgnet_cg_plan_create) keeps the fp32 steps in which the layer's kernel by triples makes the same gradient
+    // CGNET_BWD_PAIRS=0 leaves out what came with the backward by pairs in this plan too: the product tensor's gradient is made on the fp32
+    // instructions, as the layer's kernel by triples makes it, and both routes hold the same bits.
     const char* by_pairs = getenv("CGNET_BWD_PAIRS");
     p->gff_split = split_taken(L, [&](int l) { return h_t_O[l]; }) && !(by_pairs && by_pairs[0] == '0');
     for (int l = 0; l <= L; ++l) {
