@@ -40,6 +40,32 @@ def synthetic(lmax, tau, bsz, t_ff, seed=0):
     return x, w, go
 
 
+def kernel_code():
+    """Digest of the kernels' sources without comments and white space.  A counter summary names the digest of the code it was measured
+    on; figures of other code are not printed."""
+    import glob
+    import hashlib
+    import re
+    h = hashlib.sha256()
+    for path in sorted(glob.glob(os.path.join(ROOT, "cgnet_amd", "csrc", "*"))):
+        if path.endswith((".hip", ".h", ".cpp")):
+            h.update(re.sub(r"//[^\n]*|\s+", "", open(path).read()).encode())
+    return h.hexdigest()[:16]
+
+
+def profile_lines(path):
+    """The lines of a counter summary and its source revision, or (None, reason) where the summary is missing or of other code."""
+    import re
+    try:
+        lines = open(os.path.join(ROOT, path)).read().splitlines()
+    except OSError:
+        return None, "no %s" % path
+    head = dict(m.groups() for m in (re.match(r"^(source revision|kernel code):\s*(\S+)", l) for l in lines) if m)
+    if head.get("kernel code") != kernel_code():
+        return None, "%s is of other kernel code" % path
+    return lines, head.get("source revision", "unknown revision")
+
+
 TRAFFIC_PROFILE = os.path.join("profiles", "cg_layer_L11_tau12_B100_hbm_traffic_pmc.txt")
 
 
@@ -48,18 +74,14 @@ def profiled_traffic():
     summary states them (counters are not readable from inside a run; the summary names the command and
     the source revision it was measured on).  -> ({kernel: bytes}, description of the source)."""
     import re
-    path = os.path.join(ROOT, TRAFFIC_PROFILE)
-    table, rev = {}, "unknown revision"
-    try:
-        for line in open(path):
-            m = re.match(r"^(\w+)(?:<[\d,]+>)?\s+([\d.]+) MB\s+([\d.]+) MB\s+([\d.]+) MB\s+([\d.]+) MB\s+[\d.]+\s*$", line)
-            if m:
-                table[m.group(1)] = float(m.group(4)) * 1e6
-            m = re.match(r"^source revision:\s*(\S+)", line)
-            if m:
-                rev = m.group(1)
-    except OSError:
-        return {}, "no traffic profile found"
+    lines, rev = profile_lines(TRAFFIC_PROFILE)
+    if lines is None:
+        return {}, rev
+    table = {}
+    for line in lines:
+        m = re.match(r"^(\w+)(?:<[\d,]+>)?\s+([\d.]+) MB\s+([\d.]+) MB\s+([\d.]+) MB\s+([\d.]+) MB\s+[\d.]+\s*$", line)
+        if m:
+            table[m.group(1)] = float(m.group(4)) * 1e6
     return table, "%s (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE; measured at %s, not in this run)" % (TRAFFIC_PROFILE, rev)
 
 
@@ -67,20 +89,18 @@ SQ_PROFILE = os.path.join("profiles", "cg_layer_L11_tau12_B100_sq_counters_pmc.t
 
 
 def profiled_issue(kernel, avg_launch_ms):
-    """SIMD issue time of `kernel` from the committed SQ counter summary: vector and matrix instructions take turns
-    on a SIMD of this GPU but for a tenth (4 cycles per vector instruction, 32 per v_mfma_f32_16x16x4_f32; measured, see the
-    summary's header), so (4 N_vector + 32 N_matrix) / (1024 SIMDs x clock) is what they take one after the other."""
-    try:
-        for line in open(os.path.join(ROOT, SQ_PROFILE)):
-            f = line.split()
-            if len(f) >= 7 and f[0].split("<")[0] == kernel:
-                mhz, n_valu, n_mfma = float(f[2]), float(f[3]), float(f[6])
-                bound_ms = (4.0 * (n_valu - n_mfma) + 32.0 * n_mfma) / (1024 * mhz * 1e6) * 1e3
-                return {"bound_ms": round(bound_ms, 4), "frac": round(bound_ms / avg_launch_ms, 3), "clock_MHz": mhz,
-                        "vector_instructions": n_valu - n_mfma, "matrix_instructions": n_mfma,
-                        "source": SQ_PROFILE + " (counters of an earlier run, not of this one)"}
-    except (OSError, ValueError):
-        pass
+    """SIMD issue time of `kernel` from the committed SQ counter summary: what its vector instructions (4 cycles), v_mfma_f32_16x16x4_f32
+    (32 cycles, in turn with them) and v_mfma_f32_16x16x32_bf16 (16 cycles, of which vector instructions hide four) take on 1024 SIMDs
+    (profiles/matrix_vector_issue.txt)."""
+    lines, _ = profile_lines(SQ_PROFILE)
+    for line in lines or ():
+        f = line.split()
+        if len(f) >= 6 and f[0].split("<")[0] == kernel:
+            mhz, n_valu, n_f32, n_bf16 = (float(v) for v in f[2:6])
+            bound_ms = (4.0 * n_valu + 32.0 * n_f32 + 12.0 * n_bf16) / (1024 * mhz * 1e6) * 1e3
+            return {"bound_ms": round(bound_ms, 4), "frac": round(bound_ms / avg_launch_ms, 3), "clock_MHz": mhz,
+                    "vector_instructions": n_valu, "matrix_instructions_f32": n_f32, "matrix_instructions_bf16": n_bf16,
+                    "source": SQ_PROFILE + " (counters of an earlier run, not of this one)"}
     return None
 
 
