@@ -22,15 +22,16 @@
 // packed gO and packed weights by matrix instructions in the order of wmm_gradff_mfma_kernel, so that both sources hold the
 // same values to the bit; where every degree has nine output channels or more, in bfloat16 pieces (split.h).
 //
-// Bounded by issue where enough waves run: a vector multiply-add holds a SIMD for four cycles, a matrix instruction for 32, and the two
-// take turns.  lmax 11, 12 channels, B = 100, inside the layer: 8.6e7 vector and 1.1e7 matrix instructions, 75 % of the cycles of
-// 1024 SIMDs; three waves a SIMD.  That takes 168 registers and spills 41 more to 148 bytes of scratch a lane (41 .. 45 whatever the
-// output channels; from lmax 16 on 256 registers, 25 .. 35 spilled; none at lmax 12..15, 216 .. 254 registers, two waves): the
-// kernel writes 161 MB there, of which 36 are partial gradients.  The loads of packed gO and weights come out of L1, which gives 64 bytes a
+// Bounded by issue and latency: a vector multiply-add holds a SIMD for four cycles, an fp32 matrix instruction for 32, and the two take
+// turns; a bfloat16 one for 16, four of them beside vector instructions.  lmax 11, 12 channels, B = 100, inside the layer: 9.8e7 vector,
+// 4.8e6 fp32 and 6.6e6 bfloat16 matrix instructions, 68 % of the cycles of 1024 SIMDs at three waves a SIMD (G on fp32 instructions: 8.6e7
+// and 1.13e7, 75 %); lmax 20, 16 channels: 59 % at two waves.  Three waves take 168 registers, and 36 more are spilled to 128 bytes of
+// scratch a lane (41 .. 45 with G on fp32 instructions; up to lmax 7 128 registers, 6 spilled; none at lmax 12..15, 216 .. 254 registers, two
+// waves; from lmax 16 on 256 registers, 26 .. 35 spilled): the kernel writes 145 MB there, of which 36 are partial gradients.  The loads of packed gO and weights come out of L1, which gives 64 bytes a
 // cycle to loads of 4 or 16 bytes a lane and half of that to 8 bytes, and out of L2, for which the work-groups of a sample stay on one
 // XCD.  Adding the sums in LDS with ds_add_f32 is no alternative to read and write: 18 times slower (measured alone).
 // Against the kernels that work triple by triple, us (whole call, operands packed by itself): lmax 11, 12 channels, B = 100, layer
-// 568 -> 427 (this kernel 391); lmax 20, 16 channels, B = 32, layer 4021 -> 2247; lmax 15, 16 channels, B = 64, stand-alone
+// 541 -> 404 (this kernel 380; G on fp32 instructions 416); lmax 20, 16 channels, B = 32, layer 4006 -> 2047 (2238); lmax 15, 16 channels, B = 64, stand-alone
 // 1623 -> 1361; lmax 10, 4 channels, B = 100, stand-alone 106 -> 59.
 #pragma once
 #include <utility>

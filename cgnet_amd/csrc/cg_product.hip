@@ -519,7 +519,10 @@ cg_forward_mm_kernel(const float2* __restrict__ F, float2* __restrict__ FF, cons
 // unit with 45 registers spilled, 446 at two); two scaled f16 pieces (352) lose what lies 2^16 and more below the largest of the tile, and
 // showing for each sample that nothing did leaves 375, and 576 where it cannot be shown.  Fp32: a launch for each number of column
 // tiles and a barrier behind the shares 408, one launch and the shares added while the next sample runs 398.
-// What bounds it: the fp32 matrix instructions of product and mixing and the vector instructions, which take turns.
+// Those two forms over sizes, us: lmax 3, 16 channels, B = 100 35 -> 36; lmax 7, 16 channels 139 -> 140; lmax 9, 10 channels 213 -> 197; lmax 11,
+// 16 channels, MST triples, B = 32 142 -> 125; lmax 15, 16 channels, B = 32 742 -> 696, 8 channels 325 -> 316.
+// What bounds it: the fp32 matrix instructions of product and mixing (62 % of the cycles of 1024 SIMDs at lmax 11, 12 channels, B = 100) and the
+// vector instructions (19 %), which take turns.
 constexpr int kMixMaxK = 16;                   // reduction steps of one wave (64 channels)
 constexpr int kMixShares = 4;                  // shares of the reduction steps of a column tile: one wave per SIMD
 constexpr size_t kMixShareBytes = 2048;        // a share's 16 x 16 complex partial sums

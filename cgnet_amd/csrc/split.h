@@ -1,7 +1,8 @@
 // Products of fp32 operands on the 16-bit matrix instructions.
 //
 // v_mfma_f32_16x16x4_f32 holds a SIMD's vector ALUs for its 32 cycles: it and vector instructions take turns.
-// v_mfma_f32_16x16x32_bf16 takes 16 cycles for eight times the terms and runs beside vector instructions of other waves.
+// v_mfma_f32_16x16x32_bf16 takes 16 cycles for eight times the terms, of which vector instructions of other waves hide four
+// (profiles/matrix_vector_issue.txt).
 //
 // An operand is the sum of three bfloat16 pieces h + m + l, which hold its 24 bits, and six of the nine products (ml, lm and ll, together
 // at most 2^-23 of the product and mostly far less, are left out) are summed in fp32.  bfloat16 has the exponents of fp32: an entry keeps its
@@ -10,7 +11,7 @@
 // weights of any size stay in range until the result is scaled back.
 // gFF against 64 bits (rms, lmax 11, whether or not the output channels are spread over six decades): 9 channels 7.8e-8 by fp32 instructions,
 // 3.5e-8 by pieces, 12 channels 8.9e-8 and 3.6e-8, 16 channels 10.2e-8 and 3.8e-8.
-// Backward by pairs (cg_back_kernel.h), fp32 instructions -> pieces, us: lmax 11, 12 channels, B = 100: 390 -> 377; lmax 20, 16 channels,
+// Backward by pairs (cg_back_kernel.h), fp32 instructions -> pieces, us: lmax 11, 12 channels, B = 100: 390 -> 380; lmax 20, 16 channels,
 // B = 32: 2136 -> 1976; gFF alone, lmax 11, 12 channels, B = 50: 100 -> 84.  Two f16 pieces with a scale for each row and column took 381,
 // 1921 and 79, but lost what lay 2^16 and more below the largest of its row or column: output channels spread over ten decades, with
 // weights and gO that balance each other, came back with an error of 3e-3.
