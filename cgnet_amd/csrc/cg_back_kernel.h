@@ -20,18 +20,18 @@
 // degree; four lane-group swaps per register set of four degrees turn it into right operands (lane group = degree).  It is read
 // from memory (the stand-alone operator: sixteen segments of 64 bytes per load instruction) or, inside the layer, made from
 // packed gO and packed weights by matrix instructions in the order of wmm_gradff_mfma_kernel, so that both sources hold the
-// same values to the bit; where every degree has nine output channels or more, in bfloat16 pieces (split.h).
+// same values to the bit; where every degree has thirteen output channels or more, in bfloat16 pieces (split.h).
 //
 // Bounded by issue and latency: a vector multiply-add holds a SIMD for four cycles, an fp32 matrix instruction for 32, and the two take
-// turns; a bfloat16 one for 16, four of them beside vector instructions.  lmax 11, 12 channels, B = 100, inside the layer: 9.8e7 vector,
-// 4.8e6 fp32 and 6.6e6 bfloat16 matrix instructions, 68 % of the cycles of 1024 SIMDs at three waves a SIMD (G on fp32 instructions: 8.6e7
-// and 1.13e7, 75 %); lmax 20, 16 channels: 59 % at two waves.  Three waves take 168 registers, and 36 more are spilled to 128 bytes of
-// scratch a lane (41 .. 45 with G on fp32 instructions; up to lmax 7 128 registers, 6 spilled; none at lmax 12..15, 216 .. 254 registers, two
-// waves; from lmax 16 on 256 registers, 26 .. 35 spilled): the kernel writes 145 MB there, of which 36 are partial gradients.  The loads of packed gO and weights come out of L1, which gives 64 bytes a
+// turns; a bfloat16 one for 16, four of them beside vector instructions.  lmax 11, 12 channels, B = 100, inside the layer: 8.6e7 vector
+// and 1.13e7 fp32 matrix instructions, 75 % of the cycles of 1024 SIMDs at three waves a SIMD; lmax 20, 16 channels, in pieces: 59 % at two
+// waves.  Three waves take 168 registers, and 41 more are spilled to 148 bytes of scratch a lane (41 .. 45 whatever the output channels, in
+// pieces 36; up to lmax 7 128 registers, 5 or 6 spilled; none at lmax 12..15, 216 .. 254 registers, two waves; from lmax 16 on 256 registers,
+// 26 .. 35 spilled): the kernel writes 161 MB there, of which 36 are partial gradients.  The loads of packed gO and weights come out of L1, which gives 64 bytes a
 // cycle to loads of 4 or 16 bytes a lane and half of that to 8 bytes, and out of L2, for which the work-groups of a sample stay on one
 // XCD.  Adding the sums in LDS with ds_add_f32 is no alternative to read and write: 18 times slower (measured alone).
 // Against the kernels that work triple by triple, us (whole call, operands packed by itself): lmax 11, 12 channels, B = 100, layer
-// 541 -> 404 (this kernel 380; G on fp32 instructions 416); lmax 20, 16 channels, B = 32, layer 4006 -> 2047 (2238); lmax 15, 16 channels, B = 64, stand-alone
+// 541 -> 416 (this kernel 391); lmax 20, 16 channels, B = 32, layer 4006 -> 2047 (G on fp32 instructions 2238); lmax 15, 16 channels, B = 64, stand-alone
 // 1623 -> 1361; lmax 10, 4 channels, B = 100, stand-alone 106 -> 59.
 #pragma once
 #include <utility>

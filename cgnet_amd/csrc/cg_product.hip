@@ -1589,7 +1589,7 @@ cg_backward_hybrid_kernel(const float2* __restrict__ Fp, const float2* __restric
 //   A[c][(to,0)] = W_re[to][c]/div[c], A[c][(to,1)] = W_im[to][c]/div[c]
 //   B[(to,0)][(m,0)] = gO_re, B[(to,1)][(m,0)] = gO_im, B[(to,0)][(m,1)] = gO_im, B[(to,1)][(m,1)] = -gO_re
 // the arithmetic of wmm_gradff_mfma_kernel on the fp32 instructions, instruction for instruction.  Where that kernel takes them too (a
-// degree with one to eight output channels, or a mixing plan made with CGNET_BWD_PAIRS=0) the tile holds the values it would have written
+// degree with one to twelve output channels, or a mixing plan made with CGNET_BWD_PAIRS=0) the tile holds the values it would have written
 // to memory, and without the fold of the diagonal triples the result equals the two-kernel route bit for bit; in pieces (split.h) it writes
 // other roundings of the same sums.
 //

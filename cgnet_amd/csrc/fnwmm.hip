@@ -583,13 +583,15 @@ pack_w_gradff_kernel(const float2* __restrict__ W, const float* __restrict__ std
 
 // The same as pieces (split.h), a wave per tile of 16 channels: [piece][lane (k, channel)] of eight k.
 constexpr int kGffSplitBlocks = 4 * kPieces;   // blocks of 64 floats of a tile
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(256)
 pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict__ stds, float eps, const WmmDeg* __restrict__ degs,
-                           int ndeg, float* __restrict__ Ap) {
+                           int ndeg, float* __restrict__ Ap, int total_blocks) {
     __shared__ int s_tab[kMaxLookup];
-    const int blk = blockIdx.x * kGffSplitBlocks;
-    const WmmDeg d = degs[lookup_in_group(ndeg, blk, [&](int k) { return degs[k].ap_base; }, s_tab)];
-    const int lane = threadIdx.x, i = lane & 15, kk = lane >> 4, c = (blk - d.ap_base) / kGffSplitBlocks * 16 + i;
+    const int blk = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6))) * kGffSplitBlocks;
+    const int di = lookup_in_group(ndeg, blk, [&](int k) { return degs[k].ap_base; }, s_tab);
+    if (blk >= total_blocks) return;
+    const WmmDeg d = degs[di];
+    const int lane = threadIdx.x & 63, i = lane & 15, kk = lane >> 4, c = (blk - d.ap_base) / kGffSplitBlocks * 16 + i;
     const float r = stds && c < d.K ? fmaxf(eps, stds[d.cumT + c]) : 1.f;
     float v[8];
 #pragma unroll
@@ -618,7 +620,7 @@ pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict
 // NT = column tiles worked on together; ONE: these are all column tiles of the degree, so the B
 // operands are built once per sample and shared by the channel tiles.
 constexpr int kGffSub = 4;     // channel tiles per wave
-// lmax 11, 12 channels, B=50 (383 MB of gFF): fp32 steps 100 us, pieces 84.
+// lmax 11, B = 64, 16 channels (875 MB of gFF): fp32 steps 241 us, pieces 172; 12 channels, B = 50 (383 MB): fp32 steps 100.
 // Waves wanted (at least eight groups of samples are made in any case), samples a wave keeps at least: it loads its operand
 // once.  lmax 10, layers of 12..3 channels, B=100 (112 units), us: 8 groups 151, 2048 waves 95, 4096 waves 84, 8192 waves 87.
 // Both gradients together, over the shapes named at kFwdSlices: 0.80 of the time, none slower by more than 5 %.
@@ -779,6 +781,11 @@ __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, c
     store_tile(b_end - 1, nsub - 1);
 }
 
+// Fp32 steps; pieces; pieces of degrees above eleven (four column tiles and more).  Splitting gO again for every channel tile cost more than
+// the fp32 steps take, so up to six column tiles are split once.  Kernels of their own: the registers of one are no
+// concern of the others (104, 131, 173).
+enum GffForm { kGffFp32, kGffPieces, kGffWide };
+template <GffForm FORM>
 __global__ void __launch_bounds__(64)
 wmm_gradff_mfma_kernel(const float2* __restrict__ gO, const float* __restrict__ Ap, float2* __restrict__ gFF,
                        const WmmDeg* __restrict__ degs, const WmmChanUnit* __restrict__ units, int B,
@@ -789,20 +796,32 @@ wmm_gradff_mfma_kernel(const float2* __restrict__ gO, const float* __restrict__ 
     const WmmDeg d = degs[u.deg];
     const int lane = threadIdx.x;
 #define CGNET_GFF_ARGS gO, Ap, gFF, d, u, B, samples_per_group, nFF, nO, out_bytes, go_bytes, smem, lane, up.part
-#define CGNET_GFF(N_)                                                                     \
-    case N_:                                                                              \
+#define CGNET_GFF(N_) CGNET_GFF_AS(N_, N_)
+#define CGNET_GFF_AS(CASE_, N_)                                                           \
+    case CASE_:                                                                           \
         if (nct == 1) wmm_gradff_wave<N_, 1, true>(CGNET_GFF_ARGS);                       \
         else if (nct == 2) wmm_gradff_wave<N_, 2, true>(CGNET_GFF_ARGS);                  \
         else if (nct == 3) wmm_gradff_wave<N_, 3, true>(CGNET_GFF_ARGS);                  \
         else wmm_gradff_wave<N_, 3, false>(CGNET_GFF_ARGS);                               \
         break;
     const int nct = (2 * d.M + 15) >> 4;
-    switch (d.nks_b) {
-        CGNET_GFF(1) CGNET_GFF(2) CGNET_GFF(3) CGNET_GFF(4) CGNET_GFF(5) CGNET_GFF(6) CGNET_GFF(7)
-        CGNET_GFF(8) CGNET_GFF(kGffSplitBlocks)
+    if constexpr (FORM == kGffWide) {
+        if (nct == 4) wmm_gradff_wave<kGffSplitBlocks, 4, true>(CGNET_GFF_ARGS);
+        else if (nct == 5) wmm_gradff_wave<kGffSplitBlocks, 5, true>(CGNET_GFF_ARGS);
+        else if (nct == 6) wmm_gradff_wave<kGffSplitBlocks, 6, true>(CGNET_GFF_ARGS);
+        else switch (0) { CGNET_GFF_AS(0, kGffSplitBlocks) }
+    } else if constexpr (FORM == kGffPieces) {
+        if (nct == 1) wmm_gradff_wave<kGffSplitBlocks, 1, true>(CGNET_GFF_ARGS);
+        else if (nct == 2) wmm_gradff_wave<kGffSplitBlocks, 2, true>(CGNET_GFF_ARGS);
+        else wmm_gradff_wave<kGffSplitBlocks, 3, true>(CGNET_GFF_ARGS);
+    } else {
+        switch (d.nks_b) {
+            CGNET_GFF(1) CGNET_GFF(2) CGNET_GFF(3) CGNET_GFF(4) CGNET_GFF(5) CGNET_GFF(6) CGNET_GFF(7) CGNET_GFF(8)
+        }
     }
 #undef CGNET_GFF_ARGS
 #undef CGNET_GFF
+#undef CGNET_GFF_AS
 }
 
 __global__ void __launch_bounds__(256) fill_zero_kernel(float* p, size_t n) {
@@ -1247,8 +1266,8 @@ extern "C" int cgnet_FN_WMM_backward(const cgnet_wmm_plan* plan, const float* d_
             float* Ap = (float*)d_workspace;
             const int total = plan->ap_blocks * 8;    // one thread per four weights
             if (plan->gff_split)
-                CGNET_LAUNCH(pack_w_gradff_split_kernel, dim3(plan->ap_blocks / kGffSplitBlocks), dim3(64), 0, s, (const float2*)d_W,
-                             bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap);
+                CGNET_LAUNCH(pack_w_gradff_split_kernel, dim3((plan->ap_blocks / kGffSplitBlocks + 3) / 4), dim3(256), 0, s,
+                             (const float2*)d_W, bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap, plan->ap_blocks);
             else
                 CGNET_LAUNCH(pack_w_gradff_kernel, dim3((total + 255) / 256), dim3(256), 0, s, (const float2*)d_W,
                              bn ? d_stds : nullptr, eps, plan->d_degs, ndeg, Ap, plan->ap_blocks);
@@ -1258,9 +1277,14 @@ extern "C" int cgnet_FN_WMM_backward(const cgnet_wmm_plan* plan, const float* d_
             const int spg = (B + groups - 1) / groups;
             const int out_bytes = plan->gff_out_cap, go_bytes = plan->gff_go_cap;   // per wave
             const size_t lds = (size_t)out_bytes + 2 * (size_t)go_bytes;
-            CGNET_LAUNCH(wmm_gradff_mfma_kernel, dim3(grid_1d(plan->gw_units_rc0.size(), (B + spg - 1) / spg)),
-                         dim3(64), lds, s, (const float2*)d_gO, (const float*)Ap, (float2*)d_gFF, plan->d_degs,
-                         plan->d_gw_units_rc0, B, spg, plan->nFF, plan->nO, out_bytes, go_bytes);
+            auto launch = [&](auto* wmm_gradff_mfma_kernel) {
+                CGNET_LAUNCH(wmm_gradff_mfma_kernel, dim3(grid_1d(plan->gw_units_rc0.size(), (B + spg - 1) / spg)),
+                             dim3(64), lds, s, (const float2*)d_gO, (const float*)Ap, (float2*)d_gFF, plan->d_degs,
+                             plan->d_gw_units_rc0, B, spg, plan->nFF, plan->nO, out_bytes, go_bytes);
+            };
+            if (!plan->gff_split) launch(&wmm_gradff_mfma_kernel<kGffFp32>);
+            else if (plan->L <= 11) launch(&wmm_gradff_mfma_kernel<kGffPieces>);
+            else launch(&wmm_gradff_mfma_kernel<kGffWide>);
             CGNET_HIP(hipGetLastError());
             if (!plan->gff_zero_units.empty()) {
                 // degrees that produce no output channels: the general kernel writes their zeros

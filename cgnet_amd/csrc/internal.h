@@ -77,8 +77,8 @@ size_t back_bytes_up_to(const BackSet& set, int most_B, int B, Bytes&& bytes) {
 //   stand-alone, unit kernel     by the rule 0.59, 0.6 %, 1.16 times; always 0.60, 8 %, 1.66 times
 //   layer, 8..16 channels        by the rule 0.62, 1.4 %, 1.26 times (lmax 16, MST, 11 channels, B = 128: 1090 -> 1376 us); always
 //                                0.63, 14 %, 1.64 times
-//     (G on fp32 instructions; with nine output channels and more, in pieces (split.h), over 36 layers of MST triples, lmax 8..20, 9..15
-//     channels, 8..128 samples: triples are the faster wherever the rule takes them, pairs at worst 1.12 times, lmax 11, 9 channels, B = 32)
+//     (G on fp32 instructions; in pieces (split.h), over 36 layers of MST triples, lmax 8..20, 9..15 channels
+//     in and out, 8..128 samples: triples are the faster wherever the rule takes them, pairs at worst 1.12 times, lmax 11, 9 channels, B = 32)
 // A layer with other channels has no other kernel but the two of the chain: always by pairs, 0.48 of their time, 0.3 % of 2325 calls
 // slower, at worst 1.14 times.
 struct BackRule {

@@ -11,21 +11,25 @@
 // weights of any size stay in range until the result is scaled back.
 // gFF against 64 bits (rms, lmax 11, whether or not the output channels are spread over six decades): 9 channels 7.8e-8 by fp32 instructions,
 // 3.5e-8 by pieces, 12 channels 8.9e-8 and 3.6e-8, 16 channels 10.2e-8 and 3.8e-8.
-// Backward by pairs (cg_back_kernel.h), fp32 instructions -> pieces, us: lmax 11, 12 channels, B = 100: 390 -> 380; lmax 20, 16 channels,
-// B = 32: 2136 -> 1976; gFF alone, lmax 11, 12 channels, B = 50: 100 -> 84.  Two f16 pieces with a scale for each row and column took 381,
-// 1921 and 79, but lost what lay 2^16 and more below the largest of its row or column: output channels spread over ten decades, with
-// weights and gO that balance each other, came back with an error of 3e-3.
+// Backward by pairs (cg_back_kernel.h), fp32 instructions -> pieces, us: lmax 20, 16 channels, B = 32: 2136 -> 1976; gFF alone, lmax 11, 16
+// channels, B = 64: 252 -> 183.  Two f16 pieces with a scale for each row and column took 1921, but lost what lay 2^16 and more below the
+// largest of its row or column: output channels spread over ten decades, with weights and gO that balance each other, came back with an
+// error of 3e-3.
 #pragma once
 #include "common.h"
 
 namespace cgnet {
 
 // The 32 places of a product are (output channel, re / im).  Whether pieces take the place of fp32 for output channels `t` of the degrees
-// 0 .. L: every degree that has any has at least nine.  Up to eight the fp32 instructions are four at most, and a third of the operands to
-// load.  Whole step, B = 100, lmax 11, fp32 -> pieces, us: layer of 5 channels 278 -> 292, 8 channels 624 -> 650, 9 channels 796 -> 795;
-// mixing alone, 8 channels 372 -> 379, 9 channels 505 -> 505.
+// 0 .. L: every degree that has any has at least thirteen.  They replace seven or eight fp32 instructions there, five or six at nine to
+// twelve channels, and operands half as large again there, twice as large at twelve.  Kernels of a training step over lmax 2..23, 1..64 samples, fp32 -> pieces:
+//   13 .. 16 channels  layer 0.98 of the time (170 shapes, one more than 3 % slower: 54 -> 56 us), gFF alone 0.92 (14 of 170 more than 5 % slower, up
+//                      to four samples: 22 -> 25 us, at worst 79 -> 90)
+//   10 .. 12 channels  layer 1.01 (35 of 262 more than 3 % slower, 507 -> 542 us at lmax 20, 16 -> 12 channels, one sample), gFF alone 0.99 (75 of
+//                      262 more than 5 % slower, 28.6 -> 35.2 us at lmax 18, 10 channels, one sample)
+//   up to eight        layer of 5 channels at lmax 11, B = 100: 278 -> 292 us, of 8 624 -> 650
 constexpr int kPieces = 3;
-constexpr int kSplitFrom = 9, kSplitMax = 16;
+constexpr int kSplitFrom = 13, kSplitMax = 16;
 template <typename Count>
 bool split_taken(int L, Count&& t) {
     bool any = false;

@@ -168,21 +168,20 @@ def test_largest_batch_by_pairs(dev, lmax, tau, sparse, layer, most):  # noqa: F
         assert ("cg_backward_pair_kernel" in names) == (not most or bsz <= most), (bsz, names)
 
 
-@pytest.mark.parametrize("lmax,tau,bsz", [(8, 12, 70), (6, 9, 60)])
+@pytest.mark.parametrize("lmax,tau,tout,bsz", [(8, 12, 13, 70), (6, 9, 16, 60)])
 @pytest.mark.parametrize("fold", [None, "0"])
-def test_triples_beside_two_kernels(dev, monkeypatch, lmax, tau, bsz, fold):  # noqa: F811
-    """A layer of nine output channels and more, reduced triples, a batch past the rule, nothing switched: the layer's kernel makes the
+def test_triples_beside_two_kernels(dev, monkeypatch, lmax, tau, tout, bsz, fold):  # noqa: F811
+    """A layer of thirteen output channels and more, reduced triples, a batch past the rule, nothing switched: the layer's kernel makes the
     product's gradient on the fp32 instructions, the two kernels in bfloat16 pieces.  Each is as exact as chains of fp32 products, with
     the fold of the diagonal triples and without."""
     from cgnet_amd import CG_layers
     if fold:
         monkeypatch.setenv("CGNET_DIAG_FOLD", fold)
-    taus = [tau] * (lmax + 1)
-    mod = CG_layers.CGBN_cuda(lmax, taus, taus, sparse_flag=True, device=dev)
+    mod = CG_layers.CGBN_cuda(lmax, [tau] * (lmax + 1), [tout] * (lmax + 1), sparse_flag=True, device=dev)
     mod.eval()
     g = torch.Generator(device=dev).manual_seed(lmax)
     x = torch.randn(bsz, mod.cg.native_plan().nF, 2, generator=g, device=dev)
-    go = torch.randn(bsz, sum(tau * (2 * l + 1) for l in range(lmax + 1)), 2, generator=g, device=dev)
+    go = torch.randn(bsz, tout * (lmax + 1) ** 2, 2, generator=g, device=dev)
     grads = []
     for one_kernel in (True, False):
         mod.fused_backward = one_kernel
@@ -192,7 +191,7 @@ def test_triples_beside_two_kernels(dev, monkeypatch, lmax, tau, bsz, fold):  # 
         assert "cg_backward_pair_kernel" not in names
         assert {"cgbn_backward_fused_kernel"} <= names if one_kernel else {"wmm_gradff_mfma_kernel", "pack_w_gradff_split_kernel"} <= names
         grads.append(xs.grad)
-    # two roundings of the same sums: 2 tau products of a part each, then some hundred of those with fragments and coefficients; in terms
+    # two roundings of the same sums: 2 tout products of a part each, then some hundred of those with fragments and coefficients; in terms
     # of the root mean square sqrt(n) 2^-24 each, and the largest difference a few times that
     diff, size = (grads[0] - grads[1]).double(), grads[0].double()
     assert diff.norm() <= 2e-6 * size.norm() and diff.abs().max() <= 2e-5 * size.abs().max()

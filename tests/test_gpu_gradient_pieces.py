@@ -1,4 +1,4 @@
-"""Gradient of the product tensor as products of bfloat16 pieces: taken where every degree with output channels has nine to sixteen."""
+"""Gradient of the product tensor as products of bfloat16 pieces: taken where every degree with output channels has thirteen to sixteen."""
 import pytest
 import torch
 
@@ -9,13 +9,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("lmax,t_ff,t_o,bsz,spread", [
-    (0, [17], [9], 1, 0),                                   # one value of m, a tile of one channel
-    (3, [64, 16, 65, 15], [9, 16, 12, 0], 5, 0),            # tiles of channels full and not, a degree without outputs
+    (0, [17], [13], 1, 0),                                  # one value of m, a tile of one channel
+    (3, [64, 16, 65, 15], [13, 16, 14, 0], 5, 0),           # tiles of channels full and not, a degree without outputs
     (7, [40] * 8, [16] * 8, 3, 0),                          # 15 values of m: a column tile short of one
-    (11, [33] * 12, [12, 0, 13, 9] * 3, 2, 0),
-    (24, [20] * 25, [10] * 25, 1, 0),                       # more than three column tiles
-    (3, [24] * 4, [9] * 4, 4, 60),                          # rows and columns of very different size
-    (3, [24] * 4, [8] * 4, 4, 60),                          # eight channels: the fp32 instructions
+    (11, [33] * 12, [14, 0, 13, 15] * 3, 2, 0),             # the last degree of three column tiles
+    (12, [18] * 12 + [65], [13] * 12 + [15], 3, 0),         # the first of four, in a kernel of its own
+    (16, [3] * 15 + [80, 17], [16] * 17, 2, 0),             # 66 columns: the fifth tile has two
+    (19, [1] * 18 + [64, 33], [13] * 20, 1, 60),            # 78 columns
+    (23, [2] * 20 + [16, 48, 65, 20], [14] * 24, 2, 0),     # six column tiles
+    (24, [20] * 25, [13] * 25, 1, 0),                       # seven: split again for every tile of channels
+    (3, [24] * 4, [13] * 4, 4, 60),                         # rows and columns of very different size
+    (3, [24] * 4, [12] * 4, 4, 60),                         # twelve channels: the fp32 instructions
+    (13, [24] * 14, [12] * 14, 2, 60),
 ])
 def test_product_gradient(dev, lmax, t_ff, t_o, bsz, spread):  # noqa: F811
     g = torch.Generator().manual_seed(lmax + spread)
@@ -26,7 +31,7 @@ def test_product_gradient(dev, lmax, t_ff, t_o, bsz, spread):  # noqa: F811
         go.append(torch.randn(bsz, n, m, 2, generator=g) * torch.exp2(torch.randint(-spread, spread + 1, (bsz, 1, m, 1), generator=g).float()))
     std = torch.rand(sum(t_ff), generator=g) + 0.5
     names = _check(dev, w, go, std)
-    assert ("pack_w_gradff_split_kernel" in names) == (min(t for t in t_o if t) >= 9)
+    assert ("pack_w_gradff_split_kernel" in names) == (min(t for t in t_o if t) >= 13)
 
 
 def _gradient(dev, w, go, std):  # noqa: F811
@@ -82,21 +87,21 @@ def test_output_channels_of_different_scale(dev, decades):  # noqa: F811
     """An output channel that the next layer's stds divide by s sends back a gradient of 1 / s."""
     g = torch.Generator().manual_seed(decades)
     w, go = [], []
-    for l, (k, n) in enumerate([(33, 12), (16, 16), (40, 9), (17, 13)]):
+    for l, (k, n) in enumerate([(33, 14), (16, 16), (40, 13), (17, 15)]):
         r = _inverse(n, decades)
         w.append(torch.randn(n, k, 2, generator=g) * r[:, None, None])
         go.append(torch.randn(3, n, 2 * l + 1, 2, generator=g) / r[None, :, None, None])
     assert "pack_w_gradff_split_kernel" in _check(dev, w, go, torch.rand(106, generator=g) + 0.5)
 
 
-@pytest.mark.parametrize("size_w,size_go", [(-62, -62), (-20, -100), (0, -140), (62, 62), (20, 100), (-100, 100), (100, -100)])
+@pytest.mark.parametrize("size_w,size_go", [(-62, -62), (-20, -100), (0, -140), (61, 61), (20, 100), (-100, 100), (100, -100)])
 def test_sizes_of_both_operands(dev, size_w, size_go):  # noqa: F811
-    """What is in range in the result is in range on the way."""
+    """What is in range in the result is in range on the way.  (2^61 twice: 26 products of normal numbers stay below 2^6 of 2^122.)"""
     g = torch.Generator().manual_seed(5)
     w, go = [], []
     for l in range(3):
-        w.append(torch.randn(12, 20, 2, generator=g) * 2. ** size_w)
-        go.append((torch.randn(2, 12, 2 * l + 1, 2, generator=g).double() * 2. ** size_go).float())
+        w.append(torch.randn(13, 20, 2, generator=g) * 2. ** size_w)
+        go.append((torch.randn(2, 13, 2 * l + 1, 2, generator=g).double() * 2. ** size_go).float())
     if size_go >= -100:                                     # one output channel of the opposite size, whose partner is zero
         for v in w:
             v[3] = 0.
@@ -109,7 +114,7 @@ def test_sizes_of_both_operands(dev, size_w, size_go):  # noqa: F811
 
 def _draw(seed):
     g = torch.Generator().manual_seed(seed)
-    sizes = [(33, 12), (16, 16), (80, 9), (17, 13)]
+    sizes = [(33, 14), (16, 16), (80, 13), (17, 15)]
     return ([torch.randn(n, k, 2, generator=g) for k, n in sizes],
             [torch.randn(3, n, 2 * l + 1, 2, generator=g) for l, (_, n) in enumerate(sizes)])
 
@@ -137,11 +142,11 @@ def test_infinite_weight_in_a_layer(dev, lmax):  # noqa: F811
     """The layer's kernel makes of it what the two kernels make: infinities where one degree is alone, and not finite is the same place."""
     from cgnet_amd import CG_layers
     taus = [9] * (lmax + 1)
-    mod = CG_layers.CGBN_cuda(lmax, taus, taus, device=dev)
+    mod = CG_layers.CGBN_cuda(lmax, taus, [13] * (lmax + 1), device=dev)
     mod.eval()
     with torch.no_grad():
         mod.bnWMM.W[5, 0] = float("inf")
-    go = torch.randn(2, 9 * (lmax + 1) ** 2, 2, generator=torch.Generator().manual_seed(1)).to(dev)
+    go = torch.randn(2, 13 * (lmax + 1) ** 2, 2, generator=torch.Generator().manual_seed(1)).to(dev)
     grads = []
     for one_kernel in (False, True):
         mod.fused_backward = one_kernel
@@ -171,11 +176,13 @@ def test_largest_numbers(dev, which):  # noqa: F811
 
 @pytest.mark.parametrize("decades", [0, 10])
 @pytest.mark.parametrize("lmax,tin,tout,bsz,sparse", [
-    (2, [3, 1, 2], [9, 9, 9], 1, False),
-    (6, [16, 5, 9, 0, 2, 8, 12], [16, 12, 0, 13, 9, 10, 16], 5, False),
-    (9, [4] * 10, [12] * 10, 3, True),
+    (2, [3, 1, 2], [13, 13, 13], 1, False),
+    (6, [16, 5, 9, 0, 2, 8, 12], [16, 14, 0, 13, 15, 13, 16], 5, False),
+    (9, [4] * 10, [14] * 10, 3, True),
     (13, [9] * 14, [16] * 14, 2, False),
-    (18, [2] * 19, [9] * 19, 1, False),
+    (18, [2] * 19, [13] * 19, 1, False),
+    (22, [1] * 23, [15] * 23, 1, False),
+    (9, [4] * 10, [12] * 10, 3, True),                      # twelve: both on the fp32 instructions
 ])
 def test_layer_makes_the_same_gradient(dev, lmax, tin, tout, bsz, sparse, decades):  # noqa: F811
     """Inside the layer and in the mixing's kernel the products are the same and are added in the same order."""
