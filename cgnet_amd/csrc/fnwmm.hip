@@ -620,7 +620,7 @@ pack_w_gradff_split_kernel(const float2* __restrict__ W, const float* __restrict
 // NT = column tiles worked on together; ONE: these are all column tiles of the degree, so the B
 // operands are built once per sample and shared by the channel tiles.
 constexpr int kGffSub = 4;     // channel tiles per wave
-// lmax 11, B = 64, 16 channels (875 MB of gFF): fp32 steps 241 us, pieces 172; 12 channels, B = 50 (383 MB): fp32 steps 100.
+// lmax 11, B = 64, 16 channels (872 MB of gFF): fp32 steps 241 us, pieces 172; 12 channels, B = 50 (383 MB): fp32 steps 100.
 // Waves wanted (at least eight groups of samples are made in any case), samples a wave keeps at least: it loads its operand
 // once.  lmax 10, layers of 12..3 channels, B=100 (112 units), us: 8 groups 151, 2048 waves 95, 4096 waves 84, 8192 waves 87.
 // Both gradients together, over the shapes named at kFwdSlices: 0.80 of the time, none slower by more than 5 %.
@@ -782,11 +782,12 @@ __device__ __forceinline__ void wmm_gradff_wave(const float2* __restrict__ gO, c
 }
 
 // Fp32 steps; pieces; pieces of degrees above eleven (four column tiles and more).  Splitting gO again for every channel tile cost more than
-// the fp32 steps take, so up to six column tiles are split once.  Kernels of their own: the registers of one are no
-// concern of the others (104, 131, 173).
+// the fp32 steps take, so the up to six column tiles (2 l + 1 <= 47) are split once.  Kernels of their own: the registers of one are no
+// concern of the others.  Four waves a SIMD, or three (169 registers cut to 168, 37 spilled): gFF alone 0.97 of the time with two, over
+// 215 shapes of 13..16 channels, lmax 2..23.
 enum GffForm { kGffFp32, kGffPieces, kGffWide };
 template <GffForm FORM>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64, FORM == kGffWide ? 3 : 4)
 wmm_gradff_mfma_kernel(const float2* __restrict__ gO, const float* __restrict__ Ap, float2* __restrict__ gFF,
                        const WmmDeg* __restrict__ degs, const WmmChanUnit* __restrict__ units, int B,
                        int samples_per_group, int nFF, int nO, int out_bytes, int go_bytes) {
@@ -796,9 +797,8 @@ wmm_gradff_mfma_kernel(const float2* __restrict__ gO, const float* __restrict__ 
     const WmmDeg d = degs[u.deg];
     const int lane = threadIdx.x;
 #define CGNET_GFF_ARGS gO, Ap, gFF, d, u, B, samples_per_group, nFF, nO, out_bytes, go_bytes, smem, lane, up.part
-#define CGNET_GFF(N_) CGNET_GFF_AS(N_, N_)
-#define CGNET_GFF_AS(CASE_, N_)                                                           \
-    case CASE_:                                                                           \
+#define CGNET_GFF(N_)                                                                     \
+    case N_:                                                                              \
         if (nct == 1) wmm_gradff_wave<N_, 1, true>(CGNET_GFF_ARGS);                       \
         else if (nct == 2) wmm_gradff_wave<N_, 2, true>(CGNET_GFF_ARGS);                  \
         else if (nct == 3) wmm_gradff_wave<N_, 3, true>(CGNET_GFF_ARGS);                  \
@@ -809,11 +809,11 @@ wmm_gradff_mfma_kernel(const float2* __restrict__ gO, const float* __restrict__ 
         if (nct == 4) wmm_gradff_wave<kGffSplitBlocks, 4, true>(CGNET_GFF_ARGS);
         else if (nct == 5) wmm_gradff_wave<kGffSplitBlocks, 5, true>(CGNET_GFF_ARGS);
         else if (nct == 6) wmm_gradff_wave<kGffSplitBlocks, 6, true>(CGNET_GFF_ARGS);
-        else switch (0) { CGNET_GFF_AS(0, kGffSplitBlocks) }
-    } else if constexpr (FORM == kGffPieces) {
+    }
+    if constexpr (FORM != kGffFp32) {
         if (nct == 1) wmm_gradff_wave<kGffSplitBlocks, 1, true>(CGNET_GFF_ARGS);
         else if (nct == 2) wmm_gradff_wave<kGffSplitBlocks, 2, true>(CGNET_GFF_ARGS);
-        else wmm_gradff_wave<kGffSplitBlocks, 3, true>(CGNET_GFF_ARGS);
+        else if (nct == 3) wmm_gradff_wave<kGffSplitBlocks, 3, true>(CGNET_GFF_ARGS);
     } else {
         switch (d.nks_b) {
             CGNET_GFF(1) CGNET_GFF(2) CGNET_GFF(3) CGNET_GFF(4) CGNET_GFF(5) CGNET_GFF(6) CGNET_GFF(7) CGNET_GFF(8)
@@ -821,7 +821,6 @@ wmm_gradff_mfma_kernel(const float2* __restrict__ gO, const float* __restrict__ 
     }
 #undef CGNET_GFF_ARGS
 #undef CGNET_GFF
-#undef CGNET_GFF_AS
 }
 
 __global__ void __launch_bounds__(256) fill_zero_kernel(float* p, size_t n) {

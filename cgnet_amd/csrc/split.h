@@ -23,15 +23,17 @@ namespace cgnet {
 // The 32 places of a product are (output channel, re / im).  Whether pieces take the place of fp32 for output channels `t` of the degrees
 // 0 .. L: every degree that has any has at least thirteen.  They replace seven or eight fp32 instructions there, five or six at nine to
 // twelve channels, and operands half as large again there, twice as large at twelve.  Kernels of a training step over lmax 2..23, 1..64 samples, fp32 -> pieces:
-//   13 .. 16 channels  layer 0.98 of the time (170 shapes, one more than 3 % slower: 54 -> 56 us), gFF alone 0.92 (14 of 170 more than 5 % slower, up
-//                      to four samples: 22 -> 25 us, at worst 79 -> 90)
+//   13 .. 16 channels  layer 0.98 of the time (215 shapes, two more than 3 % slower: 96 -> 99 us), gFF alone 0.90 (8 of 215 more than 5 % slower, up
+//                      to four samples: 22 -> 25 us, 125 -> 135)
 //   10 .. 12 channels  layer 1.01 (35 of 262 more than 3 % slower, 507 -> 542 us at lmax 20, 16 -> 12 channels, one sample), gFF alone 0.99 (75 of
 //                      262 more than 5 % slower, 28.6 -> 35.2 us at lmax 18, 10 channels, one sample)
 //   up to eight        layer of 5 channels at lmax 11, B = 100: 278 -> 292 us, of 8 624 -> 650
+// Above degree 23, where there is no backward by pairs either, the stand-alone kernel would split gO again for every tile of channels.
 constexpr int kPieces = 3;
-constexpr int kSplitFrom = 13, kSplitMax = 16;
+constexpr int kSplitFrom = 13, kSplitMax = 16, kSplitMaxL = 23;
 template <typename Count>
 bool split_taken(int L, Count&& t) {
+    if (L > kSplitMaxL) return false;
     bool any = false;
     for (int l = 0; l <= L; ++l) {
         if (t(l) != 0 && (t(l) < kSplitFrom || t(l) > kSplitMax)) return false;
